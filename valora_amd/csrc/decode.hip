@@ -132,14 +132,13 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
   constexpr int DEC_CH = dec_ch(NB), DEC_BN = 256 * DEC_CH;   // chunks and outputs per expand item
   constexpr int KB = (NB + 1) / 2;                  // 32-wide rank blocks of the expand
   constexpr int STAGE_FLOATS = 4 * 16 * DEC_STAGE_LD;
-  constexpr int RED_FLOATS = 2 * NB * 256;          // cross-wave reduction of shrink_tile_to_lds
+  constexpr int TILE_FLOATS = shrink_lds_floats(NB);   // shrink_tile_to_lds
   constexpr int VACC_FLOATS = 16 * NB * 16;         // a tile's summed chunks (give-up path)
+  constexpr int BUF_FLOATS = TILE_FLOATS + VACC_FLOATS > STAGE_FLOATS ? TILE_FLOATS + VACC_FLOATS : STAGE_FLOATS;
   static_assert(DECODE_MAX_PRODUCERS == 16, "stamps_match reads 16 stamps");
-  static_assert(RED_FLOATS + VACC_FLOATS <= STAGE_FLOATS, "the shrink buffers alias the expand's staging tile");
-  __shared__ __align__(16) float s_buf[STAGE_FLOATS];
+  __shared__ __align__(16) float s_buf[BUF_FLOATS];   // a shrink item's tile, an expand item's staging tile
   __shared__ int32_t s_perm[16];
   __shared__ int32_t s_ready;
-  float(*red)[NB * 256] = reinterpret_cast<float(*)[NB * 256]>(s_buf);
   const int id = (int)blockIdx.x;
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -191,15 +190,14 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
     const int kbeg = s * kchunk;
     const int kend = min(h_in, kbeg + kchunk);
     const int slot = z == 0 ? sl0 : z == 1 ? sl1 : z == 2 ? sl2 : sl3;
-    shrink_tile_to_lds<T, 1, NB>(x, h_in, pool, slot, perm, r, pos0, cnt, astart, kbeg, kend, red);
+    shrink_tile_to_lds<T, 1, NB>(x, h_in, pool, slot, perm, r, pos0, cnt, astart, kbeg, kend, s_buf);
     if (wave == 0) {
       // wave 0 alone writes the partial and then the stamp: no barrier, and nothing else of its own in flight
       f32x4 *part = reinterpret_cast<f32x4 *>(tile_partial + (int64_t)item * 16 * rp);
       const int quarter = rp >> 2;
       for (int e = lane; e < 16 * quarter; e += 64) {
         const int row = e / quarter, c4 = e - row * quarter;
-        const float *src = red[1] + row * (NB * 16) + 4 * c4;
-        part[e] = f32x4{src[0], src[1], src[2], src[3]};
+        part[e] = shrink_tile_sum<NB>(s_buf, NB, row, c4);
       }
       // the partial must sit in the L2 before the stamp that announces it
       wait_vmcnt<0>();
@@ -350,14 +348,17 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
     }
   } else {
     // give-up path: the tile's chunks computed here, one after the other with the shrink item's own code
-    float *vacc = s_buf + RED_FLOATS;
+    float *vacc = s_buf + TILE_FLOATS;
     for (int e = tid; e < VACC_FLOATS; e += 256) vacc[e] = 0.f;
     const int slot_a = a.s.slots[z];
     for (int s = 0; s < a.s.ksplit; ++s) {
       const int kbeg = s * a.s.kchunk;
       const int kend = min(a.s.h_in, kbeg + a.s.kchunk);
-      shrink_tile_to_lds<T, 1, NB>(a.s.x, a.s.h_in, a.s.pool, slot_a, perm, r, pos0, cnt, astart, kbeg, kend, red);
-      for (int e = tid; e < VACC_FLOATS; e += 256) vacc[e] += red[1][e];
+      shrink_tile_to_lds<T, 1, NB, 1>(a.s.x, a.s.h_in, a.s.pool, slot_a, perm, r, pos0, cnt, astart, kbeg, kend, s_buf);
+      for (int e = tid; e < VACC_FLOATS / 4; e += 256) {
+        f32x4 *sum = reinterpret_cast<f32x4 *>(vacc) + e;
+        *sum += shrink_tile_sum<NB>(s_buf, NB, e / (NB * 4), e & (NB * 4 - 1));
+      }
       __syncthreads();
     }
 #pragma unroll

@@ -1,13 +1,12 @@
 // LoRA shrink for gfx950:  v[row, j] = T( sum_k x[t, k] * A_a[j, k] )
 //
-// One workgroup (4 waves) owns one adapter-grouped tile of up to 16*MB tokens and one K-chunk.
-// Both operands are K-contiguous in memory (token rows of x, rank rows of the pool), which is
-// exactly the per-lane layout v_mfma_f32_16x16x32 wants: lane (row = lane%16, kgroup = lane/16)
-// holds 8 consecutive K elements, so every operand is a single 16-byte global load straight
-// into the MFMA source registers -- no LDS staging, no transposes.  The four waves interleave
-// 32-element K-steps, so the workgroup reads 256 contiguous bytes of every row per round, and
-// several K-steps are loaded before any is consumed (the kernel is latency bound: what counts
-// is the number of 16-byte loads in flight per lane).
+// shrink_kernel: one workgroup (4 waves) owns one adapter-grouped tile of up to 16*MB tokens and one K chunk
+// (shrink_core.h has the loads and the products).  Bound by its chain of round trips, not by bytes: tile record ->
+// look-ups -> operand loads -> cross-wave sum -> hand-over of the K chunks.  Measured on 512 tokens over 128 adapters
+// of rank 128 (4096 wide, 122 MB of A per target) 60 -> 54 us a launch, on 77 tokens over 33 adapters of rank 8-64
+// (5120 wide) 12.7 -> 11.8, on 256 tokens over 64 adapters of rank 16 7.2 -> 7.0, by loading whole lines, one
+// round trip for all look-ups and two barriers instead of four for the cross-wave sum.
+// shrink_gemm_kernel: 128- and 256-token tiles.
 //
 // Split-K without atomics: every workgroup writes its fp32 partial tile and is done; the chunks
 // are summed in index order (bit-reproducible) by shrink_reduce_kernel or by the expand.
@@ -49,13 +48,31 @@ __device__ __forceinline__ void store_v(const ShrinkArgs &p, int pos, int t, int
   }
 }
 
-// Epilogue shared by both shrink kernels.  `tile` is the workgroup's fp32 result in LDS, row-major
+// four consecutive columns at once: one 8-byte store where they all hold values and the row allows it
+template <typename T>
+__device__ __forceinline__ void store_v4(const ShrinkArgs &p, int pos, int t, int r, int c4, f32x4 v) {
+  using Tr = Traits<T>;
+  const int col = 4 * c4;
+  uint16_t *dst = p.out + (int64_t)(p.out_by_token ? t : pos) * p.out_stride + col;
+  const bool whole = p.out_by_token ? col < r && col + 4 <= p.ncols && p.mode != MLORA_SHRINK_ACCUMULATE &&
+                                          (reinterpret_cast<uintptr_t>(dst) & 7u) == 0
+                                    : col < p.rp;
+  if (whole) {
+    if (col >= r) v = f32x4{0.f, 0.f, 0.f, 0.f};   // ranks are multiples of 8
+    *reinterpret_cast<uint2 *>(dst) = uint2{(uint32_t)Tr::from_float(v[0]) | ((uint32_t)Tr::from_float(v[1]) << 16),
+                                            (uint32_t)Tr::from_float(v[2]) | ((uint32_t)Tr::from_float(v[3]) << 16)};
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) store_v<T>(p, pos, t, r, col + i, v[i]);
+}
+
+// Epilogue of the GEMM shrink.  `tile` is the workgroup's fp32 result in LDS, row-major
 // with row stride ld: rows = tokens of the tile, columns = rank.
 //   ksplit == 1 : rounded to T and stored.
 //   ksplit  > 1 : stored as this K-chunk's fp32 partial (ordinary stores, then the workgroup is
 //                 done); a later launch on the stream -- shrink_reduce_kernel, or the expand
 //                 itself for small batches -- sums the chunks in index order and rounds once.
-// (shrink_kernel can also sum the chunks itself, see there.)
 template <typename T>
 __device__ __forceinline__ void shrink_epilogue(const ShrinkArgs &p, const float *tile, int ld, int s, int pos0,
                                                 int cnt, int r, const int32_t *perm) {
@@ -109,8 +126,10 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(ShrinkArgs args_in) 
 
 // The leading scalar parameters repeat what the first dependent load (the tile record) needs: with kernel-argument
 // preloading they arrive in registers at launch, so that load does not wait for a load of the argument block.
+// Waves per SIMD the register allocator has to leave room for: as many as do without spills.
+constexpr int shrink_min_waves(int mb, int nb) { return mb + nb <= 3 ? 4 : nb == 8 ? 3 - mb : mb * nb <= 8 ? 3 : 2; }
 template <typename T, int MB, int NB>
-__global__ __launch_bounds__(256) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
+__global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
                                                      int h_n_tiles, ShrinkArgs args_in) {
   int tile_idx, z_idx, s;
   if (h_reduce_here) {
@@ -134,7 +153,9 @@ __global__ __launch_bounds__(256) void shrink_kernel(const int32_t *tiles_base, 
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   const ShrinkArgs p = select_target(args_in, z_idx);
   constexpr int NBLK = MB * NB;
-  __shared__ float red[2][NBLK * 256];
+  constexpr int QUARTER = NB * 4;                        // groups of four columns per row, a power of two
+  constexpr int ITEMS = (MB * 16 * QUARTER + 255) / 256; // (row, group) pairs per thread
+  __shared__ __align__(16) float s_tile[shrink_lds_floats(NBLK)];
   __shared__ int s_last;
 
   const int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
@@ -142,11 +163,36 @@ __global__ __launch_bounds__(256) void shrink_kernel(const int32_t *tiles_base, 
   const int32_t *__restrict__ perm = p.plan + p.off_perm;
   const int kbeg = s * p.kchunk;
   const int kend = min(p.h_in, kbeg + p.kchunk);
-  shrink_tile_to_lds<T, MB, NB>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, kbeg, kend, red);
-  if (!p.reduce_here || p.ksplit == 1) {
-    shrink_epilogue<T>(p, red[1], NB * 16, s, pos0, cnt, r, perm);
+  const int tid = threadIdx.x;
+  const int quarter = p.rp >> 2;                         // rp is a multiple of 16, at most NB * 16
+  // thread -> (row, group of four columns); the token of the row where the result goes to token order
+  bool on[ITEMS];
+  int row[ITEMS], c4[ITEMS], tok[ITEMS];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) {
+    const int e = tid + it * 256;
+    row[it] = e / QUARTER;
+    c4[it] = e & (QUARTER - 1);
+    on[it] = row[it] < cnt && c4[it] < quarter;
+    tok[it] = (p.out_by_token && on[it]) ? perm[pos0 + row[it]] : 0;
+  }
+  shrink_tile_to_lds<T, MB, NB>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, kbeg, kend, s_tile);
+  if (p.ksplit == 1) {
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it)
+      if (on[it]) store_v4<T>(p, pos0 + row[it], tok[it], r, c4[it], shrink_tile_sum<NB>(s_tile, NBLK, row[it], c4[it]));
     return;
   }
+  // this K chunk's fp32 partial (ordinary stores).  Where the chunks are not summed here, a later launch on the
+  // stream does it -- shrink_reduce_kernel, or the expand itself for small batches -- in index order, rounding once.
+  const int pq = p.reduce_here ? p.prp >> 2 : quarter;
+  {
+    f32x4 *part = reinterpret_cast<f32x4 *>(p.partial) + ((int64_t)s * p.T + pos0) * pq;
+#pragma unroll
+    for (int it = 0; it < ITEMS; ++it)
+      if (on[it]) part[row[it] * pq + c4[it]] = shrink_tile_sum<NB>(s_tile, NBLK, row[it], c4[it]);
+  }
+  if (!p.reduce_here) return;
 
   // ---- split-K summed here: every chunk leaves its partial in the L2, the last one to arrive adds them up.
   // Partials are plain stores into rows that own whole 128-byte lines (prp floats per row), so a line never
@@ -161,16 +207,6 @@ __global__ __launch_bounds__(256) void shrink_kernel(const int32_t *tiles_base, 
   // the next launch on this plan (launches that share a plan must not overlap).
   // (Worth it for small tiles only: one workgroup reads ksplit x tile x prp x 4 bytes at L2 latency.  For
   // 128-token tiles of rank 64 that is 256 KB and measured 8.5 us, against 3.7 us for the reduce launch.)
-  const int tid = threadIdx.x;
-  const int quarter = p.rp >> 2, pq = p.prp >> 2;
-  {
-    f32x4 *part = reinterpret_cast<f32x4 *>(p.partial + ((int64_t)s * p.T + pos0) * p.prp);
-    for (int e = tid; e < cnt * quarter; e += 256) {
-      const int row = e / quarter, c4 = e - row * quarter;
-      const float *src = red[1] + row * (NB * 16) + 4 * c4;
-      part[row * pq + c4] = f32x4{src[0], src[1], src[2], src[3]};
-    }
-  }
   wait_vmcnt<0>();
   __syncthreads();
   if (tid == 0) {
@@ -189,43 +225,47 @@ __global__ __launch_bounds__(256) void shrink_kernel(const int32_t *tiles_base, 
   __syncthreads();
   const int last = s_last;
   if (last == 0) return;
+  f32x4 v[ITEMS];
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it) v[it] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (last == 1) {
-    // v[row, :] = T(0 + p_0 + p_1 + ...): the order shrink_reduce_kernel uses
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(p.partial + (int64_t)pos0 * p.prp);
+    // v[row, :] = T(0 + p_0 + p_1 + ...): the order shrink_reduce_kernel uses.  The loads of a batch of chunks are
+    // requested for all of the thread's items together.
+    constexpr int BATCH = ITEMS <= 2 ? 8 : 4;
+    const f32x4 *src = reinterpret_cast<const f32x4 *>(p.partial) + (int64_t)pos0 * pq;
     const int64_t sstride = (int64_t)p.T * pq;
-    for (int e = tid; e < cnt * quarter; e += 256) {
-      const int row = e / quarter, c4 = e - row * quarter;
-      f32x4 v = {0.f, 0.f, 0.f, 0.f};
-      for (int s0 = 0; s0 < p.ksplit; s0 += 8) {
-        f32x4 q[8];
+    for (int s0 = 0; s0 < p.ksplit; s0 += BATCH) {
+      f32x4 q[ITEMS][BATCH];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-          q[u] = (s0 + u < p.ksplit) ? src[(s0 + u) * sstride + row * pq + c4] : f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int it = 0; it < ITEMS; ++it)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) v += q[u];
-      }
-      const int t = p.out_by_token ? perm[pos0 + row] : 0;
+        for (int u = 0; u < BATCH; ++u)
+          q[it][u] = (s0 + u < p.ksplit && on[it]) ? src[(s0 + u) * sstride + row[it] * pq + c4[it]]
+                                                   : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int i = 0; i < 4; ++i) store_v<T>(p, pos0 + row, t, r, 4 * c4 + i, v[i]);
+      for (int it = 0; it < ITEMS; ++it)
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u) v[it] += q[it][u];
     }
-    return;
+  } else {
+    // the chunks were not all written through this XCD's L2 (or the caller asked for this path): compute them
+    // here, one after the other.  (The empty asm keeps the compiler from computing this path's addresses early and
+    // holding them through the ordinary one.)
+    int pos_r = pos0, astart_r = astart;
+    asm volatile("" : "+s"(pos_r), "+s"(astart_r));
+    for (int c = 0; c < p.ksplit; ++c) {
+      const int kb = c * p.kchunk;
+      __syncthreads();   // everybody has read the previous chunk's sums
+      shrink_tile_to_lds<T, MB, NB, 1>(p.x, p.h_in, p.pool, p.slot, perm, r, pos_r, cnt, astart_r, kb,
+                                       min(p.h_in, kb + p.kchunk), s_tile);
+#pragma unroll
+      for (int it = 0; it < ITEMS; ++it)
+        if (on[it]) v[it] += shrink_tile_sum<NB>(s_tile, NBLK, row[it], c4[it]);
+    }
   }
-  // the chunks were not all written through this XCD's L2 (or the caller asked for this path): compute them
-  // here, one after the other, and add them up in LDS
-  __shared__ float vacc[16 * MB * NB * 16];
-  for (int e = tid; e < 16 * MB * NB * 16; e += 256) vacc[e] = 0.f;
-  for (int c = 0; c < p.ksplit; ++c) {
-    const int kb = c * p.kchunk;
-    __syncthreads();
-    shrink_tile_to_lds<T, MB, NB>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, kb, min(p.h_in, kb + p.kchunk),
-                                  red);
-    for (int e = tid; e < 16 * MB * NB * 16; e += 256) vacc[e] += red[1][e];
-  }
-  __syncthreads();
-  for (int e = tid; e < cnt * p.rp; e += 256) {
-    const int row = e / p.rp, col = e - row * p.rp;
-    store_v<T>(p, pos0 + row, p.out_by_token ? perm[pos0 + row] : 0, r, col, vacc[row * (NB * 16) + col]);
-  }
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it)
+    if (on[it]) store_v4<T>(p, pos0 + row[it], tok[it], r, c4[it], v[it]);
 }
 
 // Prefill-sized tiles (128 tokens): GEMM structure with a three-stage LDS ring.
