@@ -14,6 +14,7 @@
 // or a matrix supplied by the caller (rows in token order).
 //
 // Reference semantics: valora/csrc/bgmv/bgmv_impl.cuh:152-207.
+#include "expand_core.h"
 #include "kernel_common.h"
 
 namespace mlora {
@@ -250,39 +251,18 @@ __global__ __launch_bounds__(256) void expand_cols_kernel(const int32_t *tiles_b
   __syncthreads();
 
   // v fragment of the tile's one 16-token block: rows = tokens (lrow), 8 consecutive rank elements per lane
+  unsigned char *const turn = reinterpret_cast<unsigned char *>(&stage[wave][0][0]);
+  static_assert(sizeof(stage) / 4 >= B_TURN_BYTES, "a wave's staging tile holds its turn");
   u32x4 vfrag[KB];
-  {
+  if constexpr (PARTIAL) {
+    v_from_partials<T, KB>(p.partial + (int64_t)pos0 * p.rp, (int64_t)p.T * p.rp, p.ksplit, p.rp, cnt, rk, lane, turn, vfrag);
+  } else {
     const bool pok = lrow < cnt;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
       const int j0 = kb * 32 + kg * 8;
-      u32x4 v = {0, 0, 0, 0};
-      if (pok && j0 < rk) {
-        if constexpr (PARTIAL) {
-          float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-          const float *src0 = p.partial + ((int64_t)pos0 + lrow) * p.rp + j0;
-          const int64_t sstride = (int64_t)p.T * p.rp;
-          for (int s0 = 0; s0 < p.ksplit; s0 += 4) {
-            f32x4 lo[4], hi[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const bool ok = s0 + u < p.ksplit;
-              const f32x4 *src = reinterpret_cast<const f32x4 *>(src0 + (int64_t)(s0 + u) * sstride);
-              lo[u] = ok ? src[0] : f32x4{0.f, 0.f, 0.f, 0.f};
-              hi[u] = ok ? src[1] : f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-              for (int i = 0; i < 4; ++i) { f[i] += lo[u][i]; f[4 + i] += hi[u][i]; }
-          }
-          v = pack8<T>(f);
-        } else {
-          const int64_t vrow = p.v_by_pos ? (int64_t)(pos0 + lrow) : (int64_t)s_perm[lrow];
-          v = load16(p.v + vrow * p.v_stride + j0);
-        }
-      }
-      vfrag[kb] = v;
+      const int64_t vrow = p.v_by_pos ? (int64_t)(pos0 + lrow) : (int64_t)s_perm[lrow];
+      vfrag[kb] = (pok && j0 < rk) ? load16(p.v + vrow * p.v_stride + j0) : u32x4{0, 0, 0, 0};
     }
   }
 
@@ -295,24 +275,22 @@ __global__ __launch_bounds__(256) void expand_cols_kernel(const int32_t *tiles_b
   for (int oc = grp * h_cl; oc < oc_end; ++oc) {
     const int o_wave = oc * EXP_BN + wave * EXP_WN;
     if (o_wave >= p.h_out) break;   // wave-uniform
-    // ---- B fragments and y rows of this chunk, all requested before any is consumed
-    u32x4 bfrag[4][KB];
+    // ---- B units and y rows of this chunk, all requested before any is consumed
+    u32x4 braw[KB][4], bfrag[4][KB];
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const int o = o_wave + nb * 16 + lrow;
+    for (int q = 0; q < KB; ++q)
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int j0 = kb * 32 + kg * 8;
-        u32x4 b = {0, 0, 0, 0};
-        if (o < p.h_out && j0 < rk) {
-          uint32_t bin, off;
-          divmod24((uint32_t)o * (uint32_t)r + (uint32_t)j0, (uint32_t)p.h_out, inv_h_out, bin, off);   // < 2^16 * 2^7
-          const int row = bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;
-          if (row >= 0) b = load16(p.pool.w + (int64_t)row * p.h_out + off);
+      for (int i = 0; i < 4; ++i) {
+        braw[q][i] = u32x4{0, 0, 0, 0};
+        if (b_any<KB>(i, (uint32_t)r)) {
+          uint32_t flat, bin, off;
+          bool ok = b_unit<KB>(q, i, lane, (uint32_t)r, flat);
+          flat += (uint32_t)o_wave * (uint32_t)r;               // < 2^16 * 2^7
+          divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off);
+          const int row = ok && bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;   // bins from r on hold -1
+          if (row >= 0) braw[q][i] = load16(p.pool.w + (int64_t)row * p.h_out + off);
         }
-        bfrag[nb][kb] = b;
       }
-    }
     u32x4 yv[2];
     uint16_t *yp[2];
     bool yok[2];
@@ -324,6 +302,7 @@ __global__ __launch_bounds__(256) void expand_cols_kernel(const int32_t *tiles_b
       yp[h] = p.y + (int64_t)t * p.h_out + o_wave + c8;
       yv[h] = yok[h] ? load16(yp[h]) : u32x4{0, 0, 0, 0};
     }
+    b_turn<KB>(braw, bfrag, (uint32_t)r, rk, lane, turn);
     // ---- delta block through the matrix cores, staged to LDS in token-major order
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {

@@ -1,0 +1,113 @@
+// Operand handling of the expand kernels.
+//
+#pragma once
+
+#include "kernel_common.h"
+
+namespace mlora {
+
+// v_mfma_f32_16x16x32 wants lane (column = lane%16, kgroup = lane/16) to hold 8 consecutive rank elements of one
+// output.  In the pool an output's r rank elements are consecutive, so lanes that load that way sit 2*r bytes apart and
+// fill the load instructions badly (half of the lanes masked at rank 16, another 128-byte line per lane from rank 64 on,
+// which costs a compute unit some 64 cycles per instruction instead of 16).  A wave's 64 outputs are one run of 128*r
+// bytes, so the column-looping expand, whose workgroups fill the device several times over, loads them in lane order
+// -- whole lines, nothing masked -- and turns them into operands through a piece of LDS of the wave's own (no barrier:
+// a wave's LDS accesses run in order; units XOR-swizzled so that the 16-byte reads, r/8 units apart, spread over the
+// banks).  Together with v_from_partials: 256 decode tokens, 64 adapters of rank 16, q+k+v 12.7 -> 11.5 us.  (The other
+// expand kernels load operands directly: there the registers and the turn cost more than the instructions, 6.2 -> 6.6 us
+// for one decode target, 26 -> 31 us for a 6749-token prefill at rank 32.)
+constexpr int B_TURN_BYTES = 4096;   // LDS of a wave's turn: 256 units of 16 bytes
+constexpr int B_OUTS = 64;           // outputs per wave
+
+__device__ __forceinline__ uint32_t b_swizzle(uint32_t q) { return q ^ (((q >> 3) ^ (q >> 6)) & 7u); }
+
+// A wave's B operands are turned in KB passes of B_OUTS / KB outputs, up to 4 instructions (256 units) each.
+// The flat element a lane's unit i of pass p starts at, relative to the wave's first output; false: no such unit.
+template <int KB>
+__device__ __forceinline__ bool b_unit(int p, int i, int lane, uint32_t r, uint32_t &flat) {
+  constexpr uint32_t OUTS = B_OUTS / KB;
+  const uint32_t q = (uint32_t)(i * 64 + lane);
+  flat = (uint32_t)p * OUTS * r + q * 8u;
+  return q < OUTS * (r >> 3);
+}
+// wave-uniform: whether instruction i of a pass has any unit
+template <int KB>
+__device__ __forceinline__ bool b_any(int i, uint32_t r) { return (uint32_t)(i * 64) < (B_OUTS / KB) * (r >> 3); }
+
+// raw[p][i] as loaded -> bfrag[nb][kb] = B^T[o = nb*16 + lane%16][kb*32 + (lane/16)*8 .. + 8), zero from rank rk on.
+// `turn`: B_TURN_BYTES of LDS of this wave.
+template <int KB>
+__device__ __forceinline__ void b_turn(const u32x4 (&raw)[KB][4], u32x4 (&bfrag)[4][KB], uint32_t r, int rk, int lane,
+                                       unsigned char *turn) {
+  const uint32_t rq = r >> 3;
+  const int lrow = lane & 15, kg = lane >> 4;
+#pragma unroll
+  for (int p = 0; p < KB; ++p) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (b_any<KB>(i, r)) *reinterpret_cast<u32x4 *>(turn + b_swizzle((uint32_t)(i * 64 + lane)) * 16u) = raw[p][i];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+    for (int n = 0; n < 4 / KB; ++n)
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const uint32_t c = (uint32_t)(kb * 4 + kg);
+        const bool ok = (int)(c * 8u) < rk;
+        const uint32_t q = (uint32_t)(n * 16 + lrow) * rq + (ok ? c : 0u);
+        const u32x4 got = *reinterpret_cast<const u32x4 *>(turn + b_swizzle(q) * 16u);
+        bfrag[p * (4 / KB) + n][kb] = ok ? got : u32x4{0, 0, 0, 0};
+      }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+// The v operand of one 16-token block from the split-K partials: `part` is the block's first row in chunk 0, rows of
+// rp floats one after the other, chunks `sstride` floats apart.  The block is one run of 64*rp bytes per chunk, loaded
+// in lane order; every lane adds up its own four columns over the chunks in index order, rounds once, and the rows
+// are turned into operands through LDS like B above.  Rows from cnt on and ranks from rk on are zero.
+template <typename T, int KB>
+__device__ __forceinline__ void v_from_partials(const float *part, int64_t sstride, int ksplit, int rp, int cnt, int rk,
+                                                int lane, unsigned char *turn, u32x4 (&vfrag)[KB]) {
+  constexpr int G = 2 * KB;                              // groups of 64 units of four floats; rp <= 32 * KB
+  const int lrow = lane & 15, kg = lane >> 4;
+  f32x4 sum[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) sum[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int n_units = cnt * (rp >> 2);                   // rows in use
+  constexpr int BATCH = 4 / KB;                          // chunks whose loads are in flight together
+  for (int s0 = 0; s0 < ksplit; s0 += BATCH) {
+    f32x4 q[BATCH][G];
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u)
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        q[u][g] = (s0 + u < ksplit && g * 64 + lane < n_units)
+                      ? *reinterpret_cast<const f32x4 *>(part + (int64_t)(s0 + u) * sstride + (g * 64 + lane) * 4)
+                      : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int u = 0; u < BATCH; ++u)
+#pragma unroll
+      for (int g = 0; g < G; ++g) sum[g] += q[u][g];
+  }
+  using Tr = Traits<T>;
+#pragma unroll
+  for (int g = 0; g < G; ++g)
+    if (g * 64 < 4 * rp)
+      *reinterpret_cast<uint2 *>(turn + (g * 64 + lane) * 8) =
+          uint2{Tr::pack2(sum[g][0], sum[g][1]), Tr::pack2(sum[g][2], sum[g][3])};
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+#pragma unroll
+  for (int kb = 0; kb < KB; ++kb) {
+    const int j0 = kb * 32 + kg * 8;
+    const bool ok = lrow < cnt && j0 < rk;
+    const u32x4 got = *reinterpret_cast<const u32x4 *>(turn + (lrow * rp + (ok ? j0 : 0)) * 2);
+    vfrag[kb] = ok ? got : u32x4{0, 0, 0, 0};
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+}  // namespace mlora

@@ -9,6 +9,8 @@ namespace mlora {
 
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
+typedef __attribute__((ext_vector_type(2))) float f32x2;
+typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 
@@ -109,6 +111,11 @@ struct Traits<_Float16> {
   }
   static __device__ __forceinline__ float to_float(uint16_t h) { return (float)as<_Float16>(h); }
   static __device__ __forceinline__ uint16_t from_float(float f) { return as<uint16_t>((_Float16)f); }
+  // two values, the first in the low half (one by one: behind a multiply-add either becomes a single mixed-precision
+  // FMA that rounds to fp16 at once, where a packed conversion would round the fp32 sum)
+  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+    return (uint32_t)from_float(lo) | ((uint32_t)from_float(hi) << 16);
+  }
 };
 
 template <>
@@ -118,12 +125,12 @@ struct Traits<__bf16> {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
   }
   static __device__ __forceinline__ float to_float(uint16_t h) { return as<float>((uint32_t)h << 16); }
-  // round to nearest even; NaN stays NaN
-  static __device__ __forceinline__ uint16_t from_float(float f) {
-    uint32_t x = as<uint32_t>(f);
-    if ((x & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((x >> 16) | 0x40u);
-    x += 0x7fffu + ((x >> 16) & 1u);
-    return (uint16_t)(x >> 16);
+  // Round to nearest even, one v_cvt_pk_bf16_f32 for two values.  (Written out in integer arithmetic the rounding is
+  // seven instructions a value, which the kernels that update y or W in place have nothing to hide behind: merging
+  // an adapter rounds every weight twice.)
+  static __device__ __forceinline__ uint16_t from_float(float f) { return as<uint16_t>((__bf16)f); }
+  static __device__ __forceinline__ uint32_t pack2(float lo, float hi) {
+    return as<uint32_t>(__builtin_convertvector((f32x2{lo, hi}), bf16x2));
   }
 };
 
@@ -144,8 +151,7 @@ template <typename T>
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
   u32x4 v;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-    v[i] = (uint32_t)Traits<T>::from_float(f[2 * i]) | ((uint32_t)Traits<T>::from_float(f[2 * i + 1]) << 16);
+  for (int i = 0; i < 4; ++i) v[i] = Traits<T>::pack2(f[2 * i], f[2 * i + 1]);
   return v;
 }
 

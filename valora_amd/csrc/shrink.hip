@@ -59,8 +59,7 @@ __device__ __forceinline__ void store_v4(const ShrinkArgs &p, int pos, int t, in
                                     : col < p.rp;
   if (whole) {
     if (col >= r) v = f32x4{0.f, 0.f, 0.f, 0.f};   // ranks are multiples of 8
-    *reinterpret_cast<uint2 *>(dst) = uint2{(uint32_t)Tr::from_float(v[0]) | ((uint32_t)Tr::from_float(v[1]) << 16),
-                                            (uint32_t)Tr::from_float(v[2]) | ((uint32_t)Tr::from_float(v[3]) << 16)};
+    *reinterpret_cast<uint2 *>(dst) = uint2{Tr::pack2(v[0], v[1]), Tr::pack2(v[2], v[3])};
     return;
   }
 #pragma unroll
