@@ -51,6 +51,21 @@ def test_merge_integer_weights_bit_exact(dev, dtype, H, ranks):
                 assert torch.equal(got[k], want[k]), f"adapter {adapter} slot {k} sign {sign}"
 
 
+@pytest.mark.parametrize("H_in,H_out,rank", [(3080, 3000, 128), (4104, 2064, 64), (136, 264, 128), (8, 4096, 64), (4096, 8, 128)])
+def test_merge_several_slices_of_A_per_workgroup(dev, H_in, H_out, rank):
+    """Shapes at the edges of the split over slices: several slices per workgroup with a ragged last one, a last
+    workgroup with fewer slices than the others, matrices smaller than a tile in either direction."""
+    g = torch.Generator().manual_seed(H_in + rank)
+    pool = W.make_pool([rank], H_in, H_out, torch.bfloat16, g, True, heads=8)
+    pool.key_buffer.copy_(torch.randint(-2, 3, pool.key_buffer.shape, generator=g))
+    pool.value_buffer.copy_(torch.randint(-2, 3, pool.value_buffer.shape, generator=g))
+    Ws = [torch.randint(-8, 9, (H_in, H_out), generator=g).to(torch.bfloat16) for _ in range(4)]
+    want = O.merge_adapter(Ws, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, 0, 1.0, sign=1)
+    got = run_merge(dev, Ws, pool, 0, 1.0, (0, 1, 2, 3), 1)
+    for k in range(4):
+        assert torch.equal(got[k], want[k]), f"slot {k}"
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_merge_random_weights_and_views(dev, dtype):
     g = torch.Generator().manual_seed(8)

@@ -14,8 +14,15 @@
 // B of a slot is [H_out, r] flat over r pool rows -- K-contiguous for the MFMA, loaded straight
 // into registers as in the expand.  A of a slot is r pool rows of H_in elements, i.e. [r, H_in]:
 // the MFMA wants 8 consecutive rank elements of ONE input row per lane, so the workgroup's
-// [r x tile height] slice of A goes through LDS and is read back transposed with 2-byte reads (the row
-// stride of tile height + 4 elements spreads the four rank groups of a wave over different banks).
+// [r x tile height] slice of A goes through LDS transposed: a thread loads an 8 x 8 block (8 rank rows, 16 bytes
+// each), transposes it in registers and writes eight 16-byte units, which the products read as they are.
+//
+// Bound by the in-place update of W (268 MB for four 4096 x 4096 slots; an in-place stream runs at 4.4-4.9 TB/s on
+// this part) up to rank 32, above that also by the operands a workgroup reads beside its share of W: B once per
+// workgroup (in lane order, expand_core.h), A once per 256 columns.  Measured, four 4096 x 4096 slots of bf16 weights,
+// before / after transposing A once instead of at every use, reading B in lane order and for several slices, and
+// rounding to bf16 in hardware: rank 16 65.9 / 59 us, rank 64 88.3 / 65, rank 128 129.9 / 81.
+#include "expand_core.h"
 #include "kernel_common.h"
 
 namespace mlora {
@@ -23,9 +30,13 @@ namespace mlora {
 namespace {
 
 constexpr int MG_BN = 256;        // output columns per workgroup, 64 per wave
-// input rows (of W) per workgroup: taller tiles re-read B less often, but the transposed LDS reads of the
-// A slice grow with the rank -- 256 rows measured faster up to rank 32, 128 rows above
+// input rows (of W) per slice of A in LDS (16 KB up to rank 64, 32 KB above)
 constexpr int merge_bm(int kb) { return kb == 1 ? 256 : 128; }
+// Workgroups resident per compute unit: four up to rank 64, two above (the B fragments of rank 128 take 64 registers).
+// Two do not keep enough of W in flight by themselves, so there the rows of W are requested an iteration ahead
+// (rank 128 85 -> 81 us; with four workgroups the extra registers cost a workgroup and 3-6 us).
+constexpr int merge_resident(int kb) { return kb == 4 ? 2 : 4; }
+constexpr bool merge_ahead(int kb) { return kb == 4; }
 constexpr int MG_STAGE_LD = 64 + 4;
 
 struct MergeArgs {
@@ -38,15 +49,16 @@ struct MergeArgs {
   int h_in, h_out;
   float scaling, sign;
   int n_ochunks;
+  int chunks;                 // slices of merge_bm() input rows per workgroup
 };
 
 template <typename T, int KB>
-__global__ __launch_bounds__(256) void merge_kernel(MergeArgs p) {
+__global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArgs p) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
   constexpr int MG_BM = merge_bm(KB);
-  constexpr int MG_RS = MG_BM + 4;   // LDS row stride of the A slice, elements (see the file header)
-  __shared__ __align__(16) uint16_t s_a[KB * 32][MG_RS];
+  constexpr int UNITS = KB * 4;      // 16-byte units (8 rank elements) per input row of the A slice
+  __shared__ __align__(16) u32x4 s_a[MG_BM * UNITS];   // unit c of row i at b_swizzle(i * UNITS + c)
   __shared__ float stage[4][16][MG_STAGE_LD];
 
   const int z = blockIdx.y;
@@ -54,7 +66,6 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs p) {
   uint16_t *__restrict__ W = p.w[z];
   const int itile = blockIdx.x / p.n_ochunks;
   const int oc = blockIdx.x - itile * p.n_ochunks;
-  const int i0 = itile * MG_BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, kg = lane >> 4;
   const int o_wave = oc * MG_BN + wave * 64;
@@ -64,27 +75,63 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs p) {
   if (r <= 0 || (r & 7) || r > KB * 32) return;      // same adapters the LoRA op accepts
   const int64_t base = p.a_start[p.adapter] + (int64_t)r * slot;
 
-  // ---- B fragments, scaled and rounded to T: bfrag[nb][kb] = T(B^T[o][j0..j0+8) * scaling)
-  u32x4 bfrag[4][KB];
+  // Row-major roles for the update of W: 8 lanes x 16 bytes cover one row of the wave's 64 outputs.
+  const int rr0 = lane >> 3, c8 = (lane & 7) * 8;
+  const bool ocol_ok = (o_wave + c8) < p.h_out;
+
+  const float inv_h_out = 1.0f / (float)p.h_out;
+  // ---- a thread's 8 x 8 block of an A slice: rank rows 8 * ac .. + 8, 16 bytes of input columns from 8 * aic on.
+  // Neighbouring threads take neighbouring chunks of the same rank rows: whole lines.  The first slice's block is
+  // requested before anything waits for B, where the registers are there (rank 64 would spill).
+  constexpr int CHUNKS = MG_BM / 8;
+  static_assert(CHUNKS * UNITS <= 256, "one block per thread");
+  const int ac = tid / CHUNKS, aic = tid - ac * CHUNKS;
+  const int row0 = itile * p.chunks * MG_BM;
+  const int n_rows = min(p.chunks * MG_BM, p.h_in - row0);        // of this workgroup
+  int arow[8];
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    const int o = o_wave + nb * 16 + lrow;
+  for (int jj = 0; jj < 8; ++jj) {
+    const int64_t ai = base + ac * 8 + jj;
+    const bool ok = ac * 8 + jj < r && ai >= 0 && ai < p.pa.a_loc_len;
+    const int64_t row = ok ? p.pa.a_loc[ai] : -1;
+    arow[jj] = row >= 0 && row < p.pa.w_rows ? (int)row : -1;     // pool rows fit 31 bits (checked on the host)
+  }
+  u32x4 ablk[8];
+  auto load_a = [&](int il0) {
+    const int il = il0 + aic * 8;
+#pragma unroll
+    for (int jj = 0; jj < 8; ++jj)
+      ablk[jj] = (arow[jj] >= 0 && il < n_rows) ? load16(p.pa.w + (int64_t)arow[jj] * p.h_in + row0 + il)
+                                                : u32x4{0, 0, 0, 0};
+  };
+  constexpr bool A_FIRST = KB != 2;
+  if constexpr (A_FIRST) load_a(0);
+
+  // ---- B fragments, scaled and rounded to T: bfrag[nb][kb] = T(B^T[o][j0..j0+8) * scaling)
+  u32x4 braw[KB][4], bfrag[4][KB];
+#pragma unroll
+  for (int q = 0; q < KB; ++q)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      braw[q][i] = u32x4{0, 0, 0, 0};
+      uint32_t flat, bin, off;
+      const bool ok = b_unit<KB>(q, i, lane, (uint32_t)r, flat);
+      flat += (uint32_t)o_wave * (uint32_t)r;                     // < 2^16 * 2^7
+      divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off);
+      const int64_t idx = base + bin;
+      if (ok && flat < (uint32_t)p.h_out * (uint32_t)r && idx >= 0 && idx < p.pb.a_loc_len) {
+        const int64_t row = p.pb.a_loc[idx];
+        if (row >= 0 && row < p.pb.w_rows) braw[q][i] = load16(p.pb.w + row * p.h_out + off);
+      }
+    }
+  static_assert(sizeof(stage) / 4 >= B_TURN_BYTES, "a wave's staging tile holds its turn");
+  b_turn<KB>(braw, bfrag, (uint32_t)r, r, lane, reinterpret_cast<unsigned char *>(&stage[wave][0][0]));
+#pragma unroll
+  for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
-      const int j0 = kb * 32 + kg * 8;
-      u32x4 b = {0, 0, 0, 0};
-      if (o < p.h_out && j0 < r) {
-        const uint32_t flat = (uint32_t)o * (uint32_t)r + (uint32_t)j0;
-        const uint32_t bin = flat / (uint32_t)p.h_out;
-        const uint32_t off = flat - bin * (uint32_t)p.h_out;
-        const int64_t idx = base + bin;
-        if (idx >= 0 && idx < p.pb.a_loc_len) {
-          const int64_t row = p.pb.a_loc[idx];
-          if (row >= 0 && row < p.pb.w_rows) b = load16(p.pb.w + row * p.h_out + off);
-        }
-      }
       float f[8];
-      unpack8<T>(b, f);
+      unpack8<T>(bfrag[nb][kb], f);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         // the reference's `B * scaling` is an fp32 product rounded to T afterwards: keep the two roundings
@@ -95,82 +142,80 @@ __global__ __launch_bounds__(256) void merge_kernel(MergeArgs p) {
       }
       bfrag[nb][kb] = pack8<T>(f);
     }
-  }
 
-  // ---- the [r x MG_BM] slice of A into LDS (rank rows beyond r are zero)
-  for (int idx = tid; idx < KB * 32 * (MG_BM / 8); idx += 256) {
-    const int j = idx / (MG_BM / 8), c = idx - j * (MG_BM / 8);
-    const int i = i0 + c * 8;
-    u32x4 a = {0, 0, 0, 0};
-    if (j < r && i < p.h_in) {
-      const int64_t ai = base + j;
-      if (ai >= 0 && ai < p.pa.a_loc_len) {
-        const int64_t row = p.pa.a_loc[ai];
-        if (row >= 0 && row < p.pa.w_rows) a = load16(p.pa.w + row * p.h_in + i);
-      }
-    }
-    uint2 *dst = reinterpret_cast<uint2 *>(&s_a[j][c * 8]);   // rows are 8-byte, not 16-byte, aligned
-    dst[0] = uint2{a[0], a[1]};
-    dst[1] = uint2{a[2], a[3]};
-  }
-  __syncthreads();
-
-  const int rr0 = lane >> 3, c8 = (lane & 7) * 8;
-  const bool ocol_ok = (o_wave + c8) < p.h_out;
-
-  for (int rb0 = 0; rb0 < MG_BM / 16; rb0 += 2) {
-    u32x4 wv[2][2];
-    uint16_t *wp[2][2];
-    bool wok[2][2];
+  uint16_t *const wbase = W + (int64_t)row0 * p.ld + o_wave + c8;
+  u32x4 wv[2][2];
+  auto load_w = [&](int il0) {
 #pragma unroll
     for (int b = 0; b < 2; ++b)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int i = i0 + (rb0 + b) * 16 + rr0 + 8 * h;
-        wok[b][h] = ocol_ok && i < p.h_in;
-        wp[b][h] = W + (int64_t)(wok[b][h] ? i : 0) * p.ld + o_wave + c8;
-        wv[b][h] = wok[b][h] ? load16(wp[b][h]) : u32x4{0, 0, 0, 0};
+        const int il = il0 + b * 16 + rr0 + 8 * h;
+        wv[b][h] = (ocol_ok && il < n_rows) ? load16(wbase + (int64_t)il * p.ld) : u32x4{0, 0, 0, 0};
       }
+  };
+  if constexpr (merge_ahead(KB)) load_w(0);
+  for (int ch = 0; ch * MG_BM < n_rows; ++ch) {
+    // ---- the [r x MG_BM] slice of A into LDS, transposed (rank rows beyond r are zero); the swizzle spreads the
+    // units of neighbouring threads over the banks
+    if (ch > 0 || !A_FIRST) load_a(ch * MG_BM);
+    if (ch > 0) __syncthreads();   // everybody has read the previous slice
+    if (tid < CHUNKS * UNITS) {
 #pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      // A^T fragment: row = input row (lrow), 8 consecutive rank elements, read transposed from LDS
-      u32x4 afrag[KB];
-      const int il = (rb0 + b) * 16 + lrow;
+      for (int e = 0; e < 8; ++e) {
+        u32x4 unit;
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int j0 = kb * 32 + kg * 8;
-        uint32_t e[8];
-#pragma unroll
-        for (int k = 0; k < 8; ++k) e[k] = s_a[j0 + k][il];
-        afrag[kb] = u32x4{e[0] | (e[1] << 16), e[2] | (e[3] << 16), e[4] | (e[5] << 16), e[6] | (e[7] << 16)};
+        for (int w = 0; w < 4; ++w)   // element e of rank rows 2w and 2w + 1
+          unit[w] = __builtin_amdgcn_perm(ablk[2 * w + 1][e >> 1], ablk[2 * w][e >> 1], (e & 1) ? 0x07060302u : 0x05040100u);
+        s_a[b_swizzle((uint32_t)((aic * 8 + e) * UNITS + ac))] = unit;
       }
+    }
+    __syncthreads();
+
+    for (int rb0 = 0; rb0 < MG_BM / 16; rb0 += 2) {
+      if constexpr (!merge_ahead(KB)) load_w(ch * MG_BM + rb0 * 16);
+      u32x4 cur[2][2];
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      for (int b = 0; b < 2; ++b)
 #pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-          if (kb * 32 < r) acc = Tr::mfma(as<vec8>(afrag[kb]), as<vec8>(bfrag[nb][kb]), acc);
+        for (int h = 0; h < 2; ++h) cur[b][h] = wv[b][h];
+      if constexpr (merge_ahead(KB)) load_w(ch * MG_BM + (rb0 + 2) * 16);
 #pragma unroll
-        for (int t = 0; t < 4; ++t) stage[wave][kg * 4 + t][nb * 16 + lrow] = acc[t];
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
+      for (int b = 0; b < 2; ++b) {
+        // A^T fragment: row = input row (lrow), 8 consecutive rank elements
+        u32x4 afrag[KB];
+        const int al = (rb0 + b) * 16 + lrow;
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (wok[b][h]) {
-          const float *srow = &stage[wave][rr0 + 8 * h][c8];
-          float f[8];
-          unpack8<T>(wv[b][h], f);
+        for (int kb = 0; kb < KB; ++kb) afrag[kb] = s_a[b_swizzle((uint32_t)(al * UNITS + kb * 4 + kg))];
 #pragma unroll
-          for (int k = 0; k < 8; ++k) {
-            const float ab = Tr::to_float(Tr::from_float(srow[k]));   // the GEMM result is a T tensor
-            f[k] += p.sign * ab;
-          }
-          store16(wp[b][h], pack8<T>(f));
+        for (int nb = 0; nb < 4; ++nb) {
+          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kb = 0; kb < KB; ++kb)
+            if (kb * 32 < r) acc = Tr::mfma(as<vec8>(afrag[kb]), as<vec8>(bfrag[nb][kb]), acc);
+#pragma unroll
+          for (int t = 0; t < 4; ++t) stage[wave][kg * 4 + t][nb * 16 + lrow] = acc[t];
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          const int il = ch * MG_BM + (rb0 + b) * 16 + rr0 + 8 * h;
+          if (ocol_ok && il < n_rows) {
+            const float *srow = &stage[wave][rr0 + 8 * h][c8];
+            float f[8];
+            unpack8<T>(cur[b][h], f);
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+              const float ab = Tr::to_float(Tr::from_float(srow[k]));   // the GEMM result is a T tensor
+              f[k] += p.sign * ab;
+            }
+            store16(wbase + (int64_t)il * p.ld, pack8<T>(f));
+          }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
       }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
     }
   }
 }
@@ -240,7 +285,16 @@ extern "C" int mlora_merge_adapter(void *stream, void *const *w, const int32_t *
   int kb = (int)((max_rank + 31) / 32);
   kb = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
   const int bm = merge_bm(kb);
-  const int64_t blocks = ((h_in + bm - 1) / bm) * a.n_ochunks;
+  // Slices per workgroup.  The grid takes so many rounds of what the device holds, each as long as a workgroup's slices
+  // and its set-up, which with the B fragments of rank 64 and more costs about one slice more (rank 128, 4096 wide: one
+  // slice 108 us, two 90, four 78; 3072 wide: 74, 72, three 58).  Up to rank 32 one slice is always fastest.
+  const int64_t slices = (h_in + bm - 1) / bm, per_slice = (int64_t)a.n_ochunks * n_targets;
+  const int64_t resident = (int64_t)merge_resident(kb) * 256;
+  auto cost = [&](int64_t c) { return ((slices + c - 1) / c * per_slice + resident - 1) / resident * (c + 1); };
+  a.chunks = 1;
+  for (int c = 2; kb > 1 && c <= 4; ++c)
+    if (cost(c) < cost(a.chunks)) a.chunks = c;
+  const int64_t blocks = (slices + a.chunks - 1) / a.chunks * a.n_ochunks;
   dim3 grid((unsigned)blocks, (unsigned)n_targets);
   return dtype == MLORA_F16 ? launch_merge_t<_Float16>((hipStream_t)stream, a, kb, grid)
                             : launch_merge_t<__bf16>((hipStream_t)stream, a, kb, grid);
