@@ -496,6 +496,122 @@ void lora_get_qkvo_fwd_expand(const at::Tensor &x, const at::Tensor &w, const at
                                 (size_t)ws.numel(), nullptr));
 }
 
+// ---- the planned op (valora_amd/plan.py) ------------------------------------------------------------------
+// What a LoraPlan holds on the native side: the plan, the index tensors it was cut from and the scratch of its calls.
+// A call checks its operands and goes straight to the C ABI.  Through ctypes a call cost 9-12 us of host time, more than
+// the GPU needs for a small decode batch (7 us); here it is the argument conversion plus the launches.
+struct NativePlan {
+  mlora_plan plan{};
+  at::Tensor buf, scratch, ids, a_start, a_len;
+  int64_t T = 0, max_rank = 0, scratch_per_target = 0;
+  int32_t n_slots = 4, bm_shrink = 0, bm_expand = 0, ksplit = 1, flags = 0;
+  c10::DeviceIndex device = 0;
+
+  NativePlan(const at::Tensor &ids_, const at::Tensor &a_start_, const at::Tensor &a_len_, int64_t max_rank_,
+             int32_t n_slots_, int32_t bm_shrink_, int32_t bm_expand_, int32_t ksplit_, int32_t flags_)
+      : ids(ids_.contiguous()), a_start(a_start_), a_len(a_len_), T(ids_.numel()), max_rank(max_rank_), n_slots(n_slots_),
+        bm_shrink(bm_shrink_), bm_expand(bm_expand_), ksplit(ksplit_), flags(flags_), device(ids_.get_device()) {
+    const int64_t A = a_start.numel();
+    buf = device_bytes(mlora_plan_bytes(T, A), ids);
+    plan.dev = buf.data_ptr();
+    plan.bytes = (size_t)buf.numel();
+    rebuild(c10::nullopt);
+    // room for a multi-target call from the start: the buffer is never replaced, so a HIP graph captured from this plan
+    // or work still queued on another stream keeps pointing at live memory
+    scratch_per_target = (int64_t)mlora_scratch_bytes(T, max_rank, ksplit);
+    size_t n = (size_t)MLORA_MAX_TARGETS * (size_t)scratch_per_target;
+    if (flags & MLORA_ONE_LAUNCH)
+      for (int t = 1; t <= MLORA_MAX_TARGETS; ++t)
+        n = std::max(n, mlora_one_launch_scratch_bytes(T, A, max_rank, ksplit, t));
+    scratch = at::empty({(int64_t)n}, ids.options().dtype(at::kByte));
+  }
+
+  hipStream_t stream() const { return c10::hip::getCurrentHIPStream(device).stream(); }
+
+  void rebuild(const c10::optional<at::Tensor> &new_ids) {
+    if (new_ids.has_value() && new_ids->defined()) {
+      if (new_ids->scalar_type() != at::kLong || new_ids->numel() != T || new_ids->device() != ids.device())
+        raise("rebuild takes " + std::to_string(T) + " int64 ids on " + ids.device().str());
+      ids = new_ids->contiguous();
+    }
+    check_rc(mlora_build_plan(stream(), &plan, static_cast<const int64_t *>(ids.data_ptr()), T,
+                              static_cast<const int64_t *>(a_start.data_ptr()),
+                              static_cast<const int64_t *>(a_len.data_ptr()), a_start.numel(), n_slots, bm_shrink,
+                              bm_expand));
+  }
+
+  mlora_pool pool(const at::Tensor &w, const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc,
+                  int64_t width) const {
+    mlora_pool p = make_pool(w, start, len, loc, width);
+    p.n_slots = n_slots;
+    return p;
+  }
+
+  void check_matrix(const at::Tensor &t) const {
+    if (t.dim() != 2 || t.size(0) != T || !t.is_contiguous())
+      raise("x and y must be contiguous [T=" + std::to_string(T) + ", H] matrices");
+  }
+
+  void apply(const at::Tensor &y, const at::Tensor &x, const at::Tensor &key_buffer, const at::Tensor &value_buffer,
+             const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc, int64_t slot, const at::Tensor &scales) {
+    if (x.dim() != 2 || y.dim() != 2 || x.size(0) != T || y.size(0) != T)
+      raise("x and y must be [T=" + std::to_string(T) + ", H] matrices");
+    if (!x.is_contiguous() || !y.is_contiguous()) raise("x and y must be contiguous");
+    const mlora_dtype code = dtype_code(x);
+    const int64_t h_in = x.size(1), h_out = y.size(1);
+    if ((int)code < 0 || y.scalar_type() != x.scalar_type() || key_buffer.scalar_type() != x.scalar_type() ||
+        value_buffer.scalar_type() != x.scalar_type())
+      no_kernel(h_in, h_out, x);
+    at::Tensor keep;
+    const void *sc = scales_ptr(scales, x, keep);
+    const mlora_pool pa = pool(key_buffer, start, len, loc, h_in), pb = pool(value_buffer, start, len, loc, h_out);
+    check_rc(mlora_lora_apply(stream(), &plan, scratch.data_ptr(), (size_t)scratch.numel(), y.data_ptr(), x.data_ptr(), T,
+                              h_in, h_out, max_rank, &pa, &pb, (int32_t)slot, sc, ksplit, flags, code));
+  }
+
+  void apply_multi(const std::vector<at::Tensor> &ys, const at::Tensor &x, const at::Tensor &key_buffer,
+                   const py::object &value_buffers, const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc,
+                   const std::vector<int64_t> &slots, const at::Tensor &scales) {
+    const size_t n = ys.size();
+    if (n < 1 || n > MLORA_MAX_TARGETS || slots.size() != n)
+      raise("apply_multi takes 1.." + std::to_string(MLORA_MAX_TARGETS) + " targets with one slot each");
+    const bool several = py::isinstance<py::list>(value_buffers) || py::isinstance<py::tuple>(value_buffers);
+    std::vector<at::Tensor> vbs;
+    if (several) vbs = value_buffers.cast<std::vector<at::Tensor>>();
+    else vbs.push_back(value_buffers.cast<at::Tensor>());
+    if (several && vbs.size() < n) raise("apply_multi takes one value buffer or one per target");
+    check_matrix(x);
+    const mlora_dtype code = dtype_code(x);
+    if ((int)code < 0 || key_buffer.scalar_type() != x.scalar_type()) no_kernel(x.size(1), x.size(1), x);
+    const int64_t h_in = x.size(1);
+    int64_t h_out = 0;
+    mlora_target tg[MLORA_MAX_TARGETS];
+    for (size_t i = 0; i < n; ++i) {
+      const at::Tensor &y = ys[i], &vb = vbs[several ? i : 0];
+      check_matrix(y);
+      if (i == 0) h_out = y.size(1);
+      if (y.scalar_type() != x.scalar_type() || vb.scalar_type() != x.scalar_type()) no_kernel(y.size(1), y.size(1), y);
+      if (y.size(1) != h_out) raise("all targets of one call must have the same output width");
+      tg[i].y = y.data_ptr();
+      tg[i].w_b = vb.data_ptr();
+      tg[i].w_b_rows = h_out > 0 ? vb.numel() / h_out : 0;
+      tg[i].slot = (int32_t)slots[i];
+    }
+    at::Tensor keep;
+    const void *sc = scales_ptr(scales, x, keep);
+    const mlora_pool pa = pool(key_buffer, start, len, loc, h_in);
+    check_rc(mlora_lora_apply_multi(stream(), &plan, scratch.data_ptr(), (size_t)scratch.numel(), x.data_ptr(), T, h_in,
+                                    h_out, max_rank, &pa, (int32_t)n, tg, sc, ksplit, flags, code));
+  }
+};
+
+// (bm_shrink, ksplit, bm_expand, flags) of a shape
+py::tuple tile_lookup(int64_t T, int64_t max_rank, int64_t hidden, int64_t n_adapters) {
+  mlora_tile_config c;
+  check_rc(mlora_tile_lookup(T, max_rank, hidden, n_adapters, &c));
+  return py::make_tuple(c.bm_shrink, c.ksplit, c.bm_expand, c.flags);
+}
+
 // ---- the cache as Python sees it ---------------------------------------------------------------------
 Key python_key(const std::vector<at::Tensor> &tensors, const std::vector<int64_t> &scalars) {
   Key key;
@@ -547,6 +663,16 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("shrink_accumulate", [](bool on) { g_sgmm_shrink_mode = on ? MLORA_SHRINK_ACCUMULATE : MLORA_SHRINK_OVERWRITE; },
         "True: the segment signature's shrink adds into y (D = X*W + C, atmm/valora/csrc/bgmv/bgmv_impl.cuh:174) "
         "instead of overwriting it.");
+  py::class_<NativePlan>(m, "NativePlan")
+      .def(py::init<const at::Tensor &, const at::Tensor &, const at::Tensor &, int64_t, int32_t, int32_t, int32_t, int32_t,
+                    int32_t>())
+      .def("apply", &NativePlan::apply)
+      .def("apply_multi", &NativePlan::apply_multi)
+      .def("rebuild", &NativePlan::rebuild)
+      .def_readonly("buf", &NativePlan::buf)
+      .def_readonly("scratch", &NativePlan::scratch)
+      .def_readonly("scratch_per_target", &NativePlan::scratch_per_target);
+  m.def("tile_lookup", &tile_lookup);
   m.def("cache_lookup", &cache_lookup);
   m.def("cache_insert", &cache_insert);
   m.def("cache_clear", [] { g_entries.clear(); });

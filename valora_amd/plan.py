@@ -15,7 +15,8 @@ from typing import Optional
 
 import torch
 
-from . import _lib, tile_table
+from . import _lib
+from ._ext import binding as _b
 
 
 class LoraPlan:
@@ -43,13 +44,13 @@ class LoraPlan:
         self.n_adapters = int(a_start.numel())
         self.n_slots = n_slots
         self.max_rank = int(max_rank)
-        cfg = tile_table.lookup(self.T, self.max_rank, hidden, self.n_adapters)
-        self.bm_shrink = cfg.bm_shrink if bm_shrink is None else bm_shrink
-        self.bm_expand = cfg.bm_expand if bm_expand is None else bm_expand
-        self.ksplit = max(1, cfg.ksplit if ksplit is None else ksplit)
-        rie = cfg.reduce_in_expand if reduce_in_expand is None else reduce_in_expand
+        t_bm_shrink, t_ksplit, t_bm_expand, t_flags = _b.tile_lookup(self.T, self.max_rank, hidden, self.n_adapters)
+        self.bm_shrink = t_bm_shrink if bm_shrink is None else bm_shrink
+        self.bm_expand = t_bm_expand if bm_expand is None else bm_expand
+        self.ksplit = max(1, t_ksplit if ksplit is None else ksplit)
+        rie = bool(t_flags & _lib.REDUCE_IN_EXPAND) if reduce_in_expand is None else reduce_in_expand
         self.flags = _lib.REDUCE_IN_EXPAND if rie else 0
-        self.one_launch = bool(cfg.one_launch if one_launch is None else one_launch)
+        self.one_launch = bool(t_flags & _lib.ONE_LAUNCH if one_launch is None else one_launch)
         if self.one_launch and (self.max_rank > 64 or bm_shrink not in (None, 16) or bm_expand not in (None, 16)):
             if one_launch:
                 raise RuntimeError("No suitable kernel. the one-launch op needs 16-token tiles and max_rank <= 64")
@@ -63,20 +64,27 @@ class LoraPlan:
             self.flags |= _lib.SHRINK_RECOMPUTE
         if expand_column_loop:
             self.flags |= _lib.EXPAND_COLUMN_LOOP
-        L = _lib.lib()
-        nbytes = int(L.mlora_plan_bytes(self.T, self.n_adapters))
-        self.buf = torch.empty(max(nbytes, 256), dtype=torch.uint8, device=self.device)
-        self.handle = _lib.Plan(_lib.ptr(self.buf), self.buf.numel(), 0, 0, 0, 0)
-        self._keep = (ids.contiguous(), a_start, a_len)
-        self.rebuild()
-        # room for a multi-target call from the start: the buffer is never replaced, so a HIP graph captured
-        # from this plan or work still queued on another stream keeps pointing at live memory
-        self.scratch_per_target = int(L.mlora_scratch_bytes(self.T, self.max_rank, self.ksplit))
-        nbytes = _lib.MAX_TARGETS * self.scratch_per_target
-        if self.one_launch:
-            nbytes = max(nbytes, max(int(L.mlora_one_launch_scratch_bytes(self.T, self.n_adapters, self.max_rank,
-                                                                          self.ksplit, n)) for n in (1, 2, 3, 4)))
-        self.scratch = torch.empty(nbytes, dtype=torch.uint8, device=self.device)
+        # plan, scratch and the calls themselves live on the native side (csrc/binding.cpp)
+        self._native = _b.NativePlan(ids, a_start, a_len, self.max_rank, n_slots, self.bm_shrink, self.bm_expand,
+                                     self.ksplit, self.flags)
+
+    @property
+    def buf(self) -> torch.Tensor:
+        return self._native.buf
+
+    @property
+    def scratch(self) -> torch.Tensor:
+        return self._native.scratch
+
+    @property
+    def scratch_per_target(self) -> int:
+        return self._native.scratch_per_target
+
+    @property
+    def handle(self):
+        """The plan as the C ABI takes it (``mlora_plan``)."""
+        buf = self._native.buf
+        return _lib.Plan(_lib.ptr(buf), buf.numel(), self.T, self.n_adapters, self.bm_shrink, self.bm_expand, self.n_slots)
 
     def rebuild(self, ids: Optional[torch.Tensor] = None) -> None:
         """Cut the tiles again, in place, for the next batch of the same size (``ids`` of the same length; None
@@ -84,14 +92,7 @@ class LoraPlan:
         stream, no allocation: a serving loop that replays one HIP graph per step captures this call at the
         head of the step and refills its ids tensor before each replay (the reference rebuilds its segment
         tensors once per forward, valora/server/router/model_infer/model_rpc.py:381)."""
-        if ids is not None:
-            if ids.dtype != torch.long or ids.numel() != self.T or ids.device != self.device:
-                raise RuntimeError(f"rebuild takes {self.T} int64 ids on {self.device}")
-            self._keep = (ids.contiguous(),) + self._keep[1:]
-        ids, a_start, a_len = self._keep
-        _lib.check(_lib.lib().mlora_build_plan(_lib.current_stream(self.device), self.handle, _lib.ptr(ids), self.T,
-                                               _lib.ptr(a_start), _lib.ptr(a_len), self.n_adapters, self.n_slots,
-                                               self.bm_shrink, self.bm_expand))
+        self._native.rebuild(ids)
 
     # -- introspection (synchronises; for tests and diagnostics) --------------------------------
     def header(self) -> dict:
@@ -165,46 +166,12 @@ class LoraPlan:
         """Several targets that read the same ``x`` (q, k, v of a layer; gate and up) in two launches:
         ``ys[i] += scale_a * (x @ A_a[slots[i]].T) @ B_a[slots[i]]``.  ``value_buffers`` is one pool tensor or
         one per target.  Same results as ``apply`` called once per target."""
-        n = len(ys)
-        if not 1 <= n <= _lib.MAX_TARGETS or len(slots) != n:
-            raise RuntimeError(f"apply_multi takes 1..{_lib.MAX_TARGETS} targets with one slot each")
-        vbs = list(value_buffers) if isinstance(value_buffers, (list, tuple)) else [value_buffers] * n
-        h_in, h_out = x.size(1), ys[0].size(1)
-        for y, vb in zip(ys, vbs):
-            self._check(x, y, key_buffer, vb)
-            if y.size(1) != h_out:
-                raise RuntimeError("all targets of one call must have the same output width")
-        if scales.dtype != x.dtype:
-            scales = scales.to(x.dtype)
-        pa = _lib.make_pool(key_buffer, a_start, a_len, a_loc, h_in, self.n_slots)
-        tg = (_lib.Target * n)()
-        for i in range(n):
-            tg[i] = _lib.Target(_lib.ptr(ys[i]), _lib.ptr(vbs[i]), vbs[i].numel() // h_out, int(slots[i]))
         # (a call whose expand half is more than 16 items per tile -- q+k+v, a 4096 -> 11008 target -- is run as two
         # launches by the library whatever the flag says: same tiles, same split, same bits)
-        flags = self.flags
-        _lib.check(_lib.lib().mlora_lora_apply_multi(
-            _lib.current_stream(self.device), self.handle, _lib.ptr(self.scratch), self.scratch.numel(), _lib.ptr(x),
-            self.T, h_in, h_out, self.max_rank, pa, n, tg, _lib.ptr(scales), int(self.ksplit), flags,
-            _lib.dtype_code(x.dtype)))
+        self._native.apply_multi(ys, x, key_buffer, value_buffers, a_start, a_len, a_loc, slots, scales)
 
     def apply(self, y: torch.Tensor, x: torch.Tensor, key_buffer: torch.Tensor, value_buffer: torch.Tensor,
               a_start: torch.Tensor, a_len: torch.Tensor, a_loc: torch.Tensor, slot: int,
               scales: torch.Tensor) -> None:
         """``y[t] += scale_a * (x[t] @ A_a.T) @ B_a`` in place for every token with an adapter."""
-        if x.dim() != 2 or y.dim() != 2 or x.size(0) != self.T or y.size(0) != self.T:
-            raise RuntimeError(f"x and y must be [T={self.T}, H] matrices")
-        if not (x.is_contiguous() and y.is_contiguous()):
-            raise RuntimeError("x and y must be contiguous")
-        code = _lib.dtype_code(x.dtype)
-        if code < 0 or y.dtype != x.dtype or key_buffer.dtype != x.dtype or value_buffer.dtype != x.dtype:
-            raise RuntimeError(f"No suitable kernel. h_in={x.size(1)} h_out={y.size(1)} dtype={x.dtype}")
-        if scales.dtype != x.dtype:
-            scales = scales.to(x.dtype)
-        h_in, h_out = x.size(1), y.size(1)
-        pa = _lib.make_pool(key_buffer, a_start, a_len, a_loc, h_in, self.n_slots)
-        pb = _lib.make_pool(value_buffer, a_start, a_len, a_loc, h_out, self.n_slots)
-        _lib.check(_lib.lib().mlora_lora_apply(
-            _lib.current_stream(self.device), self.handle, _lib.ptr(self.scratch), self.scratch.numel(),
-            _lib.ptr(y), _lib.ptr(x), self.T, h_in, h_out, self.max_rank, pa, pb, int(slot), _lib.ptr(scales),
-            int(self.ksplit), self.flags, code))
+        self._native.apply(y, x, key_buffer, value_buffer, a_start, a_len, a_loc, slot, scales)
