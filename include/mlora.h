@@ -52,9 +52,9 @@ enum {
                                  mlora_one_launch_scratch_bytes(), 128-byte aligned (the partials are
                                  handed over in cache lines that belong to one tile each; a scratch
                                  buffer aligned to less, an empty index or an empty pool make the call
-                                 run as two launches, and so does a call with more than 16 expand items
-                                 per tile -- 512-column chunks (256 above rank 32) x targets -- where two
-                                 launches measured faster).  Any batch size: items the device cannot
+                                 run as two launches, and so does a call with more than 32 expand items
+                                 per tile -- 512-column chunks x targets; above rank 32 more than 16 of
+                                 256 columns -- where two launches measured faster).  Any batch size: items the device cannot
                                  hold from the start take part in the hand-off like the others.
                                  Bit-identical to the two-launch op with MLORA_REDUCE_IN_EXPAND and the
                                  same ksplit.  Launches that share a plan must not overlap in time.  */

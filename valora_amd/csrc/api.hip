@@ -35,7 +35,7 @@ int decode_bn(int max_rank);   // output columns per expand item of the one-laun
 // limits how long a workgroup holds its slot when the producers are held up (a device shared with other work).
 constexpr int ONE_LAUNCH_WAIT_TICKS = 3000;
 // expand items per tile up to which a call that asks for one launch gets it (see mlora_lora_apply_multi)
-constexpr int ONE_LAUNCH_MAX_EXPAND_ITEMS = 16;
+constexpr int one_launch_max_expand_items(int64_t max_rank) { return max_rank <= 32 ? 32 : 16; }
 
 namespace {
 
@@ -429,13 +429,15 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   // same ksplit, which gives the same bits.
   bool use_decode = one_launch && aligned128(scratch) && pool_a->a_loc_len > 0 && pool_a->w_rows > 0;
   for (int i = 0; use_decode && i < n_targets; ++i) use_decode = targets[i].w_b_rows > 0;
-  // Where the one-launch op pays is a matter of the expand items per tile (column chunks x targets), measured on 256
-  // decode tokens over 64 adapters: up to 16 of them (one or two 4096-wide targets, an 11008 -> 4096 one) it is
-  // 2 - 2.5 us faster than two launches, with more (q+k+v: 24, one 4096 -> 11008 target: 22) the expand half is the
-  // longer one and the column-looping expand launch does it 3 us faster than these items do.
+  // Where the one-launch op pays is a matter of the expand items per tile (column chunks x targets), measured on 4 to
+  // 512 decode tokens over 8 to 64 adapters, us for two launches / one: up to rank 32 (512-column items) q+k+v of 4096
+  // columns (24 items) 10.2 / 8.9 and 15.0 / 11.4, of 5120 (30) 18.1 / 16.6, one 4096 -> 11008 target (22) 12.3 / 10.9;
+  // gate+up 4096 -> 11008 (44) 14.9 / 16.2 and 20.1 / 20.8: the expand half is the longer one there, and the
+  // column-looping expand launch does it faster than these items do.  At rank 64 (256-column items) one target of 4096
+  // columns (16) 12.9 / 9.7, q+k+v (48) 15.6 / 16.2, one of 11008 columns and more likewise slower.
   if (use_decode) {
     const int64_t bn = decode_bn((int)max_rank);
-    use_decode = (h_out + bn - 1) / bn * n_targets <= ONE_LAUNCH_MAX_EXPAND_ITEMS;
+    use_decode = (h_out + bn - 1) / bn * n_targets <= one_launch_max_expand_items(max_rank);
   }
   if (ksplit < 1 || ksplit > 64) return fail(MLORA_ERR_INVALID, "lora_apply_multi: ksplit=%d outside [1,64]", ksplit);
   const size_t per_target = scratch_bytes(T, max_rank, ksplit);

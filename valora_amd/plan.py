@@ -166,7 +166,7 @@ class LoraPlan:
         """Several targets that read the same ``x`` (q, k, v of a layer; gate and up) in two launches:
         ``ys[i] += scale_a * (x @ A_a[slots[i]].T) @ B_a[slots[i]]``.  ``value_buffers`` is one pool tensor or
         one per target.  Same results as ``apply`` called once per target."""
-        # (a call whose expand half is more than 16 items per tile -- q+k+v, a 4096 -> 11008 target -- is run as two
+        # (a call whose expand half is too many items per tile -- gate+up; from rank 64 on q+k+v too -- is run as two
         # launches by the library whatever the flag says: same tiles, same split, same bits)
         self._native.apply_multi(ys, x, key_buffer, value_buffers, a_start, a_len, a_loc, slots, scales)
 

@@ -166,7 +166,7 @@ def tune_tall_shrink(dev, n_tokens, n_adapters, rank, hidden, entry, dtype=torch
 def tune_one_launch(dev, n_tokens, n_adapters, rank, hidden, entry, dtype=torch.float16, copies=4):
     """Does the one-launch op (shrink and expand items of one grid, 16-token tiles) beat the two-launch entry of
     this shape?  Returns the entry to keep and both timings.  Only decode-like shapes qualify: rank <= 64.  The
-    library runs a call with more than 16 expand items per tile as two launches whatever the entry says, so an
+    library runs a call with too many expand items per tile as two launches whatever the entry says, so an
     MLP-wide `hidden` is measured as what it is the input of, a down projection (to a 4096- or 8192-wide output)."""
     h_out = down_projection_width(hidden)
     ids, pool, x = synthetic_batch(n_tokens, n_adapters, rank, hidden, dtype, seed=n_tokens + n_adapters + rank, h_out=h_out)
