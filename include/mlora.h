@@ -227,6 +227,22 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
                            const mlora_pool *pool_a, int32_t n_targets, const mlora_target *targets,
                            const void *scales, int32_t ksplit, int32_t flags, mlora_dtype dtype);
 
+/* ---- one adapter merged into the base weights ("deLoRA") ------------------------------------- */
+/* A plan of the tokens of every adapter but `merged` (-1 or an index outside the pool: of every token, as
+ * mlora_build_plan), for mlora_lora_compensate.                                                */
+int mlora_build_compensation_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T,
+                                  const int64_t *a_start, const int64_t *a_len, int64_t n_adapters,
+                                  int32_t n_slots, int32_t bm_shrink, int32_t bm_expand, int64_t merged);
+/* y[t] += scale_own * (x[t] A_own) B_own - scale_merged * (x[t] A_merged) B_merged for every token of such a
+ * plan: one shrink launch over both adapters of a token, one expand launch that adds the difference
+ * (the reference runs a doubled batch, valora/models/peft/lora_unordered_batch_infer.py:991-1063).
+ * scratch_bytes must be at least 2 * mlora_scratch_bytes(T, max_rank, ksplit).  Of the flags only
+ * MLORA_SHRINK_RECOMPUTE has a meaning here.                                                   */
+int mlora_lora_compensate(void *stream, const mlora_plan *plan, void *scratch, size_t scratch_bytes, void *y,
+                          const void *x, int64_t T, int64_t h_in, int64_t h_out, int64_t max_rank,
+                          const mlora_pool *pool_a, const mlora_pool *pool_b, int32_t slot, const void *scales,
+                          int32_t ksplit, int32_t flags, mlora_dtype dtype);
+
 /* ---- the reference's entry points, one call each -------------------------------------------- */
 /* Each of the four takes an optional `plan`.  NULL: the call sorts the tokens and cuts the tiles
  * itself, in `workspace` (mlora_workspace_bytes), with the tile table's configuration for the shape

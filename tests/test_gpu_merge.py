@@ -146,6 +146,39 @@ def test_delora_compensation(dev, n):
     assert err <= (6e-2 if w.dtype == torch.bfloat16 else 8e-3) * (1 + ref[has].abs().max()), err
 
 
+@pytest.mark.parametrize("ranks,T,kw", [
+    ([8], 1, {}), ([16, 8, 32], 33, {}), ([64, 8, 24], 300, dict(bm_shrink=32, ksplit=4, bm_expand=32)),
+    ([128, 16, 64], 130, dict(bm_shrink=16, ksplit=2, bm_expand=16)), ([32, 64, 8], 517, dict(bm_shrink=64, ksplit=1, bm_expand=96)),
+    ([64, 16], 700, dict(bm_shrink=128, ksplit=4, bm_expand=128)), ([16, 8, 64], 300, dict(bm_shrink=256, ksplit=2, bm_expand=48)),
+    ([16, 40], 90, dict(bm_shrink=16, ksplit=4, bm_expand=16, shrink_recompute=True))])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_compensation_shapes(dev, ranks, T, kw, dtype):
+    """The two products of a compensation call over every shrink tile height and way to finish the split-K sum: tiles
+    of the merged adapter that cross the borders of the tokens' own tiles, ragged last tiles, a merged adapter of
+    another rank, tokens without adapter, all tokens with the merged adapter, a merged adapter that does not exist."""
+    g = torch.Generator().manual_seed(T + len(ranks))
+    h_in, h_out = 520, 392
+    pool = W.make_pool(ranks, h_in, h_out, dtype, g, True, std=0.05, heads=1, scalings=[0.5 + 0.25 * i for i in range(len(ranks))])
+    pd = pool.to(dev)
+    idx = (pd.a_start, pd.a_len, pd.a_loc)
+    x, y0 = torch.randn(T, h_in, generator=g).to(dtype), torch.randn(T, h_out, generator=g).to(dtype)
+    mixed = torch.randint(-1, len(ranks), (T,), generator=g)
+    for ids, merged in ((mixed, 0), (mixed, len(ranks) - 1), (torch.zeros(T, dtype=torch.long), 0), (mixed, -1)):
+        plan = DeLoraPlan(ids.to(dev), merged, pd.a_start, pd.a_len, max(ranks), hidden=h_in, **kw)
+        for slot in (0, 3):
+            y = y0.to(dev)
+            plan.apply(y, x.to(dev), pd.key_buffer, pd.value_buffer, *idx, slot, pd.a_scaling)
+            if merged < 0:
+                want = O.lora_op(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, slot,
+                                 pool.a_scaling)
+            else:
+                want = O.delora_compensate(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc,
+                                           ids, merged, slot, pool.a_scaling)
+            assert_parity(y.cpu(), want, f"ranks {ranks} T {T} merged {merged} slot {slot}")
+            same = (ids == merged) | (ids < 0)
+            assert torch.equal(y.cpu()[same], y0[same])
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_merge_random_shapes(dev, seed):
     """Non-square weights, widths that are multiples of 8 only, 1-5 pool slots, any subset of slots,

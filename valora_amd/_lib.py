@@ -28,6 +28,7 @@ SYMBOLS = [
     "mlora_dispatch_sgmm", "mlora_prefill_shrink", "mlora_prefill_expand",
     "mlora_pool_alloc", "mlora_pool_alloc_contiguous", "mlora_pool_free", "mlora_pool_fill",
     "mlora_pool_scatter_rows", "mlora_pool_gather_rows", "mlora_index_compact", "mlora_merge_adapter",
+    "mlora_build_compensation_plan", "mlora_lora_compensate",
 ]
 
 

@@ -133,6 +133,7 @@ void set_reduce_here(ShrinkArgs &a, const mlora_plan *plan, const PlanLayout &L,
   a.prp = (int)partial_stride_lines(max_rank);
   a.n_tiles = (int)tiles_upper(plan->T, plan->n_adapters, plan->bm_shrink);
   a.arrive = reinterpret_cast<unsigned long long *>(static_cast<int32_t *>(plan->dev) + L.off_arrive);
+  a.compensate = 0;
 }
 
 struct Carver {
@@ -185,9 +186,9 @@ size_t mlora_workspace_bytes(int64_t T, int64_t n_adapters, int64_t max_rank) {
   return up(mlora_plan_bytes(T, n_adapters)) + up(scratch_bytes(T, max_rank, ks)) + up((size_t)T * 8 + 8) + 256;
 }
 
-int mlora_build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T, const int64_t *a_start,
-                     const int64_t *a_len, int64_t n_adapters, int32_t n_slots, int32_t bm_shrink,
-                     int32_t bm_expand) {
+static int build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T, const int64_t *a_start,
+                      const int64_t *a_len, int64_t n_adapters, int32_t n_slots, int32_t bm_shrink, int32_t bm_expand,
+                      int64_t merged) {
   if (!plan || !plan->dev) return fail(MLORA_ERR_INVALID, "build_plan: plan buffer is null");
   if (T < 0 || T > MAX_TOKENS) return fail(MLORA_ERR_INVALID, "build_plan: T=%lld out of range", (long long)T);
   if (n_adapters < 0 || n_adapters > MAX_ADAPTERS)
@@ -216,7 +217,19 @@ int mlora_build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t
   plan->bm_shrink = bm_shrink;
   plan->bm_expand = bm_expand;
   return launch_plan((hipStream_t)stream, static_cast<int32_t *>(plan->dev), L, ids, a_start, a_len, n_slots,
-                     bm_shrink, bm_expand);
+                     bm_shrink, bm_expand, merged >= 0 && merged < n_adapters ? (int)merged : -1);
+}
+
+int mlora_build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T, const int64_t *a_start,
+                     const int64_t *a_len, int64_t n_adapters, int32_t n_slots, int32_t bm_shrink,
+                     int32_t bm_expand) {
+  return build_plan(stream, plan, ids, T, a_start, a_len, n_adapters, n_slots, bm_shrink, bm_expand, -1);
+}
+
+int mlora_build_compensation_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T, const int64_t *a_start,
+                                  const int64_t *a_len, int64_t n_adapters, int32_t n_slots, int32_t bm_shrink,
+                                  int32_t bm_expand, int64_t merged) {
+  return build_plan(stream, plan, ids, T, a_start, a_len, n_adapters, n_slots, bm_shrink, bm_expand, merged);
 }
 
 int mlora_count_consecutive(void *stream, const int64_t *lora_rank, int64_t n_adapters, const int64_t *indicies,
@@ -354,6 +367,7 @@ int mlora_expand(void *stream, const mlora_plan *plan, void *y, int64_t T, int64
   a.slot = slot;
   a.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
   a.column_loop = (flags & MLORA_EXPAND_COLUMN_LOOP) ? 1 : 0;
+  a.compensate = 0;
   a.n_targets = 1;
   for (int i = 0; i < MLORA_MAX_TARGETS; ++i) {
     a.slots[i] = slot;
@@ -502,6 +516,7 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   e.slot = targets[0].slot;
   e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
   e.column_loop = (flags & MLORA_EXPAND_COLUMN_LOOP) ? 1 : 0;
+  e.compensate = 0;
   e.n_targets = n_targets;
   for (int i = 0; i < MLORA_MAX_TARGETS; ++i) {
     const mlora_target &t = targets[i < n_targets ? i : 0];
@@ -528,6 +543,97 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
     d.never_ready = (flags & MLORA_ONE_LAUNCH_NEVER_READY) ? 1 : 0;
     return launch_decode((hipStream_t)stream, d, (int)max_rank, dtype);
   }
+  return launch_expand((hipStream_t)stream, e, (int)max_rank, tiles_upper(T, plan->n_adapters, plan->bm_expand),
+                       plan->bm_expand, dtype);
+}
+
+int mlora_lora_compensate(void *stream, const mlora_plan *plan, void *scratch, size_t scratch_nbytes, void *y,
+                          const void *x, int64_t T, int64_t h_in, int64_t h_out, int64_t max_rank,
+                          const mlora_pool *pool_a, const mlora_pool *pool_b, int32_t slot, const void *scales,
+                          int32_t ksplit, int32_t flags, mlora_dtype dtype) {
+  if (int rc = check_dtype(dtype, h_in, h_out)) return rc;
+  if (int rc = check_dims(T, h_in, max_rank, h_in, h_out, dtype)) return rc;
+  if (int rc = check_dims(T, h_out, max_rank, h_in, h_out, dtype)) return rc;
+  if (int rc = check_plan(plan, T, "lora_compensate")) return rc;
+  if (int rc = check_pool(pool_a, "lora_compensate")) return rc;
+  if (int rc = check_pool(pool_b, "lora_compensate")) return rc;
+  if (int rc = check_plan_pool(plan, pool_a, "lora_compensate")) return rc;
+  if (int rc = check_plan_pool(plan, pool_b, "lora_compensate")) return rc;
+  if (T == 0) return MLORA_OK;
+  if (!x || !y || !scratch || !scales) return fail(MLORA_ERR_INVALID, "lora_compensate: null pointer");
+  if (!aligned16(x) || !aligned16(y) || !aligned16(scratch))
+    return fail(MLORA_ERR_INVALID, "lora_compensate: x, y and scratch must be 16-byte aligned");
+  if (slot < 0 || slot >= pool_a->n_slots) return fail(MLORA_ERR_INVALID, "lora_compensate: slot %d outside [0,%d)", slot, pool_a->n_slots);
+  if (ksplit == 0) ksplit = tile_ksplit_for(T, max_rank, h_in, plan->n_adapters, plan->bm_shrink);
+  if (ksplit < 1 || ksplit > 64) return fail(MLORA_ERR_INVALID, "lora_compensate: ksplit=%d outside [1,64]", ksplit);
+  const size_t per_target = scratch_bytes(T, max_rank, ksplit);
+  if (scratch_nbytes < 2 * per_target)
+    return fail(MLORA_ERR_WORKSPACE, "lora_compensate: scratch has %zu bytes, needs %zu", scratch_nbytes, 2 * per_target);
+  const PlanLayout L = plan_layout(plan->T, plan->n_adapters);
+  const int64_t rp = partial_stride(max_rank);
+  // shrink: "target" 0 is the tokens' own adapters, "target" 1 the merged one
+  ShrinkArgs a;
+  a.plan = static_cast<const int32_t *>(plan->dev);
+  a.off_perm = L.off_perm;
+  a.off_tiles = L.off_tiles_s;
+  a.off_prank = L.off_prank;
+  a.partial = reinterpret_cast<float *>(static_cast<char *>(scratch) + align_up(T * rp * 2, 256));
+  a.x = static_cast<const uint16_t *>(x);
+  a.pool = pool_dev(pool_a);
+  a.T = (int)T;
+  a.h_in = (int)h_in;
+  a.rp = (int)rp;
+  a.slot = slot;
+  a.ksplit = ksplit;
+  a.kchunk = (int)align_up((h_in + ksplit - 1) / ksplit, 128);
+  a.out = static_cast<uint16_t *>(scratch);
+  a.out_stride = rp;
+  a.out_by_token = 0;
+  a.mode = MLORA_SHRINK_OVERWRITE;
+  a.width = 0;
+  a.ncols = (int)rp;
+  a.partial_only = 0;
+  a.n_targets = 2;
+  for (int i = 0; i < MLORA_MAX_TARGETS; ++i) a.slots[i] = slot;
+  a.out_tstride = (int64_t)(per_target / 2);
+  a.partial_tstride = (int64_t)(per_target / 4);
+  set_reduce_here(a, plan, L, max_rank, flags);
+  a.compensate = 1;
+  if (int rc = launch_shrink((hipStream_t)stream, a, plan->bm_shrink, (int)max_rank,
+                             tiles_upper(T, plan->n_adapters, plan->bm_shrink), dtype))
+    return rc;
+  if (ksplit > 1 && !a.reduce_here)
+    if (int rc = launch_shrink_reduce((hipStream_t)stream, a, dtype)) return rc;
+
+  ExpandArgs e;
+  e.plan = a.plan;
+  e.off_perm = L.off_perm;
+  e.off_tiles = L.off_tiles_e;
+  e.y = static_cast<uint16_t *>(y);
+  e.v = static_cast<const uint16_t *>(scratch);
+  e.v_stride = rp;
+  e.v_by_pos = 1;
+  e.partial = nullptr;
+  e.ksplit = 1;
+  e.rp = (int)rp;
+  e.pool = pool_dev(pool_b);
+  e.scales = static_cast<const uint16_t *>(scales);
+  e.T = (int)T;
+  e.h_out = (int)h_out;
+  e.kmax = (int)max_rank;
+  e.slot = slot;
+  e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
+  e.column_loop = 0;
+  e.compensate = 1;
+  e.n_targets = 1;
+  for (int i = 0; i < MLORA_MAX_TARGETS; ++i) {
+    e.slots[i] = slot;
+    e.ys[i] = e.y;
+    e.ws[i] = e.pool.w;
+    e.w_rows_t[i] = e.pool.w_rows;
+  }
+  e.v_tstride = a.out_tstride;
+  e.partial_tstride = 0;
   return launch_expand((hipStream_t)stream, e, (int)max_rank, tiles_upper(T, plan->n_adapters, plan->bm_expand),
                        plan->bm_expand, dtype);
 }

@@ -504,13 +504,14 @@ struct NativePlan {
   mlora_plan plan{};
   at::Tensor buf, scratch, ids, a_start, a_len;
   int64_t T = 0, max_rank = 0, scratch_per_target = 0;
+  int64_t merged = -1;   // the adapter in the base weights of a compensation plan
   int32_t n_slots = 4, bm_shrink = 0, bm_expand = 0, ksplit = 1, flags = 0;
   c10::DeviceIndex device = 0;
 
   NativePlan(const at::Tensor &ids_, const at::Tensor &a_start_, const at::Tensor &a_len_, int64_t max_rank_,
-             int32_t n_slots_, int32_t bm_shrink_, int32_t bm_expand_, int32_t ksplit_, int32_t flags_)
-      : ids(ids_.contiguous()), a_start(a_start_), a_len(a_len_), T(ids_.numel()), max_rank(max_rank_), n_slots(n_slots_),
-        bm_shrink(bm_shrink_), bm_expand(bm_expand_), ksplit(ksplit_), flags(flags_), device(ids_.get_device()) {
+             int32_t n_slots_, int32_t bm_shrink_, int32_t bm_expand_, int32_t ksplit_, int32_t flags_, int64_t merged_)
+      : ids(ids_.contiguous()), a_start(a_start_), a_len(a_len_), T(ids_.numel()), max_rank(max_rank_), merged(merged_),
+        n_slots(n_slots_), bm_shrink(bm_shrink_), bm_expand(bm_expand_), ksplit(ksplit_), flags(flags_), device(ids_.get_device()) {
     const int64_t A = a_start.numel();
     buf = device_bytes(mlora_plan_bytes(T, A), ids);
     plan.dev = buf.data_ptr();
@@ -534,10 +535,10 @@ struct NativePlan {
         raise("rebuild takes " + std::to_string(T) + " int64 ids on " + ids.device().str());
       ids = new_ids->contiguous();
     }
-    check_rc(mlora_build_plan(stream(), &plan, static_cast<const int64_t *>(ids.data_ptr()), T,
-                              static_cast<const int64_t *>(a_start.data_ptr()),
-                              static_cast<const int64_t *>(a_len.data_ptr()), a_start.numel(), n_slots, bm_shrink,
-                              bm_expand));
+    check_rc(mlora_build_compensation_plan(stream(), &plan, static_cast<const int64_t *>(ids.data_ptr()), T,
+                                           static_cast<const int64_t *>(a_start.data_ptr()),
+                                           static_cast<const int64_t *>(a_len.data_ptr()), a_start.numel(), n_slots,
+                                           bm_shrink, bm_expand, merged));
   }
 
   mlora_pool pool(const at::Tensor &w, const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc,
@@ -554,6 +555,20 @@ struct NativePlan {
 
   void apply(const at::Tensor &y, const at::Tensor &x, const at::Tensor &key_buffer, const at::Tensor &value_buffer,
              const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc, int64_t slot, const at::Tensor &scales) {
+    one_target(mlora_lora_apply, y, x, key_buffer, value_buffer, start, len, loc, slot, scales);
+  }
+
+  // y += own adapter - merged adapter, for the tokens of a compensation plan
+  void compensate(const at::Tensor &y, const at::Tensor &x, const at::Tensor &key_buffer, const at::Tensor &value_buffer,
+                  const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc, int64_t slot,
+                  const at::Tensor &scales) {
+    one_target(mlora_lora_compensate, y, x, key_buffer, value_buffer, start, len, loc, slot, scales);
+  }
+
+  template <typename Op>
+  void one_target(Op op, const at::Tensor &y, const at::Tensor &x, const at::Tensor &key_buffer,
+                  const at::Tensor &value_buffer, const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc,
+                  int64_t slot, const at::Tensor &scales) {
     if (x.dim() != 2 || y.dim() != 2 || x.size(0) != T || y.size(0) != T)
       raise("x and y must be [T=" + std::to_string(T) + ", H] matrices");
     if (!x.is_contiguous() || !y.is_contiguous()) raise("x and y must be contiguous");
@@ -565,8 +580,8 @@ struct NativePlan {
     at::Tensor keep;
     const void *sc = scales_ptr(scales, x, keep);
     const mlora_pool pa = pool(key_buffer, start, len, loc, h_in), pb = pool(value_buffer, start, len, loc, h_out);
-    check_rc(mlora_lora_apply(stream(), &plan, scratch.data_ptr(), (size_t)scratch.numel(), y.data_ptr(), x.data_ptr(), T,
-                              h_in, h_out, max_rank, &pa, &pb, (int32_t)slot, sc, ksplit, flags, code));
+    check_rc(op(stream(), &plan, scratch.data_ptr(), (size_t)scratch.numel(), y.data_ptr(), x.data_ptr(), T, h_in, h_out,
+                max_rank, &pa, &pb, (int32_t)slot, sc, ksplit, flags, code));
   }
 
   void apply_multi(const std::vector<at::Tensor> &ys, const at::Tensor &x, const at::Tensor &key_buffer,
@@ -665,9 +680,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "instead of overwriting it.");
   py::class_<NativePlan>(m, "NativePlan")
       .def(py::init<const at::Tensor &, const at::Tensor &, const at::Tensor &, int64_t, int32_t, int32_t, int32_t, int32_t,
-                    int32_t>())
+                    int32_t, int64_t>())
       .def("apply", &NativePlan::apply)
       .def("apply_multi", &NativePlan::apply_multi)
+      .def("compensate", &NativePlan::compensate)
       .def("rebuild", &NativePlan::rebuild)
       .def_readonly("buf", &NativePlan::buf)
       .def_readonly("scratch", &NativePlan::scratch)

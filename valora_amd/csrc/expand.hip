@@ -42,11 +42,17 @@ __device__ __forceinline__ ExpandArgs select_target(const ExpandArgs &a, int z) 
 
 // Waves per SIMD the register allocator has to leave room for.  The rank-64 variant that reads a finished
 // v sits 2 registers above the 96 that allow 5 waves; held to 5 it measured 1-6 % faster on the prefill and
-// mixed shapes (more workgroups resident per round), at 6 it spills.  The others are left to the compiler.
-constexpr int expand_min_waves(int kb, bool partial) { return (kb == 2 && !partial) ? 5 : 1; }
+// mixed shapes (more workgroups resident per round), at 6 it spills.  The rank-32 one fits 7 (at 5 a 6749-token prefill
+// takes 27.5 instead of 26 us), and the one that sums partials 4.
+constexpr int expand_min_waves(int kb, bool partial, bool comp) {
+  return comp ? 1 : kb == 2 && !partial ? 5 : kb == 1 ? (partial ? 4 : 7) : 1;
+}
 
-template <typename T, int KB, bool PARTIAL>
-__global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL)) void expand_kernel(const int32_t *tiles_base, int h_n_ochunks,
+// COMP: the compensation of a request whose base weights hold another adapter (csrc/api.hip, mlora_lora_compensate):
+// y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), where v' is the "target" 1 matrix of the same positions:
+// both products in one pass over y.
+template <typename T, int KB, bool PARTIAL, bool COMP>
+__global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expand_kernel(const int32_t *tiles_base, int h_n_ochunks,
                                                                                     ExpandArgs args_in) {
   // (tiles_base, h_n_ochunks: what the first dependent load needs, in front so that kernel-argument preloading
   // delivers them in registers)
@@ -61,6 +67,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL)) void expand_ker
   const int a = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
   if (cnt <= 0) return;   // records past the last tile are zero
   const ExpandArgs p = select_target(args_in, blockIdx.y);
+  constexpr int MBU = COMP && KB == 4 ? 1 : EXP_MBU;   // two rank-128 operand sets leave registers for one block
   const int rk = min(r, p.kmax);  // rank columns the narrow operand really has (bgmv_impl.cuh:167,186)
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -76,22 +83,35 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL)) void expand_ker
   const float inv_h_out = 1.0f / (float)p.h_out;
   int64_t brow[4][KB];
   uint32_t boff[4][KB];
+  auto look_up = [&](int rr, int rrk, int64_t rbase, int64_t (&row)[4][KB], uint32_t (&off)[4][KB]) {
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    const int o = o_wave + nb * 16 + lrow;
+    for (int nb = 0; nb < 4; ++nb) {
+      const int o = o_wave + nb * 16 + lrow;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const int j0 = kb * 32 + kg * 8;
-      brow[nb][kb] = -1;
-      boff[nb][kb] = 0;
-      if (o < p.h_out && j0 < rk) {
-        const uint32_t flat = (uint32_t)o * (uint32_t)r + (uint32_t)j0;   // < 2^16 * 2^7
-        uint32_t bin;
-        divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, boff[nb][kb]);
-        const int64_t idx = base + bin;
-        if (idx >= 0 && idx < p.pool.a_loc_len) brow[nb][kb] = p.pool.a_loc[idx];
+      for (int kb = 0; kb < KB; ++kb) {
+        const int j0 = kb * 32 + kg * 8;
+        row[nb][kb] = -1;
+        off[nb][kb] = 0;
+        if (o < p.h_out && j0 < rrk) {
+          const uint32_t flat = (uint32_t)o * (uint32_t)rr + (uint32_t)j0;   // < 2^16 * 2^7
+          uint32_t bin;
+          divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off[nb][kb]);
+          const int64_t idx = rbase + bin;
+          if (idx >= 0 && idx < p.pool.a_loc_len) row[nb][kb] = p.pool.a_loc[idx];
+        }
       }
     }
+  };
+  look_up(r, rk, base, brow, boff);
+  int64_t brow2[COMP ? 4 : 1][COMP ? KB : 1];
+  uint32_t boff2[COMP ? 4 : 1][COMP ? KB : 1];
+  int rk2 = 0;
+  float scale2 = 0.f;
+  if constexpr (COMP) {
+    const int r2 = p.plan[H_MERGED_RANK];
+    rk2 = min(r2, p.kmax);
+    if (r2 > 0) scale2 = -Tr::to_float(p.scales[p.plan[H_MERGED]]);
+    look_up(r2, rk2, (int64_t)p.plan[H_MERGED_START] + (int64_t)r2 * p.slot, brow2, boff2);
   }
   s_perm[tid] = my_perm;
   // The only workgroup-wide barrier: it also drains the loads above (which everything below needs
@@ -100,15 +120,19 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL)) void expand_ker
   __syncthreads();
 
   // B fragments: bfrag[nb][kb] = B^T[o = o_wave + nb*16 + lrow][j0 .. j0+8), j0 = kb*32 + kg*8
-  u32x4 bfrag[4][KB];
+  u32x4 bfrag[4][KB], bfrag2[COMP ? 4 : 1][COMP ? KB : 1];
+  auto load_b = [&](const int64_t (&brw)[4][KB], const uint32_t (&off)[4][KB], u32x4 (&frag)[4][KB]) {
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb)
+    for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const int64_t row = brow[nb][kb];
-      bfrag[nb][kb] = (row >= 0 && row < p.pool.w_rows) ? load16(p.pool.w + row * p.h_out + boff[nb][kb])
-                                                        : u32x4{0, 0, 0, 0};
-    }
+      for (int kb = 0; kb < KB; ++kb) {
+        const int64_t row = brw[nb][kb];
+        frag[nb][kb] = (row >= 0 && row < p.pool.w_rows) ? load16(p.pool.w + row * p.h_out + off[nb][kb])
+                                                          : u32x4{0, 0, 0, 0};
+      }
+  };
+  load_b(brow, boff, bfrag);
+  if constexpr (COMP) load_b(brow2, boff2, bfrag2);
 
   // row-major roles for the y read-modify-write: 8 lanes x 16 B cover one token row of the wave's
   // 64 outputs; a wave covers 8 rows per access, two accesses per 16-token block.
@@ -118,13 +142,13 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL)) void expand_ker
   // Two 16-token blocks per iteration: their y rows and v fragments are all requested before either
   // block is consumed, so an iteration costs one memory round trip for 32 tokens.
   const int n_mb = (cnt + 15) >> 4;
-  for (int mb0 = 0; mb0 < n_mb; mb0 += EXP_MBU) {
-    u32x4 yv[EXP_MBU][2];
-    uint16_t *yp[EXP_MBU][2];
-    bool yok[EXP_MBU][2];
-    u32x4 vfrag[EXP_MBU][KB];
+  for (int mb0 = 0; mb0 < n_mb; mb0 += MBU) {
+    u32x4 yv[MBU][2];
+    uint16_t *yp[MBU][2];
+    bool yok[MBU][2];
+    u32x4 vfrag[MBU][KB], vfrag2[COMP ? MBU : 1][COMP ? KB : 1];
 #pragma unroll
-    for (int b = 0; b < EXP_MBU; ++b) {
+    for (int b = 0; b < MBU; ++b) {
       const int mb = mb0 + b;
       // ---- y rows first (the longest-latency loads of the iteration)
 #pragma unroll
@@ -170,38 +194,46 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL)) void expand_ker
           }
         }
         vfrag[b][kb] = v;
+        if constexpr (COMP)   // the same positions' rows of the merged adapter's matrix
+          vfrag2[b][kb] = (pok && j0 < rk2) ? load16(p.v + p.v_tstride + (int64_t)(pos0 + prow) * p.v_stride + j0)
+                                            : u32x4{0, 0, 0, 0};
       }
     }
 #pragma unroll
-    for (int b = 0; b < EXP_MBU; ++b) {
+    for (int b = 0; b < MBU; ++b) {
       if (mb0 + b < n_mb) {   // workgroup-uniform
-        // ---- delta block through the matrix cores, staged to LDS in token-major order
+        // ---- delta block through the matrix cores, turned through LDS into token-major order and added to the y rows
+        auto add = [&](const u32x4 (&vf)[KB], const u32x4 (&bf)[4][KB], int rkk, float sc, bool last) {
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb) {
-          f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+          for (int nb = 0; nb < 4; ++nb) {
+            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-          for (int kb = 0; kb < KB; ++kb)
-            if (kb * 32 < rk) acc = Tr::mfma(as<vec8>(vfrag[b][kb]), as<vec8>(bfrag[nb][kb]), acc);
+            for (int kb = 0; kb < KB; ++kb)
+              if (kb * 32 < rkk) acc = Tr::mfma(as<vec8>(vf[kb]), as<vec8>(bf[nb][kb]), acc);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) stage[wave][kg * 4 + i][nb * 16 + lrow] = acc[i];
-        }
-        // stage[wave] is private to this wave and a wave's LDS operations execute in order, so only
-        // the compiler has to be kept from reordering the reads below over the writes above.
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          if (yok[b][h]) {
-            const float *srow = &stage[wave][rr0 + 8 * h][c8];
-            float f[8];
-            unpack8<T>(yv[b][h], f);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) f[i] += scale * srow[i];
-            store16(yp[b][h], pack8<T>(f));
+            for (int i = 0; i < 4; ++i) stage[wave][kg * 4 + i][nb * 16 + lrow] = acc[i];
           }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
+          // stage[wave] is private to this wave and a wave's LDS operations execute in order, so only
+          // the compiler has to be kept from reordering the reads below over the writes above.
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            if (yok[b][h]) {
+              const float *srow = &stage[wave][rr0 + 8 * h][c8];
+              float f[8];
+              unpack8<T>(yv[b][h], f);
+#pragma unroll
+              for (int i = 0; i < 8; ++i) f[i] += sc * srow[i];
+              if (last) store16(yp[b][h], pack8<T>(f));
+              else yv[b][h] = pack8<T>(f);
+            }
+          }
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+        };
+        add(vfrag[b], bfrag, rk, scale, !COMP);
+        if constexpr (COMP) add(vfrag2[b], bfrag2, rk2, scale2, true);
       }
     }
   }
@@ -351,21 +383,20 @@ int launch_expand_cols_t(hipStream_t st, const ExpandArgs &a, int kb, dim3 grid,
 
 template <typename T>
 int launch_expand_t(hipStream_t st, const ExpandArgs &a, int kb, dim3 grid) {
+#define MLORA_EXPAND(KB, PARTIAL, COMP)                                                                              \
+  hipLaunchKernelGGL((expand_kernel<T, KB, PARTIAL, COMP>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a)
+#define MLORA_EXPAND_KB(KB)                                                                                          \
+  if (a.compensate) MLORA_EXPAND(KB, false, true);                                                                   \
+  else if (a.partial) MLORA_EXPAND(KB, true, false);                                                                 \
+  else MLORA_EXPAND(KB, false, false)
   switch (kb) {
-    case 1:
-      if (a.partial) hipLaunchKernelGGL((expand_kernel<T, 1, true>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a);
-      else hipLaunchKernelGGL((expand_kernel<T, 1, false>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a);
-      break;
-    case 2:
-      if (a.partial) hipLaunchKernelGGL((expand_kernel<T, 2, true>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a);
-      else hipLaunchKernelGGL((expand_kernel<T, 2, false>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a);
-      break;
-    case 4:
-      if (a.partial) hipLaunchKernelGGL((expand_kernel<T, 4, true>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a);
-      else hipLaunchKernelGGL((expand_kernel<T, 4, false>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a);
-      break;
+    case 1: MLORA_EXPAND_KB(1); break;
+    case 2: MLORA_EXPAND_KB(2); break;
+    case 4: MLORA_EXPAND_KB(4); break;
     default: return fail(MLORA_ERR_NO_KERNEL, "expand: no kernel for %d rank blocks", kb);
   }
+#undef MLORA_EXPAND_KB
+#undef MLORA_EXPAND
   return check_launch("expand_kernel");
 }
 
@@ -381,7 +412,7 @@ int launch_expand(hipStream_t st, const ExpandArgs &a, int max_rank, int64_t gri
   // such as a single 11008 -> 4096 target gets slower, 14.6 -> 16.0 us, and stays as it is)
   const int cl = 2;
   const bool many = grid_tiles * a.n_ochunks * a.n_targets >= 1920;
-  if (bm_expand == 16 && a.n_ochunks >= 2 && (many || a.column_loop)) {
+  if (bm_expand == 16 && a.n_ochunks >= 2 && (many || a.column_loop) && !a.compensate) {
     const int groups = (a.n_ochunks + cl - 1) / cl;
     const int64_t blocks = grid_tiles * groups;
     if (blocks > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "expand: grid too large");

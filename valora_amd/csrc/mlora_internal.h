@@ -25,7 +25,10 @@ constexpr int TILE_WORDS = 8;
 constexpr int32_t PLAN_MAGIC = 0x4d4c5241;
 enum Hdr {
   H_MAGIC = 0, H_T = 1, H_NADAPTERS = 2, H_NTILES_S = 3, H_NTILES_E = 4, H_NGROUPS = 5,
-  H_MAXRANK = 6, H_RESERVED = 7, H_BM_S = 8, H_BM_E = 9, H_NACTIVE = 10
+  H_MAXRANK = 6, H_RESERVED = 7, H_BM_S = 8, H_BM_E = 9, H_NACTIVE = 10,
+  // a compensation plan (mlora_build_compensation_plan): the adapter that is merged into the base weights, whose tokens
+  // are left out of the plan; -1 and rank 0 in any other plan
+  H_MERGED = 11, H_MERGED_RANK = 12, H_MERGED_START = 13
 };
 
 constexpr int64_t MAX_ADAPTERS = 8192;   // per-wave histograms live in LDS
@@ -112,6 +115,7 @@ struct ShrinkArgs {
   int prp;                    // row stride of the partials in that mode: whole 128-byte lines per row
   int n_tiles;                // upper bound of the tile count
   unsigned long long *arrive; // [tiles][MLORA_MAX_TARGETS] arrival words, zero between launches
+  int compensate;             // "target" 1 is the plan's merged adapter over all positions, see csrc/shrink.hip
 };
 
 struct ExpandArgs {
@@ -134,6 +138,7 @@ struct ExpandArgs {
   const uint16_t *scales;
   int T, h_out, kmax, slot, n_ochunks;
   int column_loop;            // force the column-looping kernel for 16-token tiles (tests); else by grid size
+  int compensate;             // every tile takes its own adapter's product minus the merged adapter's (one target)
 };
 
 
@@ -153,7 +158,7 @@ int launch_decode(hipStream_t st, const DecodeArgs &a, int max_rank, mlora_dtype
 int decode_bn(int max_rank);   // output columns per expand item of the one-launch op
 size_t decode_partial_floats(int64_t n_tiles, int n_targets, int ksplit, int64_t rp);
 int launch_plan(hipStream_t st, int32_t *plan, const PlanLayout &L, const int64_t *ids,
-                const int64_t *a_start, const int64_t *a_len, int n_slots, int bm_s, int bm_e);
+                const int64_t *a_start, const int64_t *a_len, int n_slots, int bm_s, int bm_e, int merged);
 size_t scratch_bytes(int64_t T, int64_t max_rank, int ksplit);
 int launch_count_consecutive(hipStream_t st, const int64_t *lora_rank, int64_t n_adapters,
                              const int64_t *indicies, int64_t T, int64_t *output_counts,

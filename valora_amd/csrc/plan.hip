@@ -90,7 +90,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     int32_t *__restrict__ plan, const int64_t *__restrict__ ids, const int64_t *__restrict__ a_start,
     const int64_t *__restrict__ a_len, int T, int A, int n_slots, int bm_s, int bm_e, int W,
     int64_t off_perm, int64_t off_padapter, int64_t off_prank, int64_t off_tiles_s,
-    int64_t off_tiles_e, int64_t off_counters, int64_t off_scratch, int max_tiles, int n_flag_words) {
+    int64_t off_tiles_e, int64_t off_counters, int64_t off_scratch, int max_tiles, int n_flag_words, int merged) {
   constexpr int N_WAVES = THREADS / 64;
   __shared__ int32_t whist[HIST_WORDS];
   __shared__ Quad wsum[PLAN_WAVES + 1];
@@ -115,6 +115,8 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     return (r > 0 && (r & 7) == 0 && r <= MAX_RANK) ? (int)r : 0;
   };
   auto start_of = [&](int a) -> int64_t { return SMALL ? s_astart[a] : a_start[a]; };
+
+  auto start_word = [](int64_t st) -> int32_t { return st < 0 || st > 0x7fffffff ? INT32_MIN / 2 : (int32_t)st; };
 
   // token range of each of the W histogram waves (contiguous, multiple of 64)
   const int cw = (int)align_up((T + W - 1) / W, 64);
@@ -143,7 +145,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   for (int t = t_beg + lane; t < t_end; t += 64) {
     const int64_t a64 = (t < t_beg + 64) ? id0 : ids[t];
     int a = -1, r = 0;
-    if (a64 >= 0 && a64 < A) {
+    if (a64 >= 0 && a64 < A && a64 != merged) {
       r = rank_of((int)a64);
       if (r > 0) {
         a = (int)a64;
@@ -210,7 +212,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
       r = first_r;
     } else if (t < t_end) {
       const int64_t a64 = ids[t];
-      if (a64 >= 0 && a64 < A) {
+      if (a64 >= 0 && a64 < A && a64 != merged) {
         r = rank_of((int)a64);
         if (r > 0) a = (int)a64;
       }
@@ -260,9 +262,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
       // The index has fewer than 2^31 entries (checked on the host), so a start outside 31 bits lies outside the
       // index whatever it is: it becomes a position no look-up accepts, and the adapter's rows are skipped like
       // any other row outside the pool.
-      const bool st_bad = st < 0 || st > 0x7fffffff;
-      const int32_t rec[5] = {a, rank_of(a), gstart[a] + k * bm, min(bm, c - k * bm),
-                              st_bad ? INT32_MIN / 2 : (int32_t)st};
+      const int32_t rec[5] = {a, rank_of(a), gstart[a] + k * bm, min(bm, c - k * bm), start_word(st)};
       for (int list = 0; list < (one_list ? 2 : 1); ++list) {
         int32_t *tl = (list ? plan + off_tiles_e : tiles) + (int64_t)i * TILE_WORDS;
 #pragma unroll
@@ -295,6 +295,9 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     plan[H_BM_S] = bm_s;
     plan[H_BM_E] = bm_e;
     plan[H_NACTIVE] = n_active;
+    plan[H_MERGED] = merged;
+    plan[H_MERGED_RANK] = merged >= 0 ? rank_of(merged) : 0;
+    plan[H_MERGED_START] = merged >= 0 ? start_word(start_of(merged)) : 0;
   }
 }
 
@@ -365,7 +368,7 @@ __global__ void ids_cover_requests_kernel(int64_t *ids_out, const int32_t *b_sta
 }  // namespace
 
 int launch_plan(hipStream_t st, int32_t *plan, const PlanLayout &L, const int64_t *ids,
-                const int64_t *a_start, const int64_t *a_len, int n_slots, int bm_s, int bm_e) {
+                const int64_t *a_start, const int64_t *a_len, int n_slots, int bm_s, int bm_e, int merged) {
   const int A = (int)L.A;
   int W = A > 0 ? (int)(HIST_WORDS / A) : PLAN_WAVES;
   if (W > PLAN_WAVES) W = PLAN_WAVES;
@@ -377,7 +380,7 @@ int launch_plan(hipStream_t st, int32_t *plan, const PlanLayout &L, const int64_
   hipLaunchKernelGGL((plan_kernel<SMALL, THREADS>), dim3(1), dim3(THREADS), 0, st, plan, ids, a_start, a_len,      \
                      (int)L.T, A, n_slots, bm_s, bm_e, W, L.off_perm, L.off_padapter, L.off_prank, L.off_tiles_s,  \
                      L.off_tiles_e, L.off_counters, L.off_scratch, (int)L.max_tiles,                              \
-                     (int)(L.off_scratch - L.off_counters))
+                     (int)(L.off_scratch - L.off_counters), merged)
   if (few) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL);
   else if (A <= PLAN_SMALL_A) MLORA_LAUNCH_PLAN(true, PLAN_THREADS);
   else MLORA_LAUNCH_PLAN(false, PLAN_THREADS);

@@ -30,6 +30,19 @@ __device__ __forceinline__ ShrinkArgs select_target(const ShrinkArgs &a, int z) 
   return p;
 }
 
+// A compensation call (csrc/api.hip, mlora_lora_compensate) multiplies the tokens of a plan by two adapters: each
+// token's own, tile by tile as always, and as a second "target" the one that is merged into the base weights.  The
+// second needs no tile list: its tiles are runs of `bm` positions, whatever adapters their tokens have.
+// (The flag travels beside reduce_here, in a preloaded argument: a load of the argument block in front of the tile's
+// look-ups cost every shrink launch 0.2 us.)
+constexpr int SHRINK_COMPENSATE = 4;
+__device__ __forceinline__ void merged_tile(const int32_t *plan, int tile_idx, int bm, int &r, int &pos0, int &cnt, int &astart) {
+  r = plan[H_MERGED_RANK];
+  astart = plan[H_MERGED_START];
+  pos0 = tile_idx * bm;
+  cnt = r > 0 ? min(bm, plan[H_NACTIVE] - pos0) : 0;
+}
+
 template <typename T>
 __device__ __forceinline__ void store_v(const ShrinkArgs &p, int pos, int t, int r, int col, float v) {
   using Tr = Traits<T>;
@@ -116,7 +129,7 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(ShrinkArgs args_in) 
 #pragma unroll
       for (int u = 0; u < 8; ++u) v += q[u];
     }
-    const int r = prank[pos];
+    const int r = p.compensate && blockIdx.y == 1 ? p.plan[H_MERGED_RANK] : prank[pos];
     const int t = p.out_by_token ? perm[pos] : 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) store_v<T>(p, pos, t, r, 4 * c4 + i, v[i]);
@@ -131,7 +144,8 @@ template <typename T, int MB, int NB>
 __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
                                                      int h_n_tiles, ShrinkArgs args_in) {
   int tile_idx, z_idx, s;
-  if (h_reduce_here) {
+  const bool compensate = (h_reduce_here & SHRINK_COMPENSATE) != 0;
+  if (h_reduce_here & ~SHRINK_COMPENSATE) {
     // The K chunks of a tile are summed by whichever of them finishes last, out of the L2 they share: the id
     // mod 8 selects the XCD, so all chunks (and targets) of a tile get ids that agree mod 8.
     const int per_tile = h_n_targets * h_ksplit;
@@ -157,7 +171,8 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
   __shared__ __align__(16) float s_tile[shrink_lds_floats(NBLK)];
   __shared__ int s_last;
 
-  const int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  if (compensate && z_idx == 1) merged_tile(p.plan, tile_idx, 16 * MB, r, pos0, cnt, astart);
   if (cnt <= 0) return;   // records past the last tile are zero
   const int32_t *__restrict__ perm = p.plan + p.off_perm;
   const int kbeg = s * p.kchunk;
@@ -280,14 +295,15 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
 // later ds_read_b128 of an MFMA operand (16 rows, one chunk column) over the banks.  Two stages
 // are always in flight while the third is consumed; one s_barrier per K step.
 template <typename T, int NB, int MBW>
-__global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int, int,
+__global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_flags, int,
                                                           ShrinkArgs args_in) {
   // workgroup id = (tile * targets + target) * ksplit + K chunk.  The id mod 8 selects the XCD, so
   // with the K chunk as the fast index the tiles of an adapter that share a K chunk of A, and the
   // targets that share a K chunk of x, meet in one L2.
   const int wg_tz = blockIdx.x / h_ksplit;
   const int tile_idx = wg_tz / h_n_targets;
-  const ShrinkArgs p = select_target(args_in, wg_tz - tile_idx * h_n_targets);
+  const int z_idx = wg_tz - tile_idx * h_n_targets;
+  const ShrinkArgs p = select_target(args_in, z_idx);
   const int s = blockIdx.x - wg_tz * h_ksplit;
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
@@ -304,7 +320,8 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
   __shared__ __align__(16) unsigned char s_raw[RING_BYTES > TILE_BYTES ? RING_BYTES : TILE_BYTES];
 
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
-  const int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  if ((h_flags & SHRINK_COMPENSATE) && z_idx == 1) merged_tile(p.plan, tile_idx, 64 * MBW, r, pos0, cnt, astart);
   if (cnt <= 0) return;   // records past the last tile are zero
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -447,15 +464,17 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
   shrink_epilogue<T>(p, otile, NB * 16, s, pos0, cnt, r, perm);
 }
 
+inline int head_flags(const ShrinkArgs &a) { return a.reduce_here | (a.compensate ? SHRINK_COMPENSATE : 0); }
+
 template <typename T, int MBW>
 int launch_gemm_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
   switch (nb) {
-    case 1: hipLaunchKernelGGL((shrink_gemm_kernel<T, 1, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a); break;
-    case 2: hipLaunchKernelGGL((shrink_gemm_kernel<T, 2, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a); break;
-    case 4: hipLaunchKernelGGL((shrink_gemm_kernel<T, 4, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a); break;
+    case 1: hipLaunchKernelGGL((shrink_gemm_kernel<T, 1, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
+    case 2: hipLaunchKernelGGL((shrink_gemm_kernel<T, 2, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
+    case 4: hipLaunchKernelGGL((shrink_gemm_kernel<T, 4, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
     case 8:
       if constexpr (MBW <= 2) {
-        hipLaunchKernelGGL((shrink_gemm_kernel<T, 8, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a);
+        hipLaunchKernelGGL((shrink_gemm_kernel<T, 8, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a);
         break;
       }
       return fail(MLORA_ERR_NO_KERNEL, "shrink: rank > 64 has no 256-token tile");
@@ -467,10 +486,10 @@ int launch_gemm_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
 template <typename T, int MB>
 int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
   switch (nb) {
-    case 1: hipLaunchKernelGGL((shrink_kernel<T, MB, 1>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a); break;
-    case 2: hipLaunchKernelGGL((shrink_kernel<T, MB, 2>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a); break;
-    case 4: hipLaunchKernelGGL((shrink_kernel<T, MB, 4>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a); break;
-    case 8: hipLaunchKernelGGL((shrink_kernel<T, (MB > 2 ? 2 : MB), 8>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, a.reduce_here, a.n_tiles, a); break;
+    case 1: hipLaunchKernelGGL((shrink_kernel<T, MB, 1>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
+    case 2: hipLaunchKernelGGL((shrink_kernel<T, MB, 2>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
+    case 4: hipLaunchKernelGGL((shrink_kernel<T, MB, 4>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
+    case 8: hipLaunchKernelGGL((shrink_kernel<T, (MB > 2 ? 2 : MB), 8>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
     default: return fail(MLORA_ERR_NO_KERNEL, "shrink: no kernel for rank blocks=%d", nb);
   }
   return check_launch("shrink_kernel");

@@ -10,8 +10,8 @@ The reference densifies the adapter out of the pool (lora_single_batch_infer.py:
 here one launch of ``libmlora.so`` reads the pool rows in place and updates the four weights, each
 weight element read once and written once.  For the compensation the reference duplicates the
 activations (``cat([x, x])``), runs shrink and expand over ``own adapter | merged adapter`` and adds
-``first half - second half``; here the same tokens go through two planned LoRA ops, the second with
-negated scales, without copies.
+``first half - second half``; here one shrink launch multiplies the same tokens by both adapters and one expand
+launch adds the difference, without copies.
 """
 from __future__ import annotations
 
@@ -70,13 +70,9 @@ class DeLoraPlan:
 
     def __init__(self, ids: torch.Tensor, merged_idx: int, a_start: torch.Tensor, a_len: torch.Tensor,
                  max_rank: int, hidden: int, n_slots: int = 4, **kw):
-        other = (ids != merged_idx) & (ids >= 0) & (ids < a_start.numel())
-        minus_one = torch.full_like(ids, -1)
-        self.own = LoraPlan(torch.where(other, ids, minus_one), a_start, a_len, max_rank, hidden=hidden,
-                            n_slots=n_slots, **kw)
-        self.merged = LoraPlan(torch.where(other, torch.full_like(ids, merged_idx), minus_one), a_start, a_len,
-                               max_rank, hidden=hidden, n_slots=n_slots, **kw)
+        # one plan of the tokens of every other adapter; the merged one's tokens are left out when the tiles are cut
+        self.plan = LoraPlan(ids, a_start, a_len, max_rank, hidden=hidden, n_slots=n_slots, _merged=int(merged_idx), **kw)
 
     def apply(self, y, x, key_buffer, value_buffer, a_start, a_len, a_loc, slot, scales) -> None:
-        self.own.apply(y, x, key_buffer, value_buffer, a_start, a_len, a_loc, slot, scales)
-        self.merged.apply(y, x, key_buffer, value_buffer, a_start, a_len, a_loc, slot, -scales)
+        """``y[t] += scale_own * (x[t] @ A_own.T) @ B_own - scale_merged * (x[t] @ A_merged.T) @ B_merged``."""
+        self.plan._native.compensate(y, x, key_buffer, value_buffer, a_start, a_len, a_loc, slot, scales)

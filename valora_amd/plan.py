@@ -25,7 +25,7 @@ class LoraPlan:
                  bm_expand: Optional[int] = None, ksplit: Optional[int] = None,
                  reduce_in_expand: Optional[bool] = None, one_launch: Optional[bool] = None,
                  one_launch_no_wait: bool = False, shrink_recompute: bool = False, expand_column_loop: bool = False,
-                 one_launch_never_ready: bool = False):
+                 one_launch_never_ready: bool = False, _merged: int = -1):
         """``ids``: int64 per-token adapter index (negative = no adapter); ``a_start`` / ``a_len``:
         the pool index (``a_len = n_slots * rank``); ``max_rank``: widest rank among the resident
         adapters (the reference's ``max_lora_dim``, lora_unordered_batch_infer.py:181-182).
@@ -66,7 +66,7 @@ class LoraPlan:
             self.flags |= _lib.EXPAND_COLUMN_LOOP
         # plan, scratch and the calls themselves live on the native side (csrc/binding.cpp)
         self._native = _b.NativePlan(ids, a_start, a_len, self.max_rank, n_slots, self.bm_shrink, self.bm_expand,
-                                     self.ksplit, self.flags)
+                                     self.ksplit, self.flags, int(_merged))
 
     @property
     def buf(self) -> torch.Tensor:
