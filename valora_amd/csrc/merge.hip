@@ -70,8 +70,9 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
   const int lrow = lane & 15, kg = lane >> 4;
   const int o_wave = oc * MG_BN + wave * 64;
 
+  // ranks are at most 128, so a usable length fits 32 bits (a 64-bit division would cost the set-up some 0.2 us)
   const int64_t alen = p.a_len[p.adapter];
-  const int r = (int)(alen / p.n_slots_pool);
+  const int r = alen > 0 && alen < (1 << 20) ? (int)((uint32_t)alen / (uint32_t)p.n_slots_pool) : 0;
   if (r <= 0 || (r & 7) || r > KB * 32) return;      // same adapters the LoRA op accepts
   const int64_t base = p.a_start[p.adapter] + (int64_t)r * slot;
 
@@ -88,14 +89,32 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
   const int ac = tid / CHUNKS, aic = tid - ac * CHUNKS;
   const int row0 = itile * p.chunks * MG_BM;
   const int n_rows = min(p.chunks * MG_BM, p.h_in - row0);        // of this workgroup
-  int arow[8];
+  // All look-ups in one round trip: those with nothing to look up read entry 0 (the host has checked that there is one).
+  int64_t alook[8], blook[KB][4];
+  uint32_t boff[KB][4];
+  bool aok[8], bok[KB][4];
 #pragma unroll
   for (int jj = 0; jj < 8; ++jj) {
     const int64_t ai = base + ac * 8 + jj;
-    const bool ok = ac * 8 + jj < r && ai >= 0 && ai < p.pa.a_loc_len;
-    const int64_t row = ok ? p.pa.a_loc[ai] : -1;
-    arow[jj] = row >= 0 && row < p.pa.w_rows ? (int)row : -1;     // pool rows fit 31 bits (checked on the host)
+    aok[jj] = ac * 8 + jj < r && ai >= 0 && ai < p.pa.a_loc_len;
+    alook[jj] = p.pa.a_loc[aok[jj] ? ai : 0];
   }
+#pragma unroll
+  for (int q = 0; q < KB; ++q)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      uint32_t flat, bin;
+      bok[q][i] = b_unit<KB>(q, i, lane, (uint32_t)r, flat);
+      flat += (uint32_t)o_wave * (uint32_t)r;                     // < 2^16 * 2^7
+      divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, boff[q][i]);
+      const int64_t idx = base + bin;
+      bok[q][i] = bok[q][i] && flat < (uint32_t)p.h_out * (uint32_t)r && idx >= 0 && idx < p.pb.a_loc_len;
+      blook[q][i] = p.pb.a_loc[bok[q][i] ? idx : 0];
+    }
+  int arow[8];
+#pragma unroll
+  for (int jj = 0; jj < 8; ++jj)   // pool rows fit 31 bits (checked on the host)
+    arow[jj] = aok[jj] && alook[jj] >= 0 && alook[jj] < p.pa.w_rows ? (int)alook[jj] : -1;
   u32x4 ablk[8];
   auto load_a = [&](int il0) {
     const int il = il0 + aic * 8;
@@ -104,26 +123,17 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
       ablk[jj] = (arow[jj] >= 0 && il < n_rows) ? load16(p.pa.w + (int64_t)arow[jj] * p.h_in + row0 + il)
                                                 : u32x4{0, 0, 0, 0};
   };
-  constexpr bool A_FIRST = KB != 2;
-  if constexpr (A_FIRST) load_a(0);
-
-  // ---- B fragments, scaled and rounded to T: bfrag[nb][kb] = T(B^T[o][j0..j0+8) * scaling)
+  // ---- B units, then B fragments, scaled and rounded to T: bfrag[nb][kb] = T(B^T[o][j0..j0+8) * scaling)
   u32x4 braw[KB][4], bfrag[4][KB];
 #pragma unroll
   for (int q = 0; q < KB; ++q)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      braw[q][i] = u32x4{0, 0, 0, 0};
-      uint32_t flat, bin, off;
-      const bool ok = b_unit<KB>(q, i, lane, (uint32_t)r, flat);
-      flat += (uint32_t)o_wave * (uint32_t)r;                     // < 2^16 * 2^7
-      divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off);
-      const int64_t idx = base + bin;
-      if (ok && flat < (uint32_t)p.h_out * (uint32_t)r && idx >= 0 && idx < p.pb.a_loc_len) {
-        const int64_t row = p.pb.a_loc[idx];
-        if (row >= 0 && row < p.pb.w_rows) braw[q][i] = load16(p.pb.w + row * p.h_out + off);
-      }
+      const bool ok = bok[q][i] && blook[q][i] >= 0 && blook[q][i] < p.pb.w_rows;
+      braw[q][i] = ok ? load16(p.pb.w + blook[q][i] * p.h_out + boff[q][i]) : u32x4{0, 0, 0, 0};
     }
+  constexpr bool A_FIRST = KB != 2;
+  if constexpr (A_FIRST) load_a(0);
   static_assert(sizeof(stage) / 4 >= B_TURN_BYTES, "a wave's staging tile holds its turn");
   b_turn<KB>(braw, bfrag, (uint32_t)r, r, lane, reinterpret_cast<unsigned char *>(&stage[wave][0][0]));
 #pragma unroll
@@ -155,6 +165,7 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
       }
   };
   if constexpr (merge_ahead(KB)) load_w(0);
+#pragma unroll 1
   for (int ch = 0; ch * MG_BM < n_rows; ++ch) {
     // ---- the [r x MG_BM] slice of A into LDS, transposed (rank rows beyond r are zero); the swizzle spreads the
     // units of neighbouring threads over the banks
@@ -172,6 +183,7 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
     }
     __syncthreads();
 
+#pragma unroll 1
     for (int rb0 = 0; rb0 < MG_BM / 16; rb0 += 2) {
       if constexpr (!merge_ahead(KB)) load_w(ch * MG_BM + rb0 * 16);
       u32x4 cur[2][2];
@@ -270,6 +282,7 @@ extern "C" int mlora_merge_adapter(void *stream, void *const *w, const int32_t *
     a.w[i] = static_cast<uint16_t *>(w[k]);
     a.slots[i] = slots[k];
   }
+  if (pool_a->a_loc_len < 1 || pool_b->a_loc_len < 1) return MLORA_OK;  // no rows to merge; the kernel reads entry 0
   a.ld = ld;
   a.pa = PoolDev{static_cast<const uint16_t *>(pool_a->w), pool_a->w_rows, pool_a->a_loc, pool_a->a_loc_len};
   a.pb = PoolDev{static_cast<const uint16_t *>(pool_b->w), pool_b->w_rows, pool_b->a_loc, pool_b->a_loc_len};
