@@ -294,6 +294,12 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
 // lane that fills 16-byte chunk c of row R fetches global chunk c ^ (R & 7), which spreads the
 // later ds_read_b128 of an MFMA operand (16 rows, one chunk column) over the banks.  Two stages
 // are always in flight while the third is consumed; one s_barrier per K step.
+//
+// Bound by what a compute unit takes in (x from HBM, A once per tile from L2: 33 GB/s measured with plain loads of this
+// pattern) and, on top, by what stands between a barrier and the step's loads: masks, votes and dummy loads per
+// instruction, which whole steps do without.  With that and both halves' LDS reads ahead of the products: 7600-token
+// prefill over 24 adapters of rank 32 (4 layers, shrink and expand) 739 -> 712 us, 5401 tokens of mixed ranks (two
+// layers, seven projections) 789 -> 760, 5254 tokens of rank 64 778 -> 766.
 template <typename T, int NB, int MBW>
 __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_flags, int,
                                                           ShrinkArgs args_in) {
@@ -340,7 +346,7 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
   for (int g = 0; g < XBLK; ++g) {
     const int row = wrow0 + g * 8 + grow;
     xok[g] = row < cnt;
-    const int t = xok[g] ? perm[pos0 + row] : 0;
+    const int t = perm[pos0 + (xok[g] ? row : 0)];       // (a row past the tile's end reads the first one's)
     xp[g] = p.x + (int64_t)t * p.h_in + gchunk * 8;
   }
   // A groups this wave loads: slot = wave*APW + i -> rows slot*8 .. slot*8+7 of the rank
@@ -355,7 +361,7 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
     const int64_t prow = ok ? p.pool.a_loc[idx] : 0;
     ok = ok && prow >= 0 && prow < p.pool.w_rows;
     aok[i] = ok;
-    ap[i] = p.pool.w + (ok ? prow : 0) * p.h_in + gchunk * 8;
+    ap[i] = ok ? p.pool.w + prow * p.h_in + gchunk * 8 : xp[0];   // (nothing to read: an address that is always there)
   }
 
   const int kbeg = s * p.kchunk;
@@ -382,9 +388,21 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
   };
   auto issue = [&](int step) {
     const int stage = step % STAGES;
-    const int k = kbeg + step * KC + gchunk * 8;        // first K element of this lane's chunk
-    const bool kok = k < kend;
     unsigned char *sbase = s_raw + stage * STAGE_BYTES;
+    const int off = kbeg + step * KC;
+    if (off + KC <= kend) {
+      // whole steps, all but the last one of a K that is not a multiple of 64: every lane reads, rows that do not exist
+      // somebody else's (their results are never stored), so a load is an address and an instruction
+#pragma unroll
+      for (int g = 0; g < XBLK; ++g)
+        __builtin_amdgcn_global_load_lds(GLOBAL_PTR(xp[g] + off), LDS_PTR(sbase + x_off + g * 1024), 16, 0, 0);
+#pragma unroll
+      for (int i = 0; i < APW; ++i)
+        __builtin_amdgcn_global_load_lds(GLOBAL_PTR(ap[i] + off), LDS_PTR(sbase + a_off + (wave * APW + i) * 1024), 16, 0, 0);
+      return;
+    }
+    const int k = off + gchunk * 8;                     // first K element of this lane's chunk
+    const bool kok = k < kend;
 #pragma unroll
     for (int g = 0; g < XBLK; ++g) {
       unsigned char *dst = sbase + x_off + g * 1024;
@@ -421,16 +439,22 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
     if (step + 2 < n_steps) issue(step + 2);
     const int stage = step % STAGES;
     if (wave_active) {
+      // both halves' operands are requested before the first half is used
+      u32x4 xfs[KS][MBW], bfs[KS][NB];
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
-        u32x4 xf[MBW], bf[NB];
 #pragma unroll
         for (int mb = 0; mb < MBW; ++mb)
-          xf[mb] = lds_read16(ring + stage * STAGE_BYTES + x_off + frag_off(mb * 16 + lrow, ks));
+          xfs[ks][mb] = lds_read16(ring + stage * STAGE_BYTES + x_off + frag_off(mb * 16 + lrow, ks));
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
-          bf[nb] = lds_read16(ring + stage * STAGE_BYTES + a_off + frag_off(nb * 16 + lrow, ks));
-        wait_lgkmcnt0();
+          bfs[ks][nb] = lds_read16(ring + stage * STAGE_BYTES + a_off + frag_off(nb * 16 + lrow, ks));
+      }
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        if (ks + 1 < KS) wait_lgkmcnt<MBW + NB>(); else wait_lgkmcnt<0>();
+        u32x4 (&xf)[MBW] = xfs[ks];
+        u32x4 (&bf)[NB] = bfs[ks];
 #pragma unroll
         for (int mb = 0; mb < MBW; ++mb) pin(xf[mb]);
 #pragma unroll
