@@ -108,32 +108,31 @@ __device__ __forceinline__ void shrink_epilogue(const ShrinkArgs &p, const float
 }
 
 // v[row, :] = T(sum_s partial[s][row][:]) for every row that has an adapter; one thread per four
-// columns, every chunk requested before any is consumed.  Bound by its round trips, so nothing waits for anything else:
-// how many rows have an adapter and what rank they have is requested together with the partials (rows beyond are read,
-// the buffer holds T of them, and dropped), and the four columns leave in one store.
+// columns, every chunk requested before any is consumed.
 template <typename T>
 __global__ __launch_bounds__(256) void shrink_reduce_kernel(ShrinkArgs args_in) {
   const ShrinkArgs p = select_target(args_in, blockIdx.y);
-  const uint32_t quarter = (uint32_t)p.rp >> 2;
-  const uint32_t total = (uint32_t)p.T * quarter;        // at most 2^22 * 2^5
+  const int n_active = p.plan[H_NACTIVE];
+  const int quarter = p.rp >> 2;
+  const int64_t total = (int64_t)n_active * quarter;
   const int32_t *__restrict__ perm = p.plan + p.off_perm;
   const int32_t *__restrict__ prank = p.plan + p.off_prank;
-  const f32x4 *__restrict__ src = reinterpret_cast<const f32x4 *>(p.partial);
-  for (uint32_t e = blockIdx.x * 256u + threadIdx.x; e < total; e += gridDim.x * 256u) {
-    const int pos = (int)(e / quarter), c4 = (int)(e - (uint32_t)pos * quarter);
-    const int n_active = p.plan[H_NACTIVE];
-    const int r = p.compensate && blockIdx.y == 1 ? p.plan[H_MERGED_RANK] : prank[pos];
-    const int t = p.out_by_token ? perm[pos] : 0;
+  const int64_t sstride = (int64_t)p.T * quarter;
+  const f32x4 *src = reinterpret_cast<const f32x4 *>(p.partial);
+  for (int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x; e < total; e += (int64_t)gridDim.x * 256) {
+    const int pos = (int)(e / quarter), c4 = (int)(e - (int64_t)pos * quarter);
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     for (int s0 = 0; s0 < p.ksplit; s0 += 8) {
       f32x4 q[8];
 #pragma unroll
-      for (int u = 0; u < 8; ++u)
-        q[u] = (s0 + u < p.ksplit) ? src[(int64_t)(s0 + u) * total + e] : f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int u = 0; u < 8; ++u) q[u] = (s0 + u < p.ksplit) ? src[(s0 + u) * sstride + e] : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int u = 0; u < 8; ++u) v += q[u];
     }
-    if (pos < n_active) store_v4<T>(p, pos, t, r, c4, v);
+    const int r = p.compensate && blockIdx.y == 1 ? p.plan[H_MERGED_RANK] : prank[pos];
+    const int t = p.out_by_token ? perm[pos] : 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) store_v<T>(p, pos, t, r, 4 * c4 + i, v[i]);
   }
 }
 
