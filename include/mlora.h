@@ -229,7 +229,8 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
 
 /* ---- one adapter merged into the base weights ("deLoRA") ------------------------------------- */
 /* A plan of the tokens of every adapter but `merged` (-1 or an index outside the pool: of every token, as
- * mlora_build_plan), for mlora_lora_compensate.                                                */
+ * mlora_build_plan), for mlora_lora_compensate.  A token whose own adapter has no usable rank (0, not a multiple
+ * of 8, above 128) belongs to it: the merged adapter is taken off it and nothing is added.          */
 int mlora_build_compensation_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T,
                                   const int64_t *a_start, const int64_t *a_len, int64_t n_adapters,
                                   int32_t n_slots, int32_t bm_shrink, int32_t bm_expand, int64_t merged);

@@ -179,6 +179,41 @@ def test_compensation_shapes(dev, ranks, T, kw, dtype):
             assert torch.equal(y.cpu()[same], y0[same])
 
 
+@pytest.mark.parametrize("T,kw", [
+    (1, {}), (33, {}), (300, dict(bm_shrink=16, ksplit=1, bm_expand=16)), (300, dict(bm_shrink=32, ksplit=4, bm_expand=32)),
+    (517, dict(bm_shrink=64, ksplit=2, bm_expand=96)), (700, dict(bm_shrink=128, ksplit=4, bm_expand=128)),
+    (1300, dict(bm_shrink=256, ksplit=2, bm_expand=256)), (90, dict(bm_shrink=16, ksplit=4, bm_expand=16, shrink_recompute=True))])
+def test_compensation_of_unusable_own_ranks(dev, T, kw):
+    """A token whose own adapter has no usable rank (0, not a multiple of 8, above 128) has no product of its own, and the
+    merged adapter comes off it all the same; its scale is not looked at.  With a merged adapter that has no usable rank
+    such a token is left alone."""
+    g = torch.Generator().manual_seed(T)
+    h_in, h_out, dtype = 520, 392, torch.float16
+    ranks = [32, 8, 16, 8, 64]
+    pool = W.make_pool(ranks, h_in, h_out, dtype, g, True, std=0.05, heads=1, scalings=[0.5 + 0.25 * i for i in range(len(ranks))])
+    a_len, usable = pool.a_len.clone(), pool.a_len.clone()
+    for a, rank in ((1, 0), (2, 12), (3, 136)):
+        a_len[a], usable[a] = 4 * rank, 0
+    scales = pool.a_scaling.clone()
+    scales[1:4] = torch.tensor([float("nan"), float("inf"), 2.0])
+    pd = pool.to(dev)
+    idx = (pd.a_start, a_len.to(dev), pd.a_loc)
+    x, y0 = torch.randn(T, h_in, generator=g).to(dtype), torch.randn(T, h_out, generator=g).to(dtype)
+    ids = torch.randint(-1, len(ranks), (T,), generator=g)
+    ids[0] = 1
+    for merged in (0, 4, 1, 2):
+        plan = DeLoraPlan(ids.to(dev), merged, idx[0], idx[1], 64, hidden=h_in, **kw)
+        y = y0.to(dev)
+        plan.apply(y, x.to(dev), pd.key_buffer, pd.value_buffer, *idx, 2, scales.to(dev))
+        want = O.delora_compensate(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, usable, pool.a_loc, ids, merged, 2,
+                                   scales)
+        assert_parity(y.cpu(), want, f"T {T} merged {merged}")
+        same = (ids == merged) | (ids < 0)
+        if merged in (1, 2):
+            same |= (ids >= 1) & (ids <= 3)
+        assert torch.equal(y.cpu()[same], y0[same])
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_merge_random_shapes(dev, seed):
     """Non-square weights, widths that are multiples of 8 only, 1-5 pool slots, any subset of slots,

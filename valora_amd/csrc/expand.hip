@@ -64,7 +64,8 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
   const int tile_idx = blockIdx.x / h_n_ochunks;
   const int oc = blockIdx.x - tile_idx * h_n_ochunks;
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
-  const int a = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  const int a = tile[0], r = tile[1], pos0 = tile[2], astart = tile[4];
+  const int cnt = COMP ? abs(tile[3]) : tile[3];   // (negative: no usable rank of its own, r = 0)
   if (cnt <= 0) return;   // records past the last tile are zero
   const ExpandArgs p = select_target(args_in, blockIdx.y);
   constexpr int MBU = COMP && KB == 4 ? 1 : EXP_MBU;   // two rank-128 operand sets leave registers for one block
@@ -232,7 +233,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           __builtin_amdgcn_wave_barrier();
         };
-        add(vfrag[b], bfrag, rk, scale, !COMP);
+        if (!COMP || rk > 0) add(vfrag[b], bfrag, rk, scale, !COMP);
         if constexpr (COMP) add(vfrag2[b], bfrag2, rk2, scale2, true);
       }
     }

@@ -15,7 +15,9 @@ namespace mlora {
 // perm[p]     token index at sorted position p (tokens grouped by adapter, original order kept
 //             inside a group); positions >= hdr[H_NACTIVE] are unused
 // padapter[p] adapter of position p;  prank[p] its rank
-// tile        {adapter, rank, first position, token count, a_start[adapter], 0, 0, 0}
+// tile        {adapter, rank, first position, token count, a_start[adapter], 0, 0, 0}; in a compensation plan the tile of
+//             an adapter without a usable rank has rank 0 and its token count with a minus sign: the kernels leave it as
+//             they leave an empty record, but for the compensating expand, which takes the merged adapter off its tokens
 // done, stamps  the hand-off words of the one-launch op (csrc/decode.hip): per tile a word that numbers the launches
 //             on this plan, and one stamp per shrink item; zeroed by the plan kernel
 // arrive      the arrival words of the shrink's own split-K sum (csrc/shrink.hip): one 64-bit word per tile and
@@ -27,7 +29,7 @@ enum Hdr {
   H_MAGIC = 0, H_T = 1, H_NADAPTERS = 2, H_NTILES_S = 3, H_NTILES_E = 4, H_NGROUPS = 5,
   H_MAXRANK = 6, H_RESERVED = 7, H_BM_S = 8, H_BM_E = 9, H_NACTIVE = 10,
   // a compensation plan (mlora_build_compensation_plan): the adapter that is merged into the base weights, whose tokens
-  // are left out of the plan; -1 and rank 0 in any other plan
+  // are left out of the plan (those of every other adapter are in it, whatever its rank); -1 and rank 0 in any other plan
   H_MERGED = 11, H_MERGED_RANK = 12, H_MERGED_START = 13
 };
 

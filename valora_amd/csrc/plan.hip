@@ -115,6 +115,14 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     return (r > 0 && (r & 7) == 0 && r <= MAX_RANK) ? (int)r : 0;
   };
   auto start_of = [&](int a) -> int64_t { return SMALL ? s_astart[a] : a_start[a]; };
+  // A token's adapter, -1 where the plan leaves the token out, and the adapter's usable rank.  A compensation plan keeps
+  // the tokens of adapters without a usable rank: they have no product of their own, but the merged one comes off them.
+  auto adapter_of = [&](int64_t a64, int &r) -> int {
+    r = 0;
+    if (a64 < 0 || a64 >= A || a64 == merged) return -1;
+    r = rank_of((int)a64);
+    return r > 0 || (merged >= 0 && rank_of(merged) > 0) ? (int)a64 : -1;
+  };
 
   auto start_word = [](int64_t st) -> int32_t { return st < 0 || st > 0x7fffffff ? INT32_MIN / 2 : (int32_t)st; };
 
@@ -144,14 +152,9 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   int first_a = -1, first_r = 0;
   for (int t = t_beg + lane; t < t_end; t += 64) {
     const int64_t a64 = (t < t_beg + 64) ? id0 : ids[t];
-    int a = -1, r = 0;
-    if (a64 >= 0 && a64 < A && a64 != merged) {
-      r = rank_of((int)a64);
-      if (r > 0) {
-        a = (int)a64;
-        atomicAdd(&whist[wave * A + a], 1);
-      }
-    }
+    int r;
+    const int a = adapter_of(a64, r);
+    if (a >= 0) atomicAdd(&whist[wave * A + a], 1);
     if (t < t_beg + 64) { first_a = a; first_r = r; }
   }
   __syncthreads();
@@ -211,11 +214,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
       a = first_a;
       r = first_r;
     } else if (t < t_end) {
-      const int64_t a64 = ids[t];
-      if (a64 >= 0 && a64 < A && a64 != merged) {
-        r = rank_of((int)a64);
-        if (r > 0) a = (int)a64;
-      }
+      a = adapter_of(ids[t], r);
     }
     // Lanes holding the same adapter get consecutive positions in lane order.  Which lanes hold my adapter comes from
     // one vote per bit of the adapter index (6 votes for 64 adapters), whatever the mix: one adapter for all 64 tokens
@@ -262,7 +261,9 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
       // The index has fewer than 2^31 entries (checked on the host), so a start outside 31 bits lies outside the
       // index whatever it is: it becomes a position no look-up accepts, and the adapter's rows are skipped like
       // any other row outside the pool.
-      const int32_t rec[5] = {a, rank_of(a), gstart[a] + k * bm, min(bm, c - k * bm), start_word(st)};
+      // (no usable rank, compensation plans only: the count is negative, so whoever has no use for the tile leaves)
+      const int r = rank_of(a), n = min(bm, c - k * bm);
+      const int32_t rec[5] = {a, r, gstart[a] + k * bm, r > 0 ? n : -n, start_word(st)};
       for (int list = 0; list < (one_list ? 2 : 1); ++list) {
         int32_t *tl = (list ? plan + off_tiles_e : tiles) + (int64_t)i * TILE_WORDS;
 #pragma unroll
