@@ -130,8 +130,8 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(ShrinkArgs args_in) 
       for (int u = 0; u < 8; ++u) v += q[u];
     }
     const int r = p.compensate && blockIdx.y == 1 ? p.plan[H_MERGED_RANK] : prank[pos];
-    if (r <= 0) continue;   // a token without a product (compensation plans): nothing was computed, nothing is read
     const int t = p.out_by_token ? perm[pos] : 0;
+    if (r <= 0) continue;   // a token without a product (compensation plans): nothing was computed, nothing is read
 #pragma unroll
     for (int i = 0; i < 4; ++i) store_v<T>(p, pos, t, r, 4 * c4 + i, v[i]);
   }
