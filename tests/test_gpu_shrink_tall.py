@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import lora_oracle as O
-from valora_amd import workloads as W
+from valora_amd import _lib, workloads as W
 from valora_amd.plan import LoraPlan
 from tests._util import assert_parity
 
@@ -33,3 +33,54 @@ def test_k_steps_and_rows(dev, h_in, bm, rank):
         y = y0.to(dev)
         plan.apply(y, x.to(dev), pd.key_buffer, pd.value_buffer, *idx, 1, pd.a_scaling)
         assert_parity(y.cpu(), want, f"h_in={h_in} bm={bm} rank={rank} ks={ks}")
+
+
+@pytest.mark.parametrize("bm,rank", [(16, 32), (64, 64), (128, 8), (128, 16), (128, 32), (128, 64), (128, 128), (256, 16),
+                                     (256, 32), (256, 64)])
+@pytest.mark.parametrize("h_in", [72, 512])
+def test_rows_outside_the_pool(dev, h_in, bm, rank):
+    """Rank rows whose index entry names no pool row, or that lie beyond the index, count as rows of zeros in every tile
+    height: their columns of v are zero and their part of B is skipped."""
+    g = torch.Generator().manual_seed(h_in + 10 * bm + rank)
+    dtype = torch.bfloat16 if rank == 64 else torch.float16
+    T, slot = 2 * bm + 7, 1
+    pool = W.make_pool([rank, rank, rank], h_in, 64, dtype, g, True, std=0.05, heads=1, extra_rows=1)
+    n_rows = pool.key_buffer.shape[0]
+    # the last pool row stands for "no row": zeros for the oracle, out of the pool's bounds for the op
+    pool.key_buffer[-1], pool.value_buffer[-1] = 0, 0
+    spare = n_rows - 1
+    taken = torch.where(pool.a_loc == spare)[0]
+    free = next(r for r in range(n_rows) if r not in set(pool.a_loc.tolist()))
+    pool.a_loc[taken] = free
+    seen, given = pool.a_loc.clone(), pool.a_loc.clone()
+    first = [int(s) + rank * slot for s in pool.a_start]
+    for k, bad in enumerate((-1, n_rows, 1 << 40, -(1 << 40))):
+        for at in (first[0] + (3 * k) % rank, first[1] + rank - 1 - k):
+            seen[at], given[at] = spare, bad
+    cut = first[2] + rank // 2                   # the last adapter's rows from here on lie beyond the index
+    seen[cut:] = spare
+    given = given[:cut].contiguous()
+    ids = torch.randint(-1, 3, (T,), generator=g)
+    x, y0 = torch.randn(T, h_in, generator=g).to(dtype), torch.randn(T, 64, generator=g).to(dtype)
+    v0 = torch.zeros(T, rank, dtype=dtype)
+    want_v = O.bgmv_shrink(v0, x, pool.key_buffer, pool.a_start, pool.a_len, seen, ids, slot)
+    want = O.bgmv_expand(y0, want_v, pool.value_buffer, pool.a_start, pool.a_len, seen, ids, slot, pool.a_scaling)
+    pd = pool.to(dev)
+    kb, vb = pd.key_buffer[:spare], pd.value_buffer[:spare]
+    loc, xd = given.to(dev), x.to(dev)
+    none = want_v == 0
+    for ks in (1, 2):
+        plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, rank, hidden=h_in, bm_shrink=bm, bm_expand=32, ksplit=ks,
+                        reduce_in_expand=False, one_launch=False)
+        y = y0.to(dev)
+        plan.apply(y, xd, kb, vb, pd.a_start, pd.a_len, loc, slot, pd.a_scaling)
+        assert_parity(y.cpu(), want, f"h_in={h_in} bm={bm} rank={rank} ks={ks}")
+        # the same tiles through the entry point that hands v out
+        v = v0.to(dev)
+        pa = _lib.make_pool(kb, pd.a_start, pd.a_len, loc, h_in)
+        _lib.check(_lib.lib().mlora_shrink(_lib.current_stream(dev), plan.handle, _lib.ptr(plan.scratch), plan.scratch.numel(),
+                                           _lib.ptr(xd), T, h_in, rank, pa, slot, ks, _lib.ptr(v), rank, 0, 0, 0,
+                                           _lib.dtype_code(dtype)))
+        v = v.cpu()
+        assert not v[none].any(), f"bm={bm} rank={rank} ks={ks}: a row outside the pool has a product"
+        assert_parity(v, want_v, f"v h_in={h_in} bm={bm} rank={rank} ks={ks}")

@@ -283,6 +283,9 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
     if (on[it]) store_v4<T>(p, pos0 + row[it], tok[it], r, c4[it], v[it]);
 }
 
+// What a rank row that is not there reads, K step after K step (one 128-byte line).
+__device__ const __align__(128) uint16_t g_zero_line[64] = {};
+
 // Prefill-sized tiles (128 tokens): GEMM structure with a three-stage LDS ring.
 //
 // The four waves split the tile's tokens (32 each), so no cross-wave reduction is needed.  Both
@@ -353,6 +356,7 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
   // A groups this wave loads: slot = wave*APW + i -> rows slot*8 .. slot*8+7 of the rank
   const uint16_t *ap[APW];
   bool aok[APW];
+  int astep[APW];                                       // all bits: the row moves on with K; none: it stays on its line
 #pragma unroll
   for (int i = 0; i < APW; ++i) {
     const int slot = (wave * APW + i) % ABLK;           // surplus slots duplicate real groups
@@ -362,7 +366,9 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
     const int64_t prow = ok ? p.pool.a_loc[idx] : 0;
     ok = ok && prow >= 0 && prow < p.pool.w_rows;
     aok[i] = ok;
-    ap[i] = ok ? p.pool.w + prow * p.h_in + gchunk * 8 : xp[0];   // (nothing to read: an address that is always there)
+    // a row past the rank, or outside the index or the pool, reads zeros
+    ap[i] = (ok ? p.pool.w + prow * p.h_in : g_zero_line) + gchunk * 8;
+    astep[i] = ok ? -1 : 0;
   }
 
   const int kbeg = s * p.kchunk;
@@ -378,7 +384,8 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
   // Issue every load of one K step: EXACTLY LOADS_PER_STAGE load instructions per wave, because the
   // consumer waits with a compile-time vmcnt.  A load whose lanes are all masked off would be skipped
   // by the hardware branch around it, so in that case a dummy load into a scratch block is issued
-  // instead.  Lanes beyond the end of K write zeros into their own slot (no other lane touches it).
+  // instead.  Lanes beyond the end of K, and those of rank rows that are not there, write zeros into their own slot (no
+  // other lane touches it).
   unsigned char *dummy = s_raw + STAGES * STAGE_BYTES;
   auto load_or_dummy = [&](bool c, const uint16_t *src, unsigned char *dst) {
     if (__builtin_amdgcn_ballot_w64(c) != 0ull) {
@@ -392,14 +399,15 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
     unsigned char *sbase = s_raw + stage * STAGE_BYTES;
     const int off = kbeg + step * KC;
     if (off + KC <= kend) {
-      // whole steps, all but the last one of a K that is not a multiple of 64: every lane reads, rows that do not exist
-      // somebody else's (their results are never stored), so a load is an address and an instruction
+      // whole steps, all but the last one of a K that is not a multiple of 64: every lane reads, x rows past the tile's end
+      // the first one's (their results are never stored) and rank rows that are not there the line of zeros, so a load is
+      // an address and an instruction
 #pragma unroll
       for (int g = 0; g < XBLK; ++g)
         __builtin_amdgcn_global_load_lds(GLOBAL_PTR(xp[g] + off), LDS_PTR(sbase + x_off + g * 1024), 16, 0, 0);
 #pragma unroll
       for (int i = 0; i < APW; ++i)
-        __builtin_amdgcn_global_load_lds(GLOBAL_PTR(ap[i] + off), LDS_PTR(sbase + a_off + (wave * APW + i) * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(GLOBAL_PTR(ap[i] + (off & astep[i])), LDS_PTR(sbase + a_off + (wave * APW + i) * 1024), 16, 0, 0);
       return;
     }
     const int k = off + gchunk * 8;                     // first K element of this lane's chunk
@@ -414,7 +422,7 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
     for (int i = 0; i < APW; ++i) {
       unsigned char *dst = sbase + a_off + (wave * APW + i) * 1024;
       load_or_dummy(aok[i] && kok, ap[i] + kbeg + step * KC, dst);
-      if (!kok) lds_write16(lds_offset(dst) + lane * 16, zero4);
+      if (!(aok[i] && kok)) lds_write16(lds_offset(dst) + lane * 16, zero4);
     }
   };
   // where the MFMA operand (row R of a region, K block ks) of this lane sits inside a stage
