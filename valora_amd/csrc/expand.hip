@@ -245,13 +245,14 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 // most of it the look-up chain in front of the loads, and run in three rounds.  Here a workgroup walks over `h_cl`
 // consecutive column chunks of one tile: tile record, token ids, the slot's pool rows (kept in LDS, so a chunk's B
 // addresses need no further look-up) and the v fragment are fetched once, then every chunk is one round trip (B
-// fragments and y rows requested together), and the grid is a quarter of the size.  Same arithmetic in the same
+// fragments and y rows requested together), and the grid is half the size.  Same arithmetic in the same
 // order as expand_kernel: same bits.
 template <typename T, int KB, bool PARTIAL>
-__global__ __launch_bounds__(256) void expand_cols_kernel(const int32_t *tiles_base, int h_groups, int h_cl,
-                                                          ExpandArgs args_in) {
+__global__ __launch_bounds__(256, KB == 1 ? 8 : 1) void expand_cols_kernel(const int32_t *tiles_base, int h_groups,
+                                                                                    int h_cl, ExpandArgs args_in) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
+  constexpr bool WIDER = KB * 32 < MAX_RANK;   // an adapter's rank may be above what the narrow operand holds
   __shared__ float stage[4][16][STAGE_LD];
   __shared__ int32_t s_perm[16];
   __shared__ int32_t s_row[MAX_RANK];
@@ -310,15 +311,17 @@ __global__ __launch_bounds__(256) void expand_cols_kernel(const int32_t *tiles_b
     if (o_wave >= p.h_out) break;   // wave-uniform
     // ---- B units and y rows of this chunk, all requested before any is consumed
     u32x4 braw[KB][4], bfrag[4][KB];
+    uint32_t b_own = b_lane<KB, WIDER>(lane, (uint32_t)r);
+    // (from here on: the units' shares kept from one chunk to the next would cost registers, and with them a workgroup)
+    asm volatile("" : "+v"(b_own));
 #pragma unroll
     for (int q = 0; q < KB; ++q)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         braw[q][i] = u32x4{0, 0, 0, 0};
-        if (b_any<KB>(i, (uint32_t)r)) {
+        if (b_any<KB, WIDER>(i, (uint32_t)r)) {
           uint32_t flat, bin, off;
-          bool ok = b_unit<KB>(q, i, lane, (uint32_t)r, flat);
-          flat += (uint32_t)o_wave * (uint32_t)r;               // < 2^16 * 2^7
+          const bool ok = b_unit<KB, WIDER>(q, i, lane, b_own, (uint32_t)r, (uint32_t)o_wave * (uint32_t)r, flat);   // < 2^16 * 2^7
           divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off);
           const int row = ok && bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;   // bins from r on hold -1
           if (row >= 0) braw[q][i] = load16(p.pool.w + (int64_t)row * p.h_out + off);
@@ -335,7 +338,7 @@ __global__ __launch_bounds__(256) void expand_cols_kernel(const int32_t *tiles_b
       yp[h] = p.y + (int64_t)t * p.h_out + o_wave + c8;
       yv[h] = yok[h] ? load16(yp[h]) : u32x4{0, 0, 0, 0};
     }
-    b_turn<KB>(braw, bfrag, (uint32_t)r, rk, lane, turn);
+    b_turn<KB, WIDER>(braw, bfrag, (uint32_t)r, rk, lane, turn);
     // ---- delta block through the matrix cores, staged to LDS in token-major order
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {

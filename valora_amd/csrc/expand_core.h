@@ -21,31 +21,50 @@ constexpr int B_OUTS = 64;           // outputs per wave
 
 __device__ __forceinline__ uint32_t b_swizzle(uint32_t q) { return q ^ (((q >> 3) ^ (q >> 6)) & 7u); }
 
+// Units an output has in the turn.  KB is the class of the narrow operand (up to 32 * KB columns), r the adapter's rank.
+// WIDER: r may be above the class.  What lies beyond the class meets no column of the operand: it is neither loaded nor
+// turned, so that a pass has at most 256 units whatever the rank.
+template <int KB, bool WIDER>
+__device__ __forceinline__ constexpr uint32_t b_rank_units(uint32_t r) {
+  return WIDER && r > 32u * KB ? 4u * KB : r >> 3;
+}
+static_assert(B_OUTS * 4 * 16 <= B_TURN_BYTES, "a pass, B_OUTS / KB outputs of up to 4 * KB units, fits the turn");
+
 // A wave's B operands are turned in KB passes of B_OUTS / KB outputs, up to 4 instructions (256 units) each.
-// The flat element a lane's unit i of pass p starts at, relative to the wave's first output; false: no such unit.
-template <int KB>
-__device__ __forceinline__ bool b_unit(int p, int i, int lane, uint32_t r, uint32_t &flat) {
+// A lane's own part of the flat element its units start at.
+template <int KB, bool WIDER>
+__device__ __forceinline__ uint32_t b_lane(int lane, uint32_t r) {
+  // (outputs of more units than the class uses lie apart)
+  return (uint32_t)lane * 8u + (WIDER ? (uint32_t)lane / (4u * KB) * (r - 8u * b_rank_units<KB, WIDER>(r)) : 0u);
+}
+// The flat element a lane's unit i of pass p starts at, `own` from b_lane, `first` that of the wave's first output; false:
+// no such unit.
+template <int KB, bool WIDER>
+__device__ __forceinline__ bool b_unit(int p, int i, int lane, uint32_t own, uint32_t r, uint32_t first, uint32_t &flat) {
   constexpr uint32_t OUTS = B_OUTS / KB;
-  const uint32_t q = (uint32_t)(i * 64 + lane);
-  flat = (uint32_t)p * OUTS * r + q * 8u;
-  return q < OUTS * (r >> 3);
+  const uint32_t units = b_rank_units<KB, WIDER>(r);
+  flat = first + (uint32_t)p * OUTS * r + (uint32_t)i * (512u + (WIDER ? 16u / KB * (r - 8u * units) : 0u)) + own;
+  return (uint32_t)(i * 64 + lane) < OUTS * units;
 }
 // wave-uniform: whether instruction i of a pass has any unit
-template <int KB>
-__device__ __forceinline__ bool b_any(int i, uint32_t r) { return (uint32_t)(i * 64) < (B_OUTS / KB) * (r >> 3); }
+template <int KB, bool WIDER>
+__device__ __forceinline__ bool b_any(int i, uint32_t r) {
+  return (uint32_t)(i * 64) < (B_OUTS / KB) * b_rank_units<KB, WIDER>(r);
+}
 
-// raw[p][i] as loaded -> bfrag[nb][kb] = B^T[o = nb*16 + lane%16][kb*32 + (lane/16)*8 .. + 8), zero from rank rk on.
+// raw[p][i] as loaded -> bfrag[nb][kb] = B^T[o = nb*16 + lane%16][kb*32 + (lane/16)*8 .. + 8), zero from rank rk on
+// (rk <= r, rk <= 32 * KB).
 // `turn`: B_TURN_BYTES of LDS of this wave.
-template <int KB>
+template <int KB, bool WIDER>
 __device__ __forceinline__ void b_turn(const u32x4 (&raw)[KB][4], u32x4 (&bfrag)[4][KB], uint32_t r, int rk, int lane,
                                        unsigned char *turn) {
-  const uint32_t rq = r >> 3;
+  const uint32_t rq = b_rank_units<KB, WIDER>(r);
   const int lrow = lane & 15, kg = lane >> 4;
 #pragma unroll
   for (int p = 0; p < KB; ++p) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (b_any<KB>(i, r)) *reinterpret_cast<u32x4 *>(turn + b_swizzle((uint32_t)(i * 64 + lane)) * 16u) = raw[p][i];
+      if (b_any<KB, WIDER>(i, r)) *reinterpret_cast<u32x4 *>(turn + b_swizzle((uint32_t)(i * 64 + lane)) * 16u) = raw[p][i];
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
 #pragma unroll
