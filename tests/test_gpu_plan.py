@@ -91,3 +91,48 @@ def test_count_consecutive_bit_exact(dev, T, style):
     assert P == len(want[0])
     for got, w in zip((oc, rc, li, st), want):
         assert got.dtype == torch.long and got[:P].cpu().tolist() == w
+
+
+def test_planned_calls_give_the_interpreter_lock_back(dev):
+    """With a switch interval no test outlasts, a thread that waits for the interpreter lock only gets it where the
+    thread that holds it gives it back of its own accord.  Every planned call does, around its launches."""
+    import sys
+    import threading
+    import time
+    from valora_amd import workloads as W
+    from valora_amd.merge import DeLoraPlan
+    from valora_amd.plan import LoraPlan
+    g = torch.Generator().manual_seed(1)
+    pool = W.make_pool([8, 8], 64, 64, torch.float16, g, True, heads=1).to(dev)
+    idx = (pool.a_start, pool.a_len, pool.a_loc)
+    ids = torch.zeros(4, dtype=torch.long, device=dev)
+    x, y, z = (torch.zeros(4, 64, dtype=torch.float16, device=dev) for _ in range(3))
+    plan, de = LoraPlan(ids, idx[0], idx[1], 8, hidden=64), DeLoraPlan(ids, 1, idx[0], idx[1], 8, hidden=64)
+    kb, vb, sc = pool.key_buffer, pool.value_buffer, pool.a_scaling
+    calls = {"apply": lambda: plan.apply(y, x, kb, vb, *idx, 0, sc),
+             "apply_multi": lambda: plan.apply_multi([y, z], x, kb, vb, *idx, [0, 1], sc),
+             "compensate": lambda: de.apply(y, x, kb, vb, *idx, 0, sc), "rebuild": lambda: plan.rebuild(ids)}
+    turns, stop = [0], threading.Event()
+
+    def other():
+        while not stop.is_set():
+            turns[0] += 1
+            time.sleep(0)
+
+    thread = threading.Thread(target=other)
+    was = sys.getswitchinterval()
+    sys.setswitchinterval(1000.0)
+    try:
+        thread.start()
+        seen = {}
+        for name, call in calls.items():
+            before = turns[0]
+            for _ in range(200):
+                call()
+            seen[name] = turns[0] - before
+    finally:
+        stop.set()
+        sys.setswitchinterval(was)
+        thread.join()
+    torch.cuda.synchronize()
+    assert all(n > 0 for n in seen.values()), seen

@@ -500,6 +500,18 @@ void lora_get_qkvo_fwd_expand(const at::Tensor &x, const at::Tensor &w, const at
 // What a LoraPlan holds on the native side: the plan, the index tensors it was cut from and the scratch of its calls.
 // A call checks its operands and goes straight to the C ABI.  Through ctypes a call cost 9-12 us of host time, more than
 // the GPU needs for a small decode batch (7 us); here it is the argument conversion plus the launches.
+// The C calls run without the interpreter lock (a launch waits where the device's queue is full, and other Python threads
+// go on meanwhile), on copies of what another thread's rebuild may replace.
+template <typename F>
+void check_unlocked(F call) {
+  int rc;
+  {
+    py::gil_scoped_release unlocked;
+    rc = call();
+  }
+  check_rc(rc);   // (the message belongs to this thread)
+}
+
 struct NativePlan {
   mlora_plan plan{};
   at::Tensor buf, scratch, ids, a_start, a_len;
@@ -535,10 +547,16 @@ struct NativePlan {
         raise("rebuild takes " + std::to_string(T) + " int64 ids on " + ids.device().str());
       ids = new_ids->contiguous();
     }
-    check_rc(mlora_build_compensation_plan(stream(), &plan, static_cast<const int64_t *>(ids.data_ptr()), T,
+    const at::Tensor now = ids;
+    const hipStream_t st = stream();
+    mlora_plan cut = plan;
+    check_unlocked([&] {
+      return mlora_build_compensation_plan(st, &cut, static_cast<const int64_t *>(now.data_ptr()), T,
                                            static_cast<const int64_t *>(a_start.data_ptr()),
                                            static_cast<const int64_t *>(a_len.data_ptr()), a_start.numel(), n_slots,
-                                           bm_shrink, bm_expand, merged));
+                                           bm_shrink, bm_expand, merged);
+    });
+    plan = cut;
   }
 
   mlora_pool pool(const at::Tensor &w, const at::Tensor &start, const at::Tensor &len, const at::Tensor &loc,
@@ -580,8 +598,12 @@ struct NativePlan {
     at::Tensor keep;
     const void *sc = scales_ptr(scales, x, keep);
     const mlora_pool pa = pool(key_buffer, start, len, loc, h_in), pb = pool(value_buffer, start, len, loc, h_out);
-    check_rc(op(stream(), &plan, scratch.data_ptr(), (size_t)scratch.numel(), y.data_ptr(), x.data_ptr(), T, h_in, h_out,
-                max_rank, &pa, &pb, (int32_t)slot, sc, ksplit, flags, code));
+    const mlora_plan held = plan;
+    const hipStream_t st = stream();
+    check_unlocked([&] {
+      return op(st, &held, scratch.data_ptr(), (size_t)scratch.numel(), y.data_ptr(), x.data_ptr(), T, h_in, h_out, max_rank,
+                &pa, &pb, (int32_t)slot, sc, ksplit, flags, code);
+    });
   }
 
   void apply_multi(const std::vector<at::Tensor> &ys, const at::Tensor &x, const at::Tensor &key_buffer,
@@ -615,8 +637,12 @@ struct NativePlan {
     at::Tensor keep;
     const void *sc = scales_ptr(scales, x, keep);
     const mlora_pool pa = pool(key_buffer, start, len, loc, h_in);
-    check_rc(mlora_lora_apply_multi(stream(), &plan, scratch.data_ptr(), (size_t)scratch.numel(), x.data_ptr(), T, h_in,
-                                    h_out, max_rank, &pa, (int32_t)n, tg, sc, ksplit, flags, code));
+    const mlora_plan held = plan;
+    const hipStream_t st = stream();
+    check_unlocked([&] {
+      return mlora_lora_apply_multi(st, &held, scratch.data_ptr(), (size_t)scratch.numel(), x.data_ptr(), T, h_in, h_out,
+                                    max_rank, &pa, (int32_t)n, tg, sc, ksplit, flags, code);
+    });
   }
 };
 
