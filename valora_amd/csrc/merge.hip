@@ -83,7 +83,9 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
   const float inv_h_out = 1.0f / (float)p.h_out;
   // ---- a thread's 8 x 8 block of an A slice: rank rows 8 * ac .. + 8, 16 bytes of input columns from 8 * aic on.
   // Neighbouring threads take neighbouring chunks of the same rank rows: whole lines.  The first slice's block is
-  // requested before anything waits for B, where the registers are there (rank 64 would spill).
+  // requested before anything waits for B where the registers are there: above rank 64, with two workgroups resident.
+  // (Below, with four, it spills: at ranks up to 32 without it 3072 wide 273 -> 270 us, 4096 wide 409 -> 405 for eight
+  // calls of four slots.)
   constexpr int CHUNKS = MG_BM / 8;
   static_assert(CHUNKS * UNITS <= 256, "one block per thread");
   const int ac = tid / CHUNKS, aic = tid - ac * CHUNKS;
@@ -132,7 +134,7 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
       const bool ok = bok[q][i] && blook[q][i] >= 0 && blook[q][i] < p.pb.w_rows;
       braw[q][i] = ok ? load16(p.pb.w + blook[q][i] * p.h_out + boff[q][i]) : u32x4{0, 0, 0, 0};
     }
-  constexpr bool A_FIRST = KB != 2;
+  constexpr bool A_FIRST = merge_resident(KB) <= 2;
   if constexpr (A_FIRST) load_a(0);
   static_assert(sizeof(stage) / 4 >= B_TURN_BYTES, "a wave's staging tile holds its turn");
   b_turn<KB, false>(braw, bfrag, (uint32_t)r, r, lane, reinterpret_cast<unsigned char *>(&stage[wave][0][0]));
