@@ -149,6 +149,30 @@ def test_install_aliases_registers_the_reference_import_names():
                 sys.modules[n] = m
 
 
+def test_pools_of_more_rows_than_31_bits_hold_are_refused_before_any_launch():
+    """The kernels keep pool rows and index positions in 31 bits: every entry point says so on the host.  (The pointers
+    name no memory; a call that got past its checks would fail at the launch with another status.)"""
+    import ctypes
+    L, big, some = _lib.lib(), 1 << 31, ctypes.c_void_p(4096)
+
+    def pool(w_rows=64, a_loc_len=64):
+        return _lib.Pool(some, w_rows, some, some, some, 2, a_loc_len, 4)
+
+    ws, slots = (ctypes.c_void_p * 1)(4096), (ctypes.c_int32 * 1)(0)
+    for pa, pb in ((pool(w_rows=big), pool()), (pool(), pool(w_rows=big)), (pool(a_loc_len=big), pool()),
+                   (pool(), pool(a_loc_len=big))):
+        assert L.mlora_merge_adapter(None, ws, slots, 1, 64, 64, 64, pa, pb, 0, 8, 1.0, 1, 0) == -2
+    plan = _lib.Plan(some, 1 << 20, 16, 2, 16, 16, 4)
+    tg = (_lib.Target * 2)(_lib.Target(some, some, 64, 0), _lib.Target(ctypes.c_void_p(8192), some, big, 1))
+    for flags in (0, _lib.ONE_LAUNCH):
+        assert L.mlora_lora_apply_multi(None, plan, some, 1 << 20, some, 16, 64, 64, 8, pool(), 2, tg, some, 2, flags, 0) == -2
+    for pa, pb in ((pool(w_rows=big), pool()), (pool(), pool(w_rows=big))):
+        assert L.mlora_lora_compensate(None, plan, some, 1 << 20, some, some, 16, 64, 64, 8, pa, pb, 0, some, 2, 0, 0) == -2
+        assert L.mlora_lora_apply(None, plan, some, 1 << 20, some, some, 16, 64, 64, 8, pa, pb, 0, some, 2, _lib.ONE_LAUNCH, 0) == -2
+    assert L.mlora_shrink(None, plan, some, 1 << 20, some, 16, 64, 8, pool(w_rows=big), 0, 1, None, 0, 0, 0, 0, 0) == -2
+    assert L.mlora_expand(None, plan, some, 16, 64, some, None, 0, 8, pool(w_rows=big), 0, some, 1, 0, 0) == -2
+
+
 C_PROGRAM = r"""
 #include <stdio.h>
 #include <string.h>

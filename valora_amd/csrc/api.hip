@@ -422,6 +422,8 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   for (int i = 0; i < n_targets; ++i) {
     if (!targets[i].y || !targets[i].w_b || !aligned16(targets[i].y) || !aligned16(targets[i].w_b))
       return fail(MLORA_ERR_INVALID, "lora_apply_multi: target %d has a null or misaligned pointer", i);
+    if (targets[i].w_b_rows > 0x7fffffff)
+      return fail(MLORA_ERR_NO_KERNEL, "lora_apply_multi: target %d has more than 2^31 - 1 pool rows", i);
     if (targets[i].slot < 0 || targets[i].slot >= pool_a->n_slots)
       return fail(MLORA_ERR_INVALID, "lora_apply_multi: target %d slot %d outside [0,%d)", i, targets[i].slot, pool_a->n_slots);
     for (int j = 0; j < i; ++j)

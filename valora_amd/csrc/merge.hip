@@ -271,6 +271,9 @@ extern "C" int mlora_merge_adapter(void *stream, void *const *w, const int32_t *
   if (adapter < 0 || adapter >= pool_a->n_adapters || pool_a->n_adapters != pool_b->n_adapters)
     return fail(MLORA_ERR_INVALID, "merge_adapter: adapter %lld outside [0,%lld)", (long long)adapter,
                 (long long)pool_a->n_adapters);
+  // (the kernel keeps pool rows in 31 bits)
+  if (pool_a->a_loc_len > 0x7fffffff || pool_a->w_rows > 0x7fffffff || pool_b->a_loc_len > 0x7fffffff || pool_b->w_rows > 0x7fffffff)
+    return fail(MLORA_ERR_NO_KERNEL, "merge_adapter: more than 2^31 - 1 index entries or pool rows");
   if (sign != 1 && sign != -1) return fail(MLORA_ERR_INVALID, "merge_adapter: sign must be +1 or -1");
   if (!pool_a->w || !pool_b->w || !pool_a->a_start || !pool_a->a_len || !pool_a->a_loc || !aligned16(pool_a->w) ||
       !aligned16(pool_b->w))
