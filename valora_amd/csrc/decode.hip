@@ -135,7 +135,7 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
   constexpr int TILE_FLOATS = shrink_lds_floats(NB);   // shrink_tile_to_lds
   constexpr int VACC_FLOATS = 16 * NB * 16;         // a tile's summed chunks (give-up path)
   constexpr int BUF_FLOATS = TILE_FLOATS + VACC_FLOATS > STAGE_FLOATS ? TILE_FLOATS + VACC_FLOATS : STAGE_FLOATS;
-  static_assert(DECODE_MAX_PRODUCERS == 16, "stamps_match reads 16 stamps");
+  static_assert(DECODE_MAX_PRODUCERS == 16, "stamps_state reads 16 stamps");
   __shared__ __align__(16) float s_buf[BUF_FLOATS];   // a shrink item's tile, an expand item's staging tile
   __shared__ int32_t s_perm[16];
   __shared__ int32_t s_ready;

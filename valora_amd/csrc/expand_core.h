@@ -1,5 +1,5 @@
-// Operand handling of the expand kernels.
-//
+// Operands in lane order: the B fragments and the summed split-K partials, loaded as whole lines and turned through LDS.
+// Used by the column-looping expand (csrc/expand.hip) and, for B, by the merge (csrc/merge.hip).
 #pragma once
 
 #include "kernel_common.h"

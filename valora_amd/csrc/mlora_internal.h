@@ -117,7 +117,8 @@ struct ShrinkArgs {
   int prp;                    // row stride of the partials in that mode: whole 128-byte lines per row
   int n_tiles;                // upper bound of the tile count
   unsigned long long *arrive; // [tiles][MLORA_MAX_TARGETS] arrival words, zero between launches
-  int compensate;             // "target" 1 is the plan's merged adapter over all positions, see csrc/shrink.hip
+  int compensate;             // "target" 1 is the plan's merged adapter over all positions (host side: the kernels get a
+                              // flag in their leading arguments, csrc/shrink.hip)
 };
 
 struct ExpandArgs {

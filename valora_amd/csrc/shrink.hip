@@ -33,8 +33,8 @@ __device__ __forceinline__ ShrinkArgs select_target(const ShrinkArgs &a, int z) 
 // A compensation call (csrc/api.hip, mlora_lora_compensate) multiplies the tokens of a plan by two adapters: each
 // token's own, tile by tile as always, and as a second "target" the one that is merged into the base weights.  The
 // second needs no tile list: its tiles are runs of `bm` positions, whatever adapters their tokens have.
-// (The flag travels beside reduce_here, in a preloaded argument: a load of the argument block in front of the tile's
-// look-ups cost every shrink launch 0.2 us.)
+// (The kernels take the flag from a leading argument, beside reduce_here: a load of the argument block in front of the
+// tile's look-ups cost every shrink launch 0.2 us.)
 constexpr int SHRINK_COMPENSATE = 4;
 __device__ __forceinline__ void merged_tile(const int32_t *plan, int tile_idx, int bm, int &r, int &pos0, int &cnt, int &astart) {
   r = plan[H_MERGED_RANK];
@@ -110,8 +110,9 @@ __device__ __forceinline__ void shrink_epilogue(const ShrinkArgs &p, const float
 // v[row, :] = T(sum_s partial[s][row][:]) for every row that has an adapter; one thread per four
 // columns, every chunk requested before any is consumed.
 template <typename T>
-__global__ __launch_bounds__(256) void shrink_reduce_kernel(ShrinkArgs args_in) {
+__global__ __launch_bounds__(256) void shrink_reduce_kernel(int h_flags, ShrinkArgs args_in) {
   const ShrinkArgs p = select_target(args_in, blockIdx.y);
+  const bool merged = (h_flags & SHRINK_COMPENSATE) && blockIdx.y == 1;
   const int n_active = p.plan[H_NACTIVE];
   const int quarter = p.rp >> 2;
   const int64_t total = (int64_t)n_active * quarter;
@@ -129,7 +130,7 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(ShrinkArgs args_in) 
 #pragma unroll
       for (int u = 0; u < 8; ++u) v += q[u];
     }
-    const int r = p.compensate && blockIdx.y == 1 ? p.plan[H_MERGED_RANK] : prank[pos];
+    const int r = merged ? p.plan[H_MERGED_RANK] : prank[pos];
     const int t = p.out_by_token ? perm[pos] : 0;
     if (r <= 0) continue;   // a token without a product (compensation plans): nothing was computed, nothing is read
 #pragma unroll
@@ -548,9 +549,9 @@ int launch_shrink_reduce(hipStream_t st, const ShrinkArgs &a, mlora_dtype dt) {
   if (blocks > 2048) blocks = 2048;
   if (blocks < 1) blocks = 1;
   if (dt == MLORA_F16)
-    hipLaunchKernelGGL(shrink_reduce_kernel<_Float16>, dim3((unsigned)blocks, (unsigned)a.n_targets), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(shrink_reduce_kernel<_Float16>, dim3((unsigned)blocks, (unsigned)a.n_targets), dim3(256), 0, st, head_flags(a), a);
   else
-    hipLaunchKernelGGL(shrink_reduce_kernel<__bf16>, dim3((unsigned)blocks, (unsigned)a.n_targets), dim3(256), 0, st, a);
+    hipLaunchKernelGGL(shrink_reduce_kernel<__bf16>, dim3((unsigned)blocks, (unsigned)a.n_targets), dim3(256), 0, st, head_flags(a), a);
   return check_launch("shrink_reduce_kernel");
 }
 
