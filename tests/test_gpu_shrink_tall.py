@@ -84,3 +84,32 @@ def test_rows_outside_the_pool(dev, h_in, bm, rank):
         v = v.cpu()
         assert not v[none].any(), f"bm={bm} rank={rank} ks={ks}: a row outside the pool has a product"
         assert_parity(v, want_v, f"v h_in={h_in} bm={bm} rank={rank} ks={ks}")
+
+
+@pytest.mark.parametrize("bm,rank", [(128, 8), (128, 32), (128, 64), (128, 128), (256, 16), (256, 64)])
+@pytest.mark.parametrize("h_in", [8, 64, 72, 192, 1032, 4096])
+def test_k_steps_same_bits(dev, h_in, bm, rank):
+    """Small integers: every product and sum is exact in any order (at most 4096 * 8 < 2^24), so v has one right value per
+    element and the tall tiles must give it bit for bit, whole steps and masked ones, as the 16-token tiles do."""
+    g = torch.Generator().manual_seed(h_in + bm + rank)
+    dtype = torch.bfloat16 if rank == 64 else torch.float16
+    lens = [1, 8, 31, 33, bm - 1, bm, bm + 1]
+    ids = torch.repeat_interleave(torch.arange(len(lens)), torch.tensor(lens))
+    ids = ids[torch.randperm(ids.numel(), generator=g)]
+    T = ids.numel()
+    pool = W.make_pool([rank if i % 3 else 8 for i in range(len(lens))], h_in, 64, dtype, g, True, heads=1)
+    pool.key_buffer.copy_(torch.randint(-2, 3, pool.key_buffer.shape, generator=g))
+    x = torch.randint(-4, 5, (T, h_in), generator=g).to(dtype)
+    v0 = torch.full((T, rank), 0.5, dtype=dtype)
+    want = O.bgmv_shrink(v0, x, pool.key_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 2)
+    pd, xd = pool.to(dev), x.to(dev)
+    pa = _lib.make_pool(pd.key_buffer, pd.a_start, pd.a_len, pd.a_loc, h_in)
+    for tile in (bm, 16):
+        for ks in (1, 3):
+            plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, rank, hidden=h_in, bm_shrink=tile, bm_expand=32, ksplit=ks,
+                            reduce_in_expand=False, one_launch=False)
+            v = v0.to(dev)
+            _lib.check(_lib.lib().mlora_shrink(_lib.current_stream(dev), plan.handle, _lib.ptr(plan.scratch),
+                                               plan.scratch.numel(), _lib.ptr(xd), T, h_in, rank, pa, 2, ks, _lib.ptr(v), rank,
+                                               0, 0, 0, _lib.dtype_code(dtype)))
+            assert torch.equal(v.cpu(), want), f"tile {tile} ks {ks}"
