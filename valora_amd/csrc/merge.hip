@@ -20,8 +20,9 @@
 // Bound by the in-place update of W (268 MB for four 4096 x 4096 slots; an in-place stream runs at 4.4-4.9 TB/s on
 // this part) up to rank 32, above that also by the operands a workgroup reads beside its share of W: B once per
 // workgroup (in lane order, expand_core.h), A once per 256 columns.  Measured, four 4096 x 4096 slots of bf16 weights,
-// before / after transposing A once instead of at every use, reading B in lane order and for several slices, and
-// rounding to bf16 in hardware: rank 16 65.9 / 59 us, rank 64 88.3 / 65, rank 128 129.9 / 81.
+// before / after transposing A once instead of at every use, reading B in lane order and for several slices, all
+// look-ups in one round trip, and rounding to bf16 in hardware: rank 16 63.7 / 56.5 us, rank 64 82.6 / 59.0, rank 128
+// 126.4 / 68.8.
 #include "expand_core.h"
 #include "kernel_common.h"
 
@@ -33,10 +34,7 @@ constexpr int MG_BN = 256;        // output columns per workgroup, 64 per wave
 // input rows (of W) per slice of A in LDS (16 KB up to rank 64, 32 KB above)
 constexpr int merge_bm(int kb) { return kb == 1 ? 256 : 128; }
 // Workgroups resident per compute unit: four up to rank 64, two above (the B fragments of rank 128 take 64 registers).
-// Two do not keep enough of W in flight by themselves, so there the rows of W are requested an iteration ahead
-// (rank 128 85 -> 81 us; with four workgroups the extra registers cost a workgroup and 3-6 us).
 constexpr int merge_resident(int kb) { return kb == 4 ? 2 : 4; }
-constexpr bool merge_ahead(int kb) { return kb == 4; }
 constexpr int MG_STAGE_LD = 64 + 4;
 
 struct MergeArgs {
@@ -166,7 +164,6 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
         wv[b][h] = (ocol_ok && il < n_rows) ? load16(wbase + (int64_t)il * p.ld) : u32x4{0, 0, 0, 0};
       }
   };
-  if constexpr (merge_ahead(KB)) load_w(0);
 #pragma unroll 1
   for (int ch = 0; ch * MG_BM < n_rows; ++ch) {
     // ---- the [r x MG_BM] slice of A into LDS, transposed (rank rows beyond r are zero); the swizzle spreads the
@@ -187,13 +184,7 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
 
 #pragma unroll 1
     for (int rb0 = 0; rb0 < MG_BM / 16; rb0 += 2) {
-      if constexpr (!merge_ahead(KB)) load_w(ch * MG_BM + rb0 * 16);
-      u32x4 cur[2][2];
-#pragma unroll
-      for (int b = 0; b < 2; ++b)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) cur[b][h] = wv[b][h];
-      if constexpr (merge_ahead(KB)) load_w(ch * MG_BM + (rb0 + 2) * 16);
+      load_w(ch * MG_BM + rb0 * 16);
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
         // A^T fragment: row = input row (lrow), 8 consecutive rank elements
@@ -218,7 +209,7 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
           if (ocol_ok && il < n_rows) {
             const float *srow = &stage[wave][rr0 + 8 * h][c8];
             float f[8];
-            unpack8<T>(cur[b][h], f);
+            unpack8<T>(wv[b][h], f);
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
               const float ab = Tr::to_float(Tr::from_float(srow[k]));   // the GEMM result is a T tensor
@@ -305,7 +296,8 @@ extern "C" int mlora_merge_adapter(void *stream, void *const *w, const int32_t *
   const int bm = merge_bm(kb);
   // Slices per workgroup.  The grid takes so many rounds of what the device holds, each as long as a workgroup's slices
   // and its set-up, which with the B fragments of rank 64 and more costs about one slice more (rank 128, 4096 wide: one
-  // slice 108 us, two 90, four 78; 3072 wide: 74, 72, three 58).  Up to rank 32 one slice is always fastest.
+  // slice 85.6 us, two 73.6, four 68.8; 3072 wide: 59.8, 62.8, three 51.1, four 59.1; rank 64, 4096 wide: 66.3, two 59.0,
+  // four 64.0).  Up to rank 32 one slice is always fastest (rank 16, 4096 wide: 56.5, two 59.8).
   const int64_t slices = (h_in + bm - 1) / bm, per_slice = (int64_t)a.n_ochunks * n_targets;
   const int64_t resident = (int64_t)merge_resident(kb) * 256;
   auto cost = [&](int64_t c) { return ((slices + c - 1) / c * per_slice + resident - 1) / resident * (c + 1); };
