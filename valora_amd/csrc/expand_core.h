@@ -13,9 +13,11 @@ namespace mlora {
 // bytes, so the column-looping expand, whose workgroups fill the device several times over, loads them in lane order
 // -- whole lines, nothing masked -- and turns them into operands through a piece of LDS of the wave's own (no barrier:
 // a wave's LDS accesses run in order; units XOR-swizzled so that the 16-byte reads, r/8 units apart, spread over the
-// banks).  Together with v_from_partials: 256 decode tokens, 64 adapters of rank 16, q+k+v 12.7 -> 11.5 us.  (The other
-// expand kernels load operands directly: there the registers and the turn cost more than the instructions, 6.2 -> 6.6 us
-// for one decode target, 26 -> 31 us for a 6749-token prefill at rank 32.)
+// banks).  Together with v_from_partials, direct / lane order: 77 tokens over ranks 8-64, q+k+v of 5120 columns 12.3 / 10.9
+// us with the partials summed here and 10.3 / 9.7 with a finished v; 256 tokens over 64 adapters of rank 16, q+k+v of 4096
+// columns 12.3 / 11.7 and 10.9 / 10.8; of rank 64 28.2 / 28.0 and 24.6 / 25.3; 512 tokens over 128 adapters of rank 128
+// 90.5 / 87.6 and 80.6 / 81.5.  (The other expand kernels load operands directly: there the registers and the turn cost
+// more than the instructions, 6.2 -> 6.6 us for one decode target, 26 -> 31 us for a 6749-token prefill at rank 32.)
 constexpr int B_TURN_BYTES = 4096;   // LDS of a wave's turn: 256 units of 16 bytes
 constexpr int B_OUTS = 64;           // outputs per wave
 
