@@ -304,7 +304,8 @@ __device__ const __align__(128) uint16_t g_zero_line[64] = {};
 // pattern) and, on top, by what stands between a barrier and the step's loads: masks, votes and dummy loads per
 // instruction, which whole steps do without.  With that and both halves' LDS reads ahead of the products: 7600-token
 // prefill over 24 adapters of rank 32 (4 layers, shrink and expand) 739 -> 712 us, 5401 tokens of mixed ranks (two
-// layers, seven projections) 789 -> 760, 5254 tokens of rank 64 778 -> 766.
+// layers, seven projections) 789 -> 760, 5254 tokens of rank 64 778 -> 766.  (Either alone: whole steps without masks
+// 741 -> 716, 789 -> 766, 777 -> 769; both halves read ahead 739 -> 728, 801 -> 796, 778 -> 776.)
 template <typename T, int NB, int MBW>
 __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_flags, int,
                                                           ShrinkArgs args_in) {
