@@ -445,12 +445,16 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   // same ksplit, which gives the same bits.
   bool use_decode = one_launch && aligned128(scratch) && pool_a->a_loc_len > 0 && pool_a->w_rows > 0;
   for (int i = 0; use_decode && i < n_targets; ++i) use_decode = targets[i].w_b_rows > 0;
-  // Where the one-launch op pays is a matter of the expand items per tile (column chunks x targets), measured on 4 to
-  // 512 decode tokens over 8 to 64 adapters, us for two launches / one: up to rank 32 (512-column items) q+k+v of 4096
-  // columns (24 items) 10.2 / 8.9 and 15.0 / 11.4, of 5120 (30) 18.1 / 16.6, one 4096 -> 11008 target (22) 12.3 / 10.9;
-  // gate+up 4096 -> 11008 (44) 14.9 / 16.2 and 20.1 / 20.8: the expand half is the longer one there, and the
-  // column-looping expand launch does it faster than these items do.  At rank 64 (256-column items) one target of 4096
-  // columns (16) 12.9 / 9.7, q+k+v (48) 15.6 / 16.2, one of 11008 columns and more likewise slower.
+  // Where the one-launch op pays is a matter of the expand items per tile (column chunks x targets).  Up to rank 32
+  // (512-column items) calls of 20 to 30 items -- q+k+v and gate or up of 4096- and 5120-wide models -- over 64 to 1024
+  // tokens and 1 to 128 adapters, cold operands, the table's marks: two launches take 0.86 to 1.40 times what one takes,
+  // 1.12 in the median (32 tokens over 64 adapters of rank 16: q+k+v 14.2 / 11.2 us, one 4096 -> 11008 target 12.0 / 8.5;
+  // 256 over 64: 20.8 / 20.6 and 17.4 / 17.1).  A seventh of the shapes lose, most of them where two launches' grid just
+  // reaches the size at which the expand loops over columns: 512 tokens over 2 to 32 adapters, 256 over 32 (q+k+v of rank
+  // 32 over 16 adapters 22.2 / 24.1, one 4096 -> 14336 target of rank 16 over 32 adapters 19.2 / 20.1).  gate+up 4096 ->
+  // 11008 (44 items) 14.9 / 16.2 and 20.1 / 20.8: the expand half is the longer one there, and the column-looping launch
+  // does it faster than these items do.  At rank 64 (256-column items) one target of 4096 columns (16) 12.9 / 9.7, q+k+v
+  // (48) 15.6 / 16.2, one of 11008 columns and more likewise slower.
   if (use_decode) {
     const int64_t bn = decode_bn((int)max_rank);
     use_decode = (h_out + bn - 1) / bn * n_targets <= one_launch_max_expand_items(max_rank);
