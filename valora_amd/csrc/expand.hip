@@ -252,7 +252,11 @@ __global__ __launch_bounds__(256, KB == 1 ? 8 : 1) void expand_cols_kernel(const
                                                                                     int h_cl, ExpandArgs args_in) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
-  constexpr bool WIDER = KB * 32 < MAX_RANK;   // an adapter's rank may be above what the narrow operand holds
+  // B in lane order (expand_core.h), or straight into operand order.  Lane order costs registers, and above rank 64 with
+  // them a workgroup of four; direct / turned on cold layers there: 512 tokens over 128 adapters of rank 128, one target of
+  // 4096 columns 26.2 / 28.8 us, q+k+v 81.0 / 82.2; 256 over 32, gate of 14336 columns 26.2 / 29.0, of 11008 24.8 / 25.8.
+  // Up to rank 64 it is faster in as many shapes as not (0.85 to 1.13, expand_core.h).
+  constexpr bool TURN = KB < 4;
   __shared__ float stage[4][16][STAGE_LD];
   __shared__ int32_t s_perm[16];
   __shared__ int32_t s_row[MAX_RANK];
@@ -309,24 +313,42 @@ __global__ __launch_bounds__(256, KB == 1 ? 8 : 1) void expand_cols_kernel(const
   for (int oc = grp * h_cl; oc < oc_end; ++oc) {
     const int o_wave = oc * EXP_BN + wave * EXP_WN;
     if (o_wave >= p.h_out) break;   // wave-uniform
-    // ---- B units and y rows of this chunk, all requested before any is consumed
-    u32x4 braw[KB][4], bfrag[4][KB];
-    uint32_t b_own = b_lane<KB, WIDER>(lane, (uint32_t)r);
-    // (from here on: the units' shares kept from one chunk to the next would cost registers, and with them a workgroup)
-    asm volatile("" : "+v"(b_own));
+    // ---- B and y rows of this chunk, all requested before any is consumed
+    u32x4 braw[TURN ? KB : 1][4], bfrag[4][KB];
+    if constexpr (TURN) {
+      uint32_t b_own = b_lane<KB, true>(lane, (uint32_t)r);
+      // (from here on: the units' shares kept from one chunk to the next would cost registers, and with them a workgroup)
+      asm volatile("" : "+v"(b_own));
 #pragma unroll
-    for (int q = 0; q < KB; ++q)
+      for (int q = 0; q < KB; ++q)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        braw[q][i] = u32x4{0, 0, 0, 0};
-        if (b_any<KB, WIDER>(i, (uint32_t)r)) {
-          uint32_t flat, bin, off;
-          const bool ok = b_unit<KB, WIDER>(q, i, lane, b_own, (uint32_t)r, (uint32_t)o_wave * (uint32_t)r, flat);   // < 2^16 * 2^7
-          divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off);
-          const int row = ok && bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;   // bins from r on hold -1
-          if (row >= 0) braw[q][i] = load16(p.pool.w + (int64_t)row * p.h_out + off);
+        for (int i = 0; i < 4; ++i) {
+          braw[q][i] = u32x4{0, 0, 0, 0};
+          if (b_any<KB, true>(i, (uint32_t)r)) {
+            uint32_t flat, bin, off;
+            const bool ok = b_unit<KB, true>(q, i, lane, b_own, (uint32_t)r, (uint32_t)o_wave * (uint32_t)r, flat);   // < 2^16 * 2^7
+            divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off);
+            const int row = ok && bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;   // bins from r on hold -1
+            if (row >= 0) braw[q][i] = load16(p.pool.w + (int64_t)row * p.h_out + off);
+          }
+        }
+    } else {
+#pragma unroll
+      for (int nb = 0; nb < 4; ++nb) {
+        const int o = o_wave + nb * 16 + lrow;
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const int j0 = kb * 32 + kg * 8;
+          bfrag[nb][kb] = u32x4{0, 0, 0, 0};
+          if (o < p.h_out && j0 < rk) {
+            uint32_t bin, off;
+            divmod24((uint32_t)o * (uint32_t)r + (uint32_t)j0, (uint32_t)p.h_out, inv_h_out, bin, off);   // < 2^16 * 2^7
+            const int row = bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;
+            if (row >= 0) bfrag[nb][kb] = load16(p.pool.w + (int64_t)row * p.h_out + off);
+          }
         }
       }
+    }
     u32x4 yv[2];
     uint16_t *yp[2];
     bool yok[2];
@@ -338,7 +360,7 @@ __global__ __launch_bounds__(256, KB == 1 ? 8 : 1) void expand_cols_kernel(const
       yp[h] = p.y + (int64_t)t * p.h_out + o_wave + c8;
       yv[h] = yok[h] ? load16(yp[h]) : u32x4{0, 0, 0, 0};
     }
-    b_turn<KB, WIDER>(braw, bfrag, (uint32_t)r, rk, lane, turn);
+    if constexpr (TURN) b_turn<KB, true>(braw, bfrag, (uint32_t)r, rk, lane, turn);
     // ---- delta block through the matrix cores, staged to LDS in token-major order
 #pragma unroll
     for (int nb = 0; nb < 4; ++nb) {

@@ -13,10 +13,10 @@ namespace mlora {
 // bytes, so the column-looping expand, whose workgroups fill the device several times over, loads them in lane order
 // -- whole lines, nothing masked -- and turns them into operands through a piece of LDS of the wave's own (no barrier:
 // a wave's LDS accesses run in order; units XOR-swizzled so that the 16-byte reads, r/8 units apart, spread over the
-// banks).  Together with v_from_partials, direct / lane order: 77 tokens over ranks 8-64, q+k+v of 5120 columns 12.3 / 10.9
-// us with the partials summed here and 10.3 / 9.7 with a finished v; 256 tokens over 64 adapters of rank 16, q+k+v of 4096
-// columns 12.3 / 11.7 and 10.9 / 10.8; of rank 64 28.2 / 28.0 and 24.6 / 25.3; 512 tokens over 128 adapters of rank 128
-// 90.5 / 87.6 and 80.6 / 81.5.  (The other expand kernels load operands directly: there the registers and the turn cost
+// banks).  Direct / lane order with a finished v, cold layers: 256 tokens over 64 adapters of rank 16, two targets of 3072
+// columns 7.8 / 6.6 us, q+k+v of 4096 10.9 / 11.2, gate+up of 11008 18.0 / 17.0; of rank 64 17.6 / 15.6, 25.2 / 26.5 and
+// 41.6 / 41.8; 77 tokens over ranks 8-64, gate+up of 13824 17.7 / 17.0; a decode pass of those over eight layers 701 / 686.
+// (Above rank 64, and in the other expand kernels, operands are loaded directly: there the registers and the turn cost
 // more than the instructions, 6.2 -> 6.6 us for one decode target, 26 -> 31 us for a 6749-token prefill at rank 32.)
 constexpr int B_TURN_BYTES = 4096;   // LDS of a wave's turn: 256 units of 16 bytes
 constexpr int B_OUTS = 64;           // outputs per wave
@@ -87,7 +87,9 @@ __device__ __forceinline__ void b_turn(const u32x4 (&raw)[KB][4], u32x4 (&bfrag)
 // The v operand of one 16-token block from the split-K partials: `part` is the block's first row in chunk 0, rows of
 // rp floats one after the other, chunks `sstride` floats apart.  The block is one run of 64*rp bytes per chunk, loaded
 // in lane order; every lane adds up its own four columns over the chunks in index order, rounds once, and the rows
-// are turned into operands through LDS like B above.  Rows from cnt on and ranks from rk on are zero.
+// are turned into operands through LDS like B above.  Rows from cnt on and ranks from rk on are zero.  Loaded row by row /
+// so, B directly in both: 256 tokens over 64 adapters, q+k+v of 4096 columns at rank 16 12.4 / 11.8 us, at rank 64 28.4 /
+// 26.6, one target at rank 32 8.1 / 7.7; 512 tokens over 128 adapters of rank 128, one target 31.4 / 28.8.
 template <typename T, int KB>
 __device__ __forceinline__ void v_from_partials(const float *part, int64_t sstride, int ksplit, int rp, int cnt, int rk,
                                                 int lane, unsigned char *turn, u32x4 (&vfrag)[KB]) {
