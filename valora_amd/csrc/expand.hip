@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256, KB == 1 ? 8 : 1) void expand_cols_kernel(const
   // 4096 columns 26.2 / 28.8 us, q+k+v 81.0 / 82.2; 256 over 32, gate of 14336 columns 26.2 / 29.0, of 11008 24.8 / 25.8.
   // Up to rank 64 it is faster in as many shapes as not (0.85 to 1.13, expand_core.h).
   constexpr bool TURN = KB < 4;
-  __shared__ float stage[4][16][STAGE_LD];
+  __shared__ __align__(16) float stage[4][16][STAGE_LD];   // (it also turns 16-byte units)
   __shared__ int32_t s_perm[16];
   __shared__ int32_t s_row[MAX_RANK];
 

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
   constexpr int MG_BM = merge_bm(KB);
   constexpr int UNITS = KB * 4;      // 16-byte units (8 rank elements) per input row of the A slice
   __shared__ __align__(16) u32x4 s_a[MG_BM * UNITS];   // unit c of row i at b_swizzle(i * UNITS + c)
-  __shared__ float stage[4][16][MG_STAGE_LD];
+  __shared__ __align__(16) float stage[4][16][MG_STAGE_LD];   // (it also turns 16-byte units)
 
   const int z = blockIdx.y;
   const int slot = p.slots[z];
