@@ -363,6 +363,7 @@ int mlora_expand(void *stream, const mlora_plan *plan, void *y, int64_t T, int64
   a.scales = static_cast<const uint16_t *>(scales);
   a.T = (int)T;
   a.h_out = (int)h_out;
+  a.inv_h_out = 1.0f / (float)h_out;
   a.kmax = (int)max_rank;
   a.slot = slot;
   a.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
@@ -518,6 +519,7 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   e.scales = static_cast<const uint16_t *>(scales);
   e.T = (int)T;
   e.h_out = (int)h_out;
+  e.inv_h_out = 1.0f / (float)h_out;
   e.kmax = (int)max_rank;
   e.slot = targets[0].slot;
   e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
@@ -626,6 +628,7 @@ int mlora_lora_compensate(void *stream, const mlora_plan *plan, void *scratch, s
   e.scales = static_cast<const uint16_t *>(scales);
   e.T = (int)T;
   e.h_out = (int)h_out;
+  e.inv_h_out = 1.0f / (float)h_out;
   e.kmax = (int)max_rank;
   e.slot = slot;
   e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());

@@ -240,171 +240,141 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
   }
 }
 
-// Decode-like tiles (at most 16 tokens, tile height 16): a (tile, 256-column chunk) pair is a few KB of B and y, too
-// little for a workgroup of its own -- a q+k+v call of 256 decode tokens is 3000 workgroups that live 4.7 us each,
-// most of it the look-up chain in front of the loads, and run in three rounds.  Here a workgroup walks over `h_cl`
-// consecutive column chunks of one tile: tile record, token ids, the slot's pool rows (kept in LDS, so a chunk's B
-// addresses need no further look-up) and the v fragment are fetched once, then every chunk is one round trip (B
-// fragments and y rows requested together), and the grid is half the size.  Same arithmetic in the same
-// order as expand_kernel: same bits.
-template <typename T, int KB, bool PARTIAL>
-__global__ __launch_bounds__(256, KB == 1 ? 8 : 1) void expand_cols_kernel(const int32_t *tiles_base, int h_groups,
-                                                                                    int h_cl, ExpandArgs args_in) {
+// Tiles of 16 tokens (decode batches).  Four independent waves of 64 outputs each: no LDS, no barrier (expand_core.h has
+// the loads and the product, and what it measured).  Grid: (column chunks, tiles, targets).
+// CH: column chunks of a workgroup, all their loads in flight together.  Two where every wave of a big grid would sum
+// the same split-K partials: q+k+v of 256 tokens over 64 adapters of rank 16 21.5 -> 21.1 us with its shrink, gate+up of 11008
+// columns 27.2 -> 25.8, q+k+v of 1000 tokens over 128 adapters 44.1 -> 41.9.  With a finished v one is faster (512 tokens,
+// q+k+v 26.1 against 27.5; one target of 256 tokens, 11008 columns 8.6 against 9.6), and so it is where the grid fits the
+// device or the rank is above 16 (ranks 8-64, gate+up of 13824 columns 25.2 against 27.4): built for ranks up to 16 only.
+constexpr int SMALL_GRID_Y = 65535;
+constexpr int small_min_waves(int kb, bool wide, bool comp) {   // as many as do without spills
+  return comp ? (kb <= 1 ? 7 : 1) : kb <= 1 ? 8 : kb == 2 ? (wide ? 7 : 5) : (wide ? 4 : 3);
+}
+template <typename T, int KB, int CH, bool WIDE, bool PARTIAL, bool COMP>
+__global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_small_kernel(const int32_t *tiles_base, const int32_t *perm,
+                                                                                         const int64_t *a_loc, int h_n_loc, int h_out,
+                                                                                         ExpandArgs p) {
   using Tr = Traits<T>;
-  using vec8 = typename Tr::vec8;
-  // B in lane order (expand_core.h), or straight into operand order.  Lane order costs registers, and above rank 64 with
-  // them a workgroup of four; direct / turned on cold layers there: 512 tokens over 128 adapters of rank 128, one target of
-  // 4096 columns 26.2 / 28.8 us, q+k+v 81.0 / 82.2; 256 over 32, gate of 14336 columns 26.2 / 29.0, of 11008 24.8 / 25.8.
-  // Up to rank 64 it is faster in as many shapes as not (0.85 to 1.13, expand_core.h).
-  constexpr bool TURN = KB < 4;
-  __shared__ __align__(16) float stage[4][16][STAGE_LD];   // (it also turns 16-byte units)
-  __shared__ int32_t s_perm[16];
-  __shared__ int32_t s_row[MAX_RANK];
-
-  const int tile_idx = blockIdx.x / h_groups;
-  const int grp = blockIdx.x - tile_idx * h_groups;
+  constexpr int FKB = SmallB<KB>::FRAG_KB;
+  const int tile_idx = (int)blockIdx.y + (int)(blockIdx.z >> 2) * SMALL_GRID_Y, z = (int)blockIdx.z & 3;
+  // One scalar round trip: the tile record and every argument the wave is going to use (csrc/decode.hip has the reason for the asm).
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
-  const int a = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
-  if (cnt <= 0) return;   // records past the last tile are zero
-  const ExpandArgs p = select_target(args_in, blockIdx.y);
-  const int rk = min(r, p.kmax);  // rank columns the narrow operand really has (bgmv_impl.cuh:167,186)
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lrow = lane & 15, kg = lane >> 4;
-  const int64_t base = (int64_t)astart + (int64_t)r * p.slot;
-
-  // one round trip: the tile's token indices, the pool rows of the slot and the scale
-  int my_perm = 0, my_row = -1;
-  if (tid < cnt) my_perm = p.plan[p.off_perm + pos0 + tid];
-  if (tid < r) {
-    const int64_t idx = base + tid;
-    if (idx >= 0 && idx < p.pool.a_loc_len) {
-      const int64_t row = p.pool.a_loc[idx];
-      if (row >= 0 && row < p.pool.w_rows) my_row = (int)row;   // pool rows fit 31 bits (checked on the host)
-    }
-  }
-  const float scale = Tr::to_float(p.scales[a]);
-  if (tid < 16) s_perm[tid] = my_perm;
-  if (tid < MAX_RANK) s_row[tid] = my_row;
-  __syncthreads();
-
-  // v fragment of the tile's one 16-token block: rows = tokens (lrow), 8 consecutive rank elements per lane
-  unsigned char *const turn = reinterpret_cast<unsigned char *>(&stage[wave][0][0]);
-  static_assert(sizeof(stage) / 4 >= B_TURN_BYTES, "a wave's staging tile holds its turn");
-  u32x4 vfrag[KB];
-  if constexpr (PARTIAL) {
-    v_from_partials<T, KB>(p.partial + (int64_t)pos0 * p.rp, (int64_t)p.T * p.rp, p.ksplit, p.rp, cnt, rk, lane, turn, vfrag);
-  } else {
-    const bool pok = lrow < cnt;
+  int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
+  uint16_t *y = p.ys[z];
+  const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
+  int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
+  float inv_h_out = p.inv_h_out;
+  asm volatile("" : "+s"(ad), "+s"(r), "+s"(pos0), "+s"(cnt), "+s"(astart), "+s"(slot), "+s"(kmax), "+s"(w_rows), "+s"(v_by_pos),
+                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out));
+  if (COMP) cnt = abs(cnt);                  // (negative: no usable rank of its own, r = 0)
+  if (cnt <= 0 || z >= p.n_targets) return;  // records past the last tile are zero
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int m = lane & 15, kg = lane >> 4;
+  const uint32_t o_wave = blockIdx.x * (uint32_t)(EXP_BN * CH) + (uint32_t)(wave * EXP_WN);
+  if (o_wave >= (uint32_t)h_out) return;
+  y = as_global(y);
+  w = as_global(w);
+  v = as_global(v);
+  scales = as_global(scales);
+  const bool on = m < cnt;                   // lanes without a token work on the tile's first one and store nothing
+  const int tok = perm[pos0 + (on ? m : 0)];
+  const float scale = Tr::to_float(scales[ad]);
+  const SmallPool pool = {w, a_loc, (uint32_t)h_n_loc, (uint32_t)w_rows, (uint32_t)h_out, inv_h_out, (uint32_t)(astart + r * slot), r,
+                          min(r, kmax)};
+  SmallRows<KB, WIDE> rows[CH], rows2;
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
+  for (int c = 0; c < CH; ++c) small_look_up<KB, WIDE>(pool, o_wave + c * EXP_BN, lane, rows[c]);
+  // COMP: y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), as in expand_kernel
+  SmallPool pool2 = pool;
+  float scale2 = 0.f;
+  if constexpr (COMP) {
+    const int r2 = p.plan[H_MERGED_RANK];
+    pool2.r = r2;
+    pool2.rk = min(r2, kmax);
+    pool2.base = (uint32_t)(p.plan[H_MERGED_START] + r2 * slot);
+    if (r2 > 0) scale2 = -Tr::to_float(scales[p.plan[H_MERGED]]);
+    small_look_up<KB, WIDE>(pool2, o_wave, lane, rows2);
+  }
+  const uint32_t pos = (uint32_t)(pos0 + (on ? m : 0)), vrow = v_by_pos ? pos : (uint32_t)tok;
+  auto load_v = [&](const uint16_t *src, int rk, u32x4 (&f)[FKB]) {
+#pragma unroll
+    for (int kb = 0; kb < FKB; ++kb) {
       const int j0 = kb * 32 + kg * 8;
-      const int64_t vrow = p.v_by_pos ? (int64_t)(pos0 + lrow) : (int64_t)s_perm[lrow];
-      vfrag[kb] = (pok && j0 < rk) ? load16(p.v + vrow * p.v_stride + j0) : u32x4{0, 0, 0, 0};
+      f[kb] = load16(small_source(j0 < rk, src + (uint64_t)vrow * (uint64_t)v_stride + j0));
     }
-  }
-
-  const int rr0 = lane >> 3, c8 = (lane & 7) * 8;
-  const float inv_h_out = 1.0f / (float)p.h_out;
-  // one chunk after the other: a chunk's B fragments and y rows are requested together, one round trip per chunk
-  // (both chunks' loads in flight at once measured slower, 20.5 against 19.2 us for q+k+v: the registers they take
-  // cost more resident workgroups than the round trip saves)
-  const int oc_end = min(p.n_ochunks, (grp + 1) * h_cl);
-  for (int oc = grp * h_cl; oc < oc_end; ++oc) {
-    const int o_wave = oc * EXP_BN + wave * EXP_WN;
-    if (o_wave >= p.h_out) break;   // wave-uniform
-    // ---- B and y rows of this chunk, all requested before any is consumed
-    u32x4 braw[TURN ? KB : 1][4], bfrag[4][KB];
-    if constexpr (TURN) {
-      uint32_t b_own = b_lane<KB, true>(lane, (uint32_t)r);
-      // (from here on: the units' shares kept from one chunk to the next would cost registers, and with them a workgroup)
-      asm volatile("" : "+v"(b_own));
+  };
+  u32x4 vfrag[FKB];
+  if constexpr (PARTIAL)
+    small_v_partials<T, KB>(p.partial + z * p.partial_tstride + (uint64_t)pos * (uint32_t)p.rp, (int64_t)p.T * p.rp, p.ksplit, pool.rk,
+                            lane, vfrag);
+  else
+    load_v(v + z * v_tstride, pool.rk, vfrag);
+  SmallY yy[CH];
 #pragma unroll
-      for (int q = 0; q < KB; ++q)
+  for (int c = 0; c < CH; ++c) small_load_y(yy[c], y, tok, on, o_wave + c * EXP_BN, (uint32_t)h_out, lane);
+  requested();
+  u32x4 raw[CH][SmallB<KB>::LOADS];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          braw[q][i] = u32x4{0, 0, 0, 0};
-          if (b_any<KB, true>(i, (uint32_t)r)) {
-            uint32_t flat, bin, off;
-            const bool ok = b_unit<KB, true>(q, i, lane, b_own, (uint32_t)r, (uint32_t)o_wave * (uint32_t)r, flat);   // < 2^16 * 2^7
-            divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off);
-            const int row = ok && bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;   // bins from r on hold -1
-            if (row >= 0) braw[q][i] = load16(p.pool.w + (int64_t)row * p.h_out + off);
-          }
-        }
-    } else {
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        const int o = o_wave + nb * 16 + lrow;
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          const int j0 = kb * 32 + kg * 8;
-          bfrag[nb][kb] = u32x4{0, 0, 0, 0};
-          if (o < p.h_out && j0 < rk) {
-            uint32_t bin, off;
-            divmod24((uint32_t)o * (uint32_t)r + (uint32_t)j0, (uint32_t)p.h_out, inv_h_out, bin, off);   // < 2^16 * 2^7
-            const int row = bin < (uint32_t)MAX_RANK ? s_row[bin] : -1;
-            if (row >= 0) bfrag[nb][kb] = load16(p.pool.w + (int64_t)row * p.h_out + off);
-          }
-        }
-      }
+  for (int c = 0; c < CH; ++c) small_load_b<KB, WIDE>(pool, lane, rows[c], raw[c]);
+  f32x4 acc[4];
+  if constexpr (COMP) {
+    u32x4 vfrag2[FKB], raw2[SmallB<KB>::LOADS];
+    load_v(v + v_tstride, pool2.rk, vfrag2);
+    small_load_b<KB, WIDE>(pool2, lane, rows2, raw2);
+    requested();
+    if (pool.rk > 0) {
+      small_product<T, KB>(raw[0], vfrag, pool.rk, acc);
+      small_add<T>(yy[0], acc, scale);
     }
-    u32x4 yv[2];
-    uint16_t *yp[2];
-    bool yok[2];
+    small_product<T, KB>(raw2, vfrag2, pool2.rk, acc);
+    small_add<T>(yy[0], acc, scale2);
+    small_store_y(yy[0]);
+  } else {
+    requested();
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int row = rr0 + 8 * h;
-      yok[h] = (o_wave + c8) < p.h_out && row < cnt;
-      const int t = yok[h] ? s_perm[row] : 0;
-      yp[h] = p.y + (int64_t)t * p.h_out + o_wave + c8;
-      yv[h] = yok[h] ? load16(yp[h]) : u32x4{0, 0, 0, 0};
+    for (int c = 0; c < CH; ++c) {
+      small_product<T, KB>(raw[c], vfrag, pool.rk, acc);
+      small_add<T>(yy[c], acc, scale);
+      small_store_y(yy[c]);
     }
-    if constexpr (TURN) b_turn<KB, true>(braw, bfrag, (uint32_t)r, rk, lane, turn);
-    // ---- delta block through the matrix cores, staged to LDS in token-major order
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb)
-        if (kb * 32 < rk) acc = Tr::mfma(as<vec8>(vfrag[kb]), as<vec8>(bfrag[nb][kb]), acc);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) stage[wave][kg * 4 + i][nb * 16 + lrow] = acc[i];
-    }
-    // stage[wave] is private to this wave and a wave's LDS operations execute in order, so only the compiler has to
-    // be kept from reordering the reads below over the writes above (and the next chunk's writes over these reads)
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      if (yok[h]) {
-        const float *srow = &stage[wave][rr0 + 8 * h][c8];
-        float f[8];
-        unpack8<T>(yv[h], f);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] += scale * srow[i];
-        store16(yp[h], pack8<T>(f));
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
   }
 }
 
+template <typename T, int KB>
+int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
+  const bool two = KB == 0 && !a.compensate && (a.column_loop || (a.partial && tiles * a.n_ochunks * a.n_targets >= 1920));
+  const int64_t hi = (tiles + SMALL_GRID_Y - 1) / SMALL_GRID_Y;   // grid y is 16 bits: the rest of the tile index in z, above the target
+  const dim3 grid((unsigned)(two ? (a.n_ochunks + 1) / 2 : a.n_ochunks), (unsigned)(hi > 1 ? SMALL_GRID_Y : tiles),
+                  (unsigned)(hi > 1 ? 4 * hi : a.n_targets));
+  // an index without entries: the kernel reads one all the same, and drops it
+  const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
+#define MLORA_SMALL(CH, WIDE, PARTIAL, COMP)                                                                              \
+  hipLaunchKernelGGL((expand_small_kernel<T, KB, CH, WIDE, PARTIAL, COMP>), grid, dim3(256), 0, st, a.plan + a.off_tiles, \
+                     a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
+#define MLORA_SMALL_WIDTH(CH, PARTIAL, COMP)                             \
+  if (KB > 0 && a.h_out >= SMALL_WIDE) MLORA_SMALL(CH, (KB > 0), PARTIAL, COMP); \
+  else MLORA_SMALL(CH, false, PARTIAL, COMP)
+  if (two) {
+    if constexpr (KB == 0) {
+      if (a.partial) MLORA_SMALL(2, false, true, false);
+      else MLORA_SMALL(2, false, false, false);
+    }
+  } else if (a.compensate) { MLORA_SMALL_WIDTH(1, false, true); }
+  else if (a.partial) { MLORA_SMALL_WIDTH(1, true, false); }
+  else { MLORA_SMALL_WIDTH(1, false, false); }
+#undef MLORA_SMALL_WIDTH
+#undef MLORA_SMALL
+  return check_launch("expand_small_kernel");
+}
+
 template <typename T>
-int launch_expand_cols_t(hipStream_t st, const ExpandArgs &a, int kb, dim3 grid, int groups, int cl) {
-#define MLORA_EXPAND_COLS(KB)                                                                                       \
-  if (a.partial) hipLaunchKernelGGL((expand_cols_kernel<T, KB, true>), grid, dim3(256), 0, st, a.plan + a.off_tiles, \
-                                    groups, cl, a);                                                                 \
-  else hipLaunchKernelGGL((expand_cols_kernel<T, KB, false>), grid, dim3(256), 0, st, a.plan + a.off_tiles, groups, cl, a)
-  switch (kb) {
-    case 1: MLORA_EXPAND_COLS(1); break;
-    case 2: MLORA_EXPAND_COLS(2); break;
-    case 4: MLORA_EXPAND_COLS(4); break;
-    default: return fail(MLORA_ERR_NO_KERNEL, "expand: no kernel for %d rank blocks", kb);
-  }
-#undef MLORA_EXPAND_COLS
-  return check_launch("expand_cols_kernel");
+int launch_small_t(hipStream_t st, const ExpandArgs &a, int max_rank, int64_t tiles) {
+  if (max_rank <= 16) return launch_small_kb<T, 0>(st, a, tiles);
+  if (max_rank <= 32) return launch_small_kb<T, 1>(st, a, tiles);
+  if (max_rank <= 64) return launch_small_kb<T, 2>(st, a, tiles);
+  return launch_small_kb<T, 4>(st, a, tiles);
 }
 
 template <typename T>
@@ -432,20 +402,8 @@ int launch_expand(hipStream_t st, const ExpandArgs &a, int max_rank, int64_t gri
   int kb = (max_rank + 31) / 32;
   kb = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
   if (grid_tiles <= 0) return MLORA_OK;
-  // 16-token tiles whose (tile, chunk, target) grid is well above the 1280 workgroups the device holds at once: two
-  // column chunks per workgroup (measured on 256 decode tokens / 64 adapters: q+k+v 22.6 -> 19.2 us, gate+up
-  // 4096 -> 11008 29.4 -> 23.5 us, gate 19.0 -> 15.9 us; four chunks 21.2 / 23.1 / 17.2; a 1280-workgroup grid
-  // such as a single 11008 -> 4096 target gets slower, 14.6 -> 16.0 us, and stays as it is)
-  const int cl = 2;
-  const bool many = grid_tiles * a.n_ochunks * a.n_targets >= 1920;
-  if (bm_expand == 16 && a.n_ochunks >= 2 && (many || a.column_loop) && !a.compensate) {
-    const int groups = (a.n_ochunks + cl - 1) / cl;
-    const int64_t blocks = grid_tiles * groups;
-    if (blocks > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "expand: grid too large");
-    dim3 grid((unsigned)blocks, (unsigned)a.n_targets);
-    return dt == MLORA_F16 ? launch_expand_cols_t<_Float16>(st, a, kb, grid, groups, cl)
-                           : launch_expand_cols_t<__bf16>(st, a, kb, grid, groups, cl);
-  }
+  if (bm_expand == 16)
+    return dt == MLORA_F16 ? launch_small_t<_Float16>(st, a, max_rank, grid_tiles) : launch_small_t<__bf16>(st, a, max_rank, grid_tiles);
   const int64_t blocks = grid_tiles * a.n_ochunks;
   if (blocks > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "expand: grid too large");
   dim3 grid((unsigned)blocks, (unsigned)a.n_targets);

@@ -66,6 +66,8 @@ __device__ __forceinline__ u32x4 lds_read16(uint32_t off) {
 __device__ __forceinline__ void lds_write16(uint32_t off, u32x4 v) {
   asm volatile("ds_write_b128 %0, %1" ::"v"(off), "v"(v) : "memory");
 }
+// loads requested above stay above: the compiler would rather sink them to where they are used
+__device__ __forceinline__ void requested() { asm volatile("" ::: "memory"); }
 // makes v "produced here" for the compiler, so nothing that uses it moves above a preceding wait
 __device__ __forceinline__ void pin(u32x4 &v) { asm volatile("" : "+v"(v)); }
 
@@ -75,13 +77,9 @@ __device__ __forceinline__ void pin(u32x4 &v) { asm volatile("" : "+v"(v)); }
 __device__ __forceinline__ void divmod24(uint32_t n, uint32_t d, float inv_d, uint32_t &q, uint32_t &rem) {
   q = (uint32_t)((float)n * inv_d);
   int32_t m = (int32_t)(n - q * d);
-  if (m < 0) {
-    q -= 1u;
-    m += (int32_t)d;
-  } else if (m >= (int32_t)d) {
-    q += 1u;
-    m -= (int32_t)d;
-  }
+  const bool low = m < 0, high = m >= (int32_t)d;   // (selects: a branch would cost more)
+  q += high ? 1u : low ? ~0u : 0u;
+  m += low ? (int32_t)d : high ? -(int32_t)d : 0;
   rem = (uint32_t)m;
 }
 

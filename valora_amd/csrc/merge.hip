@@ -100,13 +100,12 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
     aok[jj] = ac * 8 + jj < r && ai >= 0 && ai < p.pa.a_loc_len;
     alook[jj] = p.pa.a_loc[aok[jj] ? ai : 0];
   }
-  const uint32_t b_own = b_lane<KB, false>(lane, (uint32_t)r);
 #pragma unroll
   for (int q = 0; q < KB; ++q)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       uint32_t flat, bin;
-      bok[q][i] = b_unit<KB, false>(q, i, lane, b_own, (uint32_t)r, (uint32_t)o_wave * (uint32_t)r, flat);   // < 2^16 * 2^7
+      bok[q][i] = b_unit<KB>(q, i, lane, (uint32_t)r, (uint32_t)o_wave * (uint32_t)r, flat);   // < 2^16 * 2^7
       divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, boff[q][i]);
       const int64_t idx = base + bin;
       bok[q][i] = bok[q][i] && flat < (uint32_t)p.h_out * (uint32_t)r && idx >= 0 && idx < p.pb.a_loc_len;
@@ -136,7 +135,7 @@ __global__ __launch_bounds__(256, merge_resident(KB)) void merge_kernel(MergeArg
   constexpr bool A_FIRST = merge_resident(KB) <= 2;
   if constexpr (A_FIRST) load_a(0);
   static_assert(sizeof(stage) / 4 >= B_TURN_BYTES, "a wave's staging tile holds its turn");
-  b_turn<KB, false>(braw, bfrag, (uint32_t)r, r, lane, reinterpret_cast<unsigned char *>(&stage[wave][0][0]));
+  b_turn<KB>(braw, bfrag, (uint32_t)r, r, lane, reinterpret_cast<unsigned char *>(&stage[wave][0][0]));
 #pragma unroll
   for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
