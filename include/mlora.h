@@ -42,7 +42,9 @@ enum {
   MLORA_REDUCE_IN_EXPAND = 1, /* split-K chunks are summed by the expand launch instead of by a
                                  separate reduce launch: one launch fewer for small batches, more
                                  re-reads for large ones.  Must be given to both launches of a pair,
-                                 with the same ksplit.                                            */
+                                 with the same ksplit.  mlora_lora_apply and mlora_lora_apply_multi
+                                 follow it where it pays (16-token expand tiles: up to 10 MB of
+                                 partials read) and sum in the shrink elsewhere; same results      */
   MLORA_ONE_LAUNCH = 2,       /* mlora_lora_apply / mlora_lora_apply_multi only: shrink and expand are
                                  work items of ONE grid; an expand item requests its B and y operands,
                                  then waits (bounded: 30 us) for its tile's K-chunk partials and computes
@@ -66,11 +68,7 @@ enum {
                                  the others' partials out of the L2 it shares with them, or -- when they
                                  did not all run on its XCD -- computes them itself.  This flag makes
                                  every tile take the second path (made testable; same results, slower) */
-  MLORA_EXPAND_COLUMN_LOOP = 16, /* expand of a plan with 16-token expand tiles and ranks up to 16: a workgroup takes
-                                 two 256-column chunks of its tile instead of one.  The library does this
-                                 by itself where it sums split-K partials and the grid would otherwise be
-                                 several times what the device holds; the flag forces it for any size (made
-                                 testable; same results).  Without effect at higher ranks              */
+  MLORA_EXPAND_COLUMN_LOOP = 16, /* accepted and without effect: the expand of 16-token tiles has one form      */
   MLORA_ONE_LAUNCH_NEVER_READY = 32  /* with MLORA_ONE_LAUNCH: expand items look for a stamp that no shrink item
                                  leaves, so every one of them waits out its bound (30 us) and then computes
                                  its tile's partials itself: the way out of the bounded wait made testable

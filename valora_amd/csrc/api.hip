@@ -136,6 +136,17 @@ void set_reduce_here(ShrinkArgs &a, const mlora_plan *plan, const PlanLayout &L,
   a.compensate = 0;
 }
 
+// Whether a two-launch call leaves the sum of the split-K chunks to its expand, as its flags allow.  With 16-token expand tiles
+// every wave of 64 columns sums its tile's rows again; the shrink summing them itself costs some 1.5 us, the separate launch
+// 3.7.  Cold layers, summed in the expand / in the shrink: one target of 4096 columns at rank 16, 1 token 6.5 / 7.7 us, 128 tokens
+// 10.3 / 11.1, 256 (4.2 MB of partials read) 11.7 / 12.4; q+k+v of 32 tokens 9.9 / 10.7, of 256 (12.6 MB) 21.1 / 21.2, of 512 (25 MB)
+// 26.7 / 25.8; gate+up of 11008 columns, 256 tokens (23 MB) 25.9 / 25.1; q+k+v of 200 tokens, 5120 wide in six chunks (18 MB) 17.1 /
+// 14.1; at rank 64 and 8 chunks 77 tokens 32.5 / 23.5.  Same bits either way.
+bool sum_in_expand(int flags, int bm_expand, int64_t T, int64_t h_out, int n_targets, int ksplit, int64_t rp) {
+  if (ksplit <= 1 || !(flags & MLORA_REDUCE_IN_EXPAND)) return false;
+  return bm_expand != 16 || T * ((h_out + 63) / 64) * n_targets * ksplit * rp * 4 <= (int64_t)10 << 20;
+}
+
 struct Carver {
   char *p;
   size_t left;
@@ -367,7 +378,6 @@ int mlora_expand(void *stream, const mlora_plan *plan, void *y, int64_t T, int64
   a.kmax = (int)max_rank;
   a.slot = slot;
   a.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
-  a.column_loop = (flags & MLORA_EXPAND_COLUMN_LOOP) ? 1 : 0;
   a.compensate = 0;
   a.n_targets = 1;
   for (int i = 0; i < MLORA_MAX_TARGETS; ++i) {
@@ -398,6 +408,7 @@ int mlora_lora_apply(void *stream, const mlora_plan *plan, void *scratch, size_t
                                   scales, ksplit, flags, dtype);
   }
   if (ksplit == 0) ksplit = tile_ksplit_for(T, max_rank, h_in, plan->n_adapters, plan->bm_shrink);
+  if (!sum_in_expand(flags, plan->bm_expand, T, h_out, 1, ksplit, partial_stride(max_rank))) flags &= ~MLORA_REDUCE_IN_EXPAND;
   if (int rc = mlora_shrink(stream, plan, scratch, scratch_nbytes, x, T, h_in, max_rank, pool_a, slot, ksplit, nullptr,
                             0, MLORA_SHRINK_OVERWRITE, 0, flags, dtype))
     return rc;
@@ -469,7 +480,7 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   const PlanLayout L = plan_layout(plan->T, plan->n_adapters);
   const int64_t rp = partial_stride(max_rank);
   const int64_t v_bytes = align_up(T * rp * 2, 256);
-  const bool rie = one_launch || (ksplit > 1 && (flags & MLORA_REDUCE_IN_EXPAND));
+  const bool rie = use_decode || sum_in_expand(flags, plan->bm_expand, T, h_out, n_targets, ksplit, rp);
   ShrinkArgs a;
   a.plan = static_cast<const int32_t *>(plan->dev);
   a.off_perm = L.off_perm;
@@ -523,7 +534,6 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   e.kmax = (int)max_rank;
   e.slot = targets[0].slot;
   e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
-  e.column_loop = (flags & MLORA_EXPAND_COLUMN_LOOP) ? 1 : 0;
   e.compensate = 0;
   e.n_targets = n_targets;
   for (int i = 0; i < MLORA_MAX_TARGETS; ++i) {
@@ -632,7 +642,6 @@ int mlora_lora_compensate(void *stream, const mlora_plan *plan, void *scratch, s
   e.kmax = (int)max_rank;
   e.slot = slot;
   e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
-  e.column_loop = 0;
   e.compensate = 1;
   e.n_targets = 1;
   for (int i = 0; i < MLORA_MAX_TARGETS; ++i) {

@@ -242,16 +242,14 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 
 // Tiles of 16 tokens (decode batches).  Four independent waves of 64 outputs each: no LDS, no barrier (expand_core.h has
 // the loads and the product, and what it measured).  Grid: (column chunks, tiles, targets).
-// CH: column chunks of a workgroup, all their loads in flight together.  Two where every wave of a big grid would sum
-// the same split-K partials: q+k+v of 256 tokens over 64 adapters of rank 16 21.5 -> 21.1 us with its shrink, gate+up of 11008
-// columns 27.2 -> 25.8, q+k+v of 1000 tokens over 128 adapters 44.1 -> 41.9.  With a finished v one is faster (512 tokens,
-// q+k+v 26.1 against 27.5; one target of 256 tokens, 11008 columns 8.6 against 9.6), and so it is where the grid fits the
-// device or the rank is above 16 (ranks 8-64, gate+up of 13824 columns 25.2 against 27.4): built for ranks up to 16 only.
+// (Two or four column chunks a workgroup, all their loads in flight together, lose wherever the narrow operand is finished: 512
+// tokens, q+k+v at rank 16 26.1 / 27.5 us with its shrink, one target of 256 tokens, 11008 columns 8.6 / 9.6, ranks 8-64, gate+up
+// of 13824 columns 25.2 / 27.4.)
 constexpr int SMALL_GRID_Y = 65535;
 constexpr int small_min_waves(int kb, bool wide, bool comp) {   // as many as do without spills
   return comp ? (kb <= 1 ? 7 : 1) : kb <= 1 ? 8 : kb == 2 ? (wide ? 7 : 5) : (wide ? 4 : 3);
 }
-template <typename T, int KB, int CH, bool WIDE, bool PARTIAL, bool COMP>
+template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP>
 __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_small_kernel(const int32_t *tiles_base, const int32_t *perm,
                                                                                          const int64_t *a_loc, int h_n_loc, int h_out,
                                                                                          ExpandArgs p) {
@@ -272,7 +270,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   if (cnt <= 0 || z >= p.n_targets) return;  // records past the last tile are zero
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int m = lane & 15, kg = lane >> 4;
-  const uint32_t o_wave = blockIdx.x * (uint32_t)(EXP_BN * CH) + (uint32_t)(wave * EXP_WN);
+  const uint32_t o_wave = blockIdx.x * (uint32_t)EXP_BN + (uint32_t)(wave * EXP_WN);
   if (o_wave >= (uint32_t)h_out) return;
   y = as_global(y);
   w = as_global(w);
@@ -283,9 +281,8 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   const float scale = Tr::to_float(scales[ad]);
   const SmallPool pool = {w, a_loc, (uint32_t)h_n_loc, (uint32_t)w_rows, (uint32_t)h_out, inv_h_out, (uint32_t)(astart + r * slot), r,
                           min(r, kmax)};
-  SmallRows<KB, WIDE> rows[CH], rows2;
-#pragma unroll
-  for (int c = 0; c < CH; ++c) small_look_up<KB, WIDE>(pool, o_wave + c * EXP_BN, lane, rows[c]);
+  SmallRows<KB, WIDE> rows, rows2;
+  small_look_up<KB, WIDE>(pool, o_wave, lane, rows);
   // COMP: y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), as in expand_kernel
   SmallPool pool2 = pool;
   float scale2 = 0.f;
@@ -307,17 +304,15 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   };
   u32x4 vfrag[FKB];
   if constexpr (PARTIAL)
-    small_v_partials<T, KB>(p.partial + z * p.partial_tstride + (uint64_t)pos * (uint32_t)p.rp, (int64_t)p.T * p.rp, p.ksplit, pool.rk,
-                            lane, vfrag);
+    small_v_partials<T, KB>(as_global(p.partial) + z * p.partial_tstride + (int64_t)pos0 * p.rp, (uint32_t)((on ? m : 0) * p.rp),
+                            (int64_t)p.T * p.rp, p.ksplit, pool.rk, lane, vfrag);
   else
     load_v(v + z * v_tstride, pool.rk, vfrag);
-  SmallY yy[CH];
-#pragma unroll
-  for (int c = 0; c < CH; ++c) small_load_y(yy[c], y, tok, on, o_wave + c * EXP_BN, (uint32_t)h_out, lane);
+  SmallY yy;
+  small_load_y(yy, y, tok, on, o_wave, (uint32_t)h_out, lane);
   requested();
-  u32x4 raw[CH][SmallB<KB>::LOADS];
-#pragma unroll
-  for (int c = 0; c < CH; ++c) small_load_b<KB, WIDE>(pool, lane, rows[c], raw[c]);
+  u32x4 raw[SmallB<KB>::LOADS];
+  small_load_b<KB, WIDE>(pool, lane, rows, raw);
   f32x4 acc[4];
   if constexpr (COMP) {
     u32x4 vfrag2[FKB], raw2[SmallB<KB>::LOADS];
@@ -325,45 +320,34 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
     small_load_b<KB, WIDE>(pool2, lane, rows2, raw2);
     requested();
     if (pool.rk > 0) {
-      small_product<T, KB>(raw[0], vfrag, pool.rk, acc);
-      small_add<T>(yy[0], acc, scale);
+      small_product<T, KB>(raw, vfrag, pool.rk, lane, acc);
+      small_add<T>(yy, acc, scale);
     }
-    small_product<T, KB>(raw2, vfrag2, pool2.rk, acc);
-    small_add<T>(yy[0], acc, scale2);
-    small_store_y(yy[0]);
+    small_product<T, KB>(raw2, vfrag2, pool2.rk, lane, acc);
+    small_add<T>(yy, acc, scale2);
   } else {
     requested();
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      small_product<T, KB>(raw[c], vfrag, pool.rk, acc);
-      small_add<T>(yy[c], acc, scale);
-      small_store_y(yy[c]);
-    }
+    small_product<T, KB>(raw, vfrag, pool.rk, lane, acc);
+    small_add<T>(yy, acc, scale);
   }
+  small_store_y(yy);
 }
 
 template <typename T, int KB>
 int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
-  const bool two = KB == 0 && !a.compensate && (a.column_loop || (a.partial && tiles * a.n_ochunks * a.n_targets >= 1920));
   const int64_t hi = (tiles + SMALL_GRID_Y - 1) / SMALL_GRID_Y;   // grid y is 16 bits: the rest of the tile index in z, above the target
-  const dim3 grid((unsigned)(two ? (a.n_ochunks + 1) / 2 : a.n_ochunks), (unsigned)(hi > 1 ? SMALL_GRID_Y : tiles),
-                  (unsigned)(hi > 1 ? 4 * hi : a.n_targets));
+  const dim3 grid((unsigned)a.n_ochunks, (unsigned)(hi > 1 ? SMALL_GRID_Y : tiles), (unsigned)(hi > 1 ? 4 * hi : a.n_targets));
   // an index without entries: the kernel reads one all the same, and drops it
   const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
-#define MLORA_SMALL(CH, WIDE, PARTIAL, COMP)                                                                              \
-  hipLaunchKernelGGL((expand_small_kernel<T, KB, CH, WIDE, PARTIAL, COMP>), grid, dim3(256), 0, st, a.plan + a.off_tiles, \
+#define MLORA_SMALL(WIDE, PARTIAL, COMP)                                                                              \
+  hipLaunchKernelGGL((expand_small_kernel<T, KB, WIDE, PARTIAL, COMP>), grid, dim3(256), 0, st, a.plan + a.off_tiles, \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
-#define MLORA_SMALL_WIDTH(CH, PARTIAL, COMP)                             \
-  if (KB > 0 && a.h_out >= SMALL_WIDE) MLORA_SMALL(CH, (KB > 0), PARTIAL, COMP); \
-  else MLORA_SMALL(CH, false, PARTIAL, COMP)
-  if (two) {
-    if constexpr (KB == 0) {
-      if (a.partial) MLORA_SMALL(2, false, true, false);
-      else MLORA_SMALL(2, false, false, false);
-    }
-  } else if (a.compensate) { MLORA_SMALL_WIDTH(1, false, true); }
-  else if (a.partial) { MLORA_SMALL_WIDTH(1, true, false); }
-  else { MLORA_SMALL_WIDTH(1, false, false); }
+#define MLORA_SMALL_WIDTH(PARTIAL, COMP)                             \
+  if (KB > 0 && a.h_out >= SMALL_WIDE) MLORA_SMALL((KB > 0), PARTIAL, COMP); \
+  else MLORA_SMALL(false, PARTIAL, COMP)
+  if (a.compensate) { MLORA_SMALL_WIDTH(false, true); }
+  else if (a.partial) { MLORA_SMALL_WIDTH(true, false); }
+  else { MLORA_SMALL_WIDTH(false, false); }
 #undef MLORA_SMALL_WIDTH
 #undef MLORA_SMALL
   return check_launch("expand_small_kernel");

@@ -140,7 +140,8 @@ __device__ const __align__(128) uint16_t g_small_zeros[64] = {};
 __device__ __forceinline__ const uint16_t *small_source(bool ok, const void *src) {
   return as_global(reinterpret_cast<const uint16_t *>(ok ? src : static_cast<const void *>(g_small_zeros)));
 }
-// Requests the lane's units; units without a pool row, or beyond the narrow operand's columns, are zero.
+// Requests the lane's units; units without a pool row are zero, those beyond the narrow operand's columns are whatever stands
+// there (small_product drops them).
 template <int KB, bool WIDE>
 __device__ __forceinline__ void small_load_b(const SmallPool &p, int lane, const SmallRows<KB, WIDE> &s, u32x4 (&raw)[SmallB<KB>::LOADS]) {
   using B = SmallB<KB>;
@@ -165,12 +166,15 @@ __device__ __forceinline__ void small_load_b(const SmallPool &p, int lane, const
       src = bp[i] + s.off[i] * 2u;
       ok = bok[i];
     }
-    raw[i] = load16(small_source(ok && B::in_rank(i, lane, p.rk), src));
+    raw[i] = load16(small_source(ok, src));
   }
 }
-// acc[nb] = fragment nb of B^T times v^T
+// acc[nb] = fragment nb of B^T times v^T; units beyond the operand's columns count as zero.  (Masked here and not at the load:
+// the address of a unit that is not there and needs no pool row is as good as another, and a choice less per load; 512 tokens
+// over 128 adapters of rank 128, shrink and expand 62.7 -> 61.1 us, rank 8, gate+up of 8192 columns 27.1 -> 26.5.)
 template <typename T, int KB>
-__device__ __forceinline__ void small_product(const u32x4 (&raw)[SmallB<KB>::LOADS], const u32x4 (&vfrag)[SmallB<KB>::FRAG_KB], int rk, f32x4 (&acc)[4]) {
+__device__ __forceinline__ void small_product(const u32x4 (&raw)[SmallB<KB>::LOADS], const u32x4 (&vfrag)[SmallB<KB>::FRAG_KB], int rk, int lane,
+                                              f32x4 (&acc)[4]) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
 #pragma unroll
@@ -178,11 +182,12 @@ __device__ __forceinline__ void small_product(const u32x4 (&raw)[SmallB<KB>::LOA
   if constexpr (KB == 0) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
+      const bool in = SmallB<KB>::in_rank(i, lane, rk);
       u32x4 lo, hi;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         // lanes 32-63 of what was loaded change places with lanes 0-31 of a zero
-        const auto sw = __builtin_amdgcn_permlane32_swap(raw[i][e], 0u, false, false);
+        const auto sw = __builtin_amdgcn_permlane32_swap(in ? raw[i][e] : 0u, 0u, false, false);
         lo[e] = sw[0];
         hi[e] = sw[1];
       }
@@ -194,29 +199,37 @@ __device__ __forceinline__ void small_product(const u32x4 (&raw)[SmallB<KB>::LOA
     for (int nb = 0; nb < 4; ++nb)
 #pragma unroll
       for (int kb = 0; kb < KB; ++kb)
-        if (kb * 32 < rk) acc[nb] = Tr::mfma(as<vec8>(raw[nb * KB + kb]), as<vec8>(vfrag[kb]), acc[nb]);
+        if (kb * 32 < rk) {
+          const bool in = SmallB<KB>::in_rank(kb, lane, rk);
+          const u32x4 b = raw[nb * KB + kb];
+          acc[nb] = Tr::mfma(as<vec8>(in ? b : u32x4{0, 0, 0, 0}), as<vec8>(vfrag[kb]), acc[nb]);
+        }
   }
 }
-// The narrow operand of token lane%16 from its row of split-K partials, chunks `stride` floats apart: all of four chunks
-// requested before any is used, summed in index order, rounded once.
+// The narrow operand of the lane's token from split-K partials: its row is `row` floats behind `tile` (the same for all
+// lanes), chunks `stride` floats apart.  Four chunks are requested before any is used (the last one again where there are
+// fewer: what is loaded under a condition the compiler loads where it is used, one round trip each), summed in index order
+// and rounded once.
 template <typename T, int KB>
-__device__ __forceinline__ void small_v_partials(const float *row, int64_t stride, int ksplit, int rk, int lane,
+__device__ __forceinline__ void small_v_partials(const float *tile, uint32_t row, int64_t stride, int ksplit, int rk, int lane,
                                                  u32x4 (&vfrag)[SmallB<KB>::FRAG_KB]) {
 #pragma unroll
   for (int kb = 0; kb < SmallB<KB>::FRAG_KB; ++kb) {
     const int j0 = kb * 32 + (lane >> 4) * 8;
     const bool ok = j0 < rk;
-    const float *src0 = reinterpret_cast<const float *>(small_source(ok, row + j0));
-    const int64_t step = ok ? stride : 0;
+    const uint32_t at = (row + (uint32_t)(ok ? j0 : 0)) * 4u;
     float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    const char *chunk = reinterpret_cast<const char *>(tile);
     for (int s0 = 0; s0 < ksplit; s0 += 4) {
       f32x4 lo[4], hi[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const f32x4 *src = reinterpret_cast<const f32x4 *>(src0 + (int64_t)min(s0 + u, ksplit - 1) * step);
+        const f32x4 *src = reinterpret_cast<const f32x4 *>(chunk + at);
         lo[u] = src[0];
         hi[u] = src[1];
+        chunk += s0 + u + 1 < ksplit ? stride * 4 : 0;
       }
+      requested();
 #pragma unroll
       for (int u = 0; u < 4; ++u)
         if (s0 + u < ksplit) {   // wave-uniform
@@ -224,7 +237,8 @@ __device__ __forceinline__ void small_v_partials(const float *row, int64_t strid
           for (int i = 0; i < 4; ++i) { f[i] += lo[u][i]; f[4 + i] += hi[u][i]; }
         }
     }
-    vfrag[kb] = pack8<T>(f);
+    const u32x4 v = pack8<T>(f);
+    vfrag[kb] = ok ? v : u32x4{0, 0, 0, 0};
   }
 }
 // The lane's outputs of y: 16 from o_wave + 16 * (lane / 16) on, in two 16-byte halves.

@@ -141,7 +141,6 @@ struct ExpandArgs {
   const uint16_t *scales;
   int T, h_out, kmax, slot, n_ochunks;
   float inv_h_out;            // 1 / h_out
-  int column_loop;            // force two column chunks a workgroup for 16-token tiles (tests); else by grid size
   int compensate;             // every tile takes its own adapter's product minus the merged adapter's (one target)
 };
 

@@ -32,10 +32,8 @@ class LoraPlan:
         ``one_launch``: shrink and expand as work items of one grid (decode-like batches; forces
         16-token tiles, needs ``max_rank <= 64``); ``None`` takes the tile table's choice.
         ``one_launch_no_wait`` makes every expand item take its give-up path at once, ``one_launch_never_ready`` after
-        waiting out its bound, ``shrink_recompute`` makes the
-        128-token shrink sum its K chunks by computing them all in one workgroup, ``expand_column_loop`` makes the
-        expand of 16-token tiles take two column chunks per workgroup whatever the grid size, at ranks up to 16 (all for
-        tests)."""
+        waiting out its bound, ``shrink_recompute`` makes the 128-token shrink sum its K chunks by computing them all in
+        one workgroup (all for tests); ``expand_column_loop`` is accepted and without effect."""
         if not ids.is_cuda:
             raise RuntimeError("ids must be a CUDA tensor")
         if ids.dtype != torch.long or a_start.dtype != torch.long or a_len.dtype != torch.long:
