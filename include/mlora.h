@@ -54,9 +54,10 @@ enum {
                                  mlora_one_launch_scratch_bytes(), 128-byte aligned (the partials are
                                  handed over in cache lines that belong to one tile each; a scratch
                                  buffer aligned to less, an empty index or an empty pool make the call
-                                 run as two launches, and so does a call with more than 32 expand items
-                                 per tile -- 512-column chunks x targets; above rank 32 more than 16 of
-                                 256 columns -- where two launches measured faster).  Any batch size: items the device cannot
+                                 run as two launches, and so does what two launches measured faster for:
+                                 more than 32 expand items per tile -- 512-column chunks x targets --,
+                                 ksplit above 4, up to 4 tokens with 3 or 4 targets, ranks above 32,
+                                 big grids above rank 16).  Any batch size: items the device cannot
                                  hold from the start take part in the hand-off like the others.
                                  Bit-identical to the two-launch op with MLORA_REDUCE_IN_EXPAND and the
                                  same ksplit.  Launches that share a plan must not overlap in time.  */
@@ -119,8 +120,8 @@ size_t mlora_plan_bytes(int64_t T, int64_t n_adapters);
 /* Bytes of the scratch buffer that carries v = x*A^T from mlora_shrink to mlora_expand (a T-typed
  * [T, max_rank] matrix plus, for ksplit > 1, the fp32 split-K partials).                       */
 size_t mlora_scratch_bytes(int64_t T, int64_t max_rank, int32_t ksplit);
-/* Bytes of scratch a call with MLORA_ONE_LAUNCH needs (its K-chunk partials are laid out tile by tile, in
- * whole cache lines per tile, which takes more room than mlora_scratch_bytes gives).             */
+/* Bytes of scratch a call with MLORA_ONE_LAUNCH needs: as one launch (its K-chunk partials are laid out tile
+ * by tile, in whole cache lines per tile) or as two, whichever is more.                            */
 size_t mlora_one_launch_scratch_bytes(int64_t T, int64_t n_adapters, int64_t max_rank, int32_t ksplit,
                                       int32_t n_targets);
 /* Bytes of scratch the one-call entry points (dispatch_bgmv, dispatch_sgmm, prefill_*) need.

@@ -27,16 +27,12 @@ int check_launch(const char *what) {
 }
 
 int expand_bn();
-int decode_bn(int max_rank);   // output columns per expand item of the one-launch op
 
 // How long an expand item of the one-launch op waits for its tile's shrink items before it computes the tile's
 // partials itself, in ticks of the device's 100 MHz clock: 30 us.  The shrink items are started before the expand
 // items that wait for them and run for a few microseconds, so a healthy launch never gets near the bound; it only
 // limits how long a workgroup holds its slot when the producers are held up (a device shared with other work).
 constexpr int ONE_LAUNCH_WAIT_TICKS = 3000;
-// expand items per tile up to which a call that asks for one launch gets it (see mlora_lora_apply_multi)
-constexpr int one_launch_max_expand_items(int64_t max_rank) { return max_rank <= 32 ? 32 : 16; }
-
 namespace {
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
@@ -109,6 +105,11 @@ size_t scratch_bytes(int64_t T, int64_t max_rank, int ksplit) {
 
 namespace {
 
+size_t one_launch_bytes(int64_t T, int64_t n_adapters, int64_t max_rank, int ksplit, int n_targets) {
+  const int64_t rp = partial_stride(max_rank);
+  return (size_t)align_up(T * rp * 2, 256) + 4 * decode_partial_floats(tiles_upper(T, n_adapters, 16), n_targets, ksplit, rp);
+}
+
 PoolDev pool_dev(const mlora_pool *p) {
   PoolDev d;
   d.w = static_cast<const uint16_t *>(p->w);
@@ -145,6 +146,24 @@ void set_reduce_here(ShrinkArgs &a, const mlora_plan *plan, const PlanLayout &L,
 bool sum_in_expand(int flags, int bm_expand, int64_t T, int64_t h_out, int n_targets, int ksplit, int64_t rp) {
   if (ksplit <= 1 || !(flags & MLORA_REDUCE_IN_EXPAND)) return false;
   return bm_expand != 16 || T * ((h_out + 63) / 64) * n_targets * ksplit * rp * 4 <= (int64_t)10 << 20;
+}
+
+constexpr int64_t ONE_LAUNCH_MAX_ITEMS = 32;
+// Whether a call that asks for one launch gets it (cold layers, one launch / two, us).
+bool one_launch_pays(int64_t T, int64_t A, int64_t items, int64_t max_rank, int n_targets, int ksplit) {
+  // Expand items per tile (512-column chunks x targets), ONE_LAUNCH_MAX_ITEMS: the expand half outweighs the hand-off beyond.
+  // Up to 30 (q+k+v, or one gate / up, of 4096- and 5120-wide models) at rank 16: one target of 128 tokens 8.5 / 9.6, of 256
+  // 9.6 / 10.9; q+k+v of 64 13.3 / 14.0, of 256 19.9 / 19.5, of 512 22.1 / 24.4; gate+up of 11008 columns (44 items) 26.5 / 24.0.
+  // An expand item reads four chunks in one round trip: with more of them two launches win.  200 tokens, q+k+v of 5120 columns in five
+  // chunks: rank 8 14.3 / 13.2, rank 32 21.2 / 18.6; one target of 32 tokens of rank 32 in eight 9.0 / 8.2, of 128 10.4 / 10.8.
+  if (ksplit > 4) return false;
+  // A handful of tokens and several targets: all items of a tile run on one XCD, those of two launches on all eight.
+  // q+k+v of one token 6.5 / 6.1, two 6.8 / 6.5, four 7.0 / 6.7, eight 7.1 / 7.3.
+  if (T <= 4 && n_targets > 2) return false;
+  // Above rank 16 three workgroups fit on a compute unit instead of four, and a grid of more than about five a unit loses: rank 32, one
+  // target of 256 tokens over 16 adapters (384 workgroups) 9.2 / 10.7, over 64 (960) 14.1 / 15.3, of 400 over 128 (1836) 22.5 / 21.8; q+k+v
+  // of 256 over 16 (1152) 17.4 / 18.5, over 64 (2880) 28.6 / 28.1.
+  return max_rank <= 16 || tiles_upper(T, A, 16) * (items + ksplit * n_targets) <= 1280;
 }
 
 struct Carver {
@@ -185,9 +204,9 @@ size_t mlora_one_launch_scratch_bytes(int64_t T, int64_t n_adapters, int64_t max
   if (T < 0 || n_adapters < 0 || max_rank < 0 || n_targets < 1) return 0;
   if (ksplit < 2) ksplit = 2;
   if (ksplit * n_targets > DECODE_MAX_PRODUCERS) ksplit = DECODE_MAX_PRODUCERS / n_targets;
-  const int64_t rp = partial_stride(max_rank);
-  return (size_t)align_up(T * rp * 2, 256) +
-         4 * decode_partial_floats(tiles_upper(T, n_adapters, 16), n_targets, ksplit, rp);
+  const size_t two = scratch_bytes(T, max_rank, ksplit) * (size_t)n_targets;   // where the call runs as two launches
+  const size_t one = one_launch_bytes(T, n_adapters, max_rank, ksplit, n_targets);
+  return one > two ? one : two;
 }
 
 size_t mlora_workspace_bytes(int64_t T, int64_t n_adapters, int64_t max_rank) {
@@ -455,25 +474,16 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   // belong to one tile each (128-byte aligned), and its expand items read element 0 of the index and of every
   // target's pool where they have nothing to fetch: a call that cannot offer that runs as two launches with the
   // same ksplit, which gives the same bits.
-  bool use_decode = one_launch && aligned128(scratch) && pool_a->a_loc_len > 0 && pool_a->w_rows > 0;
+  const int64_t items = (h_out + decode_bn() - 1) / decode_bn() * n_targets;
+  bool use_decode = one_launch && max_rank <= 32 && items <= ONE_LAUNCH_MAX_ITEMS && aligned128(scratch) && pool_a->a_loc_len > 0 && pool_a->w_rows > 0;
   for (int i = 0; use_decode && i < n_targets; ++i) use_decode = targets[i].w_b_rows > 0;
-  // Where the one-launch op pays is a matter of the expand items per tile (column chunks x targets).  Up to rank 32
-  // (512-column items) calls of 20 to 30 items -- q+k+v and gate or up of 4096- and 5120-wide models -- over 64 to 1024
-  // tokens and 1 to 128 adapters, cold operands, the table's marks: two launches take 0.86 to 1.40 times what one takes,
-  // 1.12 in the median (32 tokens over 64 adapters of rank 16: q+k+v 14.2 / 11.2 us, one 4096 -> 11008 target 12.0 / 8.5;
-  // 256 over 64: 20.8 / 20.6 and 17.4 / 17.1).  A seventh of the shapes lose, most of them where two launches' grid just
-  // reaches the size at which the expand loops over columns: 512 tokens over 2 to 32 adapters, 256 over 32 (q+k+v of rank
-  // 32 over 16 adapters 22.2 / 24.1, one 4096 -> 14336 target of rank 16 over 32 adapters 19.2 / 20.1).  gate+up 4096 ->
-  // 11008 (44 items) 14.9 / 16.2 and 20.1 / 20.8: the expand half is the longer one there, and the column-looping launch
-  // does it faster than these items do.  At rank 64 (256-column items) one target of 4096 columns (16) 12.9 / 9.7, q+k+v
-  // (48) 15.6 / 16.2, one of 11008 columns and more likewise slower.
-  if (use_decode) {
-    const int64_t bn = decode_bn((int)max_rank);
-    use_decode = (h_out + bn - 1) / bn * n_targets <= one_launch_max_expand_items(max_rank);
-  }
+  // (a scratch buffer with just enough room for one launch keeps it)
+  if (use_decode && !one_launch_pays(T, plan->n_adapters, items, max_rank, n_targets, ksplit) &&
+      scratch_nbytes >= scratch_bytes(T, max_rank, ksplit) * (size_t)n_targets)
+    use_decode = false;
   if (ksplit < 1 || ksplit > 64) return fail(MLORA_ERR_INVALID, "lora_apply_multi: ksplit=%d outside [1,64]", ksplit);
   const size_t per_target = scratch_bytes(T, max_rank, ksplit);
-  const size_t scratch_need = use_decode ? mlora_one_launch_scratch_bytes(T, plan->n_adapters, max_rank, ksplit, n_targets)
+  const size_t scratch_need = use_decode ? one_launch_bytes(T, plan->n_adapters, max_rank, ksplit, n_targets)
                                          : per_target * (size_t)n_targets;
   if (scratch_nbytes < scratch_need)
     return fail(MLORA_ERR_WORKSPACE, "lora_apply_multi: scratch has %zu bytes, needs %zu", scratch_nbytes, scratch_need);
@@ -554,7 +564,7 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
     d.done = reinterpret_cast<uint32_t *>(words + L.off_counters);
     d.stamps = reinterpret_cast<uint32_t *>(words + L.off_stamps);
     d.n_tiles = (int)tiles;
-    d.e.n_ochunks = (int)((h_out + decode_bn((int)max_rank) - 1) / decode_bn((int)max_rank));
+    d.e.n_ochunks = (int)((h_out + decode_bn() - 1) / decode_bn());
     d.n_producers = ksplit * n_targets;
     d.n_consumers = d.e.n_ochunks * n_targets;
     d.spin_limit = (flags & MLORA_ONE_LAUNCH_NO_WAIT) ? 0 : ONE_LAUNCH_WAIT_TICKS;

@@ -48,6 +48,7 @@
 // Launches that share a plan must not overlap in time (they share the scratch buffer and the words above).
 //
 // Reference semantics: valora/csrc/bgmv/bgmv_impl.cuh:14-148 (shrink) and :152-207 (expand).
+#include "expand_core.h"
 #include "kernel_common.h"
 #include "shrink_core.h"
 
@@ -55,13 +56,11 @@ namespace mlora {
 
 namespace {
 
-// 256-column chunks per expand item: two (fewer, fatter items: the whole grid should be resident at once, a waiting
-// item holds its slot) up to rank 32; at rank 64 the B fragments of two chunks no longer fit the register budget of
-// three waves per SIMD (16 registers spilled), so those items take one chunk.
-constexpr int dec_ch(int nb) { return nb >= 4 ? 1 : 2; }
-constexpr int dec_nb(int max_rank) { return max_rank <= 16 ? 1 : max_rank <= 32 ? 2 : 4; }
+// 256-column chunks per expand item: two (fewer, fatter items: the whole grid should be resident at once, a waiting item holds its
+// slot).  q+k+v of 256 tokens over 64 adapters, rank 16: 19.9 us with two, 19.5 with four, which lose at one token (6.0 / 6.3);
+// rank 32: 28.5 with two, 33.7 with one.
+constexpr int DEC_CH = 2, DEC_BN = 256 * DEC_CH;   // and outputs per expand item
 constexpr int DEC_WN = 64;         // outputs per wave and chunk
-constexpr int DEC_STAGE_LD = DEC_WN + 4;
 
 // device scope: visible to every compute unit, whichever XCD it sits on; the result is not asked for
 __device__ __forceinline__ void add_device(uint32_t *p, uint32_t v) {
@@ -117,27 +116,27 @@ __device__ __forceinline__ ItemId item_of(int n_producers, int n_consumers, int 
   return it;
 }
 
-// One workgroup = one work item.  3 waves per SIMD = 3 workgroups per compute unit: an expand item keeps the B
-// fragments and y rows of 512 columns in flight, a shrink item 8 K-steps of both operands.
+// One workgroup = one work item.  4 waves per SIMD = 4 workgroups per compute unit up to rank 16 (113 registers), 3 above (157): an
+// expand item keeps the B units and y rows of 512 columns in flight, a shrink item 4 or 2 K steps of both operands.
+// Bound by the two halves' serial chains (each half's are at shrink_tile_to_lds and small_product).  With the expand item formed
+// output by token (no turn through LDS), its chunk loads not behind its B loads, and the shrink's loads without masks, cold layers,
+// rank 16, before / now: one target of one token 6.4 / 5.7 us, of 256 9.6 / 9.6, 11008 wide 15.1 / 14.1; q+k+v of 256 21.2 / 19.9, of
+// 512 23.7 / 22.1.
 // The leading scalar parameters repeat what the first dependent loads need (the tile records, the `done` words, the
 // id layout): the library is built with kernel-argument preloading, which hands the first 8 dwords of the
 // argument list to the wave in registers at launch, so the tile record can be requested without waiting for a load
 // of the argument block first (0.35 us of a 10.3 us op).
-template <typename T, int NB>
+template <typename T, int NB, bool WIDE>
 __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_base, uint32_t *done_base, int h_n_producers,
                                                         int h_n_consumers, int h_n_tiles, int h_shrink_ids,
                                                         DecodeArgs a) {
   using Tr = Traits<T>;
-  using vec8 = typename Tr::vec8;
-  constexpr int DEC_CH = dec_ch(NB), DEC_BN = 256 * DEC_CH;   // chunks and outputs per expand item
-  constexpr int KB = (NB + 1) / 2;                  // 32-wide rank blocks of the expand
-  constexpr int STAGE_FLOATS = 4 * 16 * DEC_STAGE_LD;
+  constexpr int KB = NB / 2;                        // 32-wide rank blocks of the expand, 0 for half a one (expand_core.h)
   constexpr int TILE_FLOATS = shrink_lds_floats(NB);   // shrink_tile_to_lds
   constexpr int VACC_FLOATS = 16 * NB * 16;         // a tile's summed chunks (give-up path)
-  constexpr int BUF_FLOATS = TILE_FLOATS + VACC_FLOATS > STAGE_FLOATS ? TILE_FLOATS + VACC_FLOATS : STAGE_FLOATS;
+  constexpr int BUF_FLOATS = TILE_FLOATS + VACC_FLOATS;
   static_assert(DECODE_MAX_PRODUCERS == 16, "stamps_state reads 16 stamps");
-  __shared__ __align__(16) float s_buf[BUF_FLOATS];   // a shrink item's tile, an expand item's staging tile
-  __shared__ int32_t s_perm[16];
+  __shared__ __align__(16) float s_buf[BUF_FLOATS];   // a shrink item's tile; an expand item's that computes the chunks itself
   __shared__ int32_t s_ready;
   const int id = (int)blockIdx.x;
 
@@ -193,11 +192,15 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
     shrink_tile_to_lds<T, 1, NB>(x, h_in, pool, slot, perm, r, pos0, cnt, astart, kbeg, kend, s_buf);
     if (wave == 0) {
       // wave 0 alone writes the partial and then the stamp: no barrier, and nothing else of its own in flight
-      f32x4 *part = reinterpret_cast<f32x4 *>(tile_partial + (int64_t)item * 16 * rp);
-      const int quarter = rp >> 2;
-      for (int e = lane; e < 16 * quarter; e += 64) {
-        const int row = e / quarter, c4 = e - row * quarter;
-        part[e] = shrink_tile_sum<NB>(s_buf, NB, row, c4);
+      // (no division: 16 rows x 4 quarters of a rank block are the lanes)
+      char *const part = reinterpret_cast<char *>(tile_partial + (int64_t)item * 16 * rp);
+      f32x4 sum[NB];
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) sum[nb] = shrink_tile_sum<NB>(s_buf, NB, lane >> 2, nb * 4 + (lane & 3));
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const int col = nb * 16 + (lane & 3) * 4;
+        if (col < rp) *reinterpret_cast<f32x4 *>(part + (uint32_t)((lane >> 2) * rp + col) * 4u) = sum[nb];
       }
       // the partial must sit in the L2 before the stamp that announces it
       wait_vmcnt<0>();
@@ -228,74 +231,25 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
   const uint16_t *const wB = a.e.ws[z];
   const int64_t wB_rows = a.e.w_rows_t[z];
 
-  const int lrow = lane & 15, kg = lane >> 4;
-  int o_wave[DEC_CH];
-#pragma unroll
-  for (int c = 0; c < DEC_CH; ++c) o_wave[c] = oc * DEC_BN + c * 256 + wave * DEC_WN;
-
-  // Everything that depends only on the tile record is requested first, in one round trip.  The set-up is
-  // kept to few instructions and free of branches: with every workgroup of the grid resident, the vector
-  // ALUs are what the first loads wait for.  Loads that have nothing to fetch read element 0 of their
-  // array instead of being skipped, and their result is dropped.
-  int my_perm = 0;
-  if (tid < cnt) my_perm = perm[pos0 + tid];
+  const int m = lane & 15, kg = lane >> 4;
+  const bool on = m < cnt;                // lanes without a token work on the tile's first one and store nothing
+  const uint32_t o_wave = (uint32_t)(oc * DEC_BN + __builtin_amdgcn_readfirstlane(wave) * DEC_WN);   // and 256 further on
+  const int tok = perm[pos0 + (on ? m : 0)];
   const float scale = Tr::to_float(scales[ad]);
-  const float inv_h_out = 1.0f / (float)h_out;
-  const uint32_t base32 = (uint32_t)(astart + r * slot), n_loc = (uint32_t)a_loc_len;
-  const uint32_t step16 = 16u * (uint32_t)r;
-  const bool can_step = step16 < (uint32_t)h_out;     // workgroup-uniform
-  int64_t brow[DEC_CH][4][KB];
-  uint32_t boff[DEC_CH][4][KB];
-  bool bok[DEC_CH][4][KB];
+  const SmallPool pool = {as_global(wB), as_global(a_loc), (uint32_t)a_loc_len, (uint32_t)wB_rows, (uint32_t)h_out, a.e.inv_h_out,
+                          (uint32_t)(astart + r * slot), r, rk};
+  SmallRows<KB, WIDE> rows[DEC_CH];
 #pragma unroll
-  for (int c = 0; c < DEC_CH; ++c)
+  for (int c = 0; c < DEC_CH; ++c) small_look_up<KB, WIDE>(pool, o_wave + c * 256u, lane, rows[c]);
+  // y rows and B units (expand_core.h): the loads the hand-off wait is hidden behind
+  SmallY<KB> yy[DEC_CH];
+  u32x4 raw[DEC_CH][SmallB<KB>::LOADS];
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const uint32_t j0 = (uint32_t)(kb * 32 + kg * 8);
-      BCursor cur = b_cursor((uint32_t)(o_wave[c] + lrow), (uint32_t)r, j0, (uint32_t)h_out, inv_h_out);
+  for (int c = 0; c < DEC_CH; ++c) small_load_y(yy[c], as_global(y), tok, on, o_wave + c * 256u, (uint32_t)h_out, lane);
+  requested();
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        const int o = o_wave[c] + nb * 16 + lrow;
-        if (nb > 0) {
-          if (can_step) b_advance(cur, step16, (uint32_t)h_out);
-          else cur = b_cursor((uint32_t)o, (uint32_t)r, j0, (uint32_t)h_out, inv_h_out);
-        }
-        const uint32_t idx = base32 + cur.bin;
-        const bool ok = o < h_out && (int)j0 < rk && idx < n_loc;
-        brow[c][nb][kb] = a_loc[ok ? idx : 0u];
-        boff[c][nb][kb] = cur.off;
-        bok[c][nb][kb] = ok;
-      }
-    }
-  if (tid < 16) s_perm[tid] = my_perm;
-  __syncthreads();
-
-  // B fragments and y rows: the loads the hand-off wait is hidden behind
-  u32x4 bfrag[DEC_CH][4][KB];
-#pragma unroll
-  for (int c = 0; c < DEC_CH; ++c)
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int64_t row = brow[c][nb][kb];
-        const bool ok = bok[c][nb][kb] && (uint64_t)row < (uint64_t)wB_rows;
-        const u32x4 got = load16(wB + (ok ? row * h_out + boff[c][nb][kb] : 0));
-        bfrag[c][nb][kb] = ok ? got : u32x4{0, 0, 0, 0};
-      }
-  const int rr0 = lane >> 3, c8 = (lane & 7) * 8;
-  u32x4 yv[DEC_CH][2];
-  uint16_t *yp[DEC_CH][2];
-  bool yok[DEC_CH][2];
-#pragma unroll
-  for (int c = 0; c < DEC_CH; ++c)
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int row = rr0 + 8 * h;
-      yok[c][h] = (o_wave[c] + c8) < h_out && row < cnt;
-      yp[c][h] = y + (yok[c][h] ? (int64_t)s_perm[row] * h_out + o_wave[c] + c8 : 0);
-      yv[c][h] = load16(yp[c][h]);
-    }
+  for (int c = 0; c < DEC_CH; ++c) small_load_b<KB, WIDE>(pool, lane, rows[c], raw[c]);
+  requested();
   // ---- bounded wait for the tile's stamps (one wave polls on the scalar path; the workgroup follows its
   //      verdict without draining its loads).  The producers were started before this item and run for a few
   //      microseconds; the bound (ticks of the 100 MHz clock, and a cap on the polls) only limits how long a
@@ -316,36 +270,11 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
   lds_barrier();
   const bool ready = s_ready != 0;
 
-  // ---- v fragment: rows = tokens (lrow), 8 consecutive rank elements per lane; chunks summed in index order
-  u32x4 vfrag[KB];
-  const bool pok = lrow < cnt;
+  // ---- the narrow operand of token lane%16; chunks summed in index order
+  u32x4 vfrag[SmallB<KB>::FRAG_KB];
   if (ready) {
-    const float *part = tile_partial + (int64_t)z * e_ksplit * 16 * rp;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-      const int j0 = kb * 32 + kg * 8;
-      u32x4 v = {0, 0, 0, 0};
-      if (pok && j0 < rk) {
-        float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        const float *src0 = part + lrow * rp + j0;
-        for (int s0 = 0; s0 < e_ksplit; s0 += 4) {
-          f32x4 lo[4], hi[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const bool ok = s0 + u < e_ksplit;
-            const f32x4 *src = reinterpret_cast<const f32x4 *>(src0 + (int64_t)(s0 + u) * 16 * rp);
-            lo[u] = ok ? src[0] : f32x4{0.f, 0.f, 0.f, 0.f};
-            hi[u] = ok ? src[1] : f32x4{0.f, 0.f, 0.f, 0.f};
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { f[i] += lo[u][i]; f[4 + i] += hi[u][i]; }
-        }
-        v = pack8<T>(f);
-      }
-      vfrag[kb] = v;
-    }
+    small_v_partials<T, KB>(as_global(tile_partial) + (int64_t)z * e_ksplit * 16 * rp, (uint32_t)(m * rp), (int64_t)16 * rp, e_ksplit, rk, lane,
+                            vfrag);
   } else {
     // give-up path: the tile's chunks computed here, one after the other with the shrink item's own code
     float *vacc = s_buf + TILE_FLOATS;
@@ -362,52 +291,20 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
       __syncthreads();
     }
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
+    for (int kb = 0; kb < SmallB<KB>::FRAG_KB; ++kb) {
       const int j0 = kb * 32 + kg * 8;
-      u32x4 v = {0, 0, 0, 0};
-      if (pok && j0 < rk && j0 < NB * 16) {
-        float f[8];
+      float f[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) f[i] = vacc[lrow * (NB * 16) + j0 + i];
-        v = pack8<T>(f);
-      }
-      vfrag[kb] = v;
+      for (int i = 0; i < 8; ++i) f[i] = j0 < rk && j0 < NB * 16 ? vacc[m * (NB * 16) + j0 + i] : 0.f;
+      vfrag[kb] = pack8<T>(f);
     }
-    __syncthreads();   // vacc is about to be reused as the staging tile
   }
-
-  // ---- delta blocks through the matrix cores, turned through a wave-private LDS tile for the y update
-  float(*stage)[DEC_STAGE_LD] = reinterpret_cast<float(*)[DEC_STAGE_LD]>(s_buf + wave * 16 * DEC_STAGE_LD);
 #pragma unroll
   for (int c = 0; c < DEC_CH; ++c) {
-    if (o_wave[c] < h_out) {   // wave-uniform
-#pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb)
-          if (kb * 32 < rk) acc = Tr::mfma(as<vec8>(vfrag[kb]), as<vec8>(bfrag[c][nb][kb]), acc);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) stage[kg * 4 + i][nb * 16 + lrow] = acc[i];
-      }
-      // the tile is private to this wave and a wave's LDS operations execute in order: only the compiler
-      // has to be kept from moving the reads below over the writes above
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        if (yok[c][h]) {
-          const float *srow = &stage[rr0 + 8 * h][c8];
-          float f[8];
-          unpack8<T>(yv[c][h], f);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) f[i] += scale * srow[i];
-          store16(yp[c][h], pack8<T>(f));
-        }
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-    }
+    f32x4 acc[4];
+    small_product<T, KB>(raw[c], vfrag, rk, lane, acc);
+    small_add<T, KB>(yy[c], acc, scale);
+    small_store_y(yy[c]);
   }
   // the tile's last expand item tops the tile's `done` word up to the launch's weight
   if (tid == 0 && item == h_n_consumers - 1) add_device(done_base + tile_idx, DECODE_LAUNCH_WEIGHT - (uint32_t)n_producers);
@@ -415,18 +312,19 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
 
 template <typename T>
 int launch_decode_t(hipStream_t st, const DecodeArgs &a, int nb, dim3 grid, int shrink_ids) {
-  switch (nb) {
-    case 1: hipLaunchKernelGGL((decode_kernel<T, 1>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, a.n_tiles, shrink_ids, a); break;
-    case 2: hipLaunchKernelGGL((decode_kernel<T, 2>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, a.n_tiles, shrink_ids, a); break;
-    case 4: hipLaunchKernelGGL((decode_kernel<T, 4>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, a.n_tiles, shrink_ids, a); break;
-    default: return fail(MLORA_ERR_NO_KERNEL, "one-launch op: ranks above 64 use the two-launch path");
-  }
+#define MLORA_DECODE(NB, WIDE)                                                                                                  \
+  hipLaunchKernelGGL((decode_kernel<T, NB, WIDE>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, \
+                     a.n_tiles, shrink_ids, a)
+  if (nb == 1) MLORA_DECODE(1, false);
+  else if (a.e.h_out >= SMALL_WIDE) MLORA_DECODE(2, true);
+  else MLORA_DECODE(2, false);
+#undef MLORA_DECODE
   return check_launch("decode_kernel");
 }
 
 }  // namespace
 
-int decode_bn(int max_rank) { return 256 * dec_ch(dec_nb(max_rank)); }
+int decode_bn() { return DEC_BN; }
 
 // floats of scratch the one-launch op needs for its partials: [tile][target][K chunk][16][rp]
 size_t decode_partial_floats(int64_t n_tiles, int n_targets, int ksplit, int64_t rp) {
@@ -434,9 +332,9 @@ size_t decode_partial_floats(int64_t n_tiles, int n_targets, int ksplit, int64_t
 }
 
 int launch_decode(hipStream_t st, const DecodeArgs &a, int max_rank, mlora_dtype dt) {
-  int nb = (max_rank + 15) / 16;
-  nb = nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : 8;
+  const int nb = (max_rank + 15) / 16;
   if (a.n_tiles <= 0) return MLORA_OK;
+  if (nb > 2) return fail(MLORA_ERR_NO_KERNEL, "one-launch op: ranks above 32 use the two-launch path");
   if (a.n_producers > DECODE_MAX_PRODUCERS)
     return fail(MLORA_ERR_NO_KERNEL, "one-launch op: ksplit * targets = %d exceeds %d", a.n_producers, DECODE_MAX_PRODUCERS);
   const int64_t groups = (a.n_tiles + 7) / 8;

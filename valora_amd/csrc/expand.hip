@@ -247,7 +247,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 // of 13824 columns 25.2 / 27.4.)
 constexpr int SMALL_GRID_Y = 65535;
 constexpr int small_min_waves(int kb, bool wide, bool comp) {   // as many as do without spills
-  return comp ? (kb <= 1 ? 7 : 1) : kb <= 1 ? 8 : kb == 2 ? (wide ? 7 : 5) : (wide ? 4 : 3);
+  return comp ? (kb <= 1 ? 7 : 1) : kb <= 1 ? 8 : kb == 2 ? (wide ? 6 : 5) : (wide ? 4 : 3);
 }
 template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP>
 __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_small_kernel(const int32_t *tiles_base, const int32_t *perm,
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
                             (int64_t)p.T * p.rp, p.ksplit, pool.rk, lane, vfrag);
   else
     load_v(v + z * v_tstride, pool.rk, vfrag);
-  SmallY yy;
+  SmallY<KB> yy;
   small_load_y(yy, y, tok, on, o_wave, (uint32_t)h_out, lane);
   requested();
   u32x4 raw[SmallB<KB>::LOADS];
@@ -321,14 +321,14 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
     requested();
     if (pool.rk > 0) {
       small_product<T, KB>(raw, vfrag, pool.rk, lane, acc);
-      small_add<T>(yy, acc, scale);
+      small_add<T, KB>(yy, acc, scale);
     }
     small_product<T, KB>(raw2, vfrag2, pool2.rk, lane, acc);
-    small_add<T>(yy, acc, scale2);
+    small_add<T, KB>(yy, acc, scale2);
   } else {
     requested();
     small_product<T, KB>(raw, vfrag, pool.rk, lane, acc);
-    small_add<T>(yy, acc, scale);
+    small_add<T, KB>(yy, acc, scale);
   }
   small_store_y(yy);
 }

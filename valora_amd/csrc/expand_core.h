@@ -92,11 +92,11 @@ struct SmallB {
   // what a lane fetches: LOADS units of 8 rank elements, unit i at flat element first + step(i) of the slot's B
   static __device__ __forceinline__ uint32_t lane_output(int lane) {   // of the first unit, within the wave's 64
     const int m = lane & 15;
-    return (uint32_t)((m >> 2) * 16 + (m & 3) + (KB ? 0 : (lane >> 5) * 4));
+    return KB ? (uint32_t)((m >> 2) * 16 + (m & 3)) : (uint32_t)((m >> 2) * 8 + (m & 3) + (lane >> 5) * 4);
   }
   static __device__ __forceinline__ int lane_rank(int lane) { return ((lane >> 4) & (KB ? 3 : 1)) * 8; }
   static __device__ __forceinline__ uint32_t step(int i, int r) {
-    return KB ? (uint32_t)((i / FRAG_KB) * 4 * r + (i % FRAG_KB) * 32) : (uint32_t)(i * 8 * r);
+    return KB ? (uint32_t)((i / FRAG_KB) * 4 * r + (i % FRAG_KB) * 32) : (uint32_t)(i * 32 * r);
   }
   static __device__ __forceinline__ bool in_rank(int i, int lane, int rk) { return lane_rank(lane) + (KB ? i % FRAG_KB * 32 : 0) < rk; }
 };
@@ -220,14 +220,14 @@ __device__ __forceinline__ void small_v_partials(const float *tile, uint32_t row
     const uint32_t at = (row + (uint32_t)(ok ? j0 : 0)) * 4u;
     float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     const char *chunk = reinterpret_cast<const char *>(tile);
-    for (int s0 = 0; s0 < ksplit; s0 += 4) {
+    auto add_four = [&](int s0) {
       f32x4 lo[4], hi[4];
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const f32x4 *src = reinterpret_cast<const f32x4 *>(chunk + at);
         lo[u] = src[0];
         hi[u] = src[1];
-        chunk += s0 + u + 1 < ksplit ? stride * 4 : 0;
+        chunk = next_chunk(chunk, s0 + u + 1 < ksplit, stride * 4);
       }
       requested();
 #pragma unroll
@@ -236,28 +236,34 @@ __device__ __forceinline__ void small_v_partials(const float *tile, uint32_t row
 #pragma unroll
           for (int i = 0; i < 4; ++i) { f[i] += lo[u][i]; f[4 + i] += hi[u][i]; }
         }
-    }
+    };
+    // (the first four outside the loop: a loop's loads wait for whatever was requested before it)
+    add_four(0);
+    for (int s0 = 4; s0 < ksplit; s0 += 4) add_four(s0);
     const u32x4 v = pack8<T>(f);
     vfrag[kb] = ok ? v : u32x4{0, 0, 0, 0};
   }
 }
 // The lane's outputs of y: 16 from o_wave + 16 * (lane / 16) on, in two 16-byte halves.
+template <int KB>
 struct SmallY {
   u32x4 v[2];
   uint16_t *p;
   bool ok[2];
 };
-__device__ __forceinline__ void small_load_y(SmallY &s, uint16_t *y, int tok, bool on, uint32_t o_wave, uint32_t h_out, int lane) {
-  const uint32_t o = o_wave + (uint32_t)(lane >> 4) * 16u;
+template <int KB>
+__device__ __forceinline__ void small_load_y(SmallY<KB> &s, uint16_t *y, int tok, bool on, uint32_t o_wave, uint32_t h_out, int lane) {
+  const uint32_t o = o_wave + (uint32_t)(lane >> 4) * (KB ? 16u : 8u);
+  constexpr uint32_t H = KB ? 8u : 32u;
   s.p = reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(y) + (uint64_t)(uint32_t)tok * (h_out * 2u)) + o;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    s.ok[h] = on && o + 8u * h < h_out;
-    s.v[h] = load16(o + 8u * h < h_out ? s.p + h * 8 : y);   // (lanes without a token read the first one's row)
+    s.ok[h] = on && o + H * h < h_out;
+    s.v[h] = load16(o + H * h < h_out ? s.p + h * (KB ? 8 : 32) : y);   // (lanes without a token read the first one's row)
   }
 }
-template <typename T>
-__device__ __forceinline__ void small_add(SmallY &s, const f32x4 (&acc)[4], float scale) {
+template <typename T, int KB>
+__device__ __forceinline__ void small_add(SmallY<KB> &s, const f32x4 (&acc)[4], float scale) {
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     float f[8];
@@ -267,10 +273,11 @@ __device__ __forceinline__ void small_add(SmallY &s, const f32x4 (&acc)[4], floa
     s.v[h] = pack8<T>(f);
   }
 }
-__device__ __forceinline__ void small_store_y(const SmallY &s) {
+template <int KB>
+__device__ __forceinline__ void small_store_y(const SmallY<KB> &s) {
 #pragma unroll
   for (int h = 0; h < 2; ++h)
-    if (s.ok[h]) store16(s.p + h * 8, s.v[h]);
+    if (s.ok[h]) store16(s.p + h * (KB ? 8 : 32), s.v[h]);
 }
 
 }  // namespace mlora

@@ -68,6 +68,13 @@ __device__ __forceinline__ void lds_write16(uint32_t off, u32x4 v) {
 }
 // loads requested above stay above: the compiler would rather sink them to where they are used
 __device__ __forceinline__ void requested() { asm volatile("" ::: "memory"); }
+// The next of a row of chunks that are requested together, or the same again: the compiler must not see that it may be the
+// same, or it branches around the load, one round trip per chunk.
+__device__ __forceinline__ const char *next_chunk(const char *chunk, bool more, int64_t stride) {
+  chunk += more ? stride : 0;
+  asm volatile("" : "+s"(chunk));
+  return as_global(chunk);
+}
 // makes v "produced here" for the compiler, so nothing that uses it moves above a preceding wait
 __device__ __forceinline__ void pin(u32x4 &v) { asm volatile("" : "+v"(v)); }
 

@@ -158,7 +158,7 @@ struct DecodeArgs {
   int spin_limit;             // 10 ns ticks an expand item waits for its tile's stamps before it computes the partials itself
 };
 int launch_decode(hipStream_t st, const DecodeArgs &a, int max_rank, mlora_dtype dt);
-int decode_bn(int max_rank);   // output columns per expand item of the one-launch op
+int decode_bn();   // output columns per expand item of the one-launch op
 size_t decode_partial_floats(int64_t n_tiles, int n_targets, int ksplit, int64_t rp);
 int launch_plan(hipStream_t st, int32_t *plan, const PlanLayout &L, const int64_t *ids,
                 const int64_t *a_start, const int64_t *a_len, int n_slots, int bm_s, int bm_e, int merged);

@@ -2,10 +2,7 @@
 //
 // shrink_kernel: one workgroup (4 waves) owns one adapter-grouped tile of up to 16*MB tokens and one K chunk
 // (shrink_core.h has the loads and the products).  Bound by its chain of round trips, not by bytes: tile record ->
-// look-ups -> operand loads -> cross-wave sum -> hand-over of the K chunks.  Measured on 512 tokens over 128 adapters
-// of rank 128 (4096 wide, 122 MB of A per target) 60 -> 54 us a launch, on 77 tokens over 33 adapters of rank 8-64
-// (5120 wide) 12.7 -> 11.8, on 256 tokens over 64 adapters of rank 16 7.2 -> 7.0, by loading whole lines, one
-// round trip for all look-ups and two barriers instead of four for the cross-wave sum.
+// look-ups -> operand loads -> cross-wave sum -> hand-over of the K chunks (what it measured is in shrink_core.h).
 // shrink_gemm_kernel: 128- and 256-token tiles.
 //
 // Split-K without atomics: every workgroup writes its fp32 partial tile and is done; the chunks
@@ -13,6 +10,8 @@
 //
 // Reference semantics: valora/csrc/bgmv/bgmv_impl.cuh:14-148 (per-token gather mat-vec with the
 // rank rows gathered through loc_indicies, fp32 accumulation, one T store per output).
+#include <type_traits>
+
 #include "kernel_common.h"
 #include "shrink_core.h"
 
@@ -140,21 +139,21 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(int h_flags, ShrinkA
 
 // The leading scalar parameters repeat what the first dependent load (the tile record) needs: with kernel-argument
 // preloading they arrive in registers at launch, so that load does not wait for a load of the argument block.
-// Waves per SIMD the register allocator has to leave room for: as many as do without spills.
+// Waves per SIMD the register allocator has to leave room for.  (A few tiles spill 12 to 28 registers at their look-ups; a wave less
+// for those measured slower on big grids.)
 constexpr int shrink_min_waves(int mb, int nb) { return mb + nb <= 3 ? 4 : nb == 8 ? 3 - mb : mb * nb <= 8 ? 3 : 2; }
 template <typename T, int MB, int NB>
 __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
                                                      int h_n_tiles, ShrinkArgs args_in) {
   int tile_idx, z_idx, s;
   const bool compensate = (h_reduce_here & SHRINK_COMPENSATE) != 0;
-  if (h_reduce_here & ~SHRINK_COMPENSATE) {
-    // The K chunks of a tile are summed by whichever of them finishes last, out of the L2 they share: the id
-    // mod 8 selects the XCD, so all chunks (and targets) of a tile get ids that agree mod 8.
-    const int per_tile = h_n_targets * h_ksplit;
-    const int local = blockIdx.x >> 3, tl = local / per_tile, rem = local - tl * per_tile;
-    tile_idx = tl * 8 + (blockIdx.x & 7);
-    z_idx = rem / h_ksplit;
-    s = rem - z_idx * h_ksplit;
+  const int reduce_here = h_reduce_here & ~SHRINK_COMPENSATE;
+  if (reduce_here) {
+    // The K chunks of a tile are summed by whichever of them finishes last, out of the L2 they share: the id mod 8
+    // selects the XCD, so all chunks (and targets) of a tile get ids that agree mod 8: grid (8 tiles x chunks, targets, 8 tiles).
+    s = (int)blockIdx.x >> 3;
+    z_idx = (int)blockIdx.y;
+    tile_idx = (int)blockIdx.z * 8 + ((int)blockIdx.x & 7);
     if (tile_idx >= h_n_tiles) return;
   } else {
     // workgroup id = (tile * targets + target) * ksplit + K chunk.  The id mod 8 selects the XCD, so
@@ -201,14 +200,16 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
   }
   // this K chunk's fp32 partial (ordinary stores).  Where the chunks are not summed here, a later launch on the
   // stream does it -- shrink_reduce_kernel, or the expand itself for small batches -- in index order, rounding once.
-  const int pq = p.reduce_here ? p.prp >> 2 : quarter;
-  {
-    f32x4 *part = reinterpret_cast<f32x4 *>(p.partial) + ((int64_t)s * p.T + pos0) * pq;
+  const uint32_t pq = (uint32_t)(reduce_here ? p.prp >> 2 : quarter);
+  const int64_t sstride = (int64_t)p.T * pq * 16;         // bytes between chunks
+  char *const part = as_global(reinterpret_cast<char *>(p.partial)) + (int64_t)pos0 * pq * 16;
+  uint32_t at[ITEMS];                                    // of the thread's items, lanes without one on the first
 #pragma unroll
-    for (int it = 0; it < ITEMS; ++it)
-      if (on[it]) part[row[it] * pq + c4[it]] = shrink_tile_sum<NB>(s_tile, NBLK, row[it], c4[it]);
-  }
-  if (!p.reduce_here) return;
+  for (int it = 0; it < ITEMS; ++it) at[it] = on[it] ? ((uint32_t)row[it] * pq + (uint32_t)c4[it]) * 16u : 0u;
+#pragma unroll
+  for (int it = 0; it < ITEMS; ++it)
+    if (on[it]) *reinterpret_cast<f32x4 *>(part + s * sstride + at[it]) = shrink_tile_sum<NB>(s_tile, NBLK, row[it], c4[it]);
+  if (!reduce_here) return;
 
   // ---- split-K summed here: every chunk leaves its partial in the L2, the last one to arrive adds them up.
   // Partials are plain stores into rows that own whole 128-byte lines (prp floats per row), so a line never
@@ -223,46 +224,57 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
   // the next launch on this plan (launches that share a plan must not overlap).
   // (Worth it for small tiles only: one workgroup reads ksplit x tile x prp x 4 bytes at L2 latency.  For
   // 128-token tiles of rank 64 that is 256 KB and measured 8.5 us, against 3.7 us for the reduce launch.)
+  // (With one item a thread and 64 of them, wave 0 holds them all: the others only wait for its verdict.)
+  constexpr bool ONE_WAVE = NBLK == 1;
   wait_vmcnt<0>();
-  __syncthreads();
-  if (tid == 0) {
-    const uint32_t xcd = xcd_id();
-    unsigned long long *word = p.arrive + (int64_t)tile_idx * MLORA_MAX_TARGETS + z_idx;
-    const unsigned long long add = 1ull + (xcd < 8 ? 1ull << (8 + 7 * xcd) : 0ull);
-    const unsigned long long now = __hip_atomic_fetch_add(word, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
-    int last = 0;
-    if ((int)(now & 0xffull) == p.ksplit) {
-      const bool all_here = xcd < 8 && (int)((now >> (8 + 7 * xcd)) & 0x7full) == p.ksplit;
-      last = (all_here && p.reduce_here == 1) ? 1 : 2;
-      __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (!ONE_WAVE) __syncthreads();
+  int last = 0;
+  if (!ONE_WAVE || tid < 64) {
+    if (tid == 0) {
+      const uint32_t xcd = xcd_id();
+      unsigned long long *word = p.arrive + (int64_t)tile_idx * MLORA_MAX_TARGETS + z_idx;
+      const unsigned long long add = 1ull + (xcd < 8 ? 1ull << (8 + 7 * xcd) : 0ull);
+      const unsigned long long now = __hip_atomic_fetch_add(word, add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + add;
+      if ((int)(now & 0xffull) == p.ksplit) {
+        const bool all_here = xcd < 8 && (int)((now >> (8 + 7 * xcd)) & 0x7full) == p.ksplit;
+        last = (all_here && reduce_here == 1) ? 1 : 2;
+        __hip_atomic_store(word, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      s_last = last;
     }
-    s_last = last;
   }
   __syncthreads();
-  const int last = s_last;
+  last = s_last;
   if (last == 0) return;
   f32x4 v[ITEMS];
 #pragma unroll
   for (int it = 0; it < ITEMS; ++it) v[it] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (last == 1) {
+    if (ONE_WAVE && tid >= 64) return;
     // v[row, :] = T(0 + p_0 + p_1 + ...): the order shrink_reduce_kernel uses.  The loads of a batch of chunks are
-    // requested for all of the thread's items together.
-    constexpr int BATCH = ITEMS <= 2 ? 8 : 4;
-    const f32x4 *src = reinterpret_cast<const f32x4 *>(p.partial) + (int64_t)pos0 * pq;
-    const int64_t sstride = (int64_t)p.T * pq;
-    for (int s0 = 0; s0 < p.ksplit; s0 += BATCH) {
-      f32x4 q[ITEMS][BATCH];
+    // requested for all of the thread's items together (the last chunk again where there are fewer).
+    auto add_chunks = [&](auto batch) {
+      constexpr int BATCH = decltype(batch)::value;
+      const char *chunk = part;
+      for (int s0 = 0; s0 < p.ksplit; s0 += BATCH) {
+        f32x4 q[ITEMS][BATCH];
 #pragma unroll
-      for (int it = 0; it < ITEMS; ++it)
+        for (int u = 0; u < BATCH; ++u) {
+#pragma unroll
+          for (int it = 0; it < ITEMS; ++it) q[it][u] = *reinterpret_cast<const f32x4 *>(chunk + at[it]);
+          chunk = next_chunk(chunk, s0 + u + 1 < p.ksplit, sstride);
+        }
+        requested();
 #pragma unroll
         for (int u = 0; u < BATCH; ++u)
-          q[it][u] = (s0 + u < p.ksplit && on[it]) ? src[(s0 + u) * sstride + row[it] * pq + c4[it]]
-                                                   : f32x4{0.f, 0.f, 0.f, 0.f};
+          if (s0 + u < p.ksplit) {   // wave-uniform
 #pragma unroll
-      for (int it = 0; it < ITEMS; ++it)
-#pragma unroll
-        for (int u = 0; u < BATCH; ++u) v[it] += q[it][u];
-    }
+            for (int it = 0; it < ITEMS; ++it) v[it] += q[it][u];
+          }
+      }
+    };
+    if (ITEMS > 2 || p.ksplit <= 4) add_chunks(std::integral_constant<int, 4>{});
+    else add_chunks(std::integral_constant<int, ITEMS <= 2 ? 8 : 4>{});
   } else {
     // the chunks were not all written through this XCD's L2 (or the caller asked for this path): compute them
     // here, one after the other.  (The empty asm keeps the compiler from computing this path's addresses early and
@@ -565,6 +577,8 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   if (a.reduce_here) grid_tiles = (grid_tiles + 7) / 8 * 8;   // ids are dealt to the 8 XCDs tile by tile
   if (grid_tiles * a.ksplit * a.n_targets > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");
   dim3 grid((unsigned)(grid_tiles * a.ksplit * a.n_targets));
+  if (a.reduce_here)
+    grid = dim3((unsigned)(8 * a.ksplit), (unsigned)a.n_targets, (unsigned)(grid_tiles / 8));   // at most 4096 tokens (csrc/api.hip)
   return dt == MLORA_F16 ? launch_shrink_t<_Float16>(st, a, bm, nb, grid)
                          : launch_shrink_t<__bf16>(st, a, bm, nb, grid);
 }

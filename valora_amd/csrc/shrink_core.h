@@ -40,11 +40,17 @@ __device__ __forceinline__ f32x4 shrink_tile_sum(const float *lds, int nblk, int
   return (w0 + w2) + (w1 + w3);
 }
 
+// What a lane without anything to fetch reads, as far as the steps of a batch reach.
+__device__ const __align__(128) uint16_t g_shrink_zeros[3 * 4 * SHRINK_KSTEP + SHRINK_KSTEP] = {};
+constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1; }
 // Leaves the four waves' shares of the fp32 result of K range [kbeg, kend) in `lds` (shrink_lds_floats(MB * NB) floats,
 // 16-byte aligned), for shrink_tile_sum to add up (rows = tokens of the tile, columns = rank); every thread of the
 // workgroup must call it, none may still be reading `lds`, and all have passed a barrier when it returns.
 // U: K steps in flight per wave.  The order of the sums does not depend on it.
-constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1; }
+// Bound by the instructions of one wave in a row, and by what a compute unit takes in.  Rows that are not there are a choice of
+// address, not a mask: a mask, four zeroed registers and a branch around each of a batch's 16 loads took 1400 cycles to issue.
+// One target, cold layers, masked / like this: 1 token of rank 16 4.9 / 4.0 us, 256 over 64 adapters 6.7 / 5.7, 200 over 16 of rank 32
+// 7.6 / 6.5, 77 over ranks 8-64 8.8 / 7.9, 256 over 64 of rank 64 11.6 / 10.9, 512 over 128 of rank 128 29.5 / 28.4.
 template <typename T, int MB, int NB, int U = shrink_steps(MB + NB)>
 __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ x, int h_in, const PoolDev &pool,
                                                    int slot, const int32_t *__restrict__ perm, int r, int pos0,
@@ -54,6 +60,7 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
   using vec8 = typename Tr::vec8;
   constexpr int NBLK = MB * NB;
   constexpr int BLKS = MB + NB;                         // 16-row blocks of a K step, x first
+  constexpr bool MANY = NB > 2;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, kg = lane >> 4;           // MFMA operand roles
   const int grow = lane >> 3, gcol = lane & 7;          // loader roles: row within a group of 8, 16-byte chunk
@@ -65,34 +72,43 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
   const int64_t *const a_loc = indexed ? pool.a_loc : reinterpret_cast<const int64_t *>(perm);
   int tok[MB][2];
   int64_t prow[NB][2];
-  bool ok[BLKS][2];
+  bool ok[NB][2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
 #pragma unroll
     for (int mb = 0; mb < MB; ++mb) {
       const int row = mb * 16 + u * 8 + grow;
-      ok[mb][u] = row < cnt;
-      tok[mb][u] = perm[pos0 + (row < cnt ? row : 0)];
+      tok[mb][u] = perm[pos0 + (row < cnt ? row : 0)];   // (a row past the tile's end reads the first one's)
     }
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       const int j = nb * 16 + u * 8 + grow;
-      const int64_t idx = base + j;
-      ok[MB + nb][u] = indexed && j < r && idx >= 0 && idx < pool.a_loc_len;
-      prow[nb][u] = a_loc[ok[MB + nb][u] ? idx : 0];
+      // (up to rank 32 a row past the rank reads the last one, its results are never used; above, where whole blocks may
+      // be missing, it reads zeros that stay in the cache)
+      const int64_t idx = base + (MANY ? j : min(j, r - 1));
+      ok[nb][u] = indexed && (!MANY || j < r) && idx >= 0 && idx < pool.a_loc_len;
+      prow[nb][u] = a_loc[ok[nb][u] ? idx : 0];
     }
   }
   const uint16_t *rp[BLKS][2];
+  int step[NB][2];          // MANY: all bits where the row moves on with K, none where it stays on its zeros
+  bool all = true;
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb) rp[mb][u] = x + (int64_t)tok[mb][u] * h_in + gcol * 8;
+    for (int mb = 0; mb < MB; ++mb) rp[mb][u] = x + (uint64_t)(uint32_t)tok[mb][u] * (uint32_t)h_in + gcol * 8;
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      ok[MB + nb][u] = ok[MB + nb][u] && prow[nb][u] >= 0 && prow[nb][u] < pool.w_rows;
-      rp[MB + nb][u] = pool.w + (ok[MB + nb][u] ? prow[nb][u] : 0) * h_in + gcol * 8;
+      ok[nb][u] = ok[nb][u] && prow[nb][u] >= 0 && prow[nb][u] < pool.w_rows;
+      all = all && ok[nb][u];
+      rp[MB + nb][u] = pool.w + (uint64_t)(uint32_t)(ok[nb][u] ? prow[nb][u] : 0) * (uint32_t)h_in + gcol * 8;
+      step[nb][u] = ok[nb][u] ? -1 : 0;
+      if (MANY && !ok[nb][u]) rp[MB + nb][u] = as_global(g_shrink_zeros) + gcol * 8;
     }
   }
+  // whole batches can be loaded as they are: rows that are not there read zeros anyway, or there are none
+  // (64-token tiles of rank 64: the addresses of both loops at once would spill)
+  const bool plain = MB * NB < 16 && (MANY || __builtin_amdgcn_ballot_w64(!all) == 0ull);
 
   // where this lane's chunks sit in a staged block: row u*8 + grow / chunk gcol when it writes what it loaded,
   // row lrow / chunk 4*c + kg when it reads operand c (K elements c*32 + kg*8 .. + 8 of the step)
@@ -108,20 +124,8 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // The trip count must be wave-uniform: MFMA ignores EXEC, so a lane that left the loop early
-  // would still feed its stale registers into the matrix core.  Lanes past the end load zeros.
-  for (int kb0 = kbeg + wave * SHRINK_KSTEP; kb0 < kend; kb0 += 4 * SHRINK_KSTEP * U) {
-    u32x4 buf[U * BLKS][2];
-#pragma unroll
-    for (int uu = 0; uu < U; ++uu) {
-      const int k = kb0 + uu * 4 * SHRINK_KSTEP;
-      const bool kok = k + gcol * 8 < kend;
-#pragma unroll
-      for (int b = 0; b < BLKS; ++b)
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-          buf[uu * BLKS + b][u] = (ok[b][u] && kok) ? load16(rp[b][u] + k) : u32x4{0, 0, 0, 0};
-    }
+  u32x4 buf[U * BLKS][2];
+  auto use = [&]() {
 #pragma unroll
     for (int b0 = 0; b0 < U * BLKS; b0 += SHRINK_STAGE_BLOCKS) {
 #pragma unroll
@@ -142,7 +146,7 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
 #pragma unroll
       for (int b = b0; b < b0 + SHRINK_STAGE_BLOCKS && b < U * BLKS; ++b) {
         const int uu = b / BLKS, nb = b % BLKS - MB;
-        if (nb >= 0 && nb * 16 < r) {
+        if (nb == 0 || (nb > 0 && nb * 16 < r)) {
 #pragma unroll
           for (int c = 0; c < 2; ++c)
 #pragma unroll
@@ -151,6 +155,41 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
         }
       }
     }
+  };
+  // The trip counts must be wave-uniform: MFMA ignores EXEC, so a lane that left a loop early would still feed its stale
+  // registers into the matrix core.
+  // Whole batches: a load is an instruction, the steps of a batch are offsets in it.
+  int kb0 = kbeg + wave * SHRINK_KSTEP;
+  for (; plain && kb0 + (4 * U - 3) * SHRINK_KSTEP <= kend; kb0 += 4 * SHRINK_KSTEP * U) {
+#pragma unroll
+    for (int b = 0; b < BLKS; ++b)
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        const uint16_t *const src = rp[b][u] + (MANY && b >= MB ? kb0 & step[b < MB ? 0 : b - MB][u] : kb0);
+#pragma unroll
+        for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16(src + uu * 4 * SHRINK_KSTEP);
+      }
+    requested();
+    use();
+  }
+  // what is left of the chunk, less than a batch (or all of it, where a rank row lies outside the index or the pool): steps and
+  // lanes past its end read zeros, and so do rows that are not there
+  for (; kb0 < kend; kb0 += 4 * SHRINK_KSTEP * U) {
+#pragma unroll
+    for (int uu = 0; uu < U; ++uu) {
+      const int k = kb0 + uu * 4 * SHRINK_KSTEP;
+      const bool kok = k + gcol * 8 < kend;
+#pragma unroll
+      for (int b = 0; b < BLKS; ++b)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const int nb = b < MB ? 0 : b - MB;
+          buf[uu * BLKS + b][u] = load16(as_global(kok && (b < MB || ok[nb][u]) ? rp[b][u] + k : g_shrink_zeros));
+        }
+    }
+    requested();
+    use();
+    if (MANY && MB * NB < 16) break;   // (it is less than a batch)
   }
 
   // Every wave leaves its share as it is (C layout: column = lane%16, rows = 4*(lane/16)+i) and whoever needs an

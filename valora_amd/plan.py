@@ -170,8 +170,8 @@ class LoraPlan:
         """Several targets that read the same ``x`` (q, k, v of a layer; gate and up) in two launches:
         ``ys[i] += scale_a * (x @ A_a[slots[i]].T) @ B_a[slots[i]]``.  ``value_buffers`` is one pool tensor or
         one per target.  Same results as ``apply`` called once per target."""
-        # (a call whose expand half is too many items per tile -- gate+up; from rank 64 on q+k+v too -- is run as two
-        # launches by the library whatever the flag says: same tiles, same split, same bits)
+        # (a call that two launches are faster for -- gate+up, ranks above 32, more than four K chunks -- is run as two
+        # by the library whatever the flag says: same tiles, same split, same bits)
         self._native.apply_multi(ys, x, key_buffer, value_buffers, a_start, a_len, a_loc, slots, scales)
 
     def apply(self, y: torch.Tensor, x: torch.Tensor, key_buffer: torch.Tensor, value_buffer: torch.Tensor,
