@@ -112,3 +112,52 @@ def test_one_or_two_launches(dev, rank, ksplit, T, n_targets):
     if rank <= 32 and need < _lib.lib().mlora_scratch_bytes(T, rank, two.ksplit) * n_targets:
         for a, b in zip(run(one, need), want):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("T", [1, 22, 300])
+@pytest.mark.parametrize("ksplit", [2, 4, 5, 9])
+@pytest.mark.parametrize("ranks", [[16], [24, 32], [48, 8], [64, 16], [96, 72], [128, 40]])
+def test_sum_in_a_launch_of_its_own(dev, T, ksplit, ranks):
+    """The launch that sums the chunks of tall tiles: rows of 4 to 32 quarters (12, 20 and 24 leave threads of a workgroup without
+    one), fewer and more chunks than it requests at once -- the bits of the expand that sums them itself -- and the caller's own
+    matrix in its three modes."""
+    print(T, ksplit, ranks, flush=True)
+    g = torch.Generator().manual_seed(T + ksplit)
+    A, h_in, h_out, R = len(ranks), 2312, 264, max(ranks)
+    pool = W.make_pool(ranks, h_in, h_out, torch.float16, g, True, n_slots=2, std=0.05, scalings=[0.5] * A, heads=1)
+    ids = torch.randint(-1, A, (T,), generator=g)
+    x, y0 = torch.randn(T, h_in, generator=g).half().to(dev), torch.randn(T, h_out, generator=g).half()
+    p = pool.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    got = []
+    for rie in (True, False):
+        plan = LoraPlan(ids.to(dev), *idx[:2], R, n_slots=2, hidden=h_in, bm_shrink=128, bm_expand=32, ksplit=ksplit, reduce_in_expand=rie,
+                        one_launch=False)
+        ys = [y0.to(dev), y0.to(dev)]
+        plan.apply_multi(ys, x, p.key_buffer, p.value_buffer, *idx, [1, 0], p.a_scaling)
+        got.append(ys)
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+    lib, pa = _lib.lib(), _lib.make_pool(p.key_buffer, *idx, h_in, 2)
+    rk = torch.tensor(ranks)[ids.clamp(min=0)] * (ids >= 0)
+    inside = (torch.arange(R)[None] < rk[:, None]).to(dev)
+    width = R + 8
+    before = torch.randn(T, width, generator=g).half().to(dev)
+    out = {}
+    for mode in (0, 1, 2):
+        d = before.clone()
+        _lib.check(lib.mlora_shrink(_lib.current_stream(dev), plan.handle, _lib.ptr(plan.scratch), plan.scratch.numel(), _lib.ptr(x), T, h_in, R, pa,
+                                    1, ksplit, _lib.ptr(d), width, mode, R, 0, _lib.dtype_code(torch.float16)))
+        torch.cuda.synchronize()
+        out[mode] = d
+    over, pad, acc = out[0], out[1], out[2]
+    has = (ids >= 0).to(dev)[:, None]
+    assert torch.equal(over[:, R:], before[:, R:])
+    # accumulate adds the unrounded sum: within one rounding of (what was there + the rounded sum)
+    v = torch.where(inside, over[:, :R], torch.zeros_like(before[:, :R])).float()
+    want = torch.where(inside, before[:, :R].float() + v, before[:, :R].float())
+    tol = 2.0 ** -11 * (v.abs() + 2 * want.abs()) + 2.0 ** -24
+    assert bool(((acc[:, :R].float() - want).abs() <= tol).all())
+    assert torch.equal(pad[:, :R], torch.where(has, torch.where(inside, over[:, :R], torch.zeros_like(before[:, :R])),
+                                                             before[:, :R]))
+    assert torch.equal(torch.where(inside, before[:, :R], over[:, :R]), before[:, :R])
