@@ -148,18 +148,17 @@ bool sum_in_expand(int flags, int bm_expand, int64_t T, int64_t h_out, int n_tar
   return bm_expand != 16 || T * ((h_out + 63) / 64) * n_targets * ksplit * rp * 4 <= (int64_t)10 << 20;
 }
 
+// Expand items per tile (512-column chunks x targets) up to which a call that asks for one launch gets it: beyond, the expand half
+// outweighs the hand-off.  Cold layers, one launch / two, us: up to 30 items (q+k+v, or one gate / up, of 4096- and 5120-wide models) at
+// rank 16 one target of 128 tokens 8.5 / 9.6, of 256 9.6 / 10.9; q+k+v of 64 13.3 / 14.0, of 256 19.9 / 19.5, of 512 22.1 / 24.4;
+// gate+up of 11008 columns (44 items) 26.5 / 24.0.
 constexpr int64_t ONE_LAUNCH_MAX_ITEMS = 32;
-// Whether a call that asks for one launch gets it (cold layers, one launch / two, us).
+// Whether one launch is the faster form of such a call (cold layers, one launch / two, us on the device; a call of a few tokens keeps its
+// one launch for the host's sake: q+k+v of one token 6.5 / 6.1, but 64 such calls in a row from Python 365 / 400-420).
 bool one_launch_pays(int64_t T, int64_t A, int64_t items, int64_t max_rank, int n_targets, int ksplit) {
-  // Expand items per tile (512-column chunks x targets), ONE_LAUNCH_MAX_ITEMS: the expand half outweighs the hand-off beyond.
-  // Up to 30 (q+k+v, or one gate / up, of 4096- and 5120-wide models) at rank 16: one target of 128 tokens 8.5 / 9.6, of 256
-  // 9.6 / 10.9; q+k+v of 64 13.3 / 14.0, of 256 19.9 / 19.5, of 512 22.1 / 24.4; gate+up of 11008 columns (44 items) 26.5 / 24.0.
   // An expand item reads four chunks in one round trip: with more of them two launches win.  200 tokens, q+k+v of 5120 columns in five
   // chunks: rank 8 14.3 / 13.2, rank 32 21.2 / 18.6; one target of 32 tokens of rank 32 in eight 9.0 / 8.2, of 128 10.4 / 10.8.
   if (ksplit > 4) return false;
-  // A handful of tokens and several targets: all items of a tile run on one XCD, those of two launches on all eight.
-  // q+k+v of one token 6.5 / 6.1, two 6.8 / 6.5, four 7.0 / 6.7, eight 7.1 / 7.3.
-  if (T <= 4 && n_targets > 2) return false;
   // Above rank 16 three workgroups fit on a compute unit instead of four, and a grid of more than about five a unit loses: rank 32, one
   // target of 256 tokens over 16 adapters (384 workgroups) 9.2 / 10.7, over 64 (960) 14.1 / 15.3, of 400 over 128 (1836) 22.5 / 21.8; q+k+v
   // of 256 over 16 (1152) 17.4 / 18.5, over 64 (2880) 28.6 / 28.1.

@@ -126,6 +126,9 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
   const int64_t stride = (int64_t)p.T * h_quarter * 16;
   const int32_t *__restrict__ plan = as_global(h_plan);
   const int n_active = plan[H_NACTIVE], merged_rank = plan[H_MERGED_RANK];
+  // (a compensation leaves most positions out: what it would read for them costs more than to wait for the count first; 6246
+  // tokens of rank 128, most of them with the merged adapter, a pass of 14 layers SHRINK_COMP)
+  if ((h_flags & SHRINK_COMPENSATE) && pos0 >= n_active) return;
   const int own_rank = (plan + p.off_prank)[pos], tok = (plan + p.off_perm)[pos];
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
   auto add_chunks = [&](auto batch, int s0) {
