@@ -245,10 +245,7 @@ def _layer_batches(n_tokens, n_adapters, rank, hidden, dev, dtype, copies_bytes=
             plan = LoraPlan(ids, idx[0], idx[1], rank, hidden=hidden, bm_shrink=cfg["bm_shrink"], ksplit=cfg["ksplit"],
                             bm_expand=cfg["bm_expand"], reduce_in_expand=planned and cfg["reduce_in_expand"],
                             one_launch=planned and cfg.get("one_launch", False))
-            times = []
-            for rep in range(loops + 1):
-                e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-                e0.record()
+            def run():
                 for x, attn, ys, kb, vb in layers:
                     if not planned:
                         for slot, y in enumerate(ys):
@@ -258,10 +255,22 @@ def _layer_batches(n_tokens, n_adapters, rank, hidden, dev, dtype, copies_bytes=
                         plan.apply(ys[3], attn, kb, vb, *idx, 3, scaling)
                     else:
                         plan.apply(ys[0], x, kb, vb, *idx, 0, scaling)
+
+            # replayed from a graph: what the host needs for a launch is not what a tile is chosen by
+            run()
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph):
+                run()
+            times = []
+            for rep in range(loops + 1):
+                e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+                e0.record()
+                graph.replay()
                 e1.record()
                 torch.cuda.synchronize()
                 if rep:
                     times.append(e0.elapsed_time(e1) * 1e3 / len(layers))
+            graph.reset()
             return sorted(times)[len(times) // 2]
 
         yield us
