@@ -127,7 +127,7 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
   const int32_t *__restrict__ plan = as_global(h_plan);
   const int n_active = plan[H_NACTIVE], merged_rank = plan[H_MERGED_RANK];
   // (a compensation leaves most positions out: what it would read for them costs more than to wait for the count first; 6246
-  // tokens of rank 128, most of them with the merged adapter, a pass of 14 layers SHRINK_COMP)
+  // tokens of rank 128, most of them with the merged adapter, a pass of 14 layers 4530 us, so 4349)
   if ((h_flags & SHRINK_COMPENSATE) && pos0 >= n_active) return;
   const int own_rank = (plan + p.off_prank)[pos], tok = (plan + p.off_perm)[pos];
   f32x4 v = {0.f, 0.f, 0.f, 0.f};
