@@ -56,8 +56,9 @@ enum {
                                  buffer aligned to less, an empty index or an empty pool make the call
                                  run as two launches, and so does what two launches measured faster for:
                                  more than 32 expand items per tile -- 512-column chunks x targets --,
-                                 ksplit above 4, ranks above 32, big grids above rank 16).  Any batch size: items the device cannot
-                                 hold from the start take part in the hand-off like the others.
+                                 ksplit above 4, ranks above 32, big grids above rank 16).  Any batch
+                                 size: items the device cannot hold from the start take part in the
+                                 hand-off like the others.
                                  Bit-identical to the two-launch op with MLORA_REDUCE_IN_EXPAND and the
                                  same ksplit.  Launches that share a plan must not overlap in time.  */
   MLORA_ONE_LAUNCH_NO_WAIT = 4, /* with MLORA_ONE_LAUNCH: expand items do not wait at all and always
