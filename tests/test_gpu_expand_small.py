@@ -74,3 +74,24 @@ def test_more_tiles_than_a_grid_dimension(dev):
         got.append(y)
     assert torch.equal(*got)
 
+
+
+@pytest.mark.parametrize("T", [16 * 65533, 16 * 65534, 16 * 65535 + 40])
+def test_tiles_around_a_grid_dimension_on_a_used_plan(dev, T):
+    """65535, 65536 and 65540 tile records.  The words behind them number the one-launch calls on the plan: after such a
+    call they are no longer zero, and a two-launch call on the same plan must not take them for records."""
+    p, ids, x, y0 = _case(dev, T, 8, 72, [16, 8], torch.float16, 6, hole=False)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    pools = (p.key_buffer, p.value_buffer, *idx, 1)
+    used = LoraPlan(ids, *idx[:2], 16, n_slots=2, hidden=8, ksplit=2, one_launch=True)
+    print(T, "one launch", flush=True)
+    first = y0.clone()
+    used.apply(first, x, *pools, p.a_scaling)
+    print(T, "two launches on the same plan", flush=True)
+    got = y0.clone()
+    used.shrink(x, p.key_buffer, *idx, 1)
+    used.expand(got, p.value_buffer, *idx, 1, p.a_scaling)
+    tall = LoraPlan(ids, *idx[:2], 16, n_slots=2, hidden=8, bm_shrink=16, bm_expand=128, ksplit=2, reduce_in_expand=True, one_launch=False)
+    want = y0.clone()
+    tall.apply(want, x, *pools, p.a_scaling)
+    assert torch.equal(first, want) and torch.equal(got, want)

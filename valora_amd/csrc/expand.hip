@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 // (Two or four column chunks a workgroup, all their loads in flight together, lose wherever the narrow operand is finished: 512
 // tokens, q+k+v at rank 16 26.1 / 27.5 us with its shrink, one target of 256 tokens, 11008 columns 8.6 / 9.6, ranks 8-64, gate+up
 // of 13824 columns 25.2 / 27.4.)
-constexpr int SMALL_GRID_Y = 65535;
+constexpr int64_t SMALL_MAX_TILES = 65535;   // tiles of one launch: grid y is 16 bits
 constexpr int small_min_waves(int kb, bool wide, bool comp) {   // as many as do without spills
   return comp ? (kb <= 1 ? 7 : 1) : kb <= 1 ? 8 : kb == 2 ? (wide ? 6 : 5) : (wide ? 4 : 3);
 }
@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
                                                                                          ExpandArgs p) {
   using Tr = Traits<T>;
   constexpr int FKB = SmallB<KB>::FRAG_KB;
-  const int tile_idx = (int)blockIdx.y + (int)(blockIdx.z >> 2) * SMALL_GRID_Y, z = (int)blockIdx.z & 3;
+  const int tile_idx = (int)blockIdx.y, z = (int)blockIdx.z;
   // One scalar round trip: the tile record and every argument the wave is going to use (csrc/decode.hip has the reason for the asm).
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   asm volatile("" : "+s"(ad), "+s"(r), "+s"(pos0), "+s"(cnt), "+s"(astart), "+s"(slot), "+s"(kmax), "+s"(w_rows), "+s"(v_by_pos),
                     "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out));
   if (COMP) cnt = abs(cnt);                  // (negative: no usable rank of its own, r = 0)
-  if (cnt <= 0 || z >= p.n_targets) return;  // records past the last tile are zero
+  if (cnt <= 0) return;                      // records past the last tile are zero
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int m = lane & 15, kg = lane >> 4;
   const uint32_t o_wave = blockIdx.x * (uint32_t)EXP_BN + (uint32_t)(wave * EXP_WN);
@@ -335,19 +335,23 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
 
 template <typename T, int KB>
 int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
-  const int64_t hi = (tiles + SMALL_GRID_Y - 1) / SMALL_GRID_Y;   // grid y is 16 bits: the rest of the tile index in z, above the target
-  const dim3 grid((unsigned)a.n_ochunks, (unsigned)(hi > 1 ? SMALL_GRID_Y : tiles), (unsigned)(hi > 1 ? 4 * hi : a.n_targets));
   // an index without entries: the kernel reads one all the same, and drops it
   const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
-#define MLORA_SMALL(WIDE, PARTIAL, COMP)                                                                              \
-  hipLaunchKernelGGL((expand_small_kernel<T, KB, WIDE, PARTIAL, COMP>), grid, dim3(256), 0, st, a.plan + a.off_tiles, \
+#define MLORA_SMALL(WIDE, PARTIAL, COMP)                                                                        \
+  hipLaunchKernelGGL((expand_small_kernel<T, KB, WIDE, PARTIAL, COMP>), grid, dim3(256), 0, st, records,        \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
 #define MLORA_SMALL_WIDTH(PARTIAL, COMP)                             \
   if (KB > 0 && a.h_out >= SMALL_WIDE) MLORA_SMALL((KB > 0), PARTIAL, COMP); \
   else MLORA_SMALL(false, PARTIAL, COMP)
-  if (a.compensate) { MLORA_SMALL_WIDTH(false, true); }
-  else if (a.partial) { MLORA_SMALL_WIDTH(true, false); }
-  else { MLORA_SMALL_WIDTH(false, false); }
+  // Exactly as many workgroups as there are records: what stands behind the last one is no record (the words of the one-launch
+  // op do, and a call of that kind leaves them non-zero).  More tiles than a grid's y takes (a million tokens) are several launches.
+  for (int64_t t0 = 0; t0 < tiles; t0 += SMALL_MAX_TILES) {
+    const int32_t *records = a.plan + a.off_tiles + t0 * TILE_WORDS;
+    const dim3 grid((unsigned)a.n_ochunks, (unsigned)(tiles - t0 < SMALL_MAX_TILES ? tiles - t0 : SMALL_MAX_TILES), (unsigned)a.n_targets);
+    if (a.compensate) { MLORA_SMALL_WIDTH(false, true); }
+    else if (a.partial) { MLORA_SMALL_WIDTH(true, false); }
+    else { MLORA_SMALL_WIDTH(false, false); }
+  }
 #undef MLORA_SMALL_WIDTH
 #undef MLORA_SMALL
   return check_launch("expand_small_kernel");
