@@ -149,19 +149,24 @@ bool sum_in_expand(int flags, int bm_expand, int64_t T, int64_t h_out, int n_tar
 }
 
 // Expand items per tile (512-column chunks x targets) up to which a call that asks for one launch gets it: beyond, the expand half
-// outweighs the hand-off.  Cold layers, one launch / two, us: up to 30 items (q+k+v, or one gate / up, of 4096- and 5120-wide models) at
-// rank 16 one target of 128 tokens 8.5 / 9.6, of 256 9.6 / 10.9; q+k+v of 64 13.3 / 14.0, of 256 19.9 / 19.5, of 512 22.1 / 24.4;
-// gate+up of 11008 columns (44 items) 26.5 / 24.0.
+// outweighs the hand-off (gate+up of 11008 columns, 44 items, 256 tokens 26.5 / 24.0 us in one launch / two; a limit of 16 would
+// lose q+k+v below).
 constexpr int64_t ONE_LAUNCH_MAX_ITEMS = 32;
-// Whether one launch is the faster form of such a call (cold layers, one launch / two, us on the device; a call of a few tokens keeps its
-// one launch for the host's sake: q+k+v of one token 6.5 / 6.1, but 64 such calls in a row from Python 365 / 400-420).
+// Whether one launch is the faster form of such a call.  Cold layers, four chunks, one launch / two, us on the device, rank 16, 4096
+// columns: one target of 8 to 1000 tokens over 1 to 128 adapters 0.84 to 1.00 of the two launches' time (256 tokens over 1 adapter
+// 7.2 / 7.2, over 16 7.7 / 8.9, over 64 9.8 / 11.2; 1000 over 16 12.6 / 14.8), two targets 0.87 to 1.06, 0.95 in the median, three 0.88 to
+// 1.10, 0.98 in the median (256 tokens over 64 adapters 19.4 / 19.5, over 16 13.2 / 14.4, over 4 12.4 / 12.3; 512 over 64 21.9 / 24.1; 64
+// tokens of one adapter 7.8 / 7.0).  A call of a few tokens keeps its one launch for the host's sake: q+k+v of one token
+// 6.6 / 6.5, but 64 such calls in a row from Python 365 / 400-420.  (Full tiles of three narrow targets lose most: rank 8, 2048 columns,
+// 1000 tokens over 4 adapters 17.8 / 15.3.)
 bool one_launch_pays(int64_t T, int64_t A, int64_t items, int64_t max_rank, int n_targets, int ksplit) {
   // An expand item reads four chunks in one round trip: with more of them two launches win.  200 tokens, q+k+v of 5120 columns in five
   // chunks: rank 8 14.3 / 13.2, rank 32 21.2 / 18.6; one target of 32 tokens of rank 32 in eight 9.0 / 8.2, of 128 10.4 / 10.8.
   if (ksplit > 4) return false;
   // Above rank 16 three workgroups fit on a compute unit instead of four, and a grid of more than about five a unit loses: rank 32, one
   // target of 256 tokens over 16 adapters (384 workgroups) 9.2 / 10.7, over 64 (960) 14.1 / 15.3, of 400 over 128 (1836) 22.5 / 21.8; q+k+v
-  // of 256 over 16 (1152) 17.4 / 18.5, over 64 (2880) 28.6 / 28.1.
+  // of 256 over 16 (1152) 16.9 / 18.0, over 4 (720) 15.7 / 14.6, over 64 (2880) 28.6 / 28.1.  Below the line one and two targets take 0.85 to
+  // 1.01 of the two launches' time, three 0.89 to 1.07.
   return max_rank <= 16 || tiles_upper(T, A, 16) * (items + ksplit * n_targets) <= 1280;
 }
 
