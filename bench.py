@@ -496,7 +496,7 @@ def bench_byte_heavy_decode(torch, W, LoraPlan, dev, use_graph, reps):
         nbytes = 3 * T * H * 2 + 2 * touched * r * H * 2
         out.append({"tokens": T, "rank": r, "adapters_touched": touched, "us": round(us, 2), "bytes": nbytes,
                     "gbps": round(nbytes / us / 1e3, 1), "hbm_frac": round(nbytes / us / 1e3 / HBM_PEAK_GBPS, 3),
-                    "tile": [plan.bm_shrink, plan.ksplit, plan.bm_expand], "one_launch": plan.one_launch})
+                    "tile": [plan.bm_shrink, plan.ksplit, plan.bm_expand], "one_launch": plan.runs_in_one_launch(H)})
         del pool, x, ys, plan
         torch.cuda.empty_cache()
     return out
@@ -536,7 +536,7 @@ def bench_single_adapter_vs_gemm(torch, W, LoraPlan, dev, use_graph, reps):
         nbytes = (3 * T * H + 2 * r * H) * 2
         out.append({"tokens": T, "rank": r, "us": round(us_ours, 2), "torch_mm_addmm_us": round(us_gemm, 2),
                     "gbps": round(nbytes / us_ours / 1e3, 1), "tile": [plan.bm_shrink, plan.ksplit, plan.bm_expand],
-                    "one_launch": plan.one_launch})
+                    "one_launch": plan.runs_in_one_launch(H)})
         del pool, xs, ys, vs, plan
         torch.cuda.empty_cache()
     return out
@@ -742,7 +742,7 @@ def main():
     idx = (p.a_start, p.a_len, p.a_loc)
     use_graph = not args.no_graph
 
-    fused = plan.one_launch
+    fused = plan.runs_in_one_launch(4096)
 
     def layers_only():
         for l in range(L):

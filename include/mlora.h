@@ -60,7 +60,7 @@ enum {
                                  size: items the device cannot hold from the start take part in the
                                  hand-off like the others.
                                  Bit-identical to the two-launch op with MLORA_REDUCE_IN_EXPAND and the
-                                 same ksplit.  Launches that share a plan must not overlap in time.  */
+                                 same ksplit, raised and cut as above in either form.  Launches that share a plan must not overlap in time.  */
   MLORA_ONE_LAUNCH_NO_WAIT = 4, /* with MLORA_ONE_LAUNCH: expand items do not wait at all and always
                                  compute their tile's partials themselves (the give-up path made
                                  testable; same results, slower)                                  */
@@ -124,6 +124,10 @@ size_t mlora_scratch_bytes(int64_t T, int64_t max_rank, int32_t ksplit);
  * by tile, in whole cache lines per tile) or as two, whichever is more.                            */
 size_t mlora_one_launch_scratch_bytes(int64_t T, int64_t n_adapters, int64_t max_rank, int32_t ksplit,
                                       int32_t n_targets);
+/* Whether a call with MLORA_ONE_LAUNCH of this shape runs as one launch (1) or as two (0), given an aligned scratch
+ * buffer of mlora_one_launch_scratch_bytes() and an index and pools that are not empty.             */
+int mlora_runs_in_one_launch(int64_t T, int64_t n_adapters, int64_t max_rank, int64_t h_out, int32_t ksplit,
+                             int32_t n_targets);
 /* Bytes of scratch the one-call entry points (dispatch_bgmv, dispatch_sgmm, prefill_*) need.
  * Replaces sgmm_tmp_size (atmm/valora/csrc/bgmv/bgmv_impl.cuh:128-132).                       */
 size_t mlora_workspace_bytes(int64_t T, int64_t n_adapters, int64_t max_rank);

@@ -217,3 +217,25 @@ def test_header_is_plain_c_and_a_c_program_links_against_the_library(tmp_path):
     assert r.returncode == 0, r.stderr
     r = subprocess.run([str(exe)], capture_output=True, text=True)
     assert r.returncode == 0 and r.stdout.startswith("ok"), (r.returncode, r.stdout, r.stderr)
+
+
+def test_marks_of_the_tile_table_say_something():
+    """A mark for the one-launch op either lets a call run as one launch or cuts the split of calls of up to four targets."""
+    import json
+    from valora_amd import tile_table as tt
+    with open(tt.TABLE_PATH) as f:
+        entries = json.load(f)["entries"]
+    marked = {k: v for k, v in entries.items() if v.get("one_launch")}
+    assert marked
+    for k, v in marked.items():
+        assert (v["bm_shrink"], v["bm_expand"]) == (16, 16), k
+        assert int(k.split(":")[1]) <= 32 or v["ksplit"] * _lib.MAX_TARGETS > 16, k
+
+
+@pytest.mark.parametrize("T,A,rank,h_out,ks,nt,one", [
+    (1, 8, 16, 4096, 4, 1, 1), (256, 64, 16, 4096, 4, 3, 1), (256, 64, 16, 11008, 4, 2, 0),     # 8, 24 and 44 expand items a tile
+    (64, 8, 16, 4096, 5, 1, 0), (64, 8, 16, 4096, 8, 4, 1),                                      # five chunks; eight, cut to four
+    (256, 16, 32, 4096, 4, 3, 1), (256, 64, 32, 4096, 4, 3, 0), (8, 8, 40, 4096, 2, 1, 0),       # 1152 and 2880 workgroups; rank
+    (8, 8, 16, 0, 2, 1, 0), (-1, 8, 16, 4096, 2, 1, 0), (8, 8, 16, 4096, 2, 5, 0)])
+def test_which_calls_run_in_one_launch(T, A, rank, h_out, ks, nt, one):
+    assert _lib.lib().mlora_runs_in_one_launch(T, A, rank, h_out, ks, nt) == one

@@ -403,3 +403,23 @@ def test_operands_the_one_launch_kernel_cannot_take_run_as_two_launches(dev):
     empty = torch.empty(0, dtype=torch.long, device=dev)
     pe = _lib.make_pool(p.key_buffer, p.a_start, p.a_len, empty, 512, 4)
     assert torch.equal(call(pe, full, sp, sb), y0)
+
+
+@pytest.mark.parametrize("rank,ks,h_out,nt", [(16, 4, 512, 1), (16, 4, 520, 3), (32, 4, 1032, 2), (32, 2, 24, 1), (16, 5, 512, 1), (16, 8, 512, 2),
+                                              (16, 8, 512, 4), (40, 2, 512, 1), (64, 8, 512, 3), (16, 2, 8200, 2), (32, 2, 8200, 1)])
+def test_the_form_a_call_runs_in(dev, rank, ks, h_out, nt):
+    """``runs_in_one_launch`` against what ran: one launch moves the tiles' hand-off words on, two launches leave them."""
+    g = torch.Generator().manual_seed(rank + h_out)
+    T, A = 70, 5
+    pool = W.make_pool([rank, 8] * 2 + [rank], 264, h_out, torch.float16, g, True, heads=1).to(dev)
+    ids = torch.randint(0, A, (T,), generator=g).to(dev)
+    x = torch.randn(T, 264, generator=g).half().to(dev)
+    plan = LoraPlan(ids, pool.a_start, pool.a_len, rank, hidden=264, one_launch=True, ksplit=ks)
+    ys = [torch.zeros(T, h_out, dtype=torch.float16, device=dev) for _ in range(nt)]
+    plan.apply_multi(ys, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, list(range(nt)), pool.a_scaling)
+    up8 = lambda v: (v + 7) // 8 * 8  # noqa: E731  (plan_layout, csrc/mlora_internal.h)
+    max_tiles = (T + 15) // 16 + A
+    done = up8(up8(up8(32 + T) + T) + T) + 2 * 8 * max_tiles
+    moved = bool(plan.buf.view(torch.int32)[done:done + max_tiles].any())
+    assert moved == plan.runs_in_one_launch(h_out, nt)
+    assert moved == (rank <= 32 and min(ks, 16 // nt) <= 4 and (h_out + 511) // 512 * nt <= 32)

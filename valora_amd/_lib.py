@@ -28,7 +28,7 @@ SYMBOLS = [
     "mlora_dispatch_sgmm", "mlora_prefill_shrink", "mlora_prefill_expand",
     "mlora_pool_alloc", "mlora_pool_alloc_contiguous", "mlora_pool_free", "mlora_pool_fill",
     "mlora_pool_scatter_rows", "mlora_pool_gather_rows", "mlora_index_compact", "mlora_merge_adapter",
-    "mlora_build_compensation_plan", "mlora_lora_compensate",
+    "mlora_build_compensation_plan", "mlora_lora_compensate", "mlora_runs_in_one_launch",
 ]
 
 
@@ -74,6 +74,7 @@ def lib():
     L.mlora_scratch_bytes.argtypes = [c_int64, c_int64, c_int32]
     L.mlora_workspace_bytes.argtypes = [c_int64, c_int64, c_int64]
     L.mlora_one_launch_scratch_bytes.argtypes = [c_int64, c_int64, c_int64, c_int32, c_int32]
+    L.mlora_runs_in_one_launch.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int32, c_int32]
     for n in ("mlora_tile_lookup", "mlora_tile_fallback"):
         getattr(L, n).argtypes = [c_int64, c_int64, c_int64, c_int64, POINTER(TileConfig)]
     L.mlora_build_plan.argtypes = [c_void_p, POINTER(Plan), c_void_p, c_int64, c_void_p, c_void_p,
@@ -119,7 +120,7 @@ def lib():
                                       c_void_p]
     L.mlora_merge_adapter.argtypes = [c_void_p, POINTER(c_void_p), POINTER(c_int32), c_int32, c_int64, c_int64, c_int64,
                                       POINTER(Pool), POINTER(Pool), c_int64, c_int64, ctypes.c_float, c_int32, c_int]
-    for n in SYMBOLS[6:]:  # everything after the size queries returns a status
+    for n in SYMBOLS[6:]:  # everything after the size queries returns a status (the last one a truth value)
         getattr(L, n).restype = c_int
     _lib = L
     return L

@@ -169,6 +169,16 @@ bool one_launch_pays(int64_t T, int64_t A, int64_t items, int64_t max_rank, int 
   // 1.01 of the two launches' time, three 0.89 to 1.07.
   return max_rank <= 16 || tiles_upper(T, A, 16) * (items + ksplit * n_targets) <= 1280;
 }
+int64_t one_launch_items(int64_t h_out, int n_targets) { return (h_out + decode_bn() - 1) / decode_bn() * n_targets; }
+// The split of a call with the one-launch flag, in whichever form it runs: at least two chunks (the hand-off carries partials), and no more
+// chunks of all targets together than a tile has stamps.  (Where it runs as two launches for its rank or its chunks, the cut is no
+// loss: q+k+v of 8 to 2048 tokens, 2048 to 8192 columns, the entry's own split against 16 / 3 chunks 0.99 in the median with six chunks, 1.00
+// with eight -- 0.91 up to 64 tokens of rank 16, 1.02 at rank 64 --, 1.08 with sixteen.)
+int one_launch_ksplit(int ksplit, int n_targets) {
+  if (ksplit < 2) ksplit = 2;
+  return ksplit * n_targets > DECODE_MAX_PRODUCERS ? DECODE_MAX_PRODUCERS / n_targets : ksplit;
+}
+bool one_launch_fits(int64_t max_rank, int64_t items) { return max_rank <= 32 && items <= ONE_LAUNCH_MAX_ITEMS; }
 
 struct Carver {
   char *p;
@@ -206,11 +216,17 @@ size_t mlora_scratch_bytes(int64_t T, int64_t max_rank, int32_t ksplit) {
 size_t mlora_one_launch_scratch_bytes(int64_t T, int64_t n_adapters, int64_t max_rank, int32_t ksplit,
                                       int32_t n_targets) {
   if (T < 0 || n_adapters < 0 || max_rank < 0 || n_targets < 1) return 0;
-  if (ksplit < 2) ksplit = 2;
-  if (ksplit * n_targets > DECODE_MAX_PRODUCERS) ksplit = DECODE_MAX_PRODUCERS / n_targets;
+  ksplit = one_launch_ksplit(ksplit, n_targets);
   const size_t two = scratch_bytes(T, max_rank, ksplit) * (size_t)n_targets;   // where the call runs as two launches
   const size_t one = one_launch_bytes(T, n_adapters, max_rank, ksplit, n_targets);
   return one > two ? one : two;
+}
+
+int mlora_runs_in_one_launch(int64_t T, int64_t n_adapters, int64_t max_rank, int64_t h_out, int32_t ksplit, int32_t n_targets) {
+  if (T < 0 || n_adapters < 0 || max_rank < 0 || h_out < 1 || n_targets < 1 || n_targets > MLORA_MAX_TARGETS) return 0;
+  const int64_t items = one_launch_items(h_out, n_targets);
+  return one_launch_fits(max_rank, items) &&
+         one_launch_pays(T, n_adapters, items, max_rank, n_targets, one_launch_ksplit(ksplit, n_targets));
 }
 
 size_t mlora_workspace_bytes(int64_t T, int64_t n_adapters, int64_t max_rank) {
@@ -471,15 +487,14 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
       return fail(MLORA_ERR_NO_KERNEL, "lora_apply: the one-launch op needs a plan cut with bm_shrink = bm_expand = 16 (has %d / %d)",
                   plan->bm_shrink, plan->bm_expand);
     if (max_rank > 64) return fail(MLORA_ERR_NO_KERNEL, "lora_apply: max_rank=%lld > 64 uses the two-launch op", (long long)max_rank);
-    if (ksplit < 2) ksplit = 2;   // the hand-off carries fp32 K-chunk partials
-    if (ksplit * n_targets > DECODE_MAX_PRODUCERS) ksplit = DECODE_MAX_PRODUCERS / n_targets;
+    ksplit = one_launch_ksplit(ksplit, n_targets);
   }
   // The one-launch op hands the K-chunk partials over inside the launch, through lines of the scratch buffer that
   // belong to one tile each (128-byte aligned), and its expand items read element 0 of the index and of every
   // target's pool where they have nothing to fetch: a call that cannot offer that runs as two launches with the
   // same ksplit, which gives the same bits.
-  const int64_t items = (h_out + decode_bn() - 1) / decode_bn() * n_targets;
-  bool use_decode = one_launch && max_rank <= 32 && items <= ONE_LAUNCH_MAX_ITEMS && aligned128(scratch) && pool_a->a_loc_len > 0 && pool_a->w_rows > 0;
+  const int64_t items = one_launch_items(h_out, n_targets);
+  bool use_decode = one_launch && one_launch_fits(max_rank, items) && aligned128(scratch) && pool_a->a_loc_len > 0 && pool_a->w_rows > 0;
   for (int i = 0; use_decode && i < n_targets; ++i) use_decode = targets[i].w_b_rows > 0;
   // (a scratch buffer with just enough room for one launch keeps it)
   if (use_decode && !one_launch_pays(T, plan->n_adapters, items, max_rank, n_targets, ksplit) &&

@@ -29,8 +29,9 @@ class LoraPlan:
         """``ids``: int64 per-token adapter index (negative = no adapter); ``a_start`` / ``a_len``:
         the pool index (``a_len = n_slots * rank``); ``max_rank``: widest rank among the resident
         adapters (the reference's ``max_lora_dim``, lora_unordered_batch_infer.py:181-182).
-        ``one_launch``: shrink and expand as work items of one grid (decode-like batches; forces
-        16-token tiles, needs ``max_rank <= 64``); ``None`` takes the tile table's choice.
+        ``one_launch``: asks for shrink and expand as work items of one grid (decode-like batches; forces
+        16-token tiles and at most 16 K chunks of all targets together, needs ``max_rank <= 64``; ``runs_in_one_launch`` says
+        which calls get it); ``None`` takes the tile table's choice.
         ``one_launch_no_wait`` makes every expand item take its give-up path at once, ``one_launch_never_ready`` after
         waiting out its bound, ``shrink_recompute`` makes the 128-token shrink sum its K chunks by computing them all in
         one workgroup (all for tests); ``expand_column_loop`` is accepted and without effect."""
@@ -89,6 +90,11 @@ class LoraPlan:
         """The plan as the C ABI takes it (``mlora_plan``)."""
         buf = self._native.buf
         return _lib.Plan(_lib.ptr(buf), buf.numel(), self.T, self.n_adapters, self.bm_shrink, self.bm_expand, self.n_slots)
+
+    def runs_in_one_launch(self, h_out: int, n_targets: int = 1) -> bool:
+        """Whether a call of this plan on ``n_targets`` targets of ``h_out`` columns is one launch."""
+        return self.one_launch and bool(_lib.lib().mlora_runs_in_one_launch(self.T, self.n_adapters, self.max_rank, int(h_out),
+                                                                            self.ksplit, int(n_targets)))
 
     def rebuild(self, ids: Optional[torch.Tensor] = None) -> None:
         """Cut the tiles again, in place, for the next batch of the same size (``ids`` of the same length; None

@@ -30,7 +30,7 @@ class TileConfig:
     ksplit: int      # K-chunks the shrink is split into (partials summed by the consumer)
     bm_expand: int   # tokens per expand tile: multiple of 16 up to 256
     reduce_in_expand: bool = False  # split-K chunks summed by the expand launch (small batches)
-    one_launch: bool = False        # shrink and expand as work items of one grid (decode-like batches, rank <= 64)
+    one_launch: bool = False        # calls ask for shrink and expand as work items of one grid (decode-like batches, rank <= 64)
 
 
 def _bucket(v: int, buckets) -> int:

@@ -165,9 +165,9 @@ def tune_tall_shrink(dev, n_tokens, n_adapters, rank, hidden, entry, dtype=torch
 
 def tune_one_launch(dev, n_tokens, n_adapters, rank, hidden, entry, dtype=torch.float16, copies=4):
     """Does the one-launch op (shrink and expand items of one grid, 16-token tiles) beat the two-launch entry of
-    this shape?  Returns the entry to keep and both timings.  Only decode-like shapes qualify: rank <= 64.  The
-    library runs a call with too many expand items per tile as two launches whatever the entry says, so an
-    MLP-wide `hidden` is measured as what it is the input of, a down projection (to a 4096- or 8192-wide output)."""
+    this shape?  Returns the entry to keep and both timings.  The library runs ranks above 32, splits above 4 and calls with
+    too many expand items per tile as two launches whatever the entry says: those are not tried, and an MLP-wide `hidden` is
+    measured as what it is the input of, a down projection (to a 4096- or 8192-wide output)."""
     h_out = down_projection_width(hidden)
     ids, pool, x = synthetic_batch(n_tokens, n_adapters, rank, hidden, dtype, seed=n_tokens + n_adapters + rank, h_out=h_out)
     ids, x, p = ids.to(dev), x.to(dev), pool.to(dev)
@@ -182,7 +182,7 @@ def tune_one_launch(dev, n_tokens, n_adapters, rank, hidden, entry, dtype=torch.
     two = op_us(bm_shrink=entry["bm_shrink"], ksplit=entry["ksplit"], bm_expand=entry["bm_expand"],
                 reduce_in_expand=entry.get("reduce_in_expand", False), one_launch=False)
     best = None
-    for ks in (4, 2, 3, 6, 8):
+    for ks in (4, 2, 3):
         if ks * 128 > hidden:
             continue
         us = op_us(ksplit=ks, one_launch=True)
@@ -300,6 +300,8 @@ def tune_cold(dev, n_tokens, n_adapters, rank, hidden, entry, dtype=torch.float1
             if rank > 64 or n_tokens > 2048:
                 return None
             cfg.update(bm_shrink=16, bm_expand=16, reduce_in_expand=True, ksplit=max(2, cfg["ksplit"]))
+            if rank > 32 and cfg["ksplit"] * 4 <= 16:       # two launches, whose split the flag leaves alone
+                return None
         elif cfg["ksplit"] == 1 or n_tokens > 4096:
             cfg["reduce_in_expand"] = False
         return cfg
@@ -333,7 +335,7 @@ def main():
     ap.add_argument("--ranks", type=int, nargs="+", default=list(tt.RANK_BUCKETS))
     ap.add_argument("--out", default=tt.TABLE_PATH)
     ap.add_argument("--one-launch", action="store_true",
-                    help="revisit the existing entries of decode-like shapes (<= 2048 tokens, rank <= 64; the protected "
+                    help="revisit the existing entries of decode-like shapes (<= 2048 tokens, rank <= 32; the protected "
                          "ones too) and mark those where the one-launch op is faster than the entry's two launches")
     ap.add_argument("--tall-shrink", action="store_true",
                     help="revisit the existing entries above 4096 tokens that use 128-token shrink tiles (rank <= 64, summed "
@@ -388,7 +390,7 @@ def main():
                     json.dump(table, f, indent=1)
             continue
         if args.one_launch:
-            if k in entries and n_tokens <= 2048 and rank <= 64:
+            if k in entries and n_tokens <= 2048 and rank <= 32:
                 new, two, one = tune_one_launch(dev, n_tokens, min(n_adapters, max(1, n_tokens)), rank, hidden, entries[k])
                 # a protected entry was tuned on its real workload: the synthetic batch (which may not fit the
                 # device as one grid where the real one does) can add the mark there, never take it away
