@@ -90,27 +90,6 @@ __device__ __forceinline__ void divmod24(uint32_t n, uint32_t d, float inv_d, ui
   rem = (uint32_t)m;
 }
 
-// Walks the B operand of the expand.  A slot's B block is r pool rows that, concatenated, hold [h_out, r]
-// row-major: the 8 rank elements [j0, j0 + 8) of output column o start at flat offset o*r + j0, i.e. in the
-// slot's pool row number `bin` at element `off`.  Outputs 16 apart are 16*r elements apart, so after one
-// division the cursor moves on with an add and a compare.
-struct BCursor {
-  uint32_t bin, off;
-};
-__device__ __forceinline__ BCursor b_cursor(uint32_t o, uint32_t r, uint32_t j0, uint32_t h_out, float inv_h_out) {
-  BCursor c;
-  divmod24(o * r + j0, h_out, inv_h_out, c.bin, c.off);   // o < 2^16, r <= 2^7
-  return c;
-}
-// `step` elements further on; step < h_out
-__device__ __forceinline__ void b_advance(BCursor &c, uint32_t step, uint32_t h_out) {
-  c.off += step;
-  if (c.off >= h_out) {
-    c.off -= h_out;
-    c.bin += 1u;
-  }
-}
-
 template <typename T>
 struct Traits;
 
