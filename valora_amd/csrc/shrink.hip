@@ -153,9 +153,10 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
 
 // The leading scalar parameters repeat what the first dependent load (the tile record) needs: with kernel-argument
 // preloading they arrive in registers at launch, so that load does not wait for a load of the argument block.
-// Waves per SIMD the register allocator has to leave room for.  (A few tiles spill 12 to 28 registers at their look-ups; a wave less
-// for those measured slower on big grids.)
-constexpr int shrink_min_waves(int mb, int nb) { return mb + nb <= 3 ? 4 : nb == 8 ? 3 - mb : mb * nb <= 8 ? 3 : 2; }
+// Waves per SIMD the register allocator has to leave room for: as many as do without spills.  (Three for 64-token tiles up to rank 32
+// spill 4 and 28 registers; three / two: 4000 tokens over 32 adapters of rank 32, four chunks 12.8 / 11.6 us, eight 12.9 / 11.4; 8000 over
+// 64 of rank 16 18.4 / 16.0, of rank 32 20.6 / 18.7.)
+constexpr int shrink_min_waves(int mb, int nb) { return mb + nb <= 3 ? 4 : nb == 8 ? 3 - mb : mb == 4 ? 2 : 3; }
 template <typename T, int MB, int NB>
 __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
                                                      int h_n_tiles, ShrinkArgs args_in) {

@@ -61,6 +61,7 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
   constexpr int NBLK = MB * NB;
   constexpr int BLKS = MB + NB;                         // 16-row blocks of a K step, x first
   constexpr bool MANY = NB > 2;
+  constexpr bool WHOLE = MB == 1 || NB <= 2;            // has a loop of its own for whole batches
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, kg = lane >> 4;           // MFMA operand roles
   const int grow = lane >> 3, gcol = lane & 7;          // loader roles: row within a group of 8, 16-byte chunk
@@ -106,9 +107,11 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
       if (MANY && !ok[nb][u]) rp[MB + nb][u] = as_global(g_shrink_zeros) + gcol * 8;
     }
   }
-  // whole batches can be loaded as they are: rows that are not there read zeros anyway, or there are none
-  // (64-token tiles of rank 64: the addresses of both loops at once would spill)
-  const bool plain = MB * NB < 16 && (MANY || __builtin_amdgcn_ballot_w64(!all) == 0ull);
+  // Whole batches can be loaded as they are: rows that are not there read zeros anyway, or there are none.
+  // (Tiles of several token blocks above rank 32 go without: the addresses of both loops at once spill.  32 tokens, rank 64, 13
+  // registers spilled / without that loop: 600 tokens over 16 adapters 7.1 / 6.8 us, 1152 over 64 13.9 / 12.7, 3000 over 32 17.5 / 16.1,
+  // 4000 over 128 23.4 / 22.6.)
+  const bool plain = WHOLE && (MANY || __builtin_amdgcn_ballot_w64(!all) == 0ull);
 
   // where this lane's chunks sit in a staged block: row u*8 + grow / chunk gcol when it writes what it loaded,
   // row lrow / chunk 4*c + kg when it reads operand c (K elements c*32 + kg*8 .. + 8 of the step)
@@ -189,7 +192,7 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
     }
     requested();
     use();
-    if (MANY && MB * NB < 16) break;   // (it is less than a batch)
+    if (MANY && WHOLE) break;   // (it is less than a batch)
   }
 
   // Every wave leaves its share as it is (C layout: column = lane%16, rows = 4*(lane/16)+i) and whoever needs an
