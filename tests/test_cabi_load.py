@@ -239,3 +239,12 @@ def test_marks_of_the_tile_table_say_something():
     (8, 8, 16, 0, 2, 1, 0), (-1, 8, 16, 4096, 2, 1, 0), (8, 8, 16, 4096, 2, 5, 0)])
 def test_which_calls_run_in_one_launch(T, A, rank, h_out, ks, nt, one):
     assert _lib.lib().mlora_runs_in_one_launch(T, A, rank, h_out, ks, nt) == one
+
+
+def test_large_batches_have_tall_expand_tiles():
+    """The expand of 16-token tiles fetches B once per tile: from a few thousand tokens on taller tiles win at every width."""
+    import json
+    from valora_amd import tile_table as tt
+    with open(tt.TABLE_PATH) as f:
+        entries = json.load(f)["entries"]
+    assert [k for k, v in entries.items() if int(k.split(":")[0]) > 4096 and v["bm_expand"] < 32] == []
