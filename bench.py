@@ -110,6 +110,12 @@ def time_graph(torch, fn, reps, warm, use_graph):
     return ev_ms, wall_ms
 
 
+def median_ms(torch, fn, reps, warm, use_graph, runs=5):
+    """The median of `runs` such measurements: one of a couple of milliseconds is at the mercy of a single hiccup of the host
+    (7.1 us an op measured 10.7 once)."""
+    return sorted(time_graph(torch, fn, reps, warm, use_graph)[0] for _ in range(runs))[runs // 2]
+
+
 def cpu_baseline(torch, w, budget_s=15.0):
     """The reference's per-segment PyTorch path (valora/models/bmm/lora_bmm_infer.py:342-352)
     restated in oracle/, on this host's cores: decode tokens are length-1 segments after grouping
@@ -490,8 +496,7 @@ def bench_byte_heavy_decode(torch, W, LoraPlan, dev, use_graph, reps):
             for y in ys:
                 plan.apply(y, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, 0, pool.a_scaling)
 
-        ms, _ = time_graph(torch, run, max(10, reps // 4), 3, use_graph)
-        us = ms * 1e3 / len(ys)
+        us = median_ms(torch, run, max(10, reps // 4), 3, use_graph) * 1e3 / len(ys)
         touched = len(set(ids.tolist()))
         nbytes = 3 * T * H * 2 + 2 * touched * r * H * 2
         out.append({"tokens": T, "rank": r, "adapters_touched": touched, "us": round(us, 2), "bytes": nbytes,
@@ -531,8 +536,8 @@ def bench_single_adapter_vs_gemm(torch, W, LoraPlan, dev, use_graph, reps):
                 ys[l].addmm_(vs[l], b, alpha=0.5)
 
         k = max(10, reps // 4)
-        us_ours = time_graph(torch, ours, k, 3, use_graph)[0] * 1e3 / n
-        us_gemm = time_graph(torch, gemm, k, 3, use_graph)[0] * 1e3 / n
+        us_ours = median_ms(torch, ours, k, 3, use_graph) * 1e3 / n
+        us_gemm = median_ms(torch, gemm, k, 3, use_graph) * 1e3 / n
         nbytes = (3 * T * H + 2 * r * H) * 2
         out.append({"tokens": T, "rank": r, "us": round(us_ours, 2), "torch_mm_addmm_us": round(us_gemm, 2),
                     "gbps": round(nbytes / us_ours / 1e3, 1), "tile": [plan.bm_shrink, plan.ksplit, plan.bm_expand],
