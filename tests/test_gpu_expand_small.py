@@ -35,7 +35,7 @@ def test_same_bits_as_taller_tiles(dev, T, h_out, ranks):
     print(T, h_out, ranks, dtype, flush=True)
     p, ids, x, y0 = _case(dev, T, 264, h_out, ranks, dtype, T + h_out, inf=h_out == 520)
     idx = (p.a_start, p.a_len, p.a_loc)
-    for kw in (dict(ksplit=1), dict(ksplit=2, reduce_in_expand=True), dict(ksplit=2, reduce_in_expand=True, expand_column_loop=True)):
+    for kw in (dict(ksplit=1), dict(ksplit=2, reduce_in_expand=True)):
         got = []
         for bm in (16, 32):
             plan = LoraPlan(ids, *idx[:2], max(ranks), n_slots=2, hidden=264, bm_shrink=16, bm_expand=bm, one_launch=False, **kw)
@@ -60,6 +60,18 @@ def test_compensation_same_bits_as_taller_tiles(dev, h_out, ranks):
         got.append(y)
     assert torch.equal(*got)
     assert not torch.equal(got[0], y0)
+
+
+def test_the_column_loop_flag_is_accepted(dev):
+    p, ids, x, y0 = _case(dev, 50, 264, 520, [16, 8], torch.float16, 3)
+    got = []
+    for flag in (False, True):
+        plan = LoraPlan(ids, p.a_start, p.a_len, 16, n_slots=2, hidden=264, bm_shrink=16, bm_expand=16, ksplit=2, one_launch=False,
+                        expand_column_loop=flag)
+        y = y0.clone()
+        plan.apply(y, x, p.key_buffer, p.value_buffer, p.a_start, p.a_len, p.a_loc, 1, p.a_scaling)
+        got.append(y)
+    assert torch.equal(*got) and not torch.equal(got[0], y0)
 
 
 def test_more_tiles_than_a_grid_dimension(dev):

@@ -94,8 +94,8 @@ def _wide(v, n):
 @pytest.mark.parametrize("h_out", [264, 520, 1032])
 def test_expand_operand_narrower_than_rank(dev, h_out, kmax, dtype):
     """The expand's half of the above: of an adapter whose rank exceeds the operand's columns only the first rank rows count,
-    whichever kernel the call gets.  The column-looping one turns a limited piece of B at a time; ranks up to 128 go on
-    beyond what an operand of this width can use.  Both kernels do the same arithmetic: same bits."""
+    whichever kernel the call gets (tiles of 16 tokens have one of their own); ranks up to 128 go on beyond what an operand
+    of this width can use.  Both kernels do the same arithmetic: same bits."""
     from valora_amd import _lib
     from valora_amd.plan import LoraPlan
     ranks = (128, 8, 64, 40, 32, 72, 48, 96)
@@ -105,23 +105,22 @@ def test_expand_operand_narrower_than_rank(dev, h_out, kmax, dtype):
     vd = v.to(dev)
     want = O.bgmv_expand(y0, _wide(v, R), pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 2, pool.a_scaling)
     got = []
-    for loop in (False, True):
-        plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, R, hidden=h_out, bm_shrink=16, bm_expand=16, ksplit=1,
+    for bm in (16, 32):
+        plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, R, hidden=h_out, bm_shrink=16, bm_expand=bm, ksplit=1,
                         one_launch=False)
         pb = _lib.make_pool(pd.value_buffer, pd.a_start, pd.a_len, pd.a_loc, h_out)
         y = y0.to(dev)
         _lib.check(_lib.lib().mlora_expand(_lib.current_stream(dev), plan.handle, _lib.ptr(y), 61, h_out, None, _lib.ptr(vd),
-                                           kmax, kmax, pb, 2, _lib.ptr(pd.a_scaling), 1,
-                                           _lib.EXPAND_COLUMN_LOOP if loop else 0, _lib.dtype_code(dtype)))
+                                           kmax, kmax, pb, 2, _lib.ptr(pd.a_scaling), 1, 0, _lib.dtype_code(dtype)))
         got.append(y.cpu())
-        assert_parity(got[-1], want, f"kmax {kmax} h_out {h_out} loop {loop}")
+        assert_parity(got[-1], want, f"kmax {kmax} h_out {h_out} tiles of {bm}")
     assert torch.equal(got[0], got[1])
 
 
 @pytest.mark.parametrize("max_rank", [16, 32, 64])
 def test_planned_op_of_a_lower_max_rank(dev, max_rank):
     """The planned op with a max_rank below the ranks of some adapters: the first max_rank rows of those, also where the
-    expand sums the split-K partials in its column loop."""
+    expand sums the split-K partials, in both expand kernels."""
     from valora_amd.plan import LoraPlan
     dtype = torch.float16
     pool, ids, x, y0, _, R = _case(max_rank, 90, 520, 1032, (128, 8, 64, 48, 32), dtype, id_style="holes")
@@ -132,18 +131,18 @@ def test_planned_op_of_a_lower_max_rank(dev, max_rank):
                          pool.a_scaling)
     got = []
     for rie in (False, True):
-        for loop in (False, True):
-            plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, max_rank, hidden=520, bm_shrink=16, bm_expand=16, ksplit=3,
-                            reduce_in_expand=rie, one_launch=False, expand_column_loop=loop)
+        for bm in (16, 32):
+            plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, max_rank, hidden=520, bm_shrink=16, bm_expand=bm, ksplit=3,
+                            reduce_in_expand=rie, one_launch=False)
             y = y0.to(dev)
             plan.apply(y, x.to(dev), pd.key_buffer, pd.value_buffer, pd.a_start, pd.a_len, pd.a_loc, 1, pd.a_scaling)
             got.append(y.cpu())
-            assert_parity(got[-1], want, f"max_rank {max_rank} rie {rie} loop {loop}")
+            assert_parity(got[-1], want, f"max_rank {max_rank} rie {rie} tiles of {bm}")
     assert all(torch.equal(g, got[0]) for g in got)
 
 
 def test_narrow_expand_of_a_large_decode_batch(dev):
-    """The same through dispatch_bgmv on a batch whose grid is large enough for the column loop by itself."""
+    """The same through dispatch_bgmv on a batch whose grid is several times the device."""
     from valora_amd.kernels import dispatch_bgmv
     dtype = torch.float16
     pool, ids, _, y0, v, R = _case(31, 512, 64, 4096, (64, 8) * 64, dtype)

@@ -245,11 +245,9 @@ def test_table_configurations_of_other_widths(dev, hidden, T, rank, n_adapters):
 
 
 @pytest.mark.parametrize("seed", range(300, 330))
-def test_expand_column_loop_gives_the_same_bits(dev, seed):
-    """The expand of 16-token tiles as one workgroup per (tile, 256-column chunk) and as one workgroup per two chunks
-    (what the library picks by itself for grids several times the device, forced here for any size): same bits, for
-    finished v and for split-K partials summed in the expand, one target and several, ranks up to 128, output widths
-    that end inside a chunk or leave the second chunk of a pair empty."""
+def test_expand_kernels_give_the_same_bits(dev, seed):
+    """The expand of 16-token tiles and that of taller ones, two kernels: same bits, for finished v and for split-K partials
+    summed in the expand, one target and several, ranks up to 128, output widths that end inside a column chunk."""
     rnd = random.Random(seed)
     dtype = rnd.choice([torch.float16, torch.bfloat16])
     T = rnd.choice([1, 3, 16, 17, 40, 100, 256, 300])
@@ -270,10 +268,10 @@ def test_expand_column_loop_gives_the_same_bits(dev, seed):
     pd = pool.to(dev)
     idx = (pd.a_start, pd.a_len, pd.a_loc)
     R = max(ranks)
-    kw = dict(hidden=h_in, bm_shrink=rnd.choice([16, 32]), bm_expand=16, ksplit=ksplit, reduce_in_expand=rie, one_launch=False)
+    kw = dict(hidden=h_in, bm_shrink=rnd.choice([16, 32]), ksplit=ksplit, reduce_in_expand=rie, one_launch=False)
     outs = []
-    for loop in (False, True):
-        plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, R, expand_column_loop=loop, **kw)
+    for bm in (16, rnd.choice([32, 48, 64, 128])):
+        plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, R, bm_expand=bm, **kw)
         ys = [y.to(dev) for y in y0]
         if n_targets == 1:
             plan.apply(ys[0], x.to(dev), pd.key_buffer, pd.value_buffer, *idx, 2, pd.a_scaling)

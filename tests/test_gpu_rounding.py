@@ -52,14 +52,14 @@ def bits(t):
     return t.view(torch.int16).numpy().view(np.uint16)
 
 
-def expand(dev, y, v, scale, loop, h_out=264):
+def expand(dev, y, v, scale, bm, h_out=264):
     """y + scale * (sum of v's columns), through the expand: B is ones."""
     T = y.numel()
     pool = W.make_pool([8], h_out, h_out, BF, torch.Generator().manual_seed(0), True, heads=1, scalings=[scale])
     pool.value_buffer.fill_(1.0)
     pd = pool.to(dev)
     ids = torch.zeros(T, dtype=torch.long, device=dev)
-    plan = LoraPlan(ids, pd.a_start, pd.a_len, 8, hidden=h_out, bm_shrink=16, bm_expand=16, ksplit=1, one_launch=False)
+    plan = LoraPlan(ids, pd.a_start, pd.a_len, 8, hidden=h_out, bm_shrink=16, bm_expand=bm, ksplit=1, one_launch=False)
     yd = y[:, None].expand(T, h_out).contiguous().to(dev)
     vd = torch.zeros(T, 8, dtype=BF)
     for j, col in enumerate(v):
@@ -67,39 +67,38 @@ def expand(dev, y, v, scale, loop, h_out=264):
     vd = vd.to(dev)
     pb = _lib.make_pool(pd.value_buffer, pd.a_start, pd.a_len, pd.a_loc, h_out)
     _lib.check(_lib.lib().mlora_expand(_lib.current_stream(dev), plan.handle, _lib.ptr(yd), T, h_out, None, _lib.ptr(vd), 8, 8,
-                                       pb, 0, _lib.ptr(pd.a_scaling), 1, _lib.EXPAND_COLUMN_LOOP if loop else 0,
-                                       _lib.dtype_code(BF)))
+                                       pb, 0, _lib.ptr(pd.a_scaling), 1, 0, _lib.dtype_code(BF)))
     out = yd.cpu()
     assert torch.equal(out.view(torch.int16), out.view(torch.int16)[:, :1].expand(T, h_out))
     return bits(out[:, 0].contiguous())
 
 
-@pytest.mark.parametrize("loop", [False, True])
-def test_expand_rounds_to_nearest_even(dev, loop):
+@pytest.mark.parametrize("bm", [16, 32])
+def test_expand_rounds_to_nearest_even(dev, bm):
     # the sum is put together exactly: y holds the value's upper part, the product the rest
     f = np.concatenate([patterns(30, 254, 8000, 1), np.array([3.3895314e38, 3.3961775e38, -3.3961776e38, 3.4028235e38], np.float32)])
     hi, mid, lo = parts(f, 3)
-    got = expand(dev, as_bf16(hi), [as_bf16(mid), as_bf16(lo)], 1.0, loop)
+    got = expand(dev, as_bf16(hi), [as_bf16(mid), as_bf16(lo)], 1.0, bm)
     want = rne_bits(f)
     assert (got == want).all(), [(hex(a), hex(b), float(v)) for a, b, v in zip(got, want, f) if a != b][:5]
 
 
-@pytest.mark.parametrize("loop", [False, True])
-def test_expand_rounds_subnormal_sums(dev, loop):
+@pytest.mark.parametrize("bm", [16, 32])
+def test_expand_rounds_subnormal_sums(dev, bm):
     # down to the last bit of fp32: the product is scaled into the range, y is zero
     f = np.concatenate([patterns(0, 20, 8000, 2), np.arange(1, 1 << 17, 37).astype(np.uint32).view(np.float32)])
     f = f[f != 0]
     acc = (f.astype(np.float64) * 2.0 ** 100).astype(np.float32)
-    got = expand(dev, torch.zeros(len(f), dtype=BF), [as_bf16(p) for p in parts(acc, 3)], 2.0 ** -100, loop)
+    got = expand(dev, torch.zeros(len(f), dtype=BF), [as_bf16(p) for p in parts(acc, 3)], 2.0 ** -100, bm)
     want = rne_bits(f)
     assert (got == want).all(), [(hex(a), hex(b), float(v)) for a, b, v in zip(got, want, f) if a != b][:5]
 
 
-@pytest.mark.parametrize("loop", [False, True])
-def test_expand_keeps_infinities_and_nan(dev, loop):
+@pytest.mark.parametrize("bm", [16, 32])
+def test_expand_keeps_infinities_and_nan(dev, bm):
     y = np.array([0x7F80, 0xFF80, 0x7F81, 0x7FC0, 0xFFC1, 0xFFFF, 0x7FFF], np.uint16)
     yt = torch.from_numpy(y.view(np.int16)).view(BF)
-    got = expand(dev, yt, [torch.full((len(y),), 0.5, dtype=BF)], 1.0, loop)
+    got = expand(dev, yt, [torch.full((len(y),), 0.5, dtype=BF)], 1.0, bm)
     want = np.where((y & 0x7FFF) > 0x7F80, y | 0x40, y)
     assert (got == want).all()
 

@@ -33,8 +33,8 @@ class LoraPlan:
         16-token tiles and at most 16 K chunks of all targets together, needs ``max_rank <= 64``; ``runs_in_one_launch`` says
         which calls get it); ``None`` takes the tile table's choice.
         ``one_launch_no_wait`` makes every expand item take its give-up path at once, ``one_launch_never_ready`` after
-        waiting out its bound, ``shrink_recompute`` makes the 128-token shrink sum its K chunks by computing them all in
-        one workgroup (all for tests); ``expand_column_loop`` is accepted and without effect."""
+        waiting out its bound, ``shrink_recompute`` makes a shrink that sums its K chunks inside the launch compute them all
+        in one workgroup (all for tests); ``expand_column_loop`` is accepted and without effect."""
         if not ids.is_cuda:
             raise RuntimeError("ids must be a CUDA tensor")
         if ids.dtype != torch.long or a_start.dtype != torch.long or a_len.dtype != torch.long:
