@@ -170,7 +170,7 @@ def pool_copies(p, n_max):
 def bench_all_configs(torch, W, LoraPlan, dev, path, use_graph, only=0, only_target=None):
     """Per-target timing of the other benchmark configurations and of the headline's decode batch on all seven
     projections of a layer (report only; the JSON line of the default run is config 2's q).  Each target's shrink+expand is replayed back to back on 4 copies of y
-    so that the read-modify-write does not hit the same lines (`us`: x and the pool may sit in the
+    (sixteen ops a graph: the replay of a graph of four costs the host more than such ops take) so that the read-modify-write does not hit the same lines (`us`: x and the pool may sit in the
     last-level cache), and once more over 1 GiB of x / y copies and as much of pool copies (`us_cold`: what a
     forward pass sees, where every layer has its own adapter weights)."""
     report = {}
@@ -201,10 +201,7 @@ def bench_all_configs(torch, W, LoraPlan, dev, path, use_graph, only=0, only_tar
                 for yy in ycopies:
                     plan.expand(yy, p.value_buffer, p.a_start, p.a_len, p.a_loc, t.slot, p.a_scaling)
 
-            ms, _ = time_graph(torch, fn, 30, 3, use_graph)
-            ms_s, _ = time_graph(torch, fs, 30, 3, use_graph)
-            ms_e, _ = time_graph(torch, fe, 30, 3, use_graph)
-            us = ms * 1e3 / 4
+            us, us_s, us_e = (median_ms(torch, lambda: [f() for _ in range(4)], 10, 3, use_graph, 3) * 1e3 / 16 for f in (fn, fs, fe))
             # the same op on operands no cache holds: enough copies of x and y to walk through COLD_BYTES
             n_cold = max(4, -(-COLD_BYTES // (x.numel() * 2 + ycopies[0].numel() * 2)))
             xc = [x.clone() for _ in range(n_cold)]
@@ -215,12 +212,11 @@ def bench_all_configs(torch, W, LoraPlan, dev, path, use_graph, only=0, only_tar
                 for i, (xx, yy) in enumerate(zip(xc, yc)):
                     plan.apply(yy, xx, kc[i % len(kc)], vc[i % len(vc)], p.a_start, p.a_len, p.a_loc, t.slot, p.a_scaling)
 
-            ms_c, _ = time_graph(torch, fc, 10, 2, use_graph)
-            us_cold = ms_c * 1e3 / n_cold
+            us_cold = median_ms(torch, fc, 10, 2, use_graph, 3) * 1e3 / n_cold
             del xc, yc, kc, vc
             b, f = w.algorithmic_bytes(t.name), w.flops(t.name)
             rows[t.name] = {"us": round(us, 2), "us_cold": round(us_cold, 2),
-                            "shrink_us": round(ms_s * 250, 2), "expand_us": round(ms_e * 250, 2),
+                            "shrink_us": round(us_s, 2), "expand_us": round(us_e, 2),
                             "bytes": b, "flops": f, "gbps": round(b / us / 1e3, 1),
                             "hbm_frac": round(b / us / 1e3 / HBM_PEAK_GBPS, 4), "tflops": round(f / us / 1e6, 2),
                             "tile": [plan.bm_shrink, plan.ksplit, plan.bm_expand]}
@@ -241,8 +237,7 @@ def bench_all_configs(torch, W, LoraPlan, dev, path, use_graph, only=0, only_tar
                     plan.apply_multi(ys, x, p.key_buffer, p.value_buffer, p.a_start, p.a_len, p.a_loc, slots,
                                      p.a_scaling)
 
-            ms, _ = time_graph(torch, fm, 30, 3, use_graph)
-            us = ms * 1e3 / 4
+            us = median_ms(torch, lambda: [fm() for _ in range(4)], 10, 3, use_graph, 3) * 1e3 / 16
             n_cold = max(4, -(-COLD_BYTES // (x.numel() * 2 + sum(y.numel() for y in ycopies[0]) * 2)))
             xc = [x.clone() for _ in range(n_cold)]
             yc = [[wd.y0[t.name].clone() for t in ts] for _ in range(n_cold)]
@@ -253,8 +248,7 @@ def bench_all_configs(torch, W, LoraPlan, dev, path, use_graph, only=0, only_tar
                     plan.apply_multi(ys, xx, kc[i % len(kc)], vc[i % len(vc)], p.a_start, p.a_len, p.a_loc, slots,
                                      p.a_scaling)
 
-            ms_c, _ = time_graph(torch, fmc, 10, 2, use_graph)
-            us_cold = ms_c * 1e3 / n_cold
+            us_cold = median_ms(torch, fmc, 10, 2, use_graph, 3) * 1e3 / n_cold
             del xc, yc, kc, vc
             separate = sum(rows[t.name]["us"] for t in ts)
             # x is read once for the whole group
