@@ -21,6 +21,7 @@ extern "C" {
 typedef enum { MLORA_F16 = 0, MLORA_BF16 = 1 } mlora_dtype;
 
 #define MLORA_MAX_TARGETS 4   /* targets one mlora_lora_apply_multi call can take */
+#define MLORA_MAX_PLANS 4     /* plans one mlora_build_plans call can cut */
 
 typedef enum {
   MLORA_OK = 0,
@@ -156,6 +157,11 @@ int mlora_tile_fallback(int64_t n_tokens, int64_t max_rank, int64_t hidden, int6
 int mlora_build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T,
                      const int64_t *a_start, const int64_t *a_len, int64_t n_adapters,
                      int32_t n_slots, int32_t bm_shrink, int32_t bm_expand);
+/* Several plans of one batch in one launch, each in a buffer of its own, plan i with tile heights bm_shrink[i] and
+ * bm_expand[i] (host arrays): what n_plans calls of mlora_build_plan write.                     */
+int mlora_build_plans(void *stream, mlora_plan *const *plans, int32_t n_plans, const int64_t *ids, int64_t T,
+                      const int64_t *a_start, const int64_t *a_len, int64_t n_adapters, int32_t n_slots,
+                      const int32_t *bm_shrink, const int32_t *bm_expand);
 
 /* Run-length encoding of per-token ids, bit-exact with count_consecutive_requests
  * (atmm/valora/csrc/bgmv/bgmv_impl.cuh:39-72).  Outputs are device int64 arrays with room for

@@ -70,6 +70,41 @@ def test_plan_invariants(dev, T, A, style):
         _check_plan(ids, a_len, 4, bm_s, bm_e, dev)
 
 
+@pytest.mark.parametrize("T,A", [(512, 8), (513, 8), (1024, 512), (1025, 33), (4096, 600), (4097, 3), (16385, 9), (40000, 2047), (2000, 4097)])
+def test_plan_in_parts(dev, T, A):
+    """Both sides of the sizes at which a plan is written by one, four or eight workgroups, with fewer histogram rows than
+    waves, and with rows that take more than one batch of look-ups."""
+    g = torch.Generator().manual_seed(T + A)
+    a_len = torch.randint(0, 9, (A,), generator=g) * 8 * 4
+    a_len[A // 2] = 32
+    runs = torch.repeat_interleave(torch.randint(-1, A + 1, (T,), generator=g), torch.randint(1, 300, (T,), generator=g))[:T]
+    mixed = torch.where(torch.rand(T, generator=g) < 0.5, runs, torch.randint(0, A, (T,), generator=g))
+    for ids in (runs, mixed):
+        _check_plan(ids, a_len, 4, 16, 96, dev)
+
+
+@pytest.mark.parametrize("T,A", [(1, 1), (700, 40), (5000, 33)])
+def test_plans_cut_in_one_launch(dev, T, A):
+    from valora_amd.plan import LoraPlan
+    g = torch.Generator().manual_seed(T)
+    a_len = (torch.randint(1, 9, (A,), generator=g) * 32).to(dev)
+    a_start = torch.cumsum(a_len, 0) - a_len
+    ids = torch.randint(0, A, (T,), generator=g).to(dev)
+    widths = (4096, 11008, 2048, 4096)
+    for w, p in zip(widths, LoraPlan.of_widths(ids, a_start, a_len, 64, widths)):
+        q = LoraPlan(ids, a_start, a_len, 64, hidden=w)
+        assert (p.bm_shrink, p.bm_expand, p.ksplit, p.flags) == (q.bm_shrink, q.bm_expand, q.ksplit, q.flags)
+        assert p.header() == q.header()
+        for a, b in ((p.perm(), q.perm()), (p.tiles_shrink(), q.tiles_shrink()), (p.tiles_expand(), q.tiles_expand()),
+                     (p.position_adapters(), q.position_adapters()), (p.position_ranks(), q.position_ranks())):
+            assert torch.equal(a, b)
+        p.rebuild(ids.flip(0))
+        q.rebuild(ids.flip(0))
+        assert torch.equal(p.perm(), q.perm())
+    with pytest.raises(RuntimeError):
+        LoraPlan.of_widths(ids, a_start, a_len, 64, (4096,) * 5)
+
+
 @pytest.mark.parametrize("T", [1, 2, 63, 64, 65, 1024, 1025, 5000])
 @pytest.mark.parametrize("style", ["random", "runs", "equal", "distinct"])
 def test_count_consecutive_bit_exact(dev, T, style):

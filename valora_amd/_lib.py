@@ -22,7 +22,7 @@ REDUCE_IN_EXPAND, ONE_LAUNCH, ONE_LAUNCH_NO_WAIT, SHRINK_RECOMPUTE, EXPAND_COLUM
 # every symbol include/mlora.h declares
 SYMBOLS = [
     "mlora_last_error", "mlora_version", "mlora_plan_bytes", "mlora_scratch_bytes", "mlora_one_launch_scratch_bytes",
-    "mlora_workspace_bytes", "mlora_tile_lookup", "mlora_tile_fallback", "mlora_build_plan", "mlora_count_consecutive",
+    "mlora_workspace_bytes", "mlora_tile_lookup", "mlora_tile_fallback", "mlora_build_plan", "mlora_build_plans", "mlora_count_consecutive",
     "mlora_ids_from_segments", "mlora_ids_from_requests", "mlora_shrink", "mlora_expand", "mlora_lora_apply",
     "mlora_lora_apply_multi", "mlora_dispatch_bgmv", "mlora_dispatch_bgmv_static",
     "mlora_dispatch_sgmm", "mlora_prefill_shrink", "mlora_prefill_expand",

@@ -236,10 +236,12 @@ size_t mlora_workspace_bytes(int64_t T, int64_t n_adapters, int64_t max_rank) {
   return up(mlora_plan_bytes(T, n_adapters)) + up(scratch_bytes(T, max_rank, ks)) + up((size_t)T * 8 + 8) + 256;
 }
 
-static int build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T, const int64_t *a_start,
-                      const int64_t *a_len, int64_t n_adapters, int32_t n_slots, int32_t bm_shrink, int32_t bm_expand,
-                      int64_t merged) {
-  if (!plan || !plan->dev) return fail(MLORA_ERR_INVALID, "build_plan: plan buffer is null");
+static int build_plans(void *stream, mlora_plan *const *plans, int n_plans, const int64_t *ids, int64_t T, const int64_t *a_start,
+                       const int64_t *a_len, int64_t n_adapters, int32_t n_slots, const int32_t *bm_shrink, const int32_t *bm_expand,
+                       int64_t merged) {
+  if (n_plans < 1 || n_plans > MLORA_MAX_PLANS) return fail(MLORA_ERR_INVALID, "build_plan: n_plans=%d outside [1,%d]", n_plans, MLORA_MAX_PLANS);
+  for (int i = 0; i < n_plans; ++i)
+    if (!plans[i] || !plans[i]->dev) return fail(MLORA_ERR_INVALID, "build_plan: plan buffer is null");
   if (T < 0 || T > MAX_TOKENS) return fail(MLORA_ERR_INVALID, "build_plan: T=%lld out of range", (long long)T);
   if (n_adapters < 0 || n_adapters > MAX_ADAPTERS)
     return fail(MLORA_ERR_NO_KERNEL, "build_plan: n_adapters=%lld out of range (max %lld)", (long long)n_adapters,
@@ -247,39 +249,62 @@ static int build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_
   if (T > 0 && !ids) return fail(MLORA_ERR_INVALID, "build_plan: ids is null");
   if (n_adapters > 0 && (!a_start || !a_len)) return fail(MLORA_ERR_INVALID, "build_plan: a_start / a_len is null");
   if (n_slots < 1) return fail(MLORA_ERR_INVALID, "build_plan: n_slots must be >= 1");
-  if (bm_shrink == 0 || bm_expand == 0) {   // neither rank nor width is known here: the rule's tile heights
-    const mlora_tile_config c = tile_fallback(T, 16, 4096, n_adapters);
-    if (bm_shrink == 0) bm_shrink = c.bm_shrink;
-    if (bm_expand == 0) bm_expand = c.bm_expand;
-  }
-  if (bm_shrink != 16 && bm_shrink != 32 && bm_shrink != 64 && bm_shrink != 128 && bm_shrink != 256)
-    return fail(MLORA_ERR_NO_KERNEL, "build_plan: bm_shrink=%d not in {16,32,64,128,256}", bm_shrink);
-  if (bm_expand < 16 || bm_expand > 256 || (bm_expand % 16) != 0)
-    return fail(MLORA_ERR_NO_KERNEL, "build_plan: bm_expand=%d not a multiple of 16 in [16,256]", bm_expand);
   const PlanLayout L = plan_layout(T, n_adapters);
-  if (plan->bytes < (size_t)L.total_words * 4)
-    return fail(MLORA_ERR_WORKSPACE, "build_plan: plan buffer has %zu bytes, needs %zu", plan->bytes,
-                (size_t)L.total_words * 4);
-  if (!aligned16(plan->dev)) return fail(MLORA_ERR_INVALID, "build_plan: plan buffer must be 16-byte aligned");
-  plan->T = T;
-  plan->n_adapters = n_adapters;
-  plan->n_slots = n_slots;
-  plan->bm_shrink = bm_shrink;
-  plan->bm_expand = bm_expand;
-  return launch_plan((hipStream_t)stream, static_cast<int32_t *>(plan->dev), L, ids, a_start, a_len, n_slots,
-                     bm_shrink, bm_expand, merged >= 0 && merged < n_adapters ? (int)merged : -1);
+  PlanSet set;
+  for (int i = 0; i < n_plans; ++i) {
+    const mlora_plan &plan = *plans[i];
+    int32_t bs = bm_shrink[i], be = bm_expand[i];
+    if (bs == 0 || be == 0) {   // neither rank nor width is known here: the rule's tile heights
+      const mlora_tile_config c = tile_fallback(T, 16, 4096, n_adapters);
+      if (bs == 0) bs = c.bm_shrink;
+      if (be == 0) be = c.bm_expand;
+    }
+    if (bs != 16 && bs != 32 && bs != 64 && bs != 128 && bs != 256)
+      return fail(MLORA_ERR_NO_KERNEL, "build_plan: bm_shrink=%d not in {16,32,64,128,256}", bs);
+    if (be < 16 || be > 256 || (be % 16) != 0)
+      return fail(MLORA_ERR_NO_KERNEL, "build_plan: bm_expand=%d not a multiple of 16 in [16,256]", be);
+    if (plan.bytes < (size_t)L.total_words * 4)
+      return fail(MLORA_ERR_WORKSPACE, "build_plan: plan buffer has %zu bytes, needs %zu", plan.bytes,
+                  (size_t)L.total_words * 4);
+    if (!aligned16(plan.dev)) return fail(MLORA_ERR_INVALID, "build_plan: plan buffer must be 16-byte aligned");
+    for (int j = 0; j < i; ++j)
+      if (set.plan[j] == plan.dev) return fail(MLORA_ERR_INVALID, "build_plan: plans %d and %d share a buffer", j, i);
+    set.plan[i] = static_cast<int32_t *>(plan.dev);
+    set.bm_s[i] = bs;
+    set.bm_e[i] = be;
+  }
+  for (int i = n_plans; i < MLORA_MAX_PLANS; ++i) {
+    set.plan[i] = nullptr;
+    set.bm_s[i] = set.bm_e[i] = 0;
+  }
+  for (int i = 0; i < n_plans; ++i) {
+    plans[i]->T = T;
+    plans[i]->n_adapters = n_adapters;
+    plans[i]->n_slots = n_slots;
+    plans[i]->bm_shrink = set.bm_s[i];
+    plans[i]->bm_expand = set.bm_e[i];
+  }
+  return launch_plan((hipStream_t)stream, set, n_plans, L, ids, a_start, a_len, n_slots,
+                     merged >= 0 && merged < n_adapters ? (int)merged : -1);
 }
 
 int mlora_build_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T, const int64_t *a_start,
                      const int64_t *a_len, int64_t n_adapters, int32_t n_slots, int32_t bm_shrink,
                      int32_t bm_expand) {
-  return build_plan(stream, plan, ids, T, a_start, a_len, n_adapters, n_slots, bm_shrink, bm_expand, -1);
+  return build_plans(stream, &plan, 1, ids, T, a_start, a_len, n_adapters, n_slots, &bm_shrink, &bm_expand, -1);
+}
+
+int mlora_build_plans(void *stream, mlora_plan *const *plans, int32_t n_plans, const int64_t *ids, int64_t T, const int64_t *a_start,
+                      const int64_t *a_len, int64_t n_adapters, int32_t n_slots, const int32_t *bm_shrink,
+                      const int32_t *bm_expand) {
+  if (!plans || !bm_shrink || !bm_expand) return fail(MLORA_ERR_INVALID, "build_plans: null pointer");
+  return build_plans(stream, plans, n_plans, ids, T, a_start, a_len, n_adapters, n_slots, bm_shrink, bm_expand, -1);
 }
 
 int mlora_build_compensation_plan(void *stream, mlora_plan *plan, const int64_t *ids, int64_t T, const int64_t *a_start,
                                   const int64_t *a_len, int64_t n_adapters, int32_t n_slots, int32_t bm_shrink,
                                   int32_t bm_expand, int64_t merged) {
-  return build_plan(stream, plan, ids, T, a_start, a_len, n_adapters, n_slots, bm_shrink, bm_expand, merged);
+  return build_plans(stream, &plan, 1, ids, T, a_start, a_len, n_adapters, n_slots, &bm_shrink, &bm_expand, merged);
 }
 
 int mlora_count_consecutive(void *stream, const int64_t *lora_rank, int64_t n_adapters, const int64_t *indicies,

@@ -25,6 +25,7 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
+#include <array>
 #include <cstring>
 #include <memory>
 #include <stdexcept>
@@ -521,14 +522,14 @@ struct NativePlan {
   c10::DeviceIndex device = 0;
 
   NativePlan(const at::Tensor &ids_, const at::Tensor &a_start_, const at::Tensor &a_len_, int64_t max_rank_,
-             int32_t n_slots_, int32_t bm_shrink_, int32_t bm_expand_, int32_t ksplit_, int32_t flags_, int64_t merged_)
+             int32_t n_slots_, int32_t bm_shrink_, int32_t bm_expand_, int32_t ksplit_, int32_t flags_, int64_t merged_, bool cut = true)
       : ids(ids_.contiguous()), a_start(a_start_), a_len(a_len_), T(ids_.numel()), max_rank(max_rank_), merged(merged_),
         n_slots(n_slots_), bm_shrink(bm_shrink_), bm_expand(bm_expand_), ksplit(ksplit_), flags(flags_), device(ids_.get_device()) {
     const int64_t A = a_start.numel();
     buf = device_bytes(mlora_plan_bytes(T, A), ids);
     plan.dev = buf.data_ptr();
     plan.bytes = (size_t)buf.numel();
-    rebuild(c10::nullopt);
+    if (cut) rebuild(c10::nullopt);
     // room for a multi-target call from the start: the buffer is never replaced, so a HIP graph captured from this plan
     // or work still queued on another stream keeps pointing at live memory
     scratch_per_target = (int64_t)mlora_scratch_bytes(T, max_rank, ksplit);
@@ -537,6 +538,37 @@ struct NativePlan {
       for (int t = 1; t <= MLORA_MAX_TARGETS; ++t)
         n = std::max(n, mlora_one_launch_scratch_bytes(T, A, max_rank, ksplit, t));
     scratch = at::empty({(int64_t)n}, ids.options().dtype(at::kByte));
+  }
+
+  // Plans of one batch, cut in one launch.  shapes: (bm_shrink, bm_expand, ksplit, flags) of each.
+  static py::list several(const at::Tensor &ids_, const at::Tensor &a_start_, const at::Tensor &a_len_, int64_t max_rank_,
+                          int32_t n_slots_, const std::vector<std::array<int32_t, 4>> &shapes) {
+    const size_t n = shapes.size();
+    if (n < 1 || n > MLORA_MAX_PLANS) raise("1.." + std::to_string(MLORA_MAX_PLANS) + " plans are cut together");
+    const at::Tensor all = ids_.contiguous();
+    std::vector<std::unique_ptr<NativePlan>> made;
+    mlora_plan cut[MLORA_MAX_PLANS], *plans[MLORA_MAX_PLANS];
+    int32_t bm_s[MLORA_MAX_PLANS], bm_e[MLORA_MAX_PLANS];
+    for (size_t i = 0; i < n; ++i) {
+      made.push_back(std::make_unique<NativePlan>(all, a_start_, a_len_, max_rank_, n_slots_, shapes[i][0], shapes[i][1],
+                                                  shapes[i][2], shapes[i][3], -1, false));
+      cut[i] = made[i]->plan;
+      plans[i] = &cut[i];
+      bm_s[i] = shapes[i][0];
+      bm_e[i] = shapes[i][1];
+    }
+    const hipStream_t st = made[0]->stream();
+    check_unlocked([&] {
+      return mlora_build_plans(st, plans, (int32_t)n, static_cast<const int64_t *>(all.data_ptr()), all.numel(),
+                               static_cast<const int64_t *>(a_start_.data_ptr()), static_cast<const int64_t *>(a_len_.data_ptr()),
+                               a_start_.numel(), n_slots_, bm_s, bm_e);
+    });
+    py::list out;
+    for (size_t i = 0; i < n; ++i) {
+      made[i]->plan = cut[i];
+      out.append(py::cast(std::move(made[i])));
+    }
+    return out;
   }
 
   hipStream_t stream() const { return c10::hip::getCurrentHIPStream(device).stream(); }
@@ -707,6 +739,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   py::class_<NativePlan>(m, "NativePlan")
       .def(py::init<const at::Tensor &, const at::Tensor &, const at::Tensor &, int64_t, int32_t, int32_t, int32_t, int32_t,
                     int32_t, int64_t>())
+      .def_static("several", &NativePlan::several)
       .def("apply", &NativePlan::apply)
       .def("apply_multi", &NativePlan::apply_multi)
       .def("compensate", &NativePlan::compensate)

@@ -160,8 +160,13 @@ struct DecodeArgs {
 int launch_decode(hipStream_t st, const DecodeArgs &a, int max_rank, mlora_dtype dt);
 int decode_bn();   // output columns per expand item of the one-launch op
 size_t decode_partial_floats(int64_t n_tiles, int n_targets, int ksplit, int64_t rp);
-int launch_plan(hipStream_t st, int32_t *plan, const PlanLayout &L, const int64_t *ids,
-                const int64_t *a_start, const int64_t *a_len, int n_slots, int bm_s, int bm_e, int merged);
+// plans of one batch (same tokens, same index) that differ in their tile heights only
+struct PlanSet {
+  int32_t *plan[MLORA_MAX_PLANS];
+  int bm_s[MLORA_MAX_PLANS], bm_e[MLORA_MAX_PLANS];
+};
+int launch_plan(hipStream_t st, const PlanSet &set, int n_plans, const PlanLayout &L, const int64_t *ids,
+                const int64_t *a_start, const int64_t *a_len, int n_slots, int merged);
 size_t scratch_bytes(int64_t T, int64_t max_rank, int ksplit);
 int launch_count_consecutive(hipStream_t st, const int64_t *lora_rank, int64_t n_adapters,
                              const int64_t *indicies, int64_t T, int64_t *output_counts,

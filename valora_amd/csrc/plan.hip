@@ -7,8 +7,8 @@
 //                             (atmm/valora/csrc/bgmv/bgmv_impl.cuh:39-72)
 //  * ids_fill / ids_cover_*   per-token ids from segment or per-request operands
 //
-// All are single-workgroup or trivially parallel integer kernels: the inputs are a few KB and
-// the work is launch-latency bound, so one 1024-thread workgroup with LDS histograms is used
+// All are integer kernels of one or a few workgroups, or trivially parallel: the inputs are a few KB and
+// the work is launch-latency bound, so LDS histograms in workgroups that need not talk to each other are used
 // instead of a multi-pass device-wide sort.
 #include "mlora_internal.h"
 
@@ -85,13 +85,16 @@ constexpr int PLAN_SMALL_A = 2048;   // adapters whose per-adapter tables fit in
 // lists above all) cost LDS latency instead of a global round trip each.
 // THREADS: 1024, or 256 for decode-sized batches (a few hundred tokens), where the barriers and scans of sixteen
 // waves cost more than the work they organise.
+// Grid: (parts, plans of the batch).  Every part counts all tokens and so knows every position; it then writes its share
+// of the token rows, of the tile records and of the words that start at zero.
 template <bool SMALL, int THREADS>
 __global__ __launch_bounds__(THREADS) void plan_kernel(
-    int32_t *__restrict__ plan, const int64_t *__restrict__ ids, const int64_t *__restrict__ a_start,
-    const int64_t *__restrict__ a_len, int T, int A, int n_slots, int bm_s, int bm_e, int W,
+    int32_t *plan0, const int64_t *__restrict__ ids, const int64_t *__restrict__ a_start,
+    const int64_t *__restrict__ a_len, int T, int A, int n_slots, int bm_s0, int bm_e0, int W, PlanSet set,
     int64_t off_perm, int64_t off_padapter, int64_t off_prank, int64_t off_tiles_s,
-    int64_t off_tiles_e, int64_t off_counters, int64_t off_scratch, int max_tiles, int n_flag_words, int merged) {
+    int64_t off_tiles_e, int64_t off_counters, int64_t off_scratch, int n_flag_words, int merged) {
   constexpr int N_WAVES = THREADS / 64;
+  constexpr int STEPS = THREADS == PLAN_THREADS_SMALL ? 4 : 8;   // 64-token steps whose ids are requested together
   __shared__ int32_t whist[HIST_WORDS];
   __shared__ Quad wsum[PLAN_WAVES + 1];
   __shared__ int s_wmaxr[PLAN_WAVES];
@@ -101,6 +104,14 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   __shared__ int64_t s_astart[SMALL ? PLAN_SMALL_A : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int part = (int)blockIdx.x, n_parts = (int)gridDim.x;
+  int32_t *__restrict__ plan = plan0;   // (the first plan's arguments are there at launch)
+  int bm_s = bm_s0, bm_e = bm_e0;
+  if (blockIdx.y > 0) {
+    plan = set.plan[blockIdx.y];
+    bm_s = set.bm_s[blockIdx.y];
+    bm_e = set.bm_e[blockIdx.y];
+  }
   int32_t *perm = plan + off_perm;
   int32_t *padapter = plan + off_padapter;
   int32_t *prank = plan + off_prank;
@@ -108,12 +119,13 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   int32_t *gstart = cnt + (SMALL ? PLAN_SMALL_A : A);
   int32_t *toff_s = gstart + (SMALL ? PLAN_SMALL_A : A);
   int32_t *toff_e = toff_s + (SMALL ? PLAN_SMALL_A : A);
-  // rank of adapter a (0 = not usable: ranks are multiples of 8 up to MAX_RANK) and its a_start
-  auto rank_of = [&](int a) -> int {
-    if (SMALL) return s_rank[a];
-    const int64_t r = a_len[a] / n_slots;
+  // rank of an adapter with `len` rows (0 = not usable: ranks are multiples of 8 up to MAX_RANK)
+  auto usable_rank = [&](int64_t len) -> int {
+    if (len < 0) return 0;
+    const int64_t r = len <= 0x7fffffff ? (int64_t)((uint32_t)len / (uint32_t)n_slots) : len / n_slots;
     return (r > 0 && (r & 7) == 0 && r <= MAX_RANK) ? (int)r : 0;
   };
+  auto rank_of = [&](int a) -> int { return SMALL ? s_rank[a] : usable_rank(a_len[a]); };
   auto start_of = [&](int a) -> int64_t { return SMALL ? s_astart[a] : a_start[a]; };
   // A token's adapter, -1 where the plan leaves the token out, and the adapter's usable rank.  A compensation plan keeps
   // the tokens of adapters without a usable rank: they have no product of their own, but the merged one comes off them.
@@ -126,53 +138,95 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
 
   auto start_word = [](int64_t st) -> int32_t { return st < 0 || st > 0x7fffffff ? INT32_MIN / 2 : (int32_t)st; };
 
-  // token range of each of the W histogram waves (contiguous, multiple of 64)
-  const int cw = (int)align_up((T + W - 1) / W, 64);
-  const int t_beg = wave * cw;
-  const int t_end = (wave < W) ? min(T, t_beg + cw) : 0;
+  // The tokens are cut into W rows of the histogram (runs of a multiple of 64 tokens); a wave counts `per_wave` of them.
+  const int rt = (int)align_up((T + W - 1) / W, 64);
+  const int per_wave = W > N_WAVES ? (W + N_WAVES - 1) / N_WAVES : 1;
+  const int t_beg = min(T, wave * per_wave * rt), t_end = min(T, min(W, (wave + 1) * per_wave) * rt);
+  // (tokens behind the end read the batch's last one and are dropped)
+  auto load_ids = [&](int t0, int end, int64_t (&id)[STEPS]) {
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i)
+      if (t0 + i * 64 < end) id[i] = ids[min(t0 + i * 64 + lane, T - 1)];   // wave-uniform
+    asm volatile("" ::: "memory");
+  };
+  // Which lanes hold the same adapter as this one comes from one vote per bit of the adapter index (6 votes for 64
+  // adapters), whatever the mix: one adapter for all 64 tokens of a prefill request or 64 different ones in a decode batch.
+  const int a_bits = A > 1 ? 32 - __clz(A - 1) : 0;   // bits that tell two adapter indices apart
+  auto same_adapter = [&](int a) -> unsigned long long {
+    unsigned long long same = __ballot(a >= 0);
+    if (same)   // wave-uniform
+      for (int b = 0; b < a_bits; ++b) {
+        const bool bit = (a >> b) & 1;
+        const unsigned long long m = __ballot(bit);
+        same &= bit ? m : ~m;
+      }
+    return same;
+  };
 
   // Every global load the set-up needs is requested before the first store: a wave gets its memory results in
   // issue order, so a load queued behind the zero-fill below would wait for those stores as well.
-  const int64_t id0 = (t_beg + lane < t_end) ? ids[t_beg + lane] : -1;
+  int64_t id[STEPS];
+  load_ids(t_beg, t_end, id);
   int64_t len0 = 0, start0 = 0;
   if (SMALL && tid < A) { len0 = a_len[tid]; start0 = a_start[tid]; }
 
   for (int i = tid; i < W * A; i += THREADS) whist[i] = 0;
   if (SMALL) {
     for (int a = tid; a < A; a += THREADS) {
-      const int64_t r = (a == tid ? len0 : a_len[a]) / n_slots;
-      s_rank[a] = (r > 0 && (r & 7) == 0 && r <= MAX_RANK) ? (int)r : 0;
+      s_rank[a] = usable_rank(a == tid ? len0 : a_len[a]);
       s_astart[a] = a == tid ? start0 : a_start[a];
     }
   }
   __syncthreads();
-  for (int i = tid; i < n_flag_words; i += THREADS) plan[off_counters + i] = 0;
+  for (int i = part * THREADS + tid; i < n_flag_words; i += n_parts * THREADS) plan[off_counters + i] = 0;
 
-  // 1. per-wave histogram of valid tokens (the first 64 tokens of a wave stay in registers for step 3)
-  int first_a = -1, first_r = 0;
-  for (int t = t_beg + lane; t < t_end; t += 64) {
-    const int64_t a64 = (t < t_beg + 64) ? id0 : ids[t];
-    int r;
-    const int a = adapter_of(a64, r);
-    if (a >= 0) atomicAdd(&whist[wave * A + a], 1);
-    if (t < t_beg + 64) { first_a = a; first_r = r; }
+  // 1. histogram of the tokens per row, whatever their adapters' ranks.  A step of one adapter (most of a prefill batch) is
+  // one addition: 64 lanes that add to one counter are 64 turns.
+  int row = wave * per_wave, row_end = t_beg + rt;
+  for (int t0 = t_beg; t0 < t_end; t0 += 64 * STEPS) {
+    if (t0 != t_beg) load_ids(t0, t_end, id);
+#pragma unroll
+    for (int i = 0; i < STEPS; ++i) {
+      const int t = t0 + i * 64;   // wave-uniform
+      if (t < t_end) {
+        if (t >= row_end) { ++row; row_end += rt; }
+        const uint32_t a = (uint32_t)id[i];
+        const bool ok = t + lane < t_end && (uint64_t)id[i] < (uint64_t)(uint32_t)A;
+        if (__ballot(ok && a == (uint32_t)__builtin_amdgcn_readfirstlane((int)a)) == ~0ull) {
+          if (lane == 0) atomicAdd(&whist[row * A + (int)a], 64);
+        } else if (ok) {
+          atomicAdd(&whist[row * A + (int)a], 1);
+        }
+      }
+    }
   }
   __syncthreads();
 
   // 2. per-adapter totals, group starts, tile offsets (each thread owns a run of adapters)
   const int per = (A + THREADS - 1) / THREADS;
   const int a_beg = min(A, tid * per), a_endx = min(A, a_beg + per);
+  constexpr int ROWS = THREADS == PLAN_THREADS_SMALL ? 4 : 16;   // counters of an adapter that are read in one round trip
+  auto read_hist = [&](int a, int w0, int (&h)[ROWS]) {
+#pragma unroll
+    for (int w = 0; w < ROWS; ++w) h[w] = w0 + w < W ? whist[(w0 + w) * A + a] : 0;
+  };
   int my_c = 0, my_ts = 0, my_te = 0, my_g = 0, my_maxr = 0;
   for (int a = a_beg; a < a_endx; ++a) {
-    int c = 0;
-    for (int w = 0; w < W; ++w) c += whist[w * A + a];
+    int c = 0, r;
+    const bool used = adapter_of(a, r) >= 0;   // (the plan leaves the tokens of others out)
+    for (int w0 = 0; used && w0 < W; w0 += ROWS) {
+      int h[ROWS];
+      read_hist(a, w0, h);
+#pragma unroll
+      for (int w = 0; w < ROWS; ++w) c += h[w];
+    }
     cnt[a] = c;
     if (c > 0) {
       my_c += c;
       my_ts += (c + bm_s - 1) / bm_s;
       my_te += (c + bm_e - 1) / bm_e;
       my_g += 1;
-      my_maxr = max(my_maxr, rank_of(a));
+      my_maxr = max(my_maxr, r);
     }
   }
   Quad tot;
@@ -193,10 +247,14 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     toff_s[a] = pre_ts;
     toff_e[a] = pre_te;
     int off = pre_c;
-    for (int w = 0; w < W; ++w) {  // histogram -> running write offset of (wave, adapter)
-      const int h = whist[w * A + a];
-      whist[w * A + a] = off;
-      off += h;
+    for (int w0 = 0; w0 < W; w0 += ROWS) {  // histogram -> running write offset of (row, adapter)
+      int h[ROWS];
+      read_hist(a, w0, h);
+#pragma unroll
+      for (int w = 0; w < ROWS; ++w) {
+        if (w0 + w < W) whist[(w0 + w) * A + a] = off;
+        off += h[w];
+      }
     }
     pre_c += c;
     pre_ts += (c + bm_s - 1) / bm_s;
@@ -204,51 +262,58 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   }
   __syncthreads();
 
-  // 3. stable scatter: each wave walks its range in order, 64 tokens a step; lanes holding the
+  // 3. stable scatter of the part's rows: a wave walks a row in order, 64 tokens a step; lanes holding the
   //    same adapter get consecutive positions in lane order.
-  const int a_bits = A > 1 ? 32 - __clz(A - 1) : 0;   // bits that tell two adapter indices apart
-  for (int t0 = t_beg; t0 < t_end; t0 += 64) {
-    const int t = t0 + lane;
-    int a = -1, r = 0;
-    if (t0 == t_beg) {
-      a = first_a;
-      r = first_r;
-    } else if (t < t_end) {
-      a = adapter_of(ids[t], r);
+  auto place = [&](int row, int t, int end, int64_t id64) {
+    int r = 0;
+    const int a = t < end ? adapter_of(id64, r) : -1;
+    const unsigned long long same = same_adapter(a);
+    if (a >= 0) {
+      const int slot_idx = row * A + a;
+      const int pos = whist[slot_idx] + __popcll(same & ((1ull << lane) - 1ull));
+      perm[pos] = t;
+      padapter[pos] = a;
+      prank[pos] = r;
+      __builtin_amdgcn_wave_barrier();                           // every lane of the group has read the offset ...
+      if (((same >> lane) >> 1) == 0) whist[slot_idx] = pos + 1;   // ... before its last lane moves it on
     }
-    // Lanes holding the same adapter get consecutive positions in lane order.  Which lanes hold my adapter comes from
-    // one vote per bit of the adapter index (6 votes for 64 adapters), whatever the mix: one adapter for all 64 tokens
-    // of a prefill request or 64 different ones in a decode batch.
-    const unsigned long long valid = __ballot(a >= 0);
-    if (valid) {   // wave-uniform
-      unsigned long long same = valid;
-      for (int b = 0; b < a_bits; ++b) {
-        const bool bit = (a >> b) & 1;
-        const unsigned long long m = __ballot(bit);
-        same &= bit ? m : ~m;
-      }
-      if (a >= 0) {
-        const int slot_idx = wave * A + a;
-        const int pos = whist[slot_idx] + __popcll(same & ((1ull << lane) - 1ull));
-        perm[pos] = t;
-        padapter[pos] = a;
-        prank[pos] = r;
-        __builtin_amdgcn_wave_barrier();                           // every lane of the group has read the offset ...
-        if (((same >> lane) >> 1) == 0) whist[slot_idx] = pos + 1;   // ... before its last lane moves it on
-      }
-      __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_wave_barrier();
+  };
+  // (one part and a row per wave: the ids are still in registers)
+  const bool kept = n_parts == 1 && per_wave == 1;
+  for (int k = wave; part + k * n_parts < W; k += N_WAVES) {
+    row = part + k * n_parts;
+    const int beg = min(T, row * rt), end = min(T, beg + rt);
+    for (int t0 = beg; t0 < end; t0 += 64 * STEPS) {
+      if (!kept || rt > 64 * STEPS) load_ids(t0, end, id);
+#pragma unroll
+      for (int i = 0; i < STEPS; ++i)
+        if (t0 + i * 64 < end) place(row, t0 + i * 64 + lane, end, id[i]);
     }
   }
-  __syncthreads();
 
-  // 4. tile lists: tile i belongs to the last adapter whose tile offset is <= i
+  // 4. the part's share of the tile lists: tile i belongs to the last adapter whose tile offset is <= i
   const bool one_list = bm_s == bm_e;   // then both lists are the same records (the one-launch op: 16 / 16)
   for (int pass = 0; pass < (one_list ? 1 : 2); ++pass) {
     const int n_tiles = pass ? n_te : n_ts;
     const int bm = pass ? bm_e : bm_s;
     const int32_t *toff = pass ? toff_e : toff_s;
-    int32_t *tiles = plan + (pass ? off_tiles_e : off_tiles_s);
-    for (int i = tid; i < n_tiles; i += THREADS) {
+    auto put_record = [&](int i, int4 head, int32_t start) {   // the lists begin on 32-byte boundaries of a 16-byte aligned buffer
+      static_assert(TILE_WORDS == 8, "two 16-byte stores");
+      for (int list = 0; list < (one_list ? 2 : 1); ++list) {
+        int4 *tl = reinterpret_cast<int4 *>(plan + (pass || list ? off_tiles_e : off_tiles_s) + (int64_t)i * TILE_WORDS);
+        tl[0] = head;
+        tl[1] = int4{start, 0, 0, 0};
+      }
+    };
+    // the kernels' grids are sized with the upper bound of the tile count: records past the last
+    // tile say "no tokens", so a workgroup needs no second look-up to know that it has nothing to do
+    const int upper = (T + bm - 1) / bm + min(A, T);
+    for (int i = tid * n_parts + part; i < upper; i += THREADS * n_parts) {
+      if (i >= n_tiles) {
+        put_record(i, int4{0, 0, 0, 0}, 0);
+        continue;
+      }
       int lo = 0, hi = A;  // first adapter with toff > i
       while (lo < hi) {
         const int mid = (lo + hi) >> 1;
@@ -263,26 +328,10 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
       // any other row outside the pool.
       // (no usable rank, compensation plans only: the count is negative, so whoever has no use for the tile leaves)
       const int r = rank_of(a), n = min(bm, c - k * bm);
-      const int32_t rec[5] = {a, r, gstart[a] + k * bm, r > 0 ? n : -n, start_word(st)};
-      for (int list = 0; list < (one_list ? 2 : 1); ++list) {
-        int32_t *tl = (list ? plan + off_tiles_e : tiles) + (int64_t)i * TILE_WORDS;
-#pragma unroll
-        for (int q = 0; q < TILE_WORDS; ++q) tl[q] = q < 5 ? rec[q] : 0;
-      }
-    }
-    // the kernels' grids are sized with the upper bound of the tile count: records past the last
-    // tile say "no tokens", so a workgroup needs no second look-up to know that it has nothing to do
-    const int upper = (T + bm - 1) / bm + min(A, T);
-    for (int i = n_tiles + tid; i < upper; i += THREADS) {
-      for (int list = 0; list < (one_list ? 2 : 1); ++list) {
-        int32_t *tl = (list ? plan + off_tiles_e : tiles) + (int64_t)i * TILE_WORDS;
-#pragma unroll
-        for (int k = 0; k < TILE_WORDS; ++k) tl[k] = 0;
-      }
+      put_record(i, int4{a, r, gstart[a] + k * bm, r > 0 ? n : -n}, start_word(st));
     }
   }
-  __syncthreads();
-  if (tid == 0) {
+  if (part == 0 && tid == 0) {
     plan[H_MAGIC] = PLAN_MAGIC;
     plan[H_T] = T;
     plan[H_NADAPTERS] = A;
@@ -368,19 +417,31 @@ __global__ void ids_cover_requests_kernel(int64_t *ids_out, const int32_t *b_sta
 
 }  // namespace
 
-int launch_plan(hipStream_t st, int32_t *plan, const PlanLayout &L, const int64_t *ids,
-                const int64_t *a_start, const int64_t *a_len, int n_slots, int bm_s, int bm_e, int merged) {
+int launch_plan(hipStream_t st, const PlanSet &set, int n_plans, const PlanLayout &L, const int64_t *ids,
+                const int64_t *a_start, const int64_t *a_len, int n_slots, int merged) {
   const int A = (int)L.A;
-  int W = A > 0 ? (int)(HIST_WORDS / A) : PLAN_WAVES;
-  if (W > PLAN_WAVES) W = PLAN_WAVES;
+  int W = A > 0 ? (int)(HIST_WORDS / A) : PLAN_WAVES;   // rows of the histogram
   if (W < 1) return fail(MLORA_ERR_NO_KERNEL, "plan: more than %lld adapters", (long long)MAX_ADAPTERS);
-  // the histogram is spread over as many waves as there are, W <= waves of the workgroup
   const bool few = L.T <= 1024 && A <= 512;
-  if (few && W > PLAN_THREADS_SMALL / 64) W = PLAN_THREADS_SMALL / 64;
+  // Parts and rows.  One compute unit is bound by the instructions of the scatter and by its own stores (126 KB of plan for 5400
+  // tokens); counting all tokens again in every part is cheap beside that.  us a build, back to back in a graph, 1 part / several:
+  // 918 tokens 7.4 / 6.8, 1024 over 128 adapters 8.2 / 7.4 (4 parts; 256 tokens 6.1 / 6.4, so not below 512), 5401 over 32 (8 parts)
+  // 15.2 / 10.9, 6749 over 24 17.0 / 11.3, 8192 over 64 19.4 / 13.0, 20000 over 128 38.6 / 20.3.  16 rows instead of 32: 1500 tokens 8.4 /
+  // 8.8, 5401 11.3 / 10.9, 8192 14.0 / 13.0.  (4 or 16 parts are equal to 8; 512 threads 0.5 us slower from 5000 tokens.)
+  int parts = 1, rows = PLAN_WAVES;
+  if (few) {
+    rows = L.T > 512 ? 8 : PLAN_THREADS_SMALL / 64;
+    parts = L.T > 512 ? 4 : 1;
+  } else if (A <= PLAN_SMALL_A) {
+    rows = L.T > 4096 ? 32 : 16;
+    parts = 8;
+  }
+  if (W > rows) W = rows;
+  if (parts > W) parts = W;
 #define MLORA_LAUNCH_PLAN(SMALL, THREADS)                                                                          \
-  hipLaunchKernelGGL((plan_kernel<SMALL, THREADS>), dim3(1), dim3(THREADS), 0, st, plan, ids, a_start, a_len,      \
-                     (int)L.T, A, n_slots, bm_s, bm_e, W, L.off_perm, L.off_padapter, L.off_prank, L.off_tiles_s,  \
-                     L.off_tiles_e, L.off_counters, L.off_scratch, (int)L.max_tiles,                              \
+  hipLaunchKernelGGL((plan_kernel<SMALL, THREADS>), dim3(parts, n_plans), dim3(THREADS), 0, st, set.plan[0], ids, a_start, \
+                     a_len, (int)L.T, A, n_slots, set.bm_s[0], set.bm_e[0], W, set, L.off_perm, L.off_padapter, L.off_prank,                \
+                     L.off_tiles_s, L.off_tiles_e, L.off_counters, L.off_scratch,                                 \
                      (int)(L.off_scratch - L.off_counters), merged)
   if (few) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL);
   else if (A <= PLAN_SMALL_A) MLORA_LAUNCH_PLAN(true, PLAN_THREADS);

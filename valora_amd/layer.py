@@ -62,8 +62,7 @@ class LayerPlans:
 
     def __init__(self, ids: torch.Tensor, a_start: torch.Tensor, a_len: torch.Tensor, max_rank: int, hidden: int,
                  mlp: int, n_slots: int = 4):
-        self.h = LoraPlan(ids, a_start, a_len, max_rank, n_slots=n_slots, hidden=hidden)
-        self.m = LoraPlan(ids, a_start, a_len, max_rank, n_slots=n_slots, hidden=mlp)
+        self.h, self.m = LoraPlan.of_widths(ids, a_start, a_len, max_rank, (hidden, mlp), n_slots=n_slots)
 
 
 def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float = 1e-6) -> torch.Tensor:

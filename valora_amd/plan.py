@@ -25,7 +25,7 @@ class LoraPlan:
                  bm_expand: Optional[int] = None, ksplit: Optional[int] = None,
                  reduce_in_expand: Optional[bool] = None, one_launch: Optional[bool] = None,
                  one_launch_no_wait: bool = False, shrink_recompute: bool = False, expand_column_loop: bool = False,
-                 one_launch_never_ready: bool = False, _merged: int = -1):
+                 one_launch_never_ready: bool = False, _merged: int = -1, _cut: bool = True):
         """``ids``: int64 per-token adapter index (negative = no adapter); ``a_start`` / ``a_len``:
         the pool index (``a_len = n_slots * rank``); ``max_rank``: widest rank among the resident
         adapters (the reference's ``max_lora_dim``, lora_unordered_batch_infer.py:181-182).
@@ -70,8 +70,20 @@ class LoraPlan:
         if expand_column_loop:
             self.flags |= _lib.EXPAND_COLUMN_LOOP
         # plan, scratch and the calls themselves live on the native side (csrc/binding.cpp)
-        self._native = _b.NativePlan(ids, a_start, a_len, self.max_rank, n_slots, self.bm_shrink, self.bm_expand,
-                                     self.ksplit, self.flags, int(_merged))
+        if _cut:
+            self._native = _b.NativePlan(ids, a_start, a_len, self.max_rank, n_slots, self.bm_shrink, self.bm_expand,
+                                         self.ksplit, self.flags, int(_merged))
+
+    @classmethod
+    def of_widths(cls, ids: torch.Tensor, a_start: torch.Tensor, a_len: torch.Tensor, max_rank: int, widths,
+                  n_slots: int = 4) -> list:
+        """One plan per input width, of the same batch: what ``LoraPlan(..., hidden=w)`` makes for each ``w`` of
+        ``widths`` (at most four), with the tiles of all of them cut in one launch."""
+        plans = [cls(ids, a_start, a_len, max_rank, n_slots=n_slots, hidden=w, _cut=False) for w in widths]
+        shapes = [[p.bm_shrink, p.bm_expand, p.ksplit, p.flags] for p in plans]
+        for p, native in zip(plans, _b.NativePlan.several(ids, a_start, a_len, int(max_rank), n_slots, shapes)):
+            p._native = native
+        return plans
 
     @property
     def buf(self) -> torch.Tensor:
