@@ -1,11 +1,12 @@
 // LoRA expand for gfx950:  y[t, o] = T( y[t, o] + scale_a * sum_{j<r} T(v[t, j]) * B_a[j, o] )
 //
 // The pool stores a slot's B block as [H_out, r] row-major spread over r pool rows, so output
-// column o owns r consecutive elements at flat offset o*r: the B operand of the MFMA (column =
-// output, 8 consecutive rank elements per lane) is again one 16-byte global load per lane, and
-// 16 neighbouring outputs are one contiguous 32*r-byte run.  A workgroup owns one adapter-grouped
+// column o owns r consecutive elements at flat offset o*r: a B operand of the MFMA (row =
+// output, 8 consecutive rank elements per lane) is again one 16-byte global load per lane.
+// A workgroup owns one adapter-grouped
 // tile of tokens and 256 output columns (64 per wave); each wave loads its B fragments once into
-// registers and reuses them for every 16-token block of the tile.  The fp32 MFMA result is
+// registers and reuses them for every 16-token block of the tile; the tile's v rows are loaded once
+// per workgroup into LDS.  The fp32 MFMA result is
 // turned through a small LDS tile so that the read-modify-write of y is done with 16-byte
 // accesses of 128 contiguous bytes per token row; the add is done in fp32 and rounded once.
 //
@@ -25,218 +26,221 @@ constexpr int EXP_BN = 256;       // outputs per workgroup
 constexpr int EXP_WN = 64;        // outputs per wave
 constexpr int STAGE_LD = EXP_WN + 4;
 constexpr int EXP_MBU = 2;         // 16-token blocks whose loads are in flight together
-constexpr int EXP_MAX_BM = 256;   // tallest expand tile (tokens), one thread per token at set-up
+constexpr int64_t MAX_GRID_TILES = 65535;   // tiles of one launch: grid y is 16 bits
+constexpr int EXP_V_BATCH = 3;     // chunks of v a thread requests together
+__host__ __device__ constexpr int expand_v_chunks(int kb) { return kb * 4 + 1; }   // LDS chunks of a v row, odd
 
-
-// the arguments of target z of a multi-target launch
-__device__ __forceinline__ ExpandArgs select_target(const ExpandArgs &a, int z) {
-  ExpandArgs p = a;
-  p.slot = a.slots[z];
-  p.y = a.ys[z];
-  p.pool.w = a.ws[z];
-  p.pool.w_rows = a.w_rows_t[z];
-  p.v = a.v + (int64_t)z * a.v_tstride;
-  if (a.partial) p.partial = a.partial + (int64_t)z * a.partial_tstride;
-  return p;
-}
-
-// Waves per SIMD the register allocator has to leave room for.  The rank-64 variant that reads a finished
-// v sits 2 registers above the 96 that allow 5 waves; held to 5 it measured 1-6 % faster on the prefill and
-// mixed shapes (more workgroups resident per round), at 6 it spills.  The rank-32 one fits 7 (at 5 a 6749-token prefill
-// takes 27.5 instead of 26 us), and the one that sums partials 4.
+// Waves per SIMD the register allocator has to leave room for: as many as do without spills.
 constexpr int expand_min_waves(int kb, bool partial, bool comp) {
-  return comp ? 1 : kb == 2 && !partial ? 5 : kb == 1 ? (partial ? 4 : 7) : 1;
+  return comp || partial ? 1 : kb == 1 ? 6 : kb == 2 ? 5 : 1;
 }
 
+// Tall tiles.  One scalar round trip (record, arguments), one of look-ups and v, one for B and the first y rows; then a loop
+// over 32 tokens.
+// Bound by the y stream (43 MB in place take 18.1 us as one linear pass, 231 MB 81), and before that by its own instructions and by v:
+// with a masked load for every unit, a look-up per unit and v as MFMA operands by every wave it had 670 instructions in front of
+// the loop and 450 per 32 tokens; now 500 and 190.  Cold layers, before / now, us a launch: 6749 tokens of rank 32, 4096 columns, 32-token
+// tiles 26.3 / 25.1; 5254 tokens of rank 64, 96-token tiles, one target of 4096 columns 26.4 / 22.7, three 67.4 / 57.3, two of 11008
+// 108.8 / 99.4; 5401 tokens over ranks 8-64 24.8 / 22.6, 57.9 / 54.5, 93.0 / 90.9; 10000 tokens over 8 adapters of rank 128, shrink and
+// expand 106 / 92.  (Of the 109 us, B and v together were 29, v alone 8.  One more or one less waves' worth of registers spills or gains
+// nothing; 16 instead of 8 staged tokens, 8.7 KB more LDS, 1 % slower.)
 // COMP: the compensation of a request whose base weights hold another adapter (csrc/api.hip, mlora_lora_compensate):
 // y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), where v' is the "target" 1 matrix of the same positions:
 // both products in one pass over y.
-template <typename T, int KB, bool PARTIAL, bool COMP>
-__global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expand_kernel(const int32_t *tiles_base, int h_n_ochunks,
-                                                                                    ExpandArgs args_in) {
-  // (tiles_base, h_n_ochunks: what the first dependent load needs, in front so that kernel-argument preloading
-  // delivers them in registers)
+template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP>
+__global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expand_kernel(const int32_t *tiles_base, const int32_t *perm,
+                                                                                    const int64_t *a_loc, int h_n_loc, int h_out,
+                                                                                    ExpandArgs p) {
+  // (the leading parameters: what the first dependent loads need; kernel-argument preloading delivers them in registers)
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
-  __shared__ float stage[4][16][STAGE_LD];
-  __shared__ int32_t s_perm[EXP_MAX_BM];
-
-  const int tile_idx = blockIdx.x / h_n_ochunks;
-  const int oc = blockIdx.x - tile_idx * h_n_ochunks;
-  const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
-  const int a = tile[0], r = tile[1], pos0 = tile[2], astart = tile[4];
-  const int cnt = COMP ? abs(tile[3]) : tile[3];   // (negative: no usable rank of its own, r = 0)
-  if (cnt <= 0) return;   // records past the last tile are zero
-  const ExpandArgs p = select_target(args_in, blockIdx.y);
   constexpr int MBU = COMP && KB == 4 ? 1 : EXP_MBU;   // two rank-128 operand sets leave registers for one block
-  const int rk = min(r, p.kmax);  // rank columns the narrow operand really has (bgmv_impl.cuh:167,186)
+  constexpr int VC = KB * 4, VLD = expand_v_chunks(KB);
+  __shared__ __align__(16) float stage[4][8][STAGE_LD];
+  // The tile's v rows, with COMP the merged adapter's behind them, and its token indices.  (As small as they can be: 96 tokens of
+  // rank 64 are 31.6 KB a workgroup in all, five on a compute unit.)
+  extern __shared__ __align__(16) unsigned char s_v[];
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tile_idx = (int)blockIdx.y, z = (int)blockIdx.z;
+  const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
+  int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
+  uint16_t *y = p.ys[z];
+  const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
+  int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
+  float inv_h_out = p.inv_h_out;
+  asm volatile("" : "+s"(ad), "+s"(r), "+s"(pos0), "+s"(cnt), "+s"(astart), "+s"(slot), "+s"(kmax), "+s"(w_rows), "+s"(v_by_pos),
+                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out));
+  if (COMP) cnt = abs(cnt);                  // (negative: no usable rank of its own, r = 0)
+  if (cnt <= 0) return;                      // records past the last tile are zero
+  y = as_global(y);
+  w = as_global(w);
+  v = as_global(v);
+  scales = as_global(scales);
+  const bool by_pos = PARTIAL || COMP || v_by_pos;
+  unsigned char *const s_v2 = s_v + (COMP ? cnt * VLD * 16 : 0);
+  int32_t *const s_perm = reinterpret_cast<int32_t *>(s_v + (COMP ? 2 : 1) * cnt * VLD * 16);
+
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, kg = lane >> 4;
-  const int64_t base = (int64_t)astart + (int64_t)r * p.slot;
-  const int o_wave = oc * EXP_BN + wave * EXP_WN;
+  const uint32_t o_wave = blockIdx.x * (uint32_t)EXP_BN + (uint32_t)(wave * EXP_WN);
+  const int rk = min(r, kmax);  // rank columns the narrow operand really has (bgmv_impl.cuh:167,186)
 
-  // Everything that depends only on the tile header is requested first, in one round trip:
-  // the tile's token indices, the pool rows of the B fragments and the scale.
-  int my_perm = 0;
-  if (tid < cnt) my_perm = p.plan[p.off_perm + pos0 + tid];
-  const float scale = Tr::to_float(p.scales[a]);
-  const float inv_h_out = 1.0f / (float)p.h_out;
-  int64_t brow[4][KB];
-  uint32_t boff[4][KB];
-  auto look_up = [&](int rr, int rrk, int64_t rbase, int64_t (&row)[4][KB], uint32_t (&off)[4][KB]) {
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const int o = o_wave + nb * 16 + lrow;
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int j0 = kb * 32 + kg * 8;
-        row[nb][kb] = -1;
-        off[nb][kb] = 0;
-        if (o < p.h_out && j0 < rrk) {
-          const uint32_t flat = (uint32_t)o * (uint32_t)rr + (uint32_t)j0;   // < 2^16 * 2^7
-          uint32_t bin;
-          divmod24(flat, (uint32_t)p.h_out, inv_h_out, bin, off[nb][kb]);
-          const int64_t idx = rbase + bin;
-          if (idx >= 0 && idx < p.pool.a_loc_len) row[nb][kb] = p.pool.a_loc[idx];
-        }
-      }
-    }
-  };
-  look_up(r, rk, base, brow, boff);
-  int64_t brow2[COMP ? 4 : 1][COMP ? KB : 1];
-  uint32_t boff2[COMP ? 4 : 1][COMP ? KB : 1];
-  int rk2 = 0;
+  // ---- everything that depends only on the record: token indices, pool rows of the B fragments, scale, v rows by position
+  const int my_perm = perm[pos0 + min(tid, cnt - 1)];
+  const float scale = Tr::to_float(scales[ad]);
+  const SmallPool pool = {w, a_loc, (uint32_t)h_n_loc, (uint32_t)w_rows, (uint32_t)h_out, inv_h_out, (uint32_t)(astart + r * slot), r, rk};
+  SmallRows<KB, WIDE> rows, rows2;
+  small_look_up<KB, WIDE>(pool, o_wave, lane, rows);
+  SmallPool pool2 = pool;
   float scale2 = 0.f;
   if constexpr (COMP) {
     const int r2 = p.plan[H_MERGED_RANK];
-    rk2 = min(r2, p.kmax);
-    if (r2 > 0) scale2 = -Tr::to_float(p.scales[p.plan[H_MERGED]]);
-    look_up(r2, rk2, (int64_t)p.plan[H_MERGED_START] + (int64_t)r2 * p.slot, brow2, boff2);
+    pool2.r = r2;
+    pool2.rk = min(r2, kmax);
+    pool2.base = (uint32_t)(p.plan[H_MERGED_START] + r2 * slot);
+    if (r2 > 0) scale2 = -Tr::to_float(scales[p.plan[H_MERGED]]);
+    small_look_up<KB, WIDE>(pool2, o_wave, lane, rows2);
   }
-  s_perm[tid] = my_perm;
-  // The only workgroup-wide barrier: it also drains the loads above (which everything below needs
-  // anyway).  No barrier may follow the bulk loads below -- a barrier waits for all outstanding
-  // global loads and would serialise the B, y and v traffic into separate round trips.
+  // The v rows go through LDS, whole lines, once per workgroup: loaded as MFMA operands by every wave they are as many bytes as
+  // the y rows, in a pattern that a compute unit takes 64 cycles an instruction for.  16-byte chunk c of row `row` stands at chunk
+  // row * VLD + c (VLD odd: 16 rows of one chunk spread over the banks), zeros from rank rk on.
+  // A thread's chunks are requested EXP_V_BATCH at a time, `put` writes them.
+  const int n_chunks = cnt * VC;
+  auto v_request = [&](int e0, const uint16_t *src, int rkk, bool pos, u32x4 (&q)[EXP_V_BATCH]) {
+#pragma unroll
+    for (int u = 0; u < EXP_V_BATCH; ++u) {
+      const int e = e0 + u * 256 + tid;
+      if (e0 + u * 256 + wave * 64 >= n_chunks) break;   // wave-uniform
+      const int row = min(e / VC, cnt - 1), j0 = (e % VC) * 8;
+      if constexpr (PARTIAL) {
+        // split-K partials of the shrink: four chunks are requested before any is consumed, summed in chunk order and
+        // rounded to T once
+        u32x4 f[1];
+        small_v_partials<T, 1>(as_global(p.partial) + z * p.partial_tstride + (int64_t)pos0 * p.rp, (uint32_t)(row * p.rp + (j0 < rkk ? j0 : 0)),
+                               (int64_t)p.T * p.rp, p.ksplit, 8, 0, f);
+        q[u] = j0 < rkk ? f[0] : u32x4{0, 0, 0, 0};
+      } else {
+        const uint32_t vrow = pos ? (uint32_t)(pos0 + row) : (uint32_t)s_perm[row];
+        q[u] = load16(small_source(j0 < rkk, src + (uint64_t)vrow * (uint64_t)v_stride + j0));
+      }
+    }
+  };
+  auto v_put = [&](int e0, unsigned char *dst, const u32x4 (&q)[EXP_V_BATCH]) {
+#pragma unroll
+    for (int u = 0; u < EXP_V_BATCH; ++u) {
+      const int e = e0 + u * 256 + tid;
+      if (e0 + u * 256 + wave * 64 >= n_chunks) break;
+      if (e < n_chunks) *reinterpret_cast<u32x4 *>(dst + ((e / VC) * VLD + e % VC) * 16) = q[u];
+    }
+  };
+  u32x4 q[EXP_V_BATCH];
+  if (by_pos) {
+    for (int e0 = 0; e0 < n_chunks; e0 += 256 * EXP_V_BATCH) {
+      v_request(e0, v + z * v_tstride, rk, true, q);
+      v_put(e0, s_v, q);
+    }
+    if constexpr (COMP)   // the same positions' rows of the merged adapter's matrix
+      for (int e0 = 0; e0 < n_chunks; e0 += 256 * EXP_V_BATCH) {
+        v_request(e0, v + v_tstride, pool2.rk, true, q);
+        v_put(e0, s_v2, q);
+      }
+  }
+  if (tid < cnt) s_perm[tid] = my_perm;
+  // This barrier drains the loads above, which everything below needs anyway.  None may follow the bulk loads below: a barrier
+  // waits for all outstanding global loads and would serialise the B and y traffic into separate round trips.
   __syncthreads();
 
-  // B fragments: bfrag[nb][kb] = B^T[o = o_wave + nb*16 + lrow][j0 .. j0+8), j0 = kb*32 + kg*8
-  u32x4 bfrag[4][KB], bfrag2[COMP ? 4 : 1][COMP ? KB : 1];
-  auto load_b = [&](const int64_t (&brw)[4][KB], const uint32_t (&off)[4][KB], u32x4 (&frag)[4][KB]) {
-#pragma unroll
-    for (int nb = 0; nb < 4; ++nb)
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int64_t row = brw[nb][kb];
-        frag[nb][kb] = (row >= 0 && row < p.pool.w_rows) ? load16(p.pool.w + row * p.h_out + off[nb][kb])
-                                                          : u32x4{0, 0, 0, 0};
-      }
-  };
-  load_b(brow, boff, bfrag);
-  if constexpr (COMP) load_b(brow2, boff2, bfrag2);
+  // rows of the caller's matrix are found through the tokens: requested in front of B and y, written behind
+  if (!by_pos) v_request(0, v, rk, false, q);
 
   // row-major roles for the y read-modify-write: 8 lanes x 16 B cover one token row of the wave's
-  // 64 outputs; a wave covers 8 rows per access, two accesses per 16-token block.
+  // 64 outputs; a wave covers 8 rows per access, two accesses per 16-token block.  A row or column that is not there is the
+  // tile's last row or the row's first column: read, and not stored.
   const int rr0 = lane >> 3, c8 = (lane & 7) * 8;
-  const bool ocol_ok = (o_wave + c8) < p.h_out;
-
-  // Two 16-token blocks per iteration: their y rows and v fragments are all requested before either
-  // block is consumed, so an iteration costs one memory round trip for 32 tokens.
-  const int n_mb = (cnt + 15) >> 4;
-  for (int mb0 = 0; mb0 < n_mb; mb0 += MBU) {
-    u32x4 yv[MBU][2];
-    uint16_t *yp[MBU][2];
-    bool yok[MBU][2];
-    u32x4 vfrag[MBU][KB], vfrag2[COMP ? MBU : 1][COMP ? KB : 1];
+  const bool ocol_ok = o_wave + c8 < (uint32_t)h_out;
+  uint16_t *const ycol = y + (ocol_ok ? o_wave + c8 : 0u);
+  u32x4 yv[MBU][2];
+  uint16_t *yp[MBU][2];
+  auto load_y = [&](int mb0) {
+    int t[MBU][2];
 #pragma unroll
-    for (int b = 0; b < MBU; ++b) {
-      const int mb = mb0 + b;
-      // ---- y rows first (the longest-latency loads of the iteration)
+    for (int b = 0; b < MBU; ++b)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) t[b][h] = s_perm[min((mb0 + b) * 16 + rr0 + 8 * h, cnt - 1)];
+#pragma unroll
+    for (int b = 0; b < MBU; ++b)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const int row = mb * 16 + rr0 + 8 * h;
-        yok[b][h] = ocol_ok && row < cnt;
-        const int t = yok[b][h] ? s_perm[row] : 0;
-        yp[b][h] = p.y + (int64_t)t * p.h_out + o_wave + c8;
-        yv[b][h] = yok[b][h] ? load16(yp[b][h]) : u32x4{0, 0, 0, 0};
+        yp[b][h] = ycol + (uint64_t)(uint32_t)t[b][h] * (uint32_t)h_out;
+        yv[b][h] = load16(yp[b][h]);
       }
-      // ---- v fragments: rows = tokens (lrow), 8 consecutive rank elements per lane
-      const int prow = mb * 16 + lrow;
-      const bool pok = prow < cnt;
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        const int j0 = kb * 32 + kg * 8;
-        u32x4 v = {0, 0, 0, 0};
-        if (pok && j0 < rk) {
-          if constexpr (PARTIAL) {
-            // split-K partials of the shrink: all chunks are requested before any is consumed,
-            // summed in chunk order and rounded to T once
-            float f[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            const float *src0 = p.partial + ((int64_t)pos0 + prow) * p.rp + j0;
-            const int64_t sstride = (int64_t)p.T * p.rp;
-            for (int s0 = 0; s0 < p.ksplit; s0 += 4) {
-              f32x4 lo[4], hi[4];
-#pragma unroll
-              for (int u = 0; u < 4; ++u) {
-                const bool ok = s0 + u < p.ksplit;
-                const f32x4 *src = reinterpret_cast<const f32x4 *>(src0 + (int64_t)(s0 + u) * sstride);
-                lo[u] = ok ? src[0] : f32x4{0.f, 0.f, 0.f, 0.f};
-                hi[u] = ok ? src[1] : f32x4{0.f, 0.f, 0.f, 0.f};
-              }
-#pragma unroll
-              for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) { f[i] += lo[u][i]; f[4 + i] += hi[u][i]; }
-            }
-            v = pack8<T>(f);
-          } else {
-            const int64_t vrow = p.v_by_pos ? (int64_t)(pos0 + prow) : (int64_t)s_perm[prow];
-            v = load16(p.v + vrow * p.v_stride + j0);
-          }
-        }
-        vfrag[b][kb] = v;
-        if constexpr (COMP)   // the same positions' rows of the merged adapter's matrix
-          vfrag2[b][kb] = (pok && j0 < rk2) ? load16(p.v + p.v_tstride + (int64_t)(pos0 + prow) * p.v_stride + j0)
-                                            : u32x4{0, 0, 0, 0};
-      }
+  };
+  u32x4 bfrag[4 * KB], bfrag2[COMP ? 4 * KB : 1];
+  small_load_b<KB, WIDE, true>(pool, lane, rows, bfrag);
+  if constexpr (COMP) small_load_b<KB, WIDE, true>(pool2, lane, rows2, bfrag2);
+  load_y(0);
+  requested();
+  if (!by_pos) {
+    v_put(0, s_v, q);
+    for (int e0 = 256 * EXP_V_BATCH; e0 < n_chunks; e0 += 256 * EXP_V_BATCH) {
+      v_request(e0, v, rk, false, q);
+      v_put(e0, s_v, q);
     }
+    wait_lgkmcnt0();
+    __builtin_amdgcn_s_barrier();
+    requested();
+  }
+  if (o_wave >= (uint32_t)h_out) return;
+
+  // Two 16-token blocks per iteration: their y rows are all requested before either
+  // block is consumed, so an iteration costs one memory round trip for 32 tokens.
+  for (int mb0 = 0;;) {
 #pragma unroll
     for (int b = 0; b < MBU; ++b) {
-      if (mb0 + b < n_mb) {   // workgroup-uniform
-        // ---- delta block through the matrix cores, turned through LDS into token-major order and added to the y rows
-        auto add = [&](const u32x4 (&vf)[KB], const u32x4 (&bf)[4][KB], int rkk, float sc, bool last) {
+      const int row0 = (mb0 + b) * 16;
+      if (b > 0 && row0 >= cnt) break;   // workgroup-uniform
+      // ---- delta block through the matrix cores, output by token (expand_core.h: a lane has 16 consecutive outputs of token
+      // lrow), turned through LDS into rows and added to y
+      auto add = [&](const unsigned char *vs, const u32x4 (&bf)[4 * KB], float sc, bool last) {
+        u32x4 vf[KB];
+        const unsigned char *const vrow = vs + (min(row0 + lrow, cnt - 1) * VLD + kg) * 16;
 #pragma unroll
-          for (int nb = 0; nb < 4; ++nb) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        for (int kb = 0; kb < KB; ++kb) vf[kb] = *reinterpret_cast<const u32x4 *>(vrow + kb * 64);
+        f32x4 acc[4];
 #pragma unroll
-            for (int kb = 0; kb < KB; ++kb)
-              if (kb * 32 < rkk) acc = Tr::mfma(as<vec8>(vf[kb]), as<vec8>(bf[nb][kb]), acc);
+        for (int nb = 0; nb < 4; ++nb) acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 4; ++i) stage[wave][kg * 4 + i][nb * 16 + lrow] = acc[i];
-          }
-          // stage[wave] is private to this wave and a wave's LDS operations execute in order, so only
-          // the compiler has to be kept from reordering the reads below over the writes above.
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          __builtin_amdgcn_wave_barrier();
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            if (yok[b][h]) {
-              const float *srow = &stage[wave][rr0 + 8 * h][c8];
-              float f[8];
-              unpack8<T>(yv[b][h], f);
+          for (int nb = 0; nb < 4; ++nb) acc[nb] = Tr::mfma(as<vec8>(bf[nb * KB + kb]), as<vec8>(vf[kb]), acc[nb]);
+        // Eight tokens at a time.  stage[wave] is private to this wave and a wave's LDS operations execute in order, so only
+        // the compiler has to be kept from reordering the reads below over the writes above.
 #pragma unroll
-              for (int i = 0; i < 8; ++i) f[i] += sc * srow[i];
-              if (last) store16(yp[b][h], pack8<T>(f));
-              else yv[b][h] = pack8<T>(f);
-            }
+        for (int h = 0; h < 2; ++h) {
+          if ((lrow >> 3) == h) {
+#pragma unroll
+            for (int nb = 0; nb < 4; ++nb) *reinterpret_cast<f32x4 *>(&stage[wave][lrow & 7][kg * 16 + nb * 4]) = acc[nb];
           }
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           __builtin_amdgcn_wave_barrier();
-        };
-        if (!COMP || rk > 0) add(vfrag[b], bfrag, rk, scale, !COMP);
-        if constexpr (COMP) add(vfrag2[b], bfrag2, rk2, scale2, true);
-      }
+          const float *srow = &stage[wave][rr0][c8];
+          float f[8];
+          unpack8<T>(yv[b][h], f);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) f[i] += sc * srow[i];
+          yv[b][h] = pack8<T>(f);
+          if (last && ocol_ok && row0 + rr0 + 8 * h < cnt) store16(yp[b][h], yv[b][h]);
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+        }
+      };
+      if (!COMP || rk > 0) add(s_v, bfrag, scale, !COMP);
+      if constexpr (COMP) add(s_v2, bfrag2, scale2, true);
     }
+    mb0 += MBU;
+    if (mb0 * 16 >= cnt) break;
+    load_y(mb0);
   }
 }
 
@@ -245,7 +249,6 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 // (Two or four column chunks a workgroup, all their loads in flight together, lose wherever the narrow operand is finished: 512
 // tokens, q+k+v at rank 16 26.1 / 27.5 us with its shrink, one target of 256 tokens, 11008 columns 8.6 / 9.6, ranks 8-64, gate+up
 // of 13824 columns 25.2 / 27.4.)
-constexpr int64_t SMALL_MAX_TILES = 65535;   // tiles of one launch: grid y is 16 bits
 constexpr int small_min_waves(int kb, bool wide, bool comp) {   // as many as do without spills
   return comp ? (kb <= 1 ? 7 : 1) : kb <= 1 ? 8 : kb == 2 ? (wide ? 6 : 5) : (wide ? 4 : 3);
 }
@@ -345,9 +348,9 @@ int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
   else MLORA_SMALL(false, PARTIAL, COMP)
   // Exactly as many workgroups as there are records: what stands behind the last one is no record (the words of the one-launch
   // op do, and a call of that kind leaves them non-zero).  More tiles than a grid's y takes (a million tokens) are several launches.
-  for (int64_t t0 = 0; t0 < tiles; t0 += SMALL_MAX_TILES) {
+  for (int64_t t0 = 0; t0 < tiles; t0 += MAX_GRID_TILES) {
     const int32_t *records = a.plan + a.off_tiles + t0 * TILE_WORDS;
-    const dim3 grid((unsigned)a.n_ochunks, (unsigned)(tiles - t0 < SMALL_MAX_TILES ? tiles - t0 : SMALL_MAX_TILES), (unsigned)a.n_targets);
+    const dim3 grid((unsigned)a.n_ochunks, (unsigned)(tiles - t0 < MAX_GRID_TILES ? tiles - t0 : MAX_GRID_TILES), (unsigned)a.n_targets);
     if (a.compensate) { MLORA_SMALL_WIDTH(false, true); }
     else if (a.partial) { MLORA_SMALL_WIDTH(true, false); }
     else { MLORA_SMALL_WIDTH(false, false); }
@@ -365,38 +368,44 @@ int launch_small_t(hipStream_t st, const ExpandArgs &a, int max_rank, int64_t ti
   return launch_small_kb<T, 4>(st, a, tiles);
 }
 
-template <typename T>
-int launch_expand_t(hipStream_t st, const ExpandArgs &a, int kb, dim3 grid) {
-#define MLORA_EXPAND(KB, PARTIAL, COMP)                                                                              \
-  hipLaunchKernelGGL((expand_kernel<T, KB, PARTIAL, COMP>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.n_ochunks, a)
-#define MLORA_EXPAND_KB(KB)                                                                                          \
-  if (a.compensate) MLORA_EXPAND(KB, false, true);                                                                   \
-  else if (a.partial) MLORA_EXPAND(KB, true, false);                                                                 \
-  else MLORA_EXPAND(KB, false, false)
-  switch (kb) {
-    case 1: MLORA_EXPAND_KB(1); break;
-    case 2: MLORA_EXPAND_KB(2); break;
-    case 4: MLORA_EXPAND_KB(4); break;
-    default: return fail(MLORA_ERR_NO_KERNEL, "expand: no kernel for %d rank blocks", kb);
+template <typename T, int KB>
+int launch_expand_kb(hipStream_t st, const ExpandArgs &a, int bm, int64_t tiles) {
+  // an index without entries: the kernel reads one all the same, and drops it
+  const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
+  const int lds = bm * ((a.compensate ? 2 : 1) * expand_v_chunks(KB) * 16 + 4);
+#define MLORA_EXPAND(WIDE, PARTIAL, COMP)                                                                       \
+  hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP>), grid, dim3(256), lds, st, records,            \
+                     a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
+#define MLORA_EXPAND_WIDTH(PARTIAL, COMP)                     \
+  if (a.h_out >= SMALL_WIDE) MLORA_EXPAND(true, PARTIAL, COMP); \
+  else MLORA_EXPAND(false, PARTIAL, COMP)
+  for (int64_t t0 = 0; t0 < tiles; t0 += MAX_GRID_TILES) {
+    const int32_t *records = a.plan + a.off_tiles + t0 * TILE_WORDS;
+    const dim3 grid((unsigned)a.n_ochunks, (unsigned)(tiles - t0 < MAX_GRID_TILES ? tiles - t0 : MAX_GRID_TILES), (unsigned)a.n_targets);
+    if (a.compensate) { MLORA_EXPAND_WIDTH(false, true); }
+    else if (a.partial) { MLORA_EXPAND_WIDTH(true, false); }
+    else { MLORA_EXPAND_WIDTH(false, false); }
   }
-#undef MLORA_EXPAND_KB
+#undef MLORA_EXPAND_WIDTH
 #undef MLORA_EXPAND
   return check_launch("expand_kernel");
+}
+
+template <typename T>
+int launch_expand_t(hipStream_t st, const ExpandArgs &a, int max_rank, int bm, int64_t tiles) {
+  if (max_rank <= 32) return launch_expand_kb<T, 1>(st, a, bm, tiles);
+  if (max_rank <= 64) return launch_expand_kb<T, 2>(st, a, bm, tiles);
+  return launch_expand_kb<T, 4>(st, a, bm, tiles);
 }
 
 }  // namespace
 
 int launch_expand(hipStream_t st, const ExpandArgs &a, int max_rank, int64_t grid_tiles, int bm_expand, mlora_dtype dt) {
-  int kb = (max_rank + 31) / 32;
-  kb = kb <= 1 ? 1 : kb <= 2 ? 2 : 4;
   if (grid_tiles <= 0) return MLORA_OK;
   if (bm_expand == 16)
     return dt == MLORA_F16 ? launch_small_t<_Float16>(st, a, max_rank, grid_tiles) : launch_small_t<__bf16>(st, a, max_rank, grid_tiles);
-  const int64_t blocks = grid_tiles * a.n_ochunks;
-  if (blocks > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "expand: grid too large");
-  dim3 grid((unsigned)blocks, (unsigned)a.n_targets);
-  return dt == MLORA_F16 ? launch_expand_t<_Float16>(st, a, kb, grid)
-                         : launch_expand_t<__bf16>(st, a, kb, grid);
+  return dt == MLORA_F16 ? launch_expand_t<_Float16>(st, a, max_rank, bm_expand, grid_tiles)
+                         : launch_expand_t<__bf16>(st, a, max_rank, bm_expand, grid_tiles);
 }
 
 int expand_bn() { return EXP_BN; }

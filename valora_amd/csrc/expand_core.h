@@ -140,9 +140,9 @@ __device__ const __align__(128) uint16_t g_small_zeros[64] = {};
 __device__ __forceinline__ const uint16_t *small_source(bool ok, const void *src) {
   return as_global(reinterpret_cast<const uint16_t *>(ok ? src : static_cast<const void *>(g_small_zeros)));
 }
-// Requests the lane's units; units without a pool row are zero, those beyond the narrow operand's columns are whatever stands
-// there (small_product drops them).
-template <int KB, bool WIDE>
+// Requests the lane's units; units without a pool row are zero, those beyond the narrow operand's columns are zero with IN_RANK,
+// else whatever stands there (small_product drops them).
+template <int KB, bool WIDE, bool IN_RANK = false>
 __device__ __forceinline__ void small_load_b(const SmallPool &p, int lane, const SmallRows<KB, WIDE> &s, u32x4 (&raw)[SmallB<KB>::LOADS]) {
   using B = SmallB<KB>;
   constexpr int N = SmallRows<KB, WIDE>::N;
@@ -166,7 +166,7 @@ __device__ __forceinline__ void small_load_b(const SmallPool &p, int lane, const
       src = bp[i] + s.off[i] * 2u;
       ok = bok[i];
     }
-    raw[i] = load16(small_source(ok, src));
+    raw[i] = load16(small_source(ok && (!IN_RANK || B::in_rank(i, lane, p.rk)), src));
   }
 }
 // acc[nb] = fragment nb of B^T times v^T; units beyond the operand's columns count as zero.  (Masked here and not at the load:
