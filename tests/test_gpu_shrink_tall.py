@@ -113,3 +113,34 @@ def test_k_steps_same_bits(dev, h_in, bm, rank):
                                                plan.scratch.numel(), _lib.ptr(xd), T, h_in, rank, pa, 2, ks, _lib.ptr(v), rank,
                                                0, 0, 0, _lib.dtype_code(dtype)))
             assert torch.equal(v.cpu(), want), f"tile {tile} ks {ks}"
+
+
+@pytest.mark.parametrize("bm,ranks", [(128, [8, 24, 40, 72, 128, 16]), (128, [16, 8, 32, 24]), (256, [64, 16, 40, 24, 8])])
+@pytest.mark.parametrize("h_in", [200, 320])
+def test_narrow_adapters_among_wide_ones(dev, h_in, bm, ranks):
+    """A tile takes the products of its own adapter's rank class, whatever the batch's widest.  Small integers, as above: one
+    right value per element, for every number of chunks and both ways to store it."""
+    g = torch.Generator().manual_seed(h_in + bm + len(ranks))
+    ids = torch.randint(-1, len(ranks), (3 * bm,), generator=g)
+    T, R = ids.numel(), max(ranks)
+    pool = W.make_pool(ranks, h_in, 64, torch.float16, g, True, heads=1)
+    pool.key_buffer.copy_(torch.randint(-2, 3, pool.key_buffer.shape, generator=g))
+    x = torch.randint(-4, 5, (T, h_in), generator=g).to(torch.float16)
+    v0 = torch.full((T, R), 0.5, dtype=torch.float16)
+    want = O.bgmv_shrink(v0, x, pool.key_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1)
+    pd, xd = pool.to(dev), x.to(dev)
+    pa = _lib.make_pool(pd.key_buffer, pd.a_start, pd.a_len, pd.a_loc, h_in)
+    for ks in (1, 2, 3):
+        plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, R, hidden=h_in, bm_shrink=bm, bm_expand=32, ksplit=ks,
+                        reduce_in_expand=False, one_launch=False)
+        v = v0.to(dev)
+        _lib.check(_lib.lib().mlora_shrink(_lib.current_stream(dev), plan.handle, _lib.ptr(plan.scratch), plan.scratch.numel(), _lib.ptr(xd),
+                                           T, h_in, R, pa, 1, ks, _lib.ptr(v), R, 0, 0, 0, _lib.dtype_code(torch.float16)))
+        assert torch.equal(v.cpu(), want), ks
+        plan.shrink(xd, pd.key_buffer, pd.a_start, pd.a_len, pd.a_loc, 1)
+        perm, rp = plan.perm().long().cpu(), (R + 15) // 16 * 16
+        held = plan.scratch.view(torch.float16)[:T * rp].view(T, rp)[:len(perm)].cpu()
+        for col in range(0, R, 8):
+            has = torch.tensor([ranks[int(ids[t])] > col for t in perm])
+            assert torch.equal(held[has, col:col + 8], want[perm[has], col:col + 8]), (ks, col)
+            assert not held[~has, col:col + 8].any()   # columns past a row's rank are zeros

@@ -78,34 +78,6 @@ __device__ __forceinline__ void store_v4(const ShrinkArgs &p, int pos, int t, in
   for (int i = 0; i < 4; ++i) store_v<T>(p, pos, t, r, col + i, v[i]);
 }
 
-// Epilogue of the GEMM shrink.  `tile` is the workgroup's fp32 result in LDS, row-major
-// with row stride ld: rows = tokens of the tile, columns = rank.
-//   ksplit == 1 : rounded to T and stored.
-//   ksplit  > 1 : stored as this K-chunk's fp32 partial (ordinary stores, then the workgroup is
-//                 done); a later launch on the stream -- shrink_reduce_kernel, or the expand
-//                 itself for small batches -- sums the chunks in index order and rounds once.
-template <typename T>
-__device__ __forceinline__ void shrink_epilogue(const ShrinkArgs &p, const float *tile, int ld, int s, int pos0,
-                                                int cnt, int r, const int32_t *perm) {
-  const int tid = threadIdx.x;
-  if (p.ksplit == 1) {
-    const int n_el = cnt * p.rp;
-    for (int e = tid; e < n_el; e += 256) {
-      const int row = e / p.rp, col = e - row * p.rp;
-      store_v<T>(p, pos0 + row, p.out_by_token ? perm[pos0 + row] : 0, r, col, tile[row * ld + col]);
-    }
-    return;
-  }
-  const int quarter = p.rp >> 2;       // rp is a multiple of 16
-  const int n_vec = cnt * quarter;
-  f32x4 *part = reinterpret_cast<f32x4 *>(p.partial + ((int64_t)s * p.T + pos0) * p.rp);
-  for (int e = tid; e < n_vec; e += 256) {
-    const int row = e / quarter, c4 = e - row * quarter;
-    const float *src = tile + row * ld + 4 * c4;
-    part[e] = f32x4{src[0], src[1], src[2], src[3]};
-  }
-}
-
 // v[row, :] = T(sum_s partial[s][row][:]) for every row that has an adapter; one thread per four columns, a workgroup the rows
 // that fit whole (partial rows stand one after the other: a thread's offset in the workgroup's piece is its index).
 // Bound by a launch and three round trips (arguments, chunks, store): a few MB.  Four or eight chunks are requested before any
@@ -314,150 +286,92 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
 // What a rank row that is not there reads, K step after K step (one 128-byte line).
 __device__ const __align__(128) uint16_t g_zero_line[64] = {};
 
-// Prefill-sized tiles (128 tokens): GEMM structure with a three-stage LDS ring.
+// Prefill-sized tiles (128 or 256 tokens): a GEMM tile.  The four waves split the tile's tokens, so no cross-wave reduction
+// is needed.  A K step of 64 is requested into registers as whole 128-byte lines, every wave its own x rows and a quarter
+// of the adapter's A rows, two steps before it is used, and handed over through two LDS stages; one barrier per step.
 //
-// The four waves split the tile's tokens (32 each), so no cross-wave reduction is needed.  Both
-// operands of a 64-wide K step go from global memory straight into LDS with 16-byte
-// global_load_lds (no registers are held while the data is in flight): every wave streams its
-// own x rows into a private part of the stage, the adapter's A rows are loaded once per
-// workgroup and shared by all waves.  A load instruction covers 8 rows x 128 contiguous bytes
-// (whole cache lines: asking for the two halves of a line with two instructions measured up to
-// 30 % slower) and writes them to LDS in lane order, so a stage holds rows of 128 bytes; the
-// lane that fills 16-byte chunk c of row R fetches global chunk c ^ (R & 7), which spreads the
-// later ds_read_b128 of an MFMA operand (16 rows, one chunk column) over the banks.  Two stages
-// are always in flight while the third is consumed; one s_barrier per K step.
-//
-// Bound by what a compute unit takes in (x from HBM, A once per tile from L2: 33 GB/s measured with plain loads of this
-// pattern) and, on top, by what stands between a barrier and the step's loads: masks, votes and dummy loads per
-// instruction, which whole steps do without.  With that and both halves' LDS reads ahead of the products: 7600-token
-// prefill over 24 adapters of rank 32 (4 layers, shrink and expand) 739 -> 712 us, 5401 tokens of mixed ranks (two
-// layers, seven projections) 789 -> 760, 5254 tokens of rank 64 778 -> 766.  (Either alone: whole steps without masks
-// 741 -> 716, 789 -> 766, 777 -> 769; both halves read ahead 739 -> 728, 801 -> 796, 778 -> 776.)
+// Bound by memory: x once, A once per 128 tokens, the partials, and the y lines the expand before it still has to
+// write back.  With the loads alone 17.1 of 17.9 us, with the products alone 12.3, one step only 6.6 (5254 tokens of rank 64, one
+// target in four chunks); a deeper ring, K starts spread over the channels, ids by XCD and contiguous pool rows change
+// nothing.  Direct global -> LDS loads into a three-stage ring (one or two workgroups a compute unit instead of three, LDS turn
+// of the result, zero rows read for a narrower adapter's rank) / now, behind the same expand: three targets of 5254 tokens of
+// rank 64 37.2 / 33.4 us, 5401 tokens over ranks 8-64, one target 20.4 / 19.6, two 29.5 / 25.6, three 34.5 / 30.7, `down` of 11008
+// 56.6 / 54.9.  (The chunks summed inside the launch by the last to arrive: 20.4 against 15.3 + 5.1 for the two launches, and
+// 43 against 34 + 5 for three targets of rank 64.)
+constexpr int GEMM_KC = 64;                             // K elements of a step: one 128-byte line per row
+constexpr int gemm_stage_bytes(int nb, int mbw) { return (64 * mbw + 16 * nb) * GEMM_KC * 2; }
+constexpr int GEMM_AHEAD = 2;                           // steps requested before the first is used
+
+// One tile and one K chunk, NB 16-row blocks of rank (of the tile's own adapter), MBW 16-token blocks per wave.
 template <typename T, int NB, int MBW>
-__global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_flags, int,
-                                                          ShrinkArgs args_in) {
-  // workgroup id = (tile * targets + target) * ksplit + K chunk.  The id mod 8 selects the XCD, so
-  // with the K chunk as the fast index the tiles of an adapter that share a K chunk of A, and the
-  // targets that share a K chunk of x, meet in one L2.
-  const int wg_tz = blockIdx.x / h_ksplit;
-  const int tile_idx = wg_tz / h_n_targets;
-  const int z_idx = wg_tz - tile_idx * h_n_targets;
-  const ShrinkArgs p = select_target(args_in, z_idx);
-  const int s = blockIdx.x - wg_tz * h_ksplit;
+__device__ __forceinline__ void shrink_gemm_tile(const ShrinkArgs &p, int s, int r, int pos0, int cnt, int astart, unsigned char *lds) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
-  constexpr int KC = 64, KS = KC / 32, STAGES = 3;      // MBW: 16-token blocks per wave (tile = 64 * MBW tokens)
-  static_assert(KC * 2 == 128, "a K step is one 128-byte line per row");
-  constexpr int XBLK = MBW * 2;                         // 8-row groups (1 KB) of x per wave per stage
-  constexpr int ABLK = NB * 2;                          // 8-row groups of A per stage (shared)
-  constexpr int APW = ABLK >= 4 ? ABLK / 4 : 1;         // A groups each wave loads per stage
-  constexpr int A_SLOTS = APW * 4;                      // >= ABLK; surplus slots hold duplicates
-  constexpr int STAGE_BYTES = (4 * XBLK + A_SLOTS) * 1024;
-  constexpr int TILE_BYTES = 64 * MBW * NB * 16 * 4;
-  constexpr int LOADS_PER_STAGE = XBLK + APW;           // per wave, identical for all waves
-  constexpr int RING_BYTES = STAGES * STAGE_BYTES + 1024;   // + one scratch block for dummy loads
-  __shared__ __align__(16) unsigned char s_raw[RING_BYTES > TILE_BYTES ? RING_BYTES : TILE_BYTES];
-
-  const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
-  int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
-  if ((h_flags & SHRINK_COMPENSATE) && z_idx == 1) merged_tile(p.plan, tile_idx, 64 * MBW, r, pos0, cnt, astart);
-  if (cnt <= 0) return;   // records past the last tile are zero
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  constexpr int KC = GEMM_KC, KS = KC / 32;
+  constexpr int XG = MBW * 2;                           // 8-row groups (1 KB) of x per wave and step
+  constexpr int AG = NB * 2;                            // 8-row groups of A per step, shared
+  constexpr int APW = AG >= 4 ? AG / 4 : 1;             // of which a wave loads
+  constexpr int STAGE = gemm_stage_bytes(NB, MBW);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int lrow = lane & 15, kg = lane >> 4;           // MFMA operand roles
-  const int grow = lane >> 3;                           // loader roles: row within an 8-row group,
-  const int gchunk = (lane & 7) ^ grow;                 // global 16-byte chunk this lane fetches
-  const int32_t *__restrict__ perm = p.plan + p.off_perm;
+  const int grow = lane >> 3, gcol = lane & 7;          // loader roles: row within an 8-row group, 16-byte chunk
+  const int32_t *__restrict__ perm = as_global(p.plan) + p.off_perm;
   const int64_t base = (int64_t)astart + (int64_t)r * p.slot;
   const int wrow0 = wave * 16 * MBW;
-  const bool wave_active = wrow0 < cnt;                 // wave-uniform
 
-  // this lane's global row pointers (already at its chunk)
-  const uint16_t *xp[XBLK];
-  bool xok[XBLK];
+  // this lane's global row pointers (already at its chunk), all look-ups in one round trip: a row past the tile's end reads the
+  // first one's, a rank row that is not there a line of zeros on which it stays
+  const bool indexed = p.pool.a_loc_len > 0;
+  const int64_t *const a_loc = indexed ? as_global(p.pool.a_loc) : reinterpret_cast<const int64_t *>(perm);
+  int tok[XG];
+  int64_t prow[APW];
+  bool ok[APW];
 #pragma unroll
-  for (int g = 0; g < XBLK; ++g) {
+  for (int g = 0; g < XG; ++g) {
     const int row = wrow0 + g * 8 + grow;
-    xok[g] = row < cnt;
-    const int t = perm[pos0 + (xok[g] ? row : 0)];       // (a row past the tile's end reads the first one's)
-    xp[g] = p.x + (int64_t)t * p.h_in + gchunk * 8;
+    tok[g] = perm[pos0 + (row < cnt ? row : 0)];
   }
-  // A groups this wave loads: slot = wave*APW + i -> rows slot*8 .. slot*8+7 of the rank
-  const uint16_t *ap[APW];
-  bool aok[APW];
-  int astep[APW];                                       // all bits: the row moves on with K; none: it stays on its line
 #pragma unroll
   for (int i = 0; i < APW; ++i) {
-    const int slot = (wave * APW + i) % ABLK;           // surplus slots duplicate real groups
-    const int j = slot * 8 + grow;
+    const int j = (wave * APW + i) % AG * 8 + grow;     // (rank 16 has two groups: they are loaded and written twice)
     const int64_t idx = base + j;
-    bool ok = j < r && idx >= 0 && idx < p.pool.a_loc_len;
-    const int64_t prow = ok ? p.pool.a_loc[idx] : 0;
-    ok = ok && prow >= 0 && prow < p.pool.w_rows;
-    aok[i] = ok;
-    // a row past the rank, or outside the index or the pool, reads zeros
-    ap[i] = (ok ? p.pool.w + prow * p.h_in : g_zero_line) + gchunk * 8;
-    astep[i] = ok ? -1 : 0;
+    ok[i] = indexed && j < r && idx >= 0 && idx < p.pool.a_loc_len;
+    prow[i] = a_loc[ok[i] ? idx : 0];
+  }
+  const uint16_t *xp[XG], *ap[APW];
+  int astep[APW];                                       // all bits: the row moves on with K; none: it stays on its line
+  const uint16_t *const zeros = as_global(g_zero_line) + gcol * 8;
+#pragma unroll
+  for (int g = 0; g < XG; ++g) xp[g] = as_global(p.x) + (uint64_t)(uint32_t)tok[g] * (uint32_t)p.h_in + gcol * 8;
+#pragma unroll
+  for (int i = 0; i < APW; ++i) {
+    ok[i] = ok[i] && prow[i] >= 0 && prow[i] < p.pool.w_rows;
+    ap[i] = ok[i] ? as_global(p.pool.w) + (uint64_t)(uint32_t)prow[i] * (uint32_t)p.h_in + gcol * 8 : zeros;
+    astep[i] = ok[i] ? -1 : 0;
   }
 
   const int kbeg = s * p.kchunk;
   const int kend = min(p.h_in, kbeg + p.kchunk);
-  const int n_steps = (kend - kbeg + KC - 1) / KC;
-
-  // byte offsets inside a stage: x rows of this wave, then the shared A rows
-  const uint32_t ring = lds_offset(s_raw);
-  const uint32_t x_off = (uint32_t)(wave * XBLK) * 1024u;
-  const uint32_t a_off = (uint32_t)(4 * XBLK) * 1024u;
-  const u32x4 zero4 = {0, 0, 0, 0};
-
-  // Issue every load of one K step: EXACTLY LOADS_PER_STAGE load instructions per wave, because the
-  // consumer waits with a compile-time vmcnt.  A load whose lanes are all masked off would be skipped
-  // by the hardware branch around it, so in that case a dummy load into a scratch block is issued
-  // instead.  Lanes beyond the end of K, and those of rank rows that are not there, write zeros into their own slot (no
-  // other lane touches it).
-  unsigned char *dummy = s_raw + STAGES * STAGE_BYTES;
-  auto load_or_dummy = [&](bool c, const uint16_t *src, unsigned char *dst) {
-    if (__builtin_amdgcn_ballot_w64(c) != 0ull) {
-      if (c) __builtin_amdgcn_global_load_lds(GLOBAL_PTR(src), LDS_PTR(dst), 16, 0, 0);
-    } else {
-      __builtin_amdgcn_global_load_lds(GLOBAL_PTR(p.plan), LDS_PTR(dummy), 16, 0, 0);
-    }
-  };
-  auto issue = [&](int step) {
-    const int stage = step % STAGES;
-    unsigned char *sbase = s_raw + stage * STAGE_BYTES;
+  const int n_steps = (kend - kbeg) / KC;               // whole ones
+  u32x4 rx[GEMM_AHEAD][XG], ra[GEMM_AHEAD][APW];
+  auto request = [&](int step, u32x4 (&x)[XG], u32x4 (&a)[APW]) {
     const int off = kbeg + step * KC;
-    if (off + KC <= kend) {
-      // whole steps, all but the last one of a K that is not a multiple of 64: every lane reads, x rows past the tile's end
-      // the first one's (their results are never stored) and rank rows that are not there the line of zeros, so a load is
-      // an address and an instruction
 #pragma unroll
-      for (int g = 0; g < XBLK; ++g)
-        __builtin_amdgcn_global_load_lds(GLOBAL_PTR(xp[g] + off), LDS_PTR(sbase + x_off + g * 1024), 16, 0, 0);
+    for (int g = 0; g < XG; ++g) x[g] = load16(xp[g] + off);
 #pragma unroll
-      for (int i = 0; i < APW; ++i)
-        __builtin_amdgcn_global_load_lds(GLOBAL_PTR(ap[i] + (off & astep[i])), LDS_PTR(sbase + a_off + (wave * APW + i) * 1024), 16, 0, 0);
-      return;
-    }
-    const int k = off + gchunk * 8;                     // first K element of this lane's chunk
-    const bool kok = k < kend;
-#pragma unroll
-    for (int g = 0; g < XBLK; ++g) {
-      unsigned char *dst = sbase + x_off + g * 1024;
-      load_or_dummy(xok[g] && kok, xp[g] + kbeg + step * KC, dst);
-      if (!kok) lds_write16(lds_offset(dst) + lane * 16, zero4);
-    }
-#pragma unroll
-    for (int i = 0; i < APW; ++i) {
-      unsigned char *dst = sbase + a_off + (wave * APW + i) * 1024;
-      load_or_dummy(aok[i] && kok, ap[i] + kbeg + step * KC, dst);
-      if (!(aok[i] && kok)) lds_write16(lds_offset(dst) + lane * 16, zero4);
-    }
+    for (int i = 0; i < APW; ++i) a[i] = load16(ap[i] + (off & astep[i]));
+    requested();
   };
-  // where the MFMA operand (row R of a region, K block ks) of this lane sits inside a stage
-  auto frag_off = [&](int R, int ks) -> uint32_t {
-    return (uint32_t)R * 128u + (uint32_t)(((ks * 4 + kg) ^ (R & 7)) * 16);
-  };
+  // Row R of a stage (x rows of the four waves, then A) stands at R * 128, its chunk c at chunk c ^ (R & 7): 8 lanes write one
+  // row, and the 16 rows of an MFMA operand spread over the banks.
+  unsigned char *const wx = lds + (wrow0 + grow) * 128 + ((gcol ^ grow) << 4);
+  unsigned char *const wa = lds + (64 * MBW + wave * APW % AG * 8 + grow) * 128 + ((gcol ^ grow) << 4);
+  const unsigned char *rxp[KS], *rap[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    rxp[ks] = lds + (wrow0 + lrow) * 128 + (((ks * 4 + kg) ^ (lrow & 7)) << 4);
+    rap[ks] = lds + (64 * MBW + lrow) * 128 + (((ks * 4 + kg) ^ (lrow & 7)) << 4);
+  }
 
   f32x4 acc[MBW][NB];
 #pragma unroll
@@ -465,65 +379,114 @@ __global__ __launch_bounds__(256) void shrink_gemm_kernel(const int32_t *tiles_b
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  issue(0);
-  if (n_steps > 1) issue(1);
-  for (int step = 0; step < n_steps; ++step) {
-    // wait for this step's loads (the next step's may stay in flight), then meet the other waves:
-    // after the barrier the stage is complete for everybody and the stage consumed in the previous
-    // iteration is free to be refilled
-    if (step + 1 < n_steps) wait_vmcnt<LOADS_PER_STAGE>(); else wait_vmcnt<0>();
+  auto put = [&](int stage, const u32x4 (&x)[XG], const u32x4 (&a)[APW]) {
+#pragma unroll
+    for (int g = 0; g < XG; ++g) *reinterpret_cast<u32x4 *>(wx + stage + g * 1024) = x[g];
+#pragma unroll
+    for (int i = 0; i < APW; ++i) *reinterpret_cast<u32x4 *>(wa + stage + i * 1024) = a[i];
+    requested();
+  };
+  auto multiply = [&](int stage) {
+    // behind this barrier the stage is complete, and everybody has read the other one
     wait_lgkmcnt0();
     __builtin_amdgcn_s_barrier();
-    if (step + 2 < n_steps) issue(step + 2);
-    const int stage = step % STAGES;
-    if (wave_active) {
-      // both halves' operands are requested before the first half is used
-      u32x4 xfs[KS][MBW], bfs[KS][NB];
+    requested();
+    u32x4 xf[KS][MBW], bf[KS][NB];
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
+    for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-        for (int mb = 0; mb < MBW; ++mb)
-          xfs[ks][mb] = lds_read16(ring + stage * STAGE_BYTES + x_off + frag_off(mb * 16 + lrow, ks));
+      for (int mb = 0; mb < MBW; ++mb) xf[ks][mb] = *reinterpret_cast<const u32x4 *>(rxp[ks] + stage + mb * 2048);
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) bf[ks][nb] = *reinterpret_cast<const u32x4 *>(rap[ks] + stage + nb * 2048);
+    }
+    if (MBW * NB <= 8) requested();   // (all operands of a step requested together)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+        for (int mb = 0; mb < MBW; ++mb) acc[mb][nb] = Tr::mfma(as<vec8>(bf[ks][nb]), as<vec8>(xf[ks][mb]), acc[mb][nb]);
+    requested();
+  };
+  // (the loop's requests, and those in front of it, under no condition: the compiler has to know how many are outstanding
+  // where it waits)
+  int step = 0;
+  if (n_steps >= 2 * GEMM_AHEAD) {
+#pragma unroll
+    for (int i = 0; i < GEMM_AHEAD; ++i) request(i, rx[i], ra[i]);
+    do {
+#pragma unroll
+      for (int i = 0; i < GEMM_AHEAD; ++i) {
+        put(((step + i) & 1) * STAGE, rx[i], ra[i]);
+        request(step + i + GEMM_AHEAD, rx[i], ra[i]);
+        multiply(((step + i) & 1) * STAGE);
+      }
+      step += GEMM_AHEAD;
+    } while (step + 2 * GEMM_AHEAD <= n_steps);
+  } else {
+#pragma unroll
+    for (int i = 0; i < GEMM_AHEAD; ++i)
+      if (i < n_steps) request(i, rx[i], ra[i]);
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * GEMM_AHEAD - 1; ++i)
+    if (step + i < n_steps) {
+      put(((step + i) & 1) * STAGE, rx[i % GEMM_AHEAD], ra[i % GEMM_AHEAD]);
+      if (i < GEMM_AHEAD && step + i + GEMM_AHEAD < n_steps) request(step + i + GEMM_AHEAD, rx[i % GEMM_AHEAD], ra[i % GEMM_AHEAD]);
+      multiply(((step + i) & 1) * STAGE);
+    }
+  const int off = kbeg + n_steps * KC;
+  if (off < kend) {   // the end of a K that is not a multiple of 64: chunks past it read zeros
+    const bool kok = off + gcol * 8 < kend;
+#pragma unroll
+    for (int g = 0; g < XG; ++g) rx[0][g] = load16(as_global(kok ? xp[g] + off : zeros));
+#pragma unroll
+    for (int i = 0; i < APW; ++i) ra[0][i] = load16(as_global(kok && astep[i] ? ap[i] + off : zeros));
+    put((n_steps & 1) * STAGE, rx[0], ra[0]);
+    multiply((n_steps & 1) * STAGE);
+  }
+  // A lane has four consecutive rank columns of token lrow in every block: 16-byte stores from where they are.  One chunk:
+  // rounded to T.  Several: this chunk's fp32 partial, which a later launch on the stream (shrink_reduce_kernel, or the expand for
+  // small batches) sums in index order and rounds once.
+#pragma unroll
+  for (int mb = 0; mb < MBW; ++mb) {
+    const int row = wrow0 + mb * 16 + lrow;
+    if (row < cnt) {
+      if (p.ksplit == 1) {
+        const int t = p.out_by_token ? perm[pos0 + row] : 0;
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb)
-          bfs[ks][nb] = lds_read16(ring + stage * STAGE_BYTES + a_off + frag_off(nb * 16 + lrow, ks));
-      }
+          if (nb * 16 + kg * 4 < p.rp) store_v4<T>(p, pos0 + row, t, r, nb * 4 + kg, acc[mb][nb]);
+        // columns past the tile's own rank class hold zeros, where the batch has wider ones
+        for (int c4 = NB * 4 + kg; 4 * c4 < p.rp; c4 += 4) store_v4<T>(p, pos0 + row, t, r, c4, f32x4{0.f, 0.f, 0.f, 0.f});
+      } else {
+        float *const part = as_global(p.partial) + ((int64_t)s * p.T + pos0 + row) * p.rp + kg * 4;
 #pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 1 < KS) wait_lgkmcnt<MBW + NB>(); else wait_lgkmcnt<0>();
-        u32x4 (&xf)[MBW] = xfs[ks];
-        u32x4 (&bf)[NB] = bfs[ks];
-#pragma unroll
-        for (int mb = 0; mb < MBW; ++mb) pin(xf[mb]);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) pin(bf[nb]);
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb) {
-          if (nb * 16 < r) {
-#pragma unroll
-            for (int mb = 0; mb < MBW; ++mb)
-              acc[mb][nb] = Tr::mfma(as<vec8>(xf[mb]), as<vec8>(bf[nb]), acc[mb][nb]);
-          }
-        }
+        for (int nb = 0; nb < NB; ++nb)
+          if (nb * 16 < p.rp) *reinterpret_cast<f32x4 *>(part + nb * 16) = acc[mb][nb];   // (rp: a multiple of 16)
       }
     }
   }
-  wait_lgkmcnt0();
-  __syncthreads();   // everybody is done reading the ring: reuse it for the result tile
+}
 
-  float *otile = reinterpret_cast<float *>(s_raw);
-#pragma unroll
-  for (int mb = 0; mb < MBW; ++mb)
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = wrow0 + mb * 16 + kg * 4 + i;
-        const int col = nb * 16 + lrow;
-        otile[row * (NB * 16) + col] = acc[mb][nb][i];
-      }
-  __syncthreads();
-  shrink_epilogue<T>(p, otile, NB * 16, s, pos0, cnt, r, perm);
+template <typename T, int NB, int MBW>
+__global__ __launch_bounds__(256, MBW == 2 && NB <= 4 ? 2 : 1) void shrink_gemm_kernel(const int32_t *tiles_base, int h_flags, ShrinkArgs args_in) {
+  // grid (K chunks, targets, tiles).  The workgroup id mod 8 selects the XCD, so
+  // with the K chunk as the fast index the tiles of an adapter that share a K chunk of A, and the
+  // targets that share a K chunk of x, meet in one L2.
+  const int s = (int)blockIdx.x, z_idx = (int)blockIdx.y, tile_idx = (int)blockIdx.z;
+  const ShrinkArgs p = select_target(args_in, z_idx);
+  __shared__ __align__(16) unsigned char lds[2 * gemm_stage_bytes(NB, MBW)];
+
+  const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
+  int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  if ((h_flags & SHRINK_COMPENSATE) && z_idx == 1) merged_tile(p.plan, tile_idx, 64 * MBW, r, pos0, cnt, astart);
+  if (cnt <= 0) return;   // records past the last tile are zero
+  // (a narrow adapter among wide ones takes the loads and products of its own rank)
+  if (NB > 1 && r <= 16) shrink_gemm_tile<T, 1, MBW>(p, s, r, pos0, cnt, astart, lds);
+  else if (NB > 2 && r <= 32) shrink_gemm_tile<T, 2, MBW>(p, s, r, pos0, cnt, astart, lds);
+  else if (NB > 4 && r <= 64) shrink_gemm_tile<T, 4, MBW>(p, s, r, pos0, cnt, astart, lds);
+  else shrink_gemm_tile<T, NB, MBW>(p, s, r, pos0, cnt, astart, lds);
 }
 
 inline int head_flags(const ShrinkArgs &a) { return a.reduce_here | (a.compensate ? SHRINK_COMPENSATE : 0); }
@@ -531,12 +494,12 @@ inline int head_flags(const ShrinkArgs &a) { return a.reduce_here | (a.compensat
 template <typename T, int MBW>
 int launch_gemm_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
   switch (nb) {
-    case 1: hipLaunchKernelGGL((shrink_gemm_kernel<T, 1, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
-    case 2: hipLaunchKernelGGL((shrink_gemm_kernel<T, 2, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
-    case 4: hipLaunchKernelGGL((shrink_gemm_kernel<T, 4, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
+    case 1: hipLaunchKernelGGL((shrink_gemm_kernel<T, 1, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
+    case 2: hipLaunchKernelGGL((shrink_gemm_kernel<T, 2, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
+    case 4: hipLaunchKernelGGL((shrink_gemm_kernel<T, 4, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
     case 8:
       if constexpr (MBW <= 2) {
-        hipLaunchKernelGGL((shrink_gemm_kernel<T, 8, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a);
+        hipLaunchKernelGGL((shrink_gemm_kernel<T, 8, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a);
         break;
       }
       return fail(MLORA_ERR_NO_KERNEL, "shrink: rank > 64 has no 256-token tile");
@@ -592,6 +555,10 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   if (a.reduce_here) grid_tiles = (grid_tiles + 7) / 8 * 8;   // ids are dealt to the 8 XCDs tile by tile
   if (grid_tiles * a.ksplit * a.n_targets > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");
   dim3 grid((unsigned)(grid_tiles * a.ksplit * a.n_targets));
+  if (bm >= 128) {
+    if (grid_tiles > 65535) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");   // (4M tokens of 8192 adapters have 40960)
+    grid = dim3((unsigned)a.ksplit, (unsigned)a.n_targets, (unsigned)grid_tiles);
+  }
   if (a.reduce_here)
     grid = dim3((unsigned)(8 * a.ksplit), (unsigned)a.n_targets, (unsigned)(grid_tiles / 8));   // at most 4096 tokens (csrc/api.hip)
   return dt == MLORA_F16 ? launch_shrink_t<_Float16>(st, a, bm, nb, grid)
