@@ -7,6 +7,7 @@
 #include <cstring>
 
 #include "mlora_internal.h"
+#include "one_call_tiles.h"
 
 namespace mlora {
 
@@ -135,6 +136,7 @@ void set_reduce_here(ShrinkArgs &a, const mlora_plan *plan, const PlanLayout &L,
   a.n_tiles = (int)tiles_upper(plan->T, plan->n_adapters, plan->bm_shrink);
   a.arrive = reinterpret_cast<unsigned long long *>(static_cast<int32_t *>(plan->dev) + L.off_arrive);
   a.compensate = 0;
+  a.whole = 0;
 }
 
 // Whether a two-launch call leaves the sum of the split-K chunks to its expand, as its flags allow.  With 16-token expand tiles
@@ -336,9 +338,10 @@ int mlora_ids_from_requests(void *stream, int64_t *ids_out, const int32_t *b_sta
                                   max_rows);
 }
 
-int mlora_shrink(void *stream, const mlora_plan *plan, void *scratch, size_t scratch_nbytes, const void *x, int64_t T,
-                 int64_t h_in, int64_t max_rank, const mlora_pool *pool, int32_t slot, int32_t ksplit, void *out,
-                 int64_t out_stride, int32_t mode, int32_t width, int32_t flags, mlora_dtype dtype) {
+static int shrink_call(void *stream, const mlora_plan *plan, void *scratch, size_t scratch_nbytes, const void *x, int64_t T,
+                       int64_t h_in, int64_t max_rank, const mlora_pool *pool, int32_t slot, int32_t ksplit, void *out,
+                       int64_t out_stride, int32_t mode, int32_t width, int32_t flags, int whole,
+                       mlora_dtype dtype) {
   if (int rc = check_dtype(dtype, h_in, max_rank)) return rc;
   if (int rc = check_dims(T, h_in, max_rank, h_in, max_rank, dtype)) return rc;
   if (int rc = check_plan(plan, T, "shrink")) return rc;
@@ -393,11 +396,19 @@ int mlora_shrink(void *stream, const mlora_plan *plan, void *scratch, size_t scr
     a.ncols = (int)rp;
   }
   set_reduce_here(a, plan, L, max_rank, flags);
+  a.whole = whole;
   if (int rc = launch_shrink((hipStream_t)stream, a, plan->bm_shrink, (int)max_rank,
                              tiles_upper(T, plan->n_adapters, plan->bm_shrink), dtype))
     return rc;
   if (ksplit > 1 && !a.partial_only && !a.reduce_here) return launch_shrink_reduce((hipStream_t)stream, a, dtype);
   return MLORA_OK;
+}
+
+int mlora_shrink(void *stream, const mlora_plan *plan, void *scratch, size_t scratch_nbytes, const void *x, int64_t T,
+                 int64_t h_in, int64_t max_rank, const mlora_pool *pool, int32_t slot, int32_t ksplit, void *out,
+                 int64_t out_stride, int32_t mode, int32_t width, int32_t flags, mlora_dtype dtype) {
+  return shrink_call(stream, plan, scratch, scratch_nbytes, x, T, h_in, max_rank, pool, slot, ksplit, out, out_stride, mode, width,
+                     flags, 0, dtype);
 }
 
 int mlora_expand(void *stream, const mlora_plan *plan, void *y, int64_t T, int64_t h_out, const void *scratch,
@@ -727,12 +738,14 @@ static int one_call(void *stream, void *y, const void *x, const mlora_pool *pool
   mlora_plan built;
   const mlora_plan *plan = given;
   int ksplit;
+  const int tile = expand ? 0 : one_call_tile(T, pool->n_adapters, narrow, wide);
   if (given) {
     if (int rc = check_plan(given, T, who)) return rc;
     if (int rc = check_plan_pool(given, pool, who)) return rc;
     ksplit = tile_ksplit_for(T, narrow, wide, pool->n_adapters, given->bm_shrink);
   } else {
-    const mlora_tile_config cfg = tile_lookup(T, narrow, wide, pool->n_adapters);
+    mlora_tile_config cfg = tile_lookup(T, narrow, wide, pool->n_adapters);
+    if (tile) cfg.bm_shrink = tile;
     built.bytes = mlora_plan_bytes(T, pool->n_adapters);
     built.dev = ws.take(built.bytes);
     if (!built.dev) return fail(MLORA_ERR_WORKSPACE, "%s: workspace too small (needs %zu bytes)", who,
@@ -748,13 +761,15 @@ static int one_call(void *stream, void *y, const void *x, const mlora_pool *pool
     return mlora_expand(stream, plan, y, T, h_out, nullptr, x, narrow_stride, narrow, pool, (int32_t)qkvo, scales, 1,
                         0, dtype);
   }
+  const int whole = plan->bm_shrink >= tile ? tile : 0;   // a given plan of smaller tiles keeps them
+  if (whole) ksplit = 1;
   const size_t sbytes = scratch_bytes(T, narrow, ksplit);
   void *scratch = ws.take(sbytes);
   if (!scratch) return fail(MLORA_ERR_WORKSPACE, "%s: workspace too small (needs %zu bytes)", who,
                             mlora_workspace_bytes(T, pool->n_adapters, narrow));
   if (narrow_stride == 0) narrow_stride = h_out;
-  return mlora_shrink(stream, plan, scratch, sbytes, x, T, h_in, narrow, pool, (int32_t)qkvo, ksplit, y,
-                      narrow_stride, shrink_mode, shrink_width, 0, dtype);
+  return shrink_call(stream, plan, scratch, sbytes, x, T, h_in, narrow, pool, (int32_t)qkvo, ksplit, y,
+                     narrow_stride, shrink_mode, shrink_width, 0, whole, dtype);
 }
 
 int mlora_dispatch_bgmv(void *stream, void *y, const void *x, const mlora_pool *pool, const int64_t *indicies,

@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "mlora.h"
+#include "one_call_tiles.h"
 
 namespace py = pybind11;
 
@@ -251,6 +252,7 @@ Entry *plan_for(const Key &key, hipStream_t stream, std::initializer_list<at::Te
   e->capture = capture_id(stream);
   mlora_tile_config cfg;
   check_rc(mlora_tile_lookup(T, narrow, wide, pool.n_adapters, &cfg));
+  if (const int tile = mlora::one_call_tile(T, pool.n_adapters, narrow, wide)) cfg.bm_shrink = tile;
   e->ids = make_ids();
   e->plan_buf = device_bytes(mlora_plan_bytes(T, pool.n_adapters), like);
   e->plan.dev = e->plan_buf.data_ptr();

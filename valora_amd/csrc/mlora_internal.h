@@ -117,6 +117,7 @@ struct ShrinkArgs {
   int prp;                    // row stride of the partials in that mode: whole 128-byte lines per row
   int n_tiles;                // upper bound of the tile count
   unsigned long long *arrive; // [tiles][MLORA_MAX_TARGETS] arrival words, zero between launches
+  int whole;                  // 32 or 64: all of K in one workgroup of so many tokens (no taller than the plan's tiles), else 0
   int compensate;             // "target" 1 is the plan's merged adapter over all positions (host side: the kernels get a
                               // flag in their leading arguments, csrc/shrink.hip)
 };

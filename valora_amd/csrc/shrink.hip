@@ -283,6 +283,44 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
     if (on[it]) store_v4<T>(p, pos0 + row[it], tok[it], r, c4[it], v[it]);
 }
 
+// All of K in one workgroup of eight waves, 32 or 64 tokens: no partials, no second launch (or wait for the other chunks).  The
+// tile list may be one of taller tiles, whose pieces of 16 * MB tokens the workgroups take.  csrc/one_call_tiles.h has the rule.
+// Bound by what a compute unit takes in and by HBM: 7000 tokens over 32 adapters, 4096 wide, rank 32 read 57 MB in 17.4 us (3.3
+// TB/s).  The shrink alone, cold x, 128-token tiles in four chunks and the launch that sums them / this: rank 32 22.9 / 17.4 us,
+// rank 16 17.1 / 14.4; four waves instead of eight with the same 32 tokens 19.6 / 16.4 (6749 tokens, rank 32).  Four K steps in
+// flight a wave instead of two gain nothing at 4096 and lose where they leave a remainder (7000 tokens, 3072 wide, rank 8
+// 10.8 / 12.1).
+constexpr int WHOLE_WAVES = 8;
+constexpr int WHOLE_RUN = 4;   // consecutive pieces that run on one XCD
+constexpr int whole_lds_floats(int nblk) {
+  return nblk * WHOLE_WAVES * 256 * 4 > WHOLE_WAVES * SHRINK_STAGE_WAVE ? nblk * WHOLE_WAVES * 256 : WHOLE_WAVES * SHRINK_STAGE_WAVE / 4;
+}
+template <typename T, int MB, int NB>
+__global__ __launch_bounds__(512, 2) void shrink_whole_kernel(const int32_t *tiles_base, int h_n_pieces, int h_pieces, ShrinkArgs p) {
+  // The workgroup id mod 8 selects the XCD: a run of WHOLE_RUN pieces, most of them one adapter's, meets there.
+  constexpr int H = 16 * MB;
+  const int id = (int)blockIdx.x;   // (one target)
+  const int piece = (id / (8 * WHOLE_RUN)) * (8 * WHOLE_RUN) + (id & 7) * WHOLE_RUN + (id >> 3) % WHOLE_RUN;
+  if (piece >= h_n_pieces) return;
+  const int tile_idx = piece >> h_pieces, from = (piece - (tile_idx << h_pieces)) * H;   // 1 << h_pieces pieces a tile
+  const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
+  constexpr int NBLK = MB * NB, QUARTER = NB * 4;        // groups of four columns per row, a power of two
+  __shared__ __align__(16) float s_tile[whole_lds_floats(NBLK)];
+  int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  pos0 += from;
+  cnt = min(cnt - from, H);
+  if (cnt <= 0) return;   // records past the last tile are zero
+  const int32_t *__restrict__ perm = p.plan + p.off_perm;
+  shrink_tile_to_lds<T, MB, NB, MB + NB <= 5 ? 2 : 1, WHOLE_WAVES>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, 0, p.h_in, s_tile);
+  const int quarter = p.rp >> 2;
+#pragma unroll 1
+  for (int e = threadIdx.x; e < cnt * QUARTER; e += 64 * WHOLE_WAVES) {
+    const int row = e / QUARTER, c4 = e & (QUARTER - 1);
+    if (c4 < quarter)
+      store_v4<T>(p, pos0 + row, p.out_by_token ? perm[pos0 + row] : 0, r, c4, shrink_tile_sum<NB, WHOLE_WAVES>(s_tile, NBLK, row, c4));
+  }
+}
+
 // What a rank row that is not there reads, K step after K step (one 128-byte line).
 __device__ const __align__(128) uint16_t g_zero_line[64] = {};
 
@@ -520,6 +558,25 @@ int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
   return check_launch("shrink_kernel");
 }
 
+template <typename T, int MB>
+int launch_whole(hipStream_t st, const ShrinkArgs &a, int bm, int nb, int64_t tiles) {
+  int shift = 0;
+  while ((16 * MB) << shift < bm) ++shift;
+  const int64_t pieces = tiles << shift, blocks = align_up(pieces, 8 * WHOLE_RUN);
+  if (blocks > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");
+  const dim3 grid((unsigned)blocks);
+#define MLORA_WHOLE(NB)                                                                                                        \
+  hipLaunchKernelGGL((shrink_whole_kernel<T, MB, NB>), grid, dim3(64 * WHOLE_WAVES), 0, st, a.plan + a.off_tiles,             \
+                     (int)pieces, shift, a)
+  if (nb == 1) MLORA_WHOLE(1);
+  else if constexpr (MB == 2) {
+    if (nb == 2) MLORA_WHOLE(2);
+    else MLORA_WHOLE(4);
+  }
+#undef MLORA_WHOLE
+  return check_launch("shrink_whole_kernel");
+}
+
 template <typename T>
 int launch_shrink_t(hipStream_t st, const ShrinkArgs &a, int bm, int nb, dim3 grid) {
   switch (bm) {
@@ -552,6 +609,11 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   nb = nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : 8;
   if (nb == 8 && (bm == 64 || bm == 256)) return fail(MLORA_ERR_NO_KERNEL, "shrink: rank > 64 needs tile height 16, 32 or 128");
   if (grid_tiles <= 0) return MLORA_OK;
+  if (a.whole) {
+    if (a.ksplit != 1 || bm < a.whole || nb > (a.whole == 64 ? 1 : 4)) return fail(MLORA_ERR_NO_KERNEL, "shrink: no whole-K kernel here");
+    if (a.whole == 64) return dt == MLORA_F16 ? launch_whole<_Float16, 4>(st, a, bm, nb, grid_tiles) : launch_whole<__bf16, 4>(st, a, bm, nb, grid_tiles);
+    return dt == MLORA_F16 ? launch_whole<_Float16, 2>(st, a, bm, nb, grid_tiles) : launch_whole<__bf16, 2>(st, a, bm, nb, grid_tiles);
+  }
   if (a.reduce_here) grid_tiles = (grid_tiles + 7) / 8 * 8;   // ids are dealt to the 8 XCDs tile by tile
   if (grid_tiles * a.ksplit * a.n_targets > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");
   dim3 grid((unsigned)(grid_tiles * a.ksplit * a.n_targets));

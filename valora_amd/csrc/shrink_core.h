@@ -31,17 +31,23 @@ constexpr int shrink_lds_floats(int nblk) {
 
 // four consecutive columns (4*c4 ..) of one token row of the tile shrink_tile_to_lds left in `lds`: the sum of the
 // four waves' shares, always in this order
-template <int NB>
+template <int NB, int WAVES = 4>
 __device__ __forceinline__ f32x4 shrink_tile_sum(const float *lds, int nblk, int row, int c4) {
   const int b = (row >> 4) * NB + (c4 >> 2);
   const float *src = lds + b * 256 + (row & 3) * 64 + ((row >> 2) & 3) * 16 + (c4 & 3) * 4;
   const f32x4 w0 = *reinterpret_cast<const f32x4 *>(src), w1 = *reinterpret_cast<const f32x4 *>(src + nblk * 256);
   const f32x4 w2 = *reinterpret_cast<const f32x4 *>(src + nblk * 512), w3 = *reinterpret_cast<const f32x4 *>(src + nblk * 768);
+  if constexpr (WAVES == 8) {
+    const float *const hi = src + nblk * 1024;
+    const f32x4 w4 = *reinterpret_cast<const f32x4 *>(hi), w5 = *reinterpret_cast<const f32x4 *>(hi + nblk * 256);
+    const f32x4 w6 = *reinterpret_cast<const f32x4 *>(hi + nblk * 512), w7 = *reinterpret_cast<const f32x4 *>(hi + nblk * 768);
+    return ((w0 + w4) + (w2 + w6)) + ((w1 + w5) + (w3 + w7));
+  }
   return (w0 + w2) + (w1 + w3);
 }
 
 // What a lane without anything to fetch reads, as far as the steps of a batch reach.
-__device__ const __align__(128) uint16_t g_shrink_zeros[3 * 4 * SHRINK_KSTEP + SHRINK_KSTEP] = {};
+__device__ const __align__(128) uint16_t g_shrink_zeros[3 * 8 * SHRINK_KSTEP + SHRINK_KSTEP] = {};
 constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1; }
 // Leaves the four waves' shares of the fp32 result of K range [kbeg, kend) in `lds` (shrink_lds_floats(MB * NB) floats,
 // 16-byte aligned), for shrink_tile_sum to add up (rows = tokens of the tile, columns = rank); every thread of the
@@ -51,7 +57,7 @@ constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1;
 // address, not a mask: a mask, four zeroed registers and a branch around each of a batch's 16 loads took 1400 cycles to issue.
 // One target, cold layers, masked / like this: 1 token of rank 16 4.9 / 4.0 us, 256 over 64 adapters 6.7 / 5.7, 200 over 16 of rank 32
 // 7.6 / 6.5, 77 over ranks 8-64 8.8 / 7.9, 256 over 64 of rank 64 11.6 / 10.9, 512 over 128 of rank 128 29.5 / 28.4.
-template <typename T, int MB, int NB, int U = shrink_steps(MB + NB)>
+template <typename T, int MB, int NB, int U = shrink_steps(MB + NB), int WAVES = 4>
 __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ x, int h_in, const PoolDev &pool,
                                                    int slot, const int32_t *__restrict__ perm, int r, int pos0,
                                                    int cnt, int astart, int kbeg, int kend,
@@ -163,24 +169,24 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
   // registers into the matrix core.
   // Whole batches: a load is an instruction, the steps of a batch are offsets in it.
   int kb0 = kbeg + wave * SHRINK_KSTEP;
-  for (; plain && kb0 + (4 * U - 3) * SHRINK_KSTEP <= kend; kb0 += 4 * SHRINK_KSTEP * U) {
+  for (; plain && kb0 + (WAVES * (U - 1) + 1) * SHRINK_KSTEP <= kend; kb0 += WAVES * SHRINK_KSTEP * U) {
 #pragma unroll
     for (int b = 0; b < BLKS; ++b)
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const uint16_t *const src = rp[b][u] + (MANY && b >= MB ? kb0 & step[b < MB ? 0 : b - MB][u] : kb0);
 #pragma unroll
-        for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16(src + uu * 4 * SHRINK_KSTEP);
+        for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16(src + uu * WAVES * SHRINK_KSTEP);
       }
     requested();
     use();
   }
   // what is left of the chunk, less than a batch (or all of it, where a rank row lies outside the index or the pool): steps and
   // lanes past its end read zeros, and so do rows that are not there
-  for (; kb0 < kend; kb0 += 4 * SHRINK_KSTEP * U) {
+  for (; kb0 < kend; kb0 += WAVES * SHRINK_KSTEP * U) {
 #pragma unroll
     for (int uu = 0; uu < U; ++uu) {
-      const int k = kb0 + uu * 4 * SHRINK_KSTEP;
+      const int k = kb0 + uu * WAVES * SHRINK_KSTEP;
       const bool kok = k + gcol * 8 < kend;
 #pragma unroll
       for (int b = 0; b < BLKS; ++b)
