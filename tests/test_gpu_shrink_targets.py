@@ -1,0 +1,53 @@
+"""Two or three targets of 128-token shrink tiles in one workgroup: the bits of separate calls, at the edges of tiles, K steps
+and chunks, with adapters of several rank classes and rank rows that are not in the pool, and on both sides of the rule (128 or 160
+workgroups)."""
+import pytest
+import torch
+
+from oracle import lora_oracle as O
+from valora_amd import workloads as W
+from valora_amd.plan import LoraPlan
+from tests._util import assert_parity
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("ranks", [(8, 16), (32, 8, 16, 24), (64, 8, 40, 16, 32, 56)])
+@pytest.mark.parametrize("h_in,ksplit", [(1024, 16), (1032, 15), (2048, 32), (4104, 16), (136, 2)])
+def test_bits_of_separate_calls(dev, h_in, ksplit, ranks):
+    g = torch.Generator().manual_seed(h_in + len(ranks))
+    dtype = torch.bfloat16 if len(ranks) == 4 else torch.float16
+    A, R, h_out = len(ranks), max(ranks), 72
+    for tiles in ((9, 5) if ksplit > 2 else (90, 65, 30)):   # (tiles + tails) * chunks on either side of the rule
+        lens = torch.full((A,), tiles * 128 // A)
+        lens[0], lens[-1] = lens[0] // 2 + 1, lens[-1] + 130
+        ids = torch.repeat_interleave(torch.arange(A), lens)
+        ids = ids[torch.randperm(ids.numel(), generator=g)]
+        T = ids.numel()
+        pool = W.make_pool(list(ranks), h_in, h_out, dtype, g, True, std=0.05, heads=1, extra_rows=1)
+        x = torch.randn(T, h_in, generator=g).to(dtype)
+        y0 = [torch.randn(T, h_out, generator=g).to(dtype) for _ in range(3)]
+        # the last pool row stands for "no row": zeros for the oracle, out of the pool's bounds for the op
+        spare = pool.key_buffer.shape[0] - 1
+        pool.key_buffer[-1], pool.value_buffer[-1] = 0, 0
+        pool.a_loc[torch.where(pool.a_loc == spare)[0]] = next(r for r in range(spare) if r not in set(pool.a_loc.tolist()))
+        seen = pool.a_loc.clone()
+        for slot in range(3):
+            at = int(pool.a_start[-1]) + ranks[-1] * slot + 3 * slot + 1
+            seen[at], pool.a_loc[at] = spare, (-1, spare + 1, 1 << 40)[slot]
+        pd, xd = pool.to(dev), x.to(dev)
+        idx = (pd.a_start, pd.a_len, pd.a_loc)
+        plan = LoraPlan(ids.to(dev), pd.a_start, pd.a_len, R, hidden=h_in, bm_shrink=128, bm_expand=32, ksplit=ksplit,
+                        reduce_in_expand=False, one_launch=False)
+        alone = []
+        for z in range(3):
+            y = y0[z].to(dev)
+            plan.apply(y, xd, pd.key_buffer, pd.value_buffer, *idx, z, pd.a_scaling)
+            alone.append(y.cpu())
+            want = O.lora_op(y0[z], x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, seen, ids, z, pool.a_scaling)
+            assert_parity(alone[-1], want, f"{h_in} {ksplit} {ranks} target {z}")
+        for slots in ((0, 1, 2), (2, 0)):
+            ys = [y0[z].to(dev) for z in slots]
+            plan.apply_multi(ys, xd, pd.key_buffer, pd.value_buffer, *idx, list(slots), pd.a_scaling)
+            for z, y in zip(slots, ys):
+                assert torch.equal(y.cpu(), alone[z]), f"{h_in} {ksplit} {ranks} targets {slots}, {z}"

@@ -527,6 +527,166 @@ __global__ __launch_bounds__(256, MBW == 2 && NB <= 4 ? 2 : 1) void shrink_gemm_
   else shrink_gemm_tile<T, NB, MBW>(p, s, r, pos0, cnt, astart, lds);
 }
 
+// Two or three targets of a call in one workgroup of eight waves: x is requested, written to LDS and read from it once for all
+// of them.  Tile, K steps and order of the sums are shrink_gemm_kernel's (same bits); four pairs of waves split the tokens, the
+// waves of a pair the targets' rank columns.  One step is in flight, and a step's operands are read half by half: 121 registers
+// at three targets of rank 64, so that two workgroups share a compute unit (two steps in flight: 154 registers, one workgroup,
+// 5401 tokens over ranks 8-64 32.3 us against 29.3 now).
+// Bound by memory and by what is not yet or no more streaming: launch, look-ups, first step, partials (6.6 us of one target).
+// 4430 tokens of rank 64, 4096 wide, four chunks, per target / now: two targets 25.8 / 23.3 us, three 33.3 / 27.5; 5401 tokens
+// over ranks 8-64 25.4 / 23.6, 30.6 / 29.3.
+constexpr int TARGETS_ROWS = 128;                       // tokens
+constexpr int targets_half(int nt, int nb) { return (nt * nb + 1) / 2; }   // 16-column blocks of a wave
+constexpr int targets_stage_bytes(int nt, int nb) { return (TARGETS_ROWS + 32 * targets_half(nt, nb)) * GEMM_KC * 2; }
+
+// One tile and one K chunk, NB 16-row blocks of rank (of the tile's own adapter) for each of NT targets.
+template <typename T, int NT, int NB>
+__device__ __forceinline__ void shrink_targets_tile(const ShrinkArgs &p, int s, int r, int pos0, int cnt, int astart, unsigned char *lds) {
+  using Tr = Traits<T>;
+  using vec8 = typename Tr::vec8;
+  constexpr int KC = GEMM_KC, KS = KC / 32, C = NT * NB, HB = targets_half(NT, NB);
+  constexpr int XG = 2, AG = 2 * C, APW = (AG + 7) / 8; // 8-row groups of x and A a wave loads in a step; APW waves' worth of AG
+  constexpr int STAGE = targets_stage_bytes(NT, NB);
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lrow = lane & 15, kg = lane >> 4;           // MFMA operand roles
+  const int grow = lane >> 3, gcol = lane & 7;          // loader roles: row within an 8-row group, 16-byte chunk
+  const int trow0 = (wave >> 1) * 32, b0 = (wave & 1) * HB;   // products: the wave's first token row and column block
+  const int32_t *__restrict__ perm = as_global(p.plan) + p.off_perm;
+
+  const bool indexed = p.pool.a_loc_len > 0;
+  const int64_t *const a_loc = indexed ? as_global(p.pool.a_loc) : reinterpret_cast<const int64_t *>(perm);
+  int tok[XG], group[APW];
+  int64_t prow[APW];
+  bool ok[APW];
+#pragma unroll
+  for (int g = 0; g < XG; ++g) {
+    const int row = wave * 8 * XG + g * 8 + grow;
+    tok[g] = perm[pos0 + (row < cnt ? row : 0)];
+  }
+#pragma unroll
+  for (int i = 0; i < APW; ++i) {
+    group[i] = (wave * APW + i) % AG;                   // (what goes round is loaded and written twice)
+    const int z = group[i] / (2 * NB), j = group[i] % (2 * NB) * 8 + grow;
+    const int slot = z == 0 ? p.slots[0] : z == 1 ? p.slots[1] : p.slots[2];
+    const int64_t idx = (int64_t)astart + (int64_t)r * slot + j;
+    ok[i] = indexed && j < r && idx >= 0 && idx < p.pool.a_loc_len;
+    prow[i] = a_loc[ok[i] ? idx : 0];
+  }
+  const uint16_t *xp[XG], *ap[APW];
+  int astep[APW];                                       // all bits: the row moves on with K; none: it stays on its line
+  const uint16_t *const zeros = as_global(g_zero_line) + gcol * 8;
+#pragma unroll
+  for (int g = 0; g < XG; ++g) xp[g] = as_global(p.x) + (uint64_t)(uint32_t)tok[g] * (uint32_t)p.h_in + gcol * 8;
+#pragma unroll
+  for (int i = 0; i < APW; ++i) {
+    ok[i] = ok[i] && prow[i] >= 0 && prow[i] < p.pool.w_rows;
+    ap[i] = ok[i] ? as_global(p.pool.w) + (uint64_t)(uint32_t)prow[i] * (uint32_t)p.h_in + gcol * 8 : zeros;
+    astep[i] = ok[i] ? -1 : 0;
+  }
+
+  const int kbeg = s * p.kchunk;
+  const int kend = min(p.h_in, kbeg + p.kchunk);
+  const int n_steps = (kend - kbeg) / KC;               // whole ones
+  u32x4 rx[XG], ra[APW];
+  auto request = [&](int step) {
+    const int off = kbeg + step * KC;
+#pragma unroll
+    for (int g = 0; g < XG; ++g) rx[g] = load16(xp[g] + off);
+#pragma unroll
+    for (int i = 0; i < APW; ++i) ra[i] = load16(ap[i] + (off & astep[i]));
+    requested();
+  };
+  // rows and chunks of a stage as in shrink_gemm_tile: x, then A block by block
+  unsigned char *const wx = lds + (wave * 8 * XG + grow) * 128 + ((gcol ^ grow) << 4);
+  unsigned char *wa[APW];
+#pragma unroll
+  for (int i = 0; i < APW; ++i) wa[i] = lds + (TARGETS_ROWS + group[i] * 8 + grow) * 128 + ((gcol ^ grow) << 4);
+  const unsigned char *rxp[KS], *rap[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+    rxp[ks] = lds + (trow0 + lrow) * 128 + (((ks * 4 + kg) ^ (lrow & 7)) << 4);
+    rap[ks] = lds + (TARGETS_ROWS + b0 * 16 + lrow) * 128 + (((ks * 4 + kg) ^ (lrow & 7)) << 4);
+  }
+  f32x4 acc[2][HB];
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb)
+#pragma unroll
+    for (int b = 0; b < HB; ++b) acc[mb][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto put = [&](int stage) {
+#pragma unroll
+    for (int g = 0; g < XG; ++g) *reinterpret_cast<u32x4 *>(wx + stage + g * 1024) = rx[g];
+#pragma unroll
+    for (int i = 0; i < APW; ++i) *reinterpret_cast<u32x4 *>(wa[i] + stage) = ra[i];
+    requested();
+  };
+  auto multiply = [&](int stage) {
+    // behind this barrier the stage is complete, and everybody has read the other one
+    wait_lgkmcnt0();
+    __builtin_amdgcn_s_barrier();
+    requested();
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      u32x4 xf[2], bf[HB];
+#pragma unroll
+      for (int mb = 0; mb < 2; ++mb) xf[mb] = *reinterpret_cast<const u32x4 *>(rxp[ks] + stage + mb * 2048);
+#pragma unroll
+      for (int b = 0; b < HB; ++b) bf[b] = *reinterpret_cast<const u32x4 *>(rap[ks] + stage + b * 2048);
+#pragma unroll
+      for (int b = 0; b < HB; ++b)
+#pragma unroll
+        for (int mb = 0; mb < 2; ++mb) acc[mb][b] = Tr::mfma(as<vec8>(bf[b]), as<vec8>(xf[mb]), acc[mb][b]);
+      requested();
+    }
+  };
+  // (the loop's requests under no condition: the compiler has to know how many are outstanding where it waits)
+  if (n_steps > 0) {
+    int step = 0;
+    request(0);
+    for (; step + 1 < n_steps; ++step) {
+      put((step & 1) * STAGE);
+      request(step + 1);
+      multiply((step & 1) * STAGE);
+    }
+    put((step & 1) * STAGE);
+    multiply((step & 1) * STAGE);
+  }
+  const int off = kbeg + n_steps * KC;
+  if (off < kend) {   // the end of a K that is not a multiple of 64: chunks past it read zeros
+    const bool kok = off + gcol * 8 < kend;
+#pragma unroll
+    for (int g = 0; g < XG; ++g) rx[g] = load16(as_global(kok ? xp[g] + off : zeros));
+#pragma unroll
+    for (int i = 0; i < APW; ++i) ra[i] = load16(as_global(kok && astep[i] ? ap[i] + off : zeros));
+    put((n_steps & 1) * STAGE);
+    multiply((n_steps & 1) * STAGE);
+  }
+  // as in shrink_gemm_tile: this chunk's fp32 partials, of target (b0 + b) / NB
+#pragma unroll
+  for (int mb = 0; mb < 2; ++mb) {
+    const int row = trow0 + mb * 16 + lrow;
+    if (row < cnt) {
+      float *const part = as_global(p.partial) + ((int64_t)s * p.T + pos0 + row) * p.rp + kg * 4;
+#pragma unroll
+      for (int b = 0; b < HB; ++b) {
+        const int z = (b0 + b) / NB, nb = (b0 + b) % NB;
+        if (z < NT && nb * 16 < p.rp) *reinterpret_cast<f32x4 *>(part + z * p.partial_tstride + nb * 16) = acc[mb][b];
+      }
+    }
+  }
+}
+
+template <typename T, int NT, int NB>
+__global__ __launch_bounds__(512, 4) void shrink_targets_kernel(const int32_t *tiles_base, ShrinkArgs p) {
+  // grid (K chunks, tiles)
+  __shared__ __align__(16) unsigned char lds[2 * targets_stage_bytes(NT, NB)];
+  const int32_t *__restrict__ tile = tiles_base + (int64_t)blockIdx.y * TILE_WORDS;
+  const int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4], s = (int)blockIdx.x;
+  if (cnt <= 0) return;   // records past the last tile are zero
+  if (NB > 1 && r <= 16) shrink_targets_tile<T, NT, 1>(p, s, r, pos0, cnt, astart, lds);
+  else if (NB > 2 && r <= 32) shrink_targets_tile<T, NT, 2>(p, s, r, pos0, cnt, astart, lds);
+  else shrink_targets_tile<T, NT, NB>(p, s, r, pos0, cnt, astart, lds);
+}
+
 inline int head_flags(const ShrinkArgs &a) { return a.reduce_here | (a.compensate ? SHRINK_COMPENSATE : 0); }
 
 template <typename T, int MBW>
@@ -556,6 +716,24 @@ int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
     default: return fail(MLORA_ERR_NO_KERNEL, "shrink: no kernel for rank blocks=%d", nb);
   }
   return check_launch("shrink_kernel");
+}
+
+template <typename T>
+int launch_targets(hipStream_t st, const ShrinkArgs &a, int nb, int64_t tiles) {
+  const dim3 grid((unsigned)a.ksplit, (unsigned)tiles);
+#define MLORA_TARGETS(NT, NB) \
+  hipLaunchKernelGGL((shrink_targets_kernel<T, NT, NB>), grid, dim3(512), 0, st, a.plan + a.off_tiles, a)
+  if (a.n_targets == 2) {
+    if (nb == 1) MLORA_TARGETS(2, 1);
+    else if (nb == 2) MLORA_TARGETS(2, 2);
+    else MLORA_TARGETS(2, 4);
+  } else {
+    if (nb == 1) MLORA_TARGETS(3, 1);
+    else if (nb == 2) MLORA_TARGETS(3, 2);
+    else MLORA_TARGETS(3, 4);
+  }
+#undef MLORA_TARGETS
+  return check_launch("shrink_targets_kernel");
 }
 
 template <typename T, int MB>
@@ -620,6 +798,17 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   if (bm >= 128) {
     if (grid_tiles > 65535) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");   // (4M tokens of 8192 adapters have 40960)
     grid = dim3((unsigned)a.ksplit, (unsigned)a.n_targets, (unsigned)grid_tiles);
+    // Targets together, where the fewer workgroups still fill the device evenly (two a compute unit; an adapter's last tile is half
+    // empty in the mean, one of few tokens emptier).  The whole op with a 256-wide output, rank 64, per target / together: three
+    // targets, 4096 wide, 140 workgroups (4400 tokens of one adapter) 33.2 / 36.5 us, 204 (4400 over 32) 43.8 / 37.9, 264 (4400 over
+    // 64) 52.8 / 57.3, 452 (14000 over 8) 77.0 / 63.7; two 156 (4400 over 8) 35.3 / 31.1; 8192 wide, 592 (5400 over 64) 68.7 / 74.0;
+    // 2000 tokens over 32 34.9 / 39.3.  401 shapes of 1000 to 14000 tokens, 2048 to 8192 wide, that it takes: 0.90 in the mean,
+    // 1.03 at worst.
+    const int64_t adapters = grid_tiles - (a.T + 127) / 128, wgs = (a.T / 128 + adapters / 2) * a.ksplit;
+    const bool three = a.n_targets == 3;
+    const bool even = wgs >= (three ? 160 : 128) && !(three && wgs > 256 && wgs <= 320) && !(wgs > 512 && wgs <= 704) && a.T >= 64 * adapters;
+    if (even && bm == 128 && nb <= 4 && (three || a.n_targets == 2) && a.ksplit > 1 && !a.compensate)
+      return dt == MLORA_F16 ? launch_targets<_Float16>(st, a, nb, grid_tiles) : launch_targets<__bf16>(st, a, nb, grid_tiles);
   }
   if (a.reduce_here)
     grid = dim3((unsigned)(8 * a.ksplit), (unsigned)a.n_targets, (unsigned)(grid_tiles / 8));   // at most 4096 tokens (csrc/api.hip)
