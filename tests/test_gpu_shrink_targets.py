@@ -12,7 +12,7 @@ from tests._util import assert_parity
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ranks", [(8, 16), (32, 8, 16, 24), (64, 8, 40, 16, 32, 56)])
+@pytest.mark.parametrize("ranks", [(8, 16), (32, 8, 16, 24), (64, 8, 40, 16, 32, 56), (128, 8, 72, 16, 104, 56)])
 @pytest.mark.parametrize("h_in,ksplit", [(1024, 16), (1032, 15), (2048, 32), (4104, 16), (136, 2)])
 def test_bits_of_separate_calls(dev, h_in, ksplit, ranks):
     g = torch.Generator().manual_seed(h_in + len(ranks))

@@ -508,7 +508,7 @@ __device__ __forceinline__ void shrink_gemm_tile(const ShrinkArgs &p, int s, int
 }
 
 template <typename T, int NB, int MBW>
-__global__ __launch_bounds__(256, MBW == 2 && NB <= 4 ? 2 : 1) void shrink_gemm_kernel(const int32_t *tiles_base, int h_flags, ShrinkArgs args_in) {
+__global__ __launch_bounds__(256, MBW == 2 ? 2 : 1) void shrink_gemm_kernel(const int32_t *tiles_base, int h_flags, ShrinkArgs args_in) {
   // grid (K chunks, targets, tiles).  The workgroup id mod 8 selects the XCD, so
   // with the K chunk as the fast index the tiles of an adapter that share a K chunk of A, and the
   // targets that share a K chunk of x, meet in one L2.
@@ -523,18 +523,19 @@ __global__ __launch_bounds__(256, MBW == 2 && NB <= 4 ? 2 : 1) void shrink_gemm_
   // (a narrow adapter among wide ones takes the loads and products of its own rank)
   if (NB > 1 && r <= 16) shrink_gemm_tile<T, 1, MBW>(p, s, r, pos0, cnt, astart, lds);
   else if (NB > 2 && r <= 32) shrink_gemm_tile<T, 2, MBW>(p, s, r, pos0, cnt, astart, lds);
-  else if (NB > 4 && r <= 64) shrink_gemm_tile<T, 4, MBW>(p, s, r, pos0, cnt, astart, lds);
   else shrink_gemm_tile<T, NB, MBW>(p, s, r, pos0, cnt, astart, lds);
 }
 
-// Two or three targets of a call in one workgroup of eight waves: x is requested, written to LDS and read from it once for all
-// of them.  Tile, K steps and order of the sums are shrink_gemm_kernel's (same bits); four pairs of waves split the tokens, the
-// waves of a pair the targets' rank columns.  One step is in flight, and a step's operands are read half by half: 121 registers
-// at three targets of rank 64, so that two workgroups share a compute unit (two steps in flight: 154 registers, one workgroup,
-// 5401 tokens over ranks 8-64 32.3 us against 29.3 now).
+// The same tile in eight waves, for NT targets of a call together (x is requested, written to LDS and read from it once for all
+// of them), or for one of rank above 64.  Tile, K steps and order of the sums are shrink_gemm_kernel's (same bits); four pairs of
+// waves split the tokens, the waves of a pair the rank columns.  One step is in flight, and a step's operands are read half by
+// half, so that two workgroups share a compute unit up to 192 columns (two steps in flight at three targets of rank 64: 154
+// registers, one workgroup, 5401 tokens over ranks 8-64 32.3 us against 29.3 now).
 // Bound by memory and by what is not yet or no more streaming: launch, look-ups, first step, partials (6.6 us of one target).
-// 4430 tokens of rank 64, 4096 wide, four chunks, per target / now: two targets 25.8 / 23.3 us, three 33.3 / 27.5; 5401 tokens
-// over ranks 8-64 25.4 / 23.6, 30.6 / 29.3.
+// 4430 tokens of rank 64, 4096 wide, four chunks, per target / together: two targets 25.8 / 23.3 us, three 33.3 / 27.5; 5401 tokens
+// over ranks 8-64 25.4 / 23.6, 30.6 / 29.3.  One target of rank 128, four waves (280 registers, one workgroup a compute unit) /
+// eight, the whole op: 3000 tokens over 64 adapters, 5120 wide 47.8 / 43.0; 113 shapes 0.965 in the mean.  (Up to rank 64 one target is
+// better off with four waves of two 16-token blocks each: 0.98 to 1.05.)
 constexpr int TARGETS_ROWS = 128;                       // tokens
 constexpr int targets_half(int nt, int nb) { return (nt * nb + 1) / 2; }   // 16-column blocks of a wave
 constexpr int targets_stage_bytes(int nt, int nb) { return (TARGETS_ROWS + 32 * targets_half(nt, nb)) * GEMM_KC * 2; }
@@ -567,7 +568,7 @@ __device__ __forceinline__ void shrink_targets_tile(const ShrinkArgs &p, int s, 
   for (int i = 0; i < APW; ++i) {
     group[i] = (wave * APW + i) % AG;                   // (what goes round is loaded and written twice)
     const int z = group[i] / (2 * NB), j = group[i] % (2 * NB) * 8 + grow;
-    const int slot = z == 0 ? p.slots[0] : z == 1 ? p.slots[1] : p.slots[2];
+    const int slot = NT == 1 ? p.slot : z == 0 ? p.slots[0] : z == 1 ? p.slots[1] : p.slots[2];
     const int64_t idx = (int64_t)astart + (int64_t)r * slot + j;
     ok[i] = indexed && j < r && idx >= 0 && idx < p.pool.a_loc_len;
     prow[i] = a_loc[ok[i] ? idx : 0];
@@ -660,30 +661,49 @@ __device__ __forceinline__ void shrink_targets_tile(const ShrinkArgs &p, int s, 
     put((n_steps & 1) * STAGE);
     multiply((n_steps & 1) * STAGE);
   }
-  // as in shrink_gemm_tile: this chunk's fp32 partials, of target (b0 + b) / NB
+  // A lane has four consecutive rank columns of token lrow in every block: 16-byte stores from where they are.  One chunk:
+  // rounded to T.  Several: this chunk's fp32 partial, which a later launch on the stream (shrink_reduce_kernel, or the expand for
+  // small batches) sums in index order and rounds once.  Block b0 + b is target (b0 + b) / NB's.
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb) {
     const int row = trow0 + mb * 16 + lrow;
     if (row < cnt) {
-      float *const part = as_global(p.partial) + ((int64_t)s * p.T + pos0 + row) * p.rp + kg * 4;
+      if (NT == 1 && p.ksplit == 1) {                   // (targets go together only where K is split)
+        const int t = p.out_by_token ? perm[pos0 + row] : 0;
 #pragma unroll
-      for (int b = 0; b < HB; ++b) {
-        const int z = (b0 + b) / NB, nb = (b0 + b) % NB;
-        if (z < NT && nb * 16 < p.rp) *reinterpret_cast<f32x4 *>(part + z * p.partial_tstride + nb * 16) = acc[mb][b];
+        for (int b = 0; b < HB; ++b) {
+          const int c4 = (b0 + b) * 4 + kg;
+          if (b0 + b < NB && 4 * c4 < p.rp) store_v4<T>(p, pos0 + row, t, r, c4, acc[mb][b]);
+        }
+        // columns past the tile's own rank class hold zeros, where the batch has wider ones
+        if (b0 == 0)
+          for (int c4 = NB * 4 + kg; 4 * c4 < p.rp; c4 += 4) store_v4<T>(p, pos0 + row, t, r, c4, f32x4{0.f, 0.f, 0.f, 0.f});
+      } else {
+        float *const part = as_global(p.partial) + ((int64_t)s * p.T + pos0 + row) * p.rp + kg * 4;
+#pragma unroll
+        for (int b = 0; b < HB; ++b) {
+          const int z = (b0 + b) / NB, nb = (b0 + b) % NB;
+          if (z < NT && nb * 16 < p.rp) *reinterpret_cast<f32x4 *>(part + z * p.partial_tstride + nb * 16) = acc[mb][b];   // (rp: a multiple of 16)
+        }
       }
     }
   }
 }
 
 template <typename T, int NT, int NB>
-__global__ __launch_bounds__(512, 4) void shrink_targets_kernel(const int32_t *tiles_base, ShrinkArgs p) {
-  // grid (K chunks, tiles)
+__global__ __launch_bounds__(512, NT * NB <= 12 ? 4 : 2) void shrink_targets_kernel(const int32_t *tiles_base, int h_flags, ShrinkArgs args_in) {
+  // grid (K chunks, groups of NT targets, tiles)
+  const ShrinkArgs p = NT == 1 ? select_target(args_in, blockIdx.y) : args_in;
   __shared__ __align__(16) unsigned char lds[2 * targets_stage_bytes(NT, NB)];
-  const int32_t *__restrict__ tile = tiles_base + (int64_t)blockIdx.y * TILE_WORDS;
-  const int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4], s = (int)blockIdx.x;
+  const int32_t *__restrict__ tile = tiles_base + (int64_t)blockIdx.z * TILE_WORDS;
+  int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  const int s = (int)blockIdx.x;
+  if (NT == 1 && (h_flags & SHRINK_COMPENSATE) && blockIdx.y == 1) merged_tile(p.plan, (int)blockIdx.z, TARGETS_ROWS, r, pos0, cnt, astart);
   if (cnt <= 0) return;   // records past the last tile are zero
+  // (a narrow adapter among wide ones takes the loads and products of its own rank)
   if (NB > 1 && r <= 16) shrink_targets_tile<T, NT, 1>(p, s, r, pos0, cnt, astart, lds);
   else if (NB > 2 && r <= 32) shrink_targets_tile<T, NT, 2>(p, s, r, pos0, cnt, astart, lds);
+  else if (NB > 4 && r <= 64) shrink_targets_tile<T, NT, 4>(p, s, r, pos0, cnt, astart, lds);
   else shrink_targets_tile<T, NT, NB>(p, s, r, pos0, cnt, astart, lds);
 }
 
@@ -695,12 +715,6 @@ int launch_gemm_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
     case 1: hipLaunchKernelGGL((shrink_gemm_kernel<T, 1, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
     case 2: hipLaunchKernelGGL((shrink_gemm_kernel<T, 2, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
     case 4: hipLaunchKernelGGL((shrink_gemm_kernel<T, 4, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
-    case 8:
-      if constexpr (MBW <= 2) {
-        hipLaunchKernelGGL((shrink_gemm_kernel<T, 8, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a);
-        break;
-      }
-      return fail(MLORA_ERR_NO_KERNEL, "shrink: rank > 64 has no 256-token tile");
     default: return fail(MLORA_ERR_NO_KERNEL, "shrink: no kernel for rank blocks=%d", nb);
   }
   return check_launch("shrink_gemm_kernel");
@@ -718,19 +732,18 @@ int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
   return check_launch("shrink_kernel");
 }
 
-template <typename T>
+template <typename T, int NT>
 int launch_targets(hipStream_t st, const ShrinkArgs &a, int nb, int64_t tiles) {
-  const dim3 grid((unsigned)a.ksplit, (unsigned)tiles);
-#define MLORA_TARGETS(NT, NB) \
-  hipLaunchKernelGGL((shrink_targets_kernel<T, NT, NB>), grid, dim3(512), 0, st, a.plan + a.off_tiles, a)
-  if (a.n_targets == 2) {
-    if (nb == 1) MLORA_TARGETS(2, 1);
-    else if (nb == 2) MLORA_TARGETS(2, 2);
-    else MLORA_TARGETS(2, 4);
+  const dim3 grid((unsigned)a.ksplit, (unsigned)(a.n_targets / NT), (unsigned)tiles);
+#define MLORA_TARGETS(NB) \
+  hipLaunchKernelGGL((shrink_targets_kernel<T, NT, NB>), grid, dim3(512), 0, st, a.plan + a.off_tiles, head_flags(a), a)
+  if constexpr (NT == 1) {   // (above rank 64)
+    MLORA_TARGETS(8);
   } else {
-    if (nb == 1) MLORA_TARGETS(3, 1);
-    else if (nb == 2) MLORA_TARGETS(3, 2);
-    else MLORA_TARGETS(3, 4);
+    if (nb == 1) MLORA_TARGETS(1);
+    else if (nb == 2) MLORA_TARGETS(2);
+    else if (nb == 4) MLORA_TARGETS(4);
+    else MLORA_TARGETS(8);
   }
 #undef MLORA_TARGETS
   return check_launch("shrink_targets_kernel");
@@ -798,17 +811,22 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   if (bm >= 128) {
     if (grid_tiles > 65535) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");   // (4M tokens of 8192 adapters have 40960)
     grid = dim3((unsigned)a.ksplit, (unsigned)a.n_targets, (unsigned)grid_tiles);
-    // Targets together, where the fewer workgroups still fill the device evenly (two a compute unit; an adapter's last tile is half
-    // empty in the mean, one of few tokens emptier).  The whole op with a 256-wide output, rank 64, per target / together: three
-    // targets, 4096 wide, 140 workgroups (4400 tokens of one adapter) 33.2 / 36.5 us, 204 (4400 over 32) 43.8 / 37.9, 264 (4400 over
-    // 64) 52.8 / 57.3, 452 (14000 over 8) 77.0 / 63.7; two 156 (4400 over 8) 35.3 / 31.1; 8192 wide, 592 (5400 over 64) 68.7 / 74.0;
-    // 2000 tokens over 32 34.9 / 39.3.  401 shapes of 1000 to 14000 tokens, 2048 to 8192 wide, that it takes: 0.90 in the mean,
-    // 1.03 at worst.
+    // Targets together, where the fewer workgroups still fill the device evenly (two a compute unit, one above rank 64; an adapter's
+    // last tile is half empty in the mean, one of few tokens emptier).  The whole op with a 256-wide output, rank 64, per target /
+    // together: three targets, 4096 wide, 140 workgroups (4400 tokens of one adapter) 33.2 / 36.5 us, 204 (4400 over 32) 43.8 / 37.9,
+    // 264 (4400 over 64) 52.8 / 57.3, 452 (14000 over 8) 77.0 / 63.7; two 156 (4400 over 8) 35.3 / 31.1; 8192 wide, 592 (5400 over
+    // 64) 68.7 / 74.0; 2000 tokens over 32 34.9 / 39.3.  401 shapes of 1000 to 14000 tokens, 2048 to 8192 wide, that it takes: 0.90 in
+    // the mean, 1.03 at worst.  Rank 128, three targets: 250 workgroups (14000 over 32, 8192 wide) 247 / 173 us, 256 to 320 1.13 in
+    // the mean of 28 shapes.
     const int64_t adapters = grid_tiles - (a.T + 127) / 128, wgs = (a.T / 128 + adapters / 2) * a.ksplit;
     const bool three = a.n_targets == 3;
-    const bool even = wgs >= (three ? 160 : 128) && !(three && wgs > 256 && wgs <= 320) && !(wgs > 512 && wgs <= 704) && a.T >= 64 * adapters;
-    if (even && bm == 128 && nb <= 4 && (three || a.n_targets == 2) && a.ksplit > 1 && !a.compensate)
-      return dt == MLORA_F16 ? launch_targets<_Float16>(st, a, nb, grid_tiles) : launch_targets<__bf16>(st, a, nb, grid_tiles);
+    const bool even = wgs >= (three ? 160 : 128) && a.T >= 64 * adapters &&
+                      (nb == 8 ? wgs <= 256 : !(three && wgs > 256 && wgs <= 320) && !(wgs > 512 && wgs <= 704));
+    if (even && bm == 128 && (three || a.n_targets == 2) && a.ksplit > 1 && !a.compensate) {
+      if (three) return dt == MLORA_F16 ? launch_targets<_Float16, 3>(st, a, nb, grid_tiles) : launch_targets<__bf16, 3>(st, a, nb, grid_tiles);
+      return dt == MLORA_F16 ? launch_targets<_Float16, 2>(st, a, nb, grid_tiles) : launch_targets<__bf16, 2>(st, a, nb, grid_tiles);
+    }
+    if (nb == 8) return dt == MLORA_F16 ? launch_targets<_Float16, 1>(st, a, nb, grid_tiles) : launch_targets<__bf16, 1>(st, a, nb, grid_tiles);
   }
   if (a.reduce_here)
     grid = dim3((unsigned)(8 * a.ksplit), (unsigned)a.n_targets, (unsigned)(grid_tiles / 8));   // at most 4096 tokens (csrc/api.hip)
