@@ -3,10 +3,12 @@
 // shrink_kernel: one workgroup (4 waves) owns one adapter-grouped tile of up to 16*MB tokens and one K chunk
 // (shrink_core.h has the loads and the products).  Bound by its chain of round trips, not by bytes: tile record ->
 // look-ups -> operand loads -> cross-wave sum -> hand-over of the K chunks (what it measured is in shrink_core.h).
-// shrink_gemm_kernel: 128- and 256-token tiles.
+// shrink_whole_kernel: the same with all of K in one workgroup of eight waves, for one-call entry points.
+// shrink_gemm_kernel: 128- and 256-token tiles, one target of rank up to 64.  shrink_targets_kernel: 128-token tiles, several
+// targets together, or one above rank 64.
 //
-// Split-K without atomics: every workgroup writes its fp32 partial tile and is done; the chunks
-// are summed in index order (bit-reproducible) by shrink_reduce_kernel or by the expand.
+// Split-K without atomics on values: every workgroup writes its fp32 partial tile; the chunks are summed in index order
+// (bit-reproducible) by the last chunk of a small tile to arrive, by shrink_reduce_kernel or by the expand.
 //
 // Reference semantics: valora/csrc/bgmv/bgmv_impl.cuh:14-148 (per-token gather mat-vec with the
 // rank rows gathered through loc_indicies, fp32 accumulation, one T store per output).
@@ -334,8 +336,8 @@ __device__ const __align__(128) uint16_t g_zero_line[64] = {};
 // nothing.  Direct global -> LDS loads into a three-stage ring (one or two workgroups a compute unit instead of three, LDS turn
 // of the result, zero rows read for a narrower adapter's rank) / now, behind the same expand: three targets of 5254 tokens of
 // rank 64 37.2 / 33.4 us, 5401 tokens over ranks 8-64, one target 20.4 / 19.6, two 29.5 / 25.6, three 34.5 / 30.7, `down` of 11008
-// 56.6 / 54.9.  (The chunks summed inside the launch by the last to arrive: 20.4 against 15.3 + 5.1 for the two launches, and
-// 43 against 34 + 5 for three targets of rank 64.)
+// 56.6 / 54.9 (targets together: shrink_targets_kernel, below).  (The chunks summed inside the launch by the last to arrive: 20.4
+// against 15.3 + 5.1 for the two launches, and 43 against 34 + 5 for three targets of rank 64.)
 constexpr int GEMM_KC = 64;                             // K elements of a step: one 128-byte line per row
 constexpr int gemm_stage_bytes(int nb, int mbw) { return (64 * mbw + 16 * nb) * GEMM_KC * 2; }
 constexpr int GEMM_AHEAD = 2;                           // steps requested before the first is used
