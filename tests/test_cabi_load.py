@@ -248,3 +248,13 @@ def test_large_batches_have_tall_expand_tiles():
     with open(tt.TABLE_PATH) as f:
         entries = json.load(f)["entries"]
     assert [k for k, v in entries.items() if int(k.split(":")[0]) > 4096 and v["bm_expand"] < 32] == []
+
+
+def test_small_batches_have_shrink_tiles_of_their_own_size():
+    """A shrink tile takes one adapter's tokens and loads as many rows as it is tall: no entry's tiles are taller than its
+    batches (rows past a tile's end are copies of its first one)."""
+    import json
+    from valora_amd import tile_table as tt
+    with open(tt.TABLE_PATH) as f:
+        entries = json.load(f)["entries"]
+    assert [k for k, v in entries.items() if v["bm_shrink"] > max(16, int(k.split(":")[0]))] == []
