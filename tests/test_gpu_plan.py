@@ -83,6 +83,22 @@ def test_plan_in_parts(dev, T, A):
         _check_plan(ids, a_len, 4, 16, 96, dev)
 
 
+@pytest.mark.parametrize("T,A", [(7, 2048), (7, 2049), (600, 2049), (3000, 2049), (8, 8192)])
+def test_compensation_plan_keeps_adapters_without_a_rank(dev, T, A):
+    """Their tokens have no product of their own, but the merged adapter's comes off them: on both sides of the number of
+    adapters whose tables fit in LDS."""
+    from valora_amd.plan import LoraPlan
+    g = torch.Generator().manual_seed(T + A)
+    rank = torch.randint(0, 3, (A,), generator=g) * 16
+    rank[1] = 16
+    ids = torch.where(torch.rand(T, generator=g) < 0.3, 1, torch.randint(-1, A + 1, (T,), generator=g))
+    plan = LoraPlan(ids.to(dev), (torch.cumsum(rank, 0) * 4 - rank * 4).to(dev), (rank * 4).to(dev), 32, bm_shrink=32, bm_expand=48,
+                    ksplit=1, _merged=1)
+    want = sorted((t for t in range(T) if 0 <= ids[t] < A and ids[t] != 1), key=lambda t: (int(ids[t]), t))
+    assert plan.perm().cpu().tolist() == want
+    assert plan.position_ranks().cpu().tolist() == [int(rank[ids[t]]) for t in want]
+
+
 @pytest.mark.parametrize("T,A", [(1, 1), (700, 40), (5000, 33)])
 def test_plans_cut_in_one_launch(dev, T, A):
     from valora_amd.plan import LoraPlan

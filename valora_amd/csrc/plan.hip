@@ -129,11 +129,13 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   auto start_of = [&](int a) -> int64_t { return SMALL ? s_astart[a] : a_start[a]; };
   // A token's adapter, -1 where the plan leaves the token out, and the adapter's usable rank.  A compensation plan keeps
   // the tokens of adapters without a usable rank: they have no product of their own, but the merged one comes off them.
+  // (Looked up once: inside adapter_of the compiler's code for tables in global memory dropped those tokens all the same.)
+  const bool keep_rankless = merged >= 0 && usable_rank(a_len[merged]) > 0;
   auto adapter_of = [&](int64_t a64, int &r) -> int {
     r = 0;
     if (a64 < 0 || a64 >= A || a64 == merged) return -1;
     r = rank_of((int)a64);
-    return r > 0 || (merged >= 0 && rank_of(merged) > 0) ? (int)a64 : -1;
+    return r > 0 || keep_rankless ? (int)a64 : -1;
   };
 
   auto start_word = [](int64_t st) -> int32_t { return st < 0 || st > 0x7fffffff ? INT32_MIN / 2 : (int32_t)st; };
