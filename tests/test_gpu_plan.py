@@ -99,6 +99,37 @@ def test_compensation_plan_keeps_adapters_without_a_rank(dev, T, A):
     assert plan.position_ranks().cpu().tolist() == [int(rank[ids[t]]) for t in want]
 
 
+@pytest.mark.parametrize("T,A", [(256, 512), (257, 512), (64, 513), (900, 2048), (901, 2048), (901, 513), (600, 2049), (601, 2049), (8, 8192)])
+@pytest.mark.parametrize("merged", [-1, 1])
+def test_plan_forms(dev, T, A, merged):
+    """Both sides of the sizes at which the one-part form of the kernel ends, with unusable ranks, ids outside the index and
+    several plans in one launch; a compensation plan leaves the merged adapter out and keeps adapters without a rank."""
+    from valora_amd.plan import LoraPlan
+    g = torch.Generator().manual_seed(T + A)
+    rank = torch.randint(0, 3, (A,), generator=g) * 16
+    rank[merged] = 16
+    ids = torch.where(torch.rand(T, generator=g) < 0.3, 1, torch.randint(-1, A + 1, (T,), generator=g))
+    a_len, a_start = rank * 4, torch.cumsum(rank * 4, 0) - rank * 4
+    index = (ids.to(dev), a_start.to(dev), a_len.to(dev))
+    plans = [LoraPlan(*index, 32, bm_shrink=32, bm_expand=48, ksplit=1, _merged=merged)]
+    if merged < 0:
+        plans += LoraPlan.of_widths(*index, 32, (4096, 11008))
+    kept = [t for t in range(T) if 0 <= ids[t] < A and ids[t] != merged and (merged >= 0 or rank[ids[t]] > 0)]
+    want = sorted(kept, key=lambda t: (int(ids[t]), t))   # stable, by adapter
+    for p in plans:
+        assert p.perm().cpu().tolist() == want
+        assert p.position_adapters().cpu().tolist() == [int(ids[t]) for t in want]
+        assert p.position_ranks().cpu().tolist() == [int(rank[ids[t]]) for t in want]
+        for tiles, bm in ((p.tiles_shrink().cpu(), p.bm_shrink), (p.tiles_expand().cpu(), p.bm_expand)):
+            at, seen = 0, []
+            while at < len(want):
+                a = int(ids[want[at]])
+                n = min(bm, sum(1 for t in want[at:at + bm] if int(ids[t]) == a))
+                seen.append([a, int(rank[a]), at, n if rank[a] > 0 else -n, int(a_start[a])])
+                at += n
+            assert tiles[:, :5].tolist() == seen
+
+
 @pytest.mark.parametrize("T,A", [(1, 1), (700, 40), (5000, 33)])
 def test_plans_cut_in_one_launch(dev, T, A):
     from valora_amd.plan import LoraPlan

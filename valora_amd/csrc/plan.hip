@@ -87,14 +87,16 @@ constexpr int PLAN_SMALL_A = 2048;   // adapters whose per-adapter tables fit in
 // waves cost more than the work they organise.
 // Grid: (parts, plans of the batch).  Every part counts all tokens and so knows every position; it then writes its share
 // of the token rows, of the tile records and of the words that start at zero.
-template <bool SMALL, int THREADS>
+// PARTS: several parts a plan, and several steps of 64 tokens requested together.  Without, one part, a row of the histogram per
+// wave and a step at a time: half the code, and a launch finds none of it in the instruction cache.
+template <bool SMALL, int THREADS, bool PARTS>
 __global__ __launch_bounds__(THREADS) void plan_kernel(
     int32_t *plan0, const int64_t *__restrict__ ids, const int64_t *__restrict__ a_start,
     const int64_t *__restrict__ a_len, int T, int A, int n_slots, int bm_s0, int bm_e0, int W, PlanSet set,
     int64_t off_perm, int64_t off_padapter, int64_t off_prank, int64_t off_tiles_s,
     int64_t off_tiles_e, int64_t off_counters, int64_t off_scratch, int n_flag_words, int merged) {
   constexpr int N_WAVES = THREADS / 64;
-  constexpr int STEPS = THREADS == PLAN_THREADS_SMALL ? 4 : 8;   // 64-token steps whose ids are requested together
+  constexpr int STEPS = !PARTS ? 1 : THREADS == PLAN_THREADS_SMALL ? 4 : 8;   // 64-token steps whose ids are requested together
   __shared__ int32_t whist[HIST_WORDS];
   __shared__ Quad wsum[PLAN_WAVES + 1];
   __shared__ int s_wmaxr[PLAN_WAVES];
@@ -104,7 +106,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   __shared__ int64_t s_astart[SMALL ? PLAN_SMALL_A : 1];
 
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int part = (int)blockIdx.x, n_parts = (int)gridDim.x;
+  const int part = PARTS ? (int)blockIdx.x : 0, n_parts = PARTS ? (int)gridDim.x : 1;
   int32_t *__restrict__ plan = plan0;   // (the first plan's arguments are there at launch)
   int bm_s = bm_s0, bm_e = bm_e0;
   if (blockIdx.y > 0) {
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
 
   // The tokens are cut into W rows of the histogram (runs of a multiple of 64 tokens); a wave counts `per_wave` of them.
   const int rt = (int)align_up((T + W - 1) / W, 64);
-  const int per_wave = W > N_WAVES ? (W + N_WAVES - 1) / N_WAVES : 1;
+  const int per_wave = PARTS && W > N_WAVES ? (W + N_WAVES - 1) / N_WAVES : 1;
   const int t_beg = min(T, wave * per_wave * rt), t_end = min(T, min(W, (wave + 1) * per_wave) * rt);
   // (tokens behind the end read the batch's last one and are dropped)
   auto load_ids = [&](int t0, int end, int64_t (&id)[STEPS]) {
@@ -182,24 +184,36 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   __syncthreads();
   for (int i = part * THREADS + tid; i < n_flag_words; i += n_parts * THREADS) plan[off_counters + i] = 0;
 
-  // 1. histogram of the tokens per row, whatever their adapters' ranks.  A step of one adapter (most of a prefill batch) is
-  // one addition: 64 lanes that add to one counter are 64 turns.
+  // 1. histogram of the tokens per row.  A step of one adapter (most of a prefill batch) is one addition: 64 lanes that add to
+  // one counter are 64 turns.
   int row = wave * per_wave, row_end = t_beg + rt;
+  int first_a = -1, first_r = 0;   // without PARTS: the row's first 64 tokens, kept for step 3
   for (int t0 = t_beg; t0 < t_end; t0 += 64 * STEPS) {
     if (t0 != t_beg) load_ids(t0, t_end, id);
+    if constexpr (PARTS) {   // whatever the adapters' ranks: step 2 drops the counts of those that the plan leaves out
 #pragma unroll
-    for (int i = 0; i < STEPS; ++i) {
-      const int t = t0 + i * 64;   // wave-uniform
-      if (t < t_end) {
-        if (t >= row_end) { ++row; row_end += rt; }
-        const uint32_t a = (uint32_t)id[i];
-        const bool ok = t + lane < t_end && (uint64_t)id[i] < (uint64_t)(uint32_t)A;
-        if (__ballot(ok && a == (uint32_t)__builtin_amdgcn_readfirstlane((int)a)) == ~0ull) {
-          if (lane == 0) atomicAdd(&whist[row * A + (int)a], 64);
-        } else if (ok) {
-          atomicAdd(&whist[row * A + (int)a], 1);
+      for (int i = 0; i < STEPS; ++i) {
+        const int t = t0 + i * 64;   // wave-uniform
+        if (t < t_end) {
+          if (t >= row_end) { ++row; row_end += rt; }
+          const uint32_t a = (uint32_t)id[i];
+          const bool ok = t + lane < t_end && (uint64_t)id[i] < (uint64_t)(uint32_t)A;
+          if (__ballot(ok && a == (uint32_t)__builtin_amdgcn_readfirstlane((int)a)) == ~0ull) {
+            if (lane == 0) atomicAdd(&whist[row * A + (int)a], 64);
+          } else if (ok) {
+            atomicAdd(&whist[row * A + (int)a], 1);
+          }
         }
       }
+    } else {
+      int r = 0;
+      const int a = t0 + lane < t_end ? adapter_of(id[0], r) : -1;
+      if (__ballot(a >= 0 && a == __builtin_amdgcn_readfirstlane(a)) == ~0ull) {
+        if (lane == 0) atomicAdd(&whist[row * A + a], 64);
+      } else if (a >= 0) {
+        atomicAdd(&whist[row * A + a], 1);
+      }
+      if (t0 == t_beg) { first_a = a; first_r = r; }
     }
   }
   __syncthreads();
@@ -207,28 +221,28 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   // 2. per-adapter totals, group starts, tile offsets (each thread owns a run of adapters)
   const int per = (A + THREADS - 1) / THREADS;
   const int a_beg = min(A, tid * per), a_endx = min(A, a_beg + per);
-  constexpr int ROWS = THREADS == PLAN_THREADS_SMALL ? 4 : 16;   // counters of an adapter that are read in one round trip
+  constexpr int ROWS = !PARTS || THREADS == PLAN_THREADS_SMALL ? 4 : 16;   // counters of an adapter that are read in one round trip
   auto read_hist = [&](int a, int w0, int (&h)[ROWS]) {
 #pragma unroll
     for (int w = 0; w < ROWS; ++w) h[w] = w0 + w < W ? whist[(w0 + w) * A + a] : 0;
   };
   int my_c = 0, my_ts = 0, my_te = 0, my_g = 0, my_maxr = 0;
   for (int a = a_beg; a < a_endx; ++a) {
-    int c = 0, r;
-    const bool used = adapter_of(a, r) >= 0;   // (the plan leaves the tokens of others out)
-    for (int w0 = 0; used && w0 < W; w0 += ROWS) {
+    int c = 0, r = 0;
+    for (int w0 = 0; w0 < W; w0 += ROWS) {
       int h[ROWS];
       read_hist(a, w0, h);
 #pragma unroll
       for (int w = 0; w < ROWS; ++w) c += h[w];
     }
+    if (PARTS && c > 0 && adapter_of(a, r) < 0) c = 0;   // (the plan leaves its tokens out)
     cnt[a] = c;
     if (c > 0) {
       my_c += c;
       my_ts += (c + bm_s - 1) / bm_s;
       my_te += (c + bm_e - 1) / bm_e;
       my_g += 1;
-      my_maxr = max(my_maxr, r);
+      my_maxr = max(my_maxr, PARTS ? r : rank_of(a));
     }
   }
   Quad tot;
@@ -266,9 +280,9 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
 
   // 3. stable scatter of the part's rows: a wave walks a row in order, 64 tokens a step; lanes holding the
   //    same adapter get consecutive positions in lane order.
-  auto place = [&](int row, int t, int end, int64_t id64) {
-    int r = 0;
-    const int a = t < end ? adapter_of(id64, r) : -1;
+  auto place = [&](int row, int t, int end, int64_t id64, bool known) {   // known: first_a and first_r
+    int r = known ? first_r : 0;
+    const int a = known ? first_a : t < end ? adapter_of(id64, r) : -1;
     const unsigned long long same = same_adapter(a);
     if (a >= 0) {
       const int slot_idx = row * A + a;
@@ -281,16 +295,22 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     }
     __builtin_amdgcn_wave_barrier();
   };
-  // (one part and a row per wave: the ids are still in registers)
-  const bool kept = n_parts == 1 && per_wave == 1;
-  for (int k = wave; part + k * n_parts < W; k += N_WAVES) {
-    row = part + k * n_parts;
-    const int beg = min(T, row * rt), end = min(T, beg + rt);
-    for (int t0 = beg; t0 < end; t0 += 64 * STEPS) {
-      if (!kept || rt > 64 * STEPS) load_ids(t0, end, id);
+  if constexpr (PARTS) {
+    const bool kept = n_parts == 1 && per_wave == 1;   // (one part and a row per wave: the ids are still in registers)
+    for (int k = wave; part + k * n_parts < W; k += N_WAVES) {
+      row = part + k * n_parts;
+      const int beg = min(T, row * rt), end = min(T, beg + rt);
+      for (int t0 = beg; t0 < end; t0 += 64 * STEPS) {
+        if (!kept || rt > 64 * STEPS) load_ids(t0, end, id);
 #pragma unroll
-      for (int i = 0; i < STEPS; ++i)
-        if (t0 + i * 64 < end) place(row, t0 + i * 64 + lane, end, id[i]);
+        for (int i = 0; i < STEPS; ++i)
+          if (t0 + i * 64 < end) place(row, t0 + i * 64 + lane, end, id[i], false);
+      }
+    }
+  } else {
+    for (int t0 = t_beg; t0 < t_end; t0 += 64) {
+      if (t0 != t_beg) load_ids(t0, t_end, id);
+      place(row, t0 + lane, t_end, id[0], t0 == t_beg);
     }
   }
 
@@ -427,27 +447,34 @@ int launch_plan(hipStream_t st, const PlanSet &set, int n_plans, const PlanLayou
   const bool few = L.T <= 1024 && A <= 512;
   // Parts and rows.  One compute unit is bound by the instructions of the scatter and by its own stores (126 KB of plan for 5400
   // tokens); counting all tokens again in every part is cheap beside that.  us a build, back to back in a graph, 1 part / several:
-  // 918 tokens 7.4 / 6.8, 1024 over 128 adapters 8.2 / 7.4 (4 parts; 256 tokens 6.1 / 6.4, so not below 512), 5401 over 32 (8 parts)
-  // 15.2 / 10.9, 6749 over 24 17.0 / 11.3, 8192 over 64 19.4 / 13.0, 20000 over 128 38.6 / 20.3.  16 rows instead of 32: 1500 tokens 8.4 /
-  // 8.8, 5401 11.3 / 10.9, 8192 14.0 / 13.0.  (4 or 16 parts are equal to 8; 512 threads 0.5 us slower from 5000 tokens.)
+  // 300 tokens over 300 adapters 9.1 / 8.3, 512 over 32 6.7 / 6.4, 1024 over 128 9.4 / 7.5 (4 parts; 256 tokens 5.7 / 6.4), 5401 over 32 (8
+  // parts) 15.2 / 10.9, 6749 over 24 17.0 / 11.3, 20000 over 128 38.6 / 20.3; 512 to 2048 adapters, where counting them again costs more:
+  // 800 tokens over 600 8.4 / 8.8, 1000 9.8 / 9.4.  16 rows instead of 32: 1500 tokens 8.4 / 8.8, 5401 11.3 / 10.9, 8192 14.0 / 13.0.
+  // (4 or 16 parts are equal to 8; 512 threads 0.5 us slower from 5000 tokens.)
+  // The code of one part (PARTS off) against that of several, both with one part: one token 5.1 / 5.4, 64 over 600 adapters 7.6 / 8.3, over
+  // 2000 9.0 / 10.8, over 4000 12.9 / 15.5; above 2048 adapters 600 tokens 20.5 / 20.5, 4000 64.6 / 58.0.
   int parts = 1, rows = PLAN_WAVES;
   if (few) {
-    rows = L.T > 512 ? 8 : PLAN_THREADS_SMALL / 64;
-    parts = L.T > 512 ? 4 : 1;
-  } else if (A <= PLAN_SMALL_A) {
+    rows = L.T > 256 ? 8 : PLAN_THREADS_SMALL / 64;
+    parts = L.T > 256 ? 4 : 1;
+  } else if (A <= PLAN_SMALL_A && L.T > 900) {
     rows = L.T > 4096 ? 32 : 16;
     parts = 8;
   }
   if (W > rows) W = rows;
   if (parts > W) parts = W;
-#define MLORA_LAUNCH_PLAN(SMALL, THREADS)                                                                          \
-  hipLaunchKernelGGL((plan_kernel<SMALL, THREADS>), dim3(parts, n_plans), dim3(THREADS), 0, st, set.plan[0], ids, a_start, \
+  const bool small_a = A <= PLAN_SMALL_A;
+#define MLORA_LAUNCH_PLAN(SMALL, THREADS, PARTS)                                                                      \
+  hipLaunchKernelGGL((plan_kernel<SMALL, THREADS, PARTS>), dim3(parts, n_plans), dim3(THREADS), 0, st, set.plan[0], ids, a_start, \
                      a_len, (int)L.T, A, n_slots, set.bm_s[0], set.bm_e[0], W, set, L.off_perm, L.off_padapter, L.off_prank,                \
                      L.off_tiles_s, L.off_tiles_e, L.off_counters, L.off_scratch,                                 \
                      (int)(L.off_scratch - L.off_counters), merged)
-  if (few) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL);
-  else if (A <= PLAN_SMALL_A) MLORA_LAUNCH_PLAN(true, PLAN_THREADS);
-  else MLORA_LAUNCH_PLAN(false, PLAN_THREADS);
+  if (few && parts == 1) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL, false);
+  else if (few) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL, true);
+  else if (small_a && parts > 1) MLORA_LAUNCH_PLAN(true, PLAN_THREADS, true);
+  else if (small_a) MLORA_LAUNCH_PLAN(true, PLAN_THREADS, false);
+  else if (L.T > 600) MLORA_LAUNCH_PLAN(false, PLAN_THREADS, true);
+  else MLORA_LAUNCH_PLAN(false, PLAN_THREADS, false);
 #undef MLORA_LAUNCH_PLAN
   return check_launch("plan_kernel");
 }
