@@ -129,6 +129,10 @@ size_t mlora_one_launch_scratch_bytes(int64_t T, int64_t n_adapters, int64_t max
  * buffer of mlora_one_launch_scratch_bytes() and an index and pools that are not empty.             */
 int mlora_runs_in_one_launch(int64_t T, int64_t n_adapters, int64_t max_rank, int64_t h_out, int32_t ksplit,
                              int32_t n_targets);
+/* Whether the shrink of a call with n_targets targets multiplies them in one workgroup, which loads x once (1), or each in
+ * workgroups of its own (0).  Same bits either way.                                             */
+int mlora_targets_together(int64_t T, int64_t n_adapters, int64_t max_rank, int32_t bm_shrink, int32_t ksplit,
+                           int32_t n_targets);
 /* Bytes of scratch the one-call entry points (dispatch_bgmv, dispatch_sgmm, prefill_*) need.
  * Replaces sgmm_tmp_size (atmm/valora/csrc/bgmv/bgmv_impl.cuh:128-132).                       */
 size_t mlora_workspace_bytes(int64_t T, int64_t n_adapters, int64_t max_rank);

@@ -241,6 +241,16 @@ def test_which_calls_run_in_one_launch(T, A, rank, h_out, ks, nt, one):
     assert _lib.lib().mlora_runs_in_one_launch(T, A, rank, h_out, ks, nt) == one
 
 
+@pytest.mark.parametrize("T,A,rank,bm,ks,nt,together", [
+    (6749, 24, 32, 128, 4, 3, 1), (5254, 20, 64, 128, 4, 3, 1), (5254, 20, 64, 128, 4, 2, 1), (14000, 32, 128, 128, 2, 3, 1),
+    # slower together: many adapters of which the batch touches few, few tokens in many chunks, a second round of workgroups
+    (2622, 40, 128, 128, 4, 3, 0), (4409, 46, 128, 128, 4, 3, 0), (6604, 103, 128, 128, 4, 3, 0), (1276, 15, 128, 128, 8, 2, 0),
+    (1482, 22, 128, 128, 8, 3, 0), (2505, 19, 64, 128, 8, 3, 0), (4280, 42, 64, 128, 8, 3, 0), (7062, 32, 32, 128, 4, 3, 0),
+    (6749, 24, 32, 128, 4, 1, 0), (6749, 24, 32, 128, 4, 4, 0), (6749, 24, 32, 128, 1, 3, 0), (6749, 24, 32, 64, 4, 3, 0), (6749, 24, 32, 256, 4, 3, 0)])
+def test_which_targets_go_together(T, A, rank, bm, ks, nt, together):
+    assert _lib.lib().mlora_targets_together(T, A, rank, bm, ks, nt) == together
+
+
 def test_large_batches_have_tall_expand_tiles():
     """The expand of 16-token tiles fetches B once per tile: from a few thousand tokens on taller tiles win at every width."""
     import json

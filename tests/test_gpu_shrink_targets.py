@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from oracle import lora_oracle as O
-from valora_amd import workloads as W
+from valora_amd import _lib, workloads as W
 from valora_amd.plan import LoraPlan
 from tests._util import assert_parity
 
@@ -51,3 +51,28 @@ def test_bits_of_separate_calls(dev, h_in, ksplit, ranks):
             plan.apply_multi(ys, xd, pd.key_buffer, pd.value_buffer, *idx, list(slots), pd.a_scaling)
             for z, y in zip(slots, ys):
                 assert torch.equal(y.cpu(), alone[z]), f"{h_in} {ksplit} {ranks} targets {slots}, {z}"
+
+
+@pytest.mark.parametrize("T,h_in,ksplit,rank,n,together", [
+    (5249, 1032, 4, 16, 3, 1),     # 42 tiles: the odd block of columns and a K remainder, together
+    (5120, 1032, 4, 64, 3, 1), (4992, 1032, 4, 64, 3, 0),       # 160 and 156 workgroups at least
+    (4096, 1032, 4, 40, 2, 1), (3968, 1032, 4, 40, 2, 0),       # 128 and 124
+    (8064, 1032, 4, 32, 3, 1), (8192, 1032, 4, 32, 3, 0), (10624, 264, 4, 32, 3, 0), (10752, 264, 4, 32, 3, 1),   # 256, 260, 336, 340 usually
+    (3968, 2056, 16, 24, 2, 1), (4096, 2056, 16, 24, 2, 0), (5504, 2056, 16, 16, 3, 0), (5632, 2056, 16, 16, 3, 1),   # 512, 528, 704, 720
+    (5760, 1032, 4, 128, 3, 1), (5632, 1032, 4, 128, 3, 0), (4736, 1032, 4, 72, 2, 1), (4608, 1032, 4, 72, 2, 0),
+])
+def test_both_sides_of_the_rule(dev, T, h_in, ksplit, rank, n, together):
+    """The route a call takes, and the bits of separate calls on it."""
+    ranks = (rank, 8)
+    assert _lib.lib().mlora_targets_together(T, len(ranks), rank, 128, ksplit, n) == together
+    g = torch.Generator().manual_seed(T + h_in)
+    ids = torch.where(torch.arange(T) < T // 3 + 5, 1, 0)[torch.randperm(T, generator=g)]
+    pool = W.make_pool(list(ranks), h_in, 72, torch.float16, g, True, std=0.05, heads=1).to(dev)
+    x = torch.randn(T, h_in, generator=g).to(torch.float16).to(dev)
+    idx = (pool.a_start, pool.a_len, pool.a_loc)
+    plan = LoraPlan(ids.to(dev), *idx[:2], rank, hidden=h_in, bm_shrink=128, bm_expand=32, ksplit=ksplit, reduce_in_expand=False, one_launch=False)
+    ys = [torch.zeros(T, 72, dtype=torch.float16, device=dev) for _ in range(2 * n)]
+    plan.apply_multi(ys[:n], x, pool.key_buffer, pool.value_buffer, *idx, list(range(n)), pool.a_scaling)
+    for z in range(n):
+        plan.apply(ys[n + z], x, pool.key_buffer, pool.value_buffer, *idx, z, pool.a_scaling)
+        assert ys[z].any() and torch.equal(ys[z], ys[n + z]), z

@@ -29,6 +29,7 @@ SYMBOLS = [
     "mlora_pool_alloc", "mlora_pool_alloc_contiguous", "mlora_pool_free", "mlora_pool_fill",
     "mlora_pool_scatter_rows", "mlora_pool_gather_rows", "mlora_index_compact", "mlora_merge_adapter",
     "mlora_build_compensation_plan", "mlora_lora_compensate", "mlora_runs_in_one_launch",
+    "mlora_targets_together",
 ]
 
 
@@ -75,6 +76,7 @@ def lib():
     L.mlora_workspace_bytes.argtypes = [c_int64, c_int64, c_int64]
     L.mlora_one_launch_scratch_bytes.argtypes = [c_int64, c_int64, c_int64, c_int32, c_int32]
     L.mlora_runs_in_one_launch.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int32, c_int32]
+    L.mlora_targets_together.argtypes = [c_int64, c_int64, c_int64, c_int32, c_int32, c_int32]
     for n in ("mlora_tile_lookup", "mlora_tile_fallback"):
         getattr(L, n).argtypes = [c_int64, c_int64, c_int64, c_int64, POINTER(TileConfig)]
     L.mlora_build_plan.argtypes = [c_void_p, POINTER(Plan), c_void_p, c_int64, c_void_p, c_void_p,

@@ -231,6 +231,11 @@ int mlora_runs_in_one_launch(int64_t T, int64_t n_adapters, int64_t max_rank, in
          one_launch_pays(T, n_adapters, items, max_rank, n_targets, one_launch_ksplit(ksplit, n_targets));
 }
 
+int mlora_targets_together(int64_t T, int64_t n_adapters, int64_t max_rank, int32_t bm_shrink, int32_t ksplit, int32_t n_targets) {
+  if (T < 1 || n_adapters < 1 || max_rank < 1) return 0;
+  return shrink_targets_together(T, n_adapters < T ? n_adapters : T, max_rank, bm_shrink, ksplit, n_targets);
+}
+
 size_t mlora_workspace_bytes(int64_t T, int64_t n_adapters, int64_t max_rank) {
   if (T < 0 || n_adapters < 0 || max_rank < 0) return 0;
   auto up = [](size_t n) { return (n + 255) & ~(size_t)255; };

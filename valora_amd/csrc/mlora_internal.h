@@ -181,6 +181,7 @@ int launch_ids_from_requests(hipStream_t st, int64_t *ids_out, const int32_t *b_
                              int64_t T, int64_t max_rows);
 int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int64_t grid_tiles,
                   mlora_dtype dt);
+bool shrink_targets_together(int64_t T, int64_t adapters, int64_t max_rank, int bm, int ksplit, int n_targets);   // at most `adapters` of them have tokens
 int launch_shrink_reduce(hipStream_t st, const ShrinkArgs &a, mlora_dtype dt);
 int launch_expand(hipStream_t st, const ExpandArgs &a, int max_rank, int64_t grid_tiles, int bm_expand,
                   mlora_dtype dt);

@@ -796,6 +796,30 @@ int launch_shrink_reduce(hipStream_t st, const ShrinkArgs &a, mlora_dtype dt) {
   return check_launch("shrink_reduce_kernel");
 }
 
+// Two or three targets of 128-token tiles together, where the fewer workgroups still fill the device evenly: two a compute unit, one
+// above rank 64, so that some 270 or 540 of them need a second or third round.  How many there are depends on how many of the index's
+// adapters the batch touches, which the host does not know: the least (all tokens of one adapter) must be enough, and the
+// number when all adapters end in a half-empty tile not too many.  Above four K chunks a workgroup has few K steps behind its
+// launch, look-ups and first loads, and sharing x gains less than the fewer workgroups lose.
+// The whole op with a 256-wide output, per target / together, us.  Rank 64, three targets, 4096 wide: 140 workgroups (4400 tokens of one
+// adapter) 33.2 / 36.5, 204 (4400 over 32) 43.8 / 37.9, 264 (4400 over 64) 52.8 / 57.3, 452 (14000 over 8) 77.0 / 63.7; eight chunks, 160
+// (2505 over one, 8192 wide) 37.5 / 39.8; two targets 156 (4400 over 8) 35.3 / 31.1, 592 (5400 over 64, 8192 wide) 68.7 / 74.0.  Rank 128,
+// three targets: 250 workgroups (14000 over 32, 8192 wide) 247 / 173, 144 (4409 over 4, 3072 wide) 41.6 / 51.6; two, eight chunks: 112
+// (1276 over 7, 3072 wide) 23.0 / 27.1.  1500 shapes of 1000 to 16000 tokens, 2048 to 14336 wide, batches of one to all of up to 150 adapters,
+// the ones it takes: rank up to 64 0.92 (two targets) and 0.88 (three), above 0.95 and 0.93 in the mean; 22 of 830 above 1.02, 1.10 at worst.
+bool shrink_targets_together(int64_t T, int64_t adapters, int64_t max_rank, int bm, int ksplit, int n_targets) {
+  if (bm != 128 || ksplit < 2 || (n_targets != 2 && n_targets != 3) || T < 64 * adapters) return false;
+  const int64_t least = (T + 127) / 128 * ksplit, usual = (T / 128 + adapters / 2) * ksplit;
+  const bool three = n_targets == 3, many = ksplit > 4;
+  if (max_rank > 64) {
+    if (usual > (many ? 240 : 256 - 2 * ksplit)) return false;   // (one round of one per unit; sizes of tails vary)
+    return least >= (three ? many ? 208 : 180 : many ? 168 : 148);
+  }
+  if (usual > 512 && usual <= 704) return false;   // into the third round
+  if (!three) return least >= 128;
+  return many ? least >= 176 && (usual <= 232 || usual > 704) : least >= 160 && (usual <= 256 || usual > 336);
+}
+
 int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int64_t grid_tiles,
                   mlora_dtype dt) {
   int nb = (max_rank + 15) / 16;
@@ -813,19 +837,8 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   if (bm >= 128) {
     if (grid_tiles > 65535) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");   // (4M tokens of 8192 adapters have 40960)
     grid = dim3((unsigned)a.ksplit, (unsigned)a.n_targets, (unsigned)grid_tiles);
-    // Targets together, where the fewer workgroups still fill the device evenly (two a compute unit, one above rank 64; an adapter's
-    // last tile is half empty in the mean, one of few tokens emptier).  The whole op with a 256-wide output, rank 64, per target /
-    // together: three targets, 4096 wide, 140 workgroups (4400 tokens of one adapter) 33.2 / 36.5 us, 204 (4400 over 32) 43.8 / 37.9,
-    // 264 (4400 over 64) 52.8 / 57.3, 452 (14000 over 8) 77.0 / 63.7; two 156 (4400 over 8) 35.3 / 31.1; 8192 wide, 592 (5400 over
-    // 64) 68.7 / 74.0; 2000 tokens over 32 34.9 / 39.3.  401 shapes of 1000 to 14000 tokens, 2048 to 8192 wide, that it takes: 0.90 in
-    // the mean, 1.03 at worst.  Rank 128, three targets: 250 workgroups (14000 over 32, 8192 wide) 247 / 173 us, 256 to 320 1.13 in
-    // the mean of 28 shapes.
-    const int64_t adapters = grid_tiles - (a.T + 127) / 128, wgs = (a.T / 128 + adapters / 2) * a.ksplit;
-    const bool three = a.n_targets == 3;
-    const bool even = wgs >= (three ? 160 : 128) && a.T >= 64 * adapters &&
-                      (nb == 8 ? wgs <= 256 : !(three && wgs > 256 && wgs <= 320) && !(wgs > 512 && wgs <= 704));
-    if (even && bm == 128 && (three || a.n_targets == 2) && a.ksplit > 1 && !a.compensate) {
-      if (three) return dt == MLORA_F16 ? launch_targets<_Float16, 3>(st, a, nb, grid_tiles) : launch_targets<__bf16, 3>(st, a, nb, grid_tiles);
+    if (!a.compensate && shrink_targets_together(a.T, grid_tiles - (a.T + 127) / 128, max_rank, bm, a.ksplit, a.n_targets)) {
+      if (a.n_targets == 3) return dt == MLORA_F16 ? launch_targets<_Float16, 3>(st, a, nb, grid_tiles) : launch_targets<__bf16, 3>(st, a, nb, grid_tiles);
       return dt == MLORA_F16 ? launch_targets<_Float16, 2>(st, a, nb, grid_tiles) : launch_targets<__bf16, 2>(st, a, nb, grid_tiles);
     }
     if (nb == 8) return dt == MLORA_F16 ? launch_targets<_Float16, 1>(st, a, nb, grid_tiles) : launch_targets<__bf16, 1>(st, a, nb, grid_tiles);
