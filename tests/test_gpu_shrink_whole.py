@@ -89,3 +89,40 @@ def test_entry_points(dev, T, h_in, ranks):
     lora_get_qkvo_fwd_shrink(xd, pd.key_buffer.view(-1, h_in), o, pd.a_loc, pd.a_start, pd.a_len, start.to(dev), seq.to(dev),
                              req.to(dev), h_in, slot, R, int(seq.max()))
     assert_parity(o.cpu(), fresh.to(dtype), f"prefill shrink {T} {h_in}")
+
+
+@pytest.mark.parametrize("T,h_in,ranks,tile", [
+    (4480, 72, (16,), 32), (4479, 72, (16,), 0), (8000, 264, (16,), 32), (8001, 264, (16,), 0),     # 250 pieces
+    (4600, 136, (32,) * 212, 32), (4600, 136, (32,) * 214, 0),                                      # and 106 or 107 tails
+    (5001, 2048, (32, 8), 32), (5001, 2056, (32, 8), 0), (5001, 3064, (32, 8), 0), (5001, 3072, (32, 8), 32),
+    (6368, 3080, (32, 16), 0), (6369, 3080, (32, 16), 32), (4600, 1032, (64, 16), 32),              # 199 and 200 pieces at least
+    (10176, 3080, (16,), 0), (10177, 3080, (16, 8, 8), 64), (15872, 3072, (8,), 64), (15873, 3072, (8,), 0), (12000, 3064, (16,), 0),
+])
+@pytest.mark.parametrize("missing", [False, True])
+def test_both_sides_of_the_rule(dev, T, h_in, ranks, tile, missing):
+    """Which calls take the kernel, and their results with every pool row there and with rows outside the index or the pool."""
+    from valora_amd._ext import binding
+    from valora_amd.kernels import dispatch_bgmv
+    A, R, slot = len(ranks), max(ranks), 1
+    assert binding.one_call_tile(T, A, R, h_in) == tile
+    g = torch.Generator().manual_seed(T + h_in)
+    dtype = torch.bfloat16 if T % 2 else torch.float16
+    pool = W.make_pool(list(ranks), h_in, h_in, dtype, g, True, std=0.05, heads=1, extra_rows=1)
+    seen = pool.a_loc.clone()
+    if missing:
+        spare = pool.key_buffer.shape[0] - 1   # zeros for the oracle, out of the pool's bounds for the op
+        pool.key_buffer[-1] = 0
+        pool.a_loc[pool.a_loc == spare] = 0
+        seen = pool.a_loc.clone()
+        for a in range(0, A, 2):
+            for i, bad in enumerate((-1, spare + 1, 1 << 40)):
+                at = int(pool.a_start[a]) + ranks[a] * slot + 2 * i + 1
+                seen[at], pool.a_loc[at] = spare, bad
+    ids = torch.randint(-1, A, (T,), generator=g)
+    x, d0 = torch.randn(T, h_in, generator=g).to(dtype), torch.randn(T, R, generator=g).to(dtype)
+    want = O.bgmv_shrink(d0, x, pool.key_buffer, pool.a_start, pool.a_len, seen, ids, slot)
+    pd, d = pool.to(dev), d0.to(dev)
+    dispatch_bgmv(d, x.to(dev), pd.key_buffer, pd.a_start, pd.a_len, pd.a_loc, ids.to(dev), slot, pd.a_scaling)
+    assert_parity(d.cpu(), want, f"{T} {h_in} {missing}")
+    had = (torch.tensor(ranks)[ids.clamp(min=0)].unsqueeze(1) > torch.arange(R)) & (ids >= 0).unsqueeze(1)
+    assert torch.equal(d.cpu()[~had], d0[~had])

@@ -750,6 +750,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def_readonly("scratch", &NativePlan::scratch)
       .def_readonly("scratch_per_target", &NativePlan::scratch_per_target);
   m.def("tile_lookup", &tile_lookup);
+  m.def("one_call_tile", &mlora::one_call_tile);
   m.def("cache_lookup", &cache_lookup);
   m.def("cache_insert", &cache_insert);
   m.def("cache_clear", [] { g_entries.clear(); });
