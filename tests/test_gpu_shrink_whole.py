@@ -92,11 +92,11 @@ def test_entry_points(dev, T, h_in, ranks):
 
 
 @pytest.mark.parametrize("T,h_in,ranks,tile", [
-    (4480, 72, (16,), 32), (4479, 72, (16,), 0), (8000, 264, (16,), 32), (8001, 264, (16,), 0),     # 250 pieces
-    (4600, 136, (32,) * 212, 32), (4600, 136, (32,) * 214, 0),                                      # and 106 or 107 tails
-    (5001, 2048, (32, 8), 32), (5001, 2056, (32, 8), 0), (5001, 3064, (32, 8), 0), (5001, 3072, (32, 8), 32),
+    (4480, 72, (16,), 32), (4479, 72, (16,), 0), (8192, 264, (16,), 32), (8193, 264, (16,), 0),     # 256 pieces
+    (4600, 136, (32,) * 212, 32), (4600, 136, (32,) * 214, 0),                                      # 144 and 112 or 113 tails
+    (5001, 2048, (32, 8), 32), (5001, 2056, (32, 8), 0), (5001, 2056, (32, 8) * 4, 32), (5001, 3064, (32, 8), 0), (5001, 3072, (32, 8), 32),
     (6368, 3080, (32, 16), 0), (6369, 3080, (32, 16), 32), (4600, 1032, (64, 16), 32),              # 199 and 200 pieces at least
-    (10176, 3080, (16,), 0), (10177, 3080, (16, 8, 8), 64), (15872, 3072, (8,), 64), (15873, 3072, (8,), 0), (12000, 3064, (16,), 0),
+    (8896, 3080, (16,), 0), (8897, 3080, (16, 8, 8), 64), (16384, 3072, (8,), 64), (16385, 3072, (8,), 0), (12000, 3064, (16,), 0),
 ])
 @pytest.mark.parametrize("missing", [False, True])
 def test_both_sides_of_the_rule(dev, T, h_in, ranks, tile, missing):

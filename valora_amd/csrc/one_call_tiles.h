@@ -17,19 +17,20 @@ namespace mlora {
 //   rank 32 18.5 / 20.2); 14000 over 32, rank 16, 64 a workgroup 28.3 / 24.9 (rank 32 31.4 / 31.1); 3500 over 8, rank 8 9.6 / 10.7
 //   5000 over 32: 5120 wide, rank 16 19.6 / 15.6, 3072 wide, rank 16 12.9 / 10.2 (8192 wide, rank 16 23.1 / 23.8)
 //   2048 wide, rank 64: 6700 over 64 19.9 / 14.8 (10000 over 32, rank 32 by 64 a workgroup 15.0 / 17.3); 2560 wide, rank 32: 7554 over one
-//   adapter 15.4 / 15.9
+//   adapter 15.4 / 15.9, batches of more than ten adapters 0.86 in the mean
 //   64 a workgroup: 7186 over 42 of 168, rank 8, 3072 wide, 127 workgroups 16.1 / 19.4; 15521 over 19, rank 16, 2560 wide, 258 21.8 / 27.6
 // Through the entry points, 1500 shapes of 4480 to 17000 tokens, 1024 to 5120 wide, batches of one to all of up to 220 adapters: 0.90 in
-// the mean of the 1031 that it takes, 11 above 1.02.  Values that are not the rounded exact sum: 0.138 / 0.124 %.
+// the mean of the 1113 that it takes, 14 above 1.02.  Values that are not the rounded exact sum: 0.138 / 0.124 %.
 inline int one_call_tile(int64_t T, int64_t A, int64_t max_rank, int64_t h_in) {
   if (T < 4480 || max_rank > 64 || h_in > 5120 || h_in * max_rank > 131072) return 0;
-  const int64_t tails = (A < T ? A : T) / 2, least32 = (T + 31) / 32, least64 = (T + 63) / 64;
-  if (least32 + tails <= 250) {
+  const int64_t touched = A < T ? A : T, least32 = (T + 31) / 32, least64 = (T + 63) / 64;
+  const int64_t tails = touched / 2 + (touched < 12 ? touched : 12) / 2;   // (the second term: room for more than the mean)
+  if (least32 + tails <= 256) {
     if (max_rank <= 16 || h_in <= 2048) return 32;
-    if (h_in < 3072) return 0;
+    if (h_in < 3072) return A >= 8 ? 32 : 0;
     return h_in <= 3072 || least32 >= 200 ? 32 : 0;
   }
-  return max_rank <= 16 && h_in >= 3072 && least64 >= 160 && least64 + tails <= 248 ? 64 : 0;
+  return max_rank <= 16 && h_in >= 3072 && least64 >= 140 && least64 + tails <= 256 ? 64 : 0;
 }
 
 }  // namespace mlora
