@@ -456,7 +456,6 @@ int mlora_expand(void *stream, const mlora_plan *plan, void *y, int64_t T, int64
   a.h_out = (int)h_out;
   a.inv_h_out = 1.0f / (float)h_out;
   a.kmax = (int)max_rank;
-  a.slot = slot;
   a.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
   a.compensate = 0;
   a.n_targets = 1;
@@ -602,7 +601,6 @@ int mlora_lora_apply_multi(void *stream, const mlora_plan *plan, void *scratch, 
   e.h_out = (int)h_out;
   e.inv_h_out = 1.0f / (float)h_out;
   e.kmax = (int)max_rank;
-  e.slot = targets[0].slot;
   e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
   e.compensate = 0;
   e.n_targets = n_targets;
@@ -710,7 +708,6 @@ int mlora_lora_compensate(void *stream, const mlora_plan *plan, void *scratch, s
   e.h_out = (int)h_out;
   e.inv_h_out = 1.0f / (float)h_out;
   e.kmax = (int)max_rank;
-  e.slot = slot;
   e.n_ochunks = (int)((h_out + expand_bn() - 1) / expand_bn());
   e.compensate = 1;
   e.n_targets = 1;

@@ -24,9 +24,6 @@ __device__ __forceinline__ To as(const From &v) {
 __device__ __forceinline__ u32x4 load16(const uint16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
 __device__ __forceinline__ void store16(uint16_t *p, u32x4 v) { *reinterpret_cast<u32x4 *>(p) = v; }
 
-// Direct global -> LDS load: each active lane copies 16 bytes from its own global address to
-// lds_base + lane*16 (lds_base is wave-uniform); completion is tracked by vmcnt.
-#define GLOBAL_PTR(p) (reinterpret_cast<const __attribute__((address_space(1))) void *>(reinterpret_cast<uintptr_t>(p)))
 // A pointer that went through an inline asm operand has lost what the compiler knew about it; telling it again that
 // the memory is global keeps its loads and stores on the global path (flat accesses count against two wait counters)
 template <typename P>
@@ -34,38 +31,16 @@ __device__ __forceinline__ P *as_global(P *p) {
   typedef __attribute__((address_space(1))) P *GP;
   return (P *)(GP)(uintptr_t)p;
 }
-#define LDS_PTR(p) ((__attribute__((address_space(3))) void *)(p))
 
-// wait until at most N vector-memory loads of this wave are outstanding (loads retire in order)
+// wait until at most N vector-memory accesses of this wave are outstanding (they retire in order)
 template <int N>
 __device__ __forceinline__ void wait_vmcnt() {
   static_assert(N >= 0 && N < 64, "vmcnt is a 6-bit counter");
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
-// the same for LDS accesses, which complete in order as well
-template <int N>
-__device__ __forceinline__ void wait_lgkmcnt() {
-  static_assert(N >= 0 && N < 16, "lgkmcnt is a 4-bit counter");
-  asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(N) : "memory");
-}
+// wait until none of its LDS accesses and scalar loads is outstanding
 __device__ __forceinline__ void wait_lgkmcnt0() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 
-// LDS accesses the compiler does not see as LDS accesses.  Around direct-to-LDS loads the
-// compiler's own wait insertion is conservative (it drains ALL outstanding loads before any LDS
-// access that might alias their destination), which would serialise a multi-stage ring; with
-// these the kernel orders things itself: wait_vmcnt<N>() before reading a stage,
-// wait_lgkmcnt0() + pin() before using what lds_read16 returned.
-__device__ __forceinline__ uint32_t lds_offset(const void *p) {
-  return (uint32_t)(uintptr_t)LDS_PTR(const_cast<void *>(p));
-}
-__device__ __forceinline__ u32x4 lds_read16(uint32_t off) {
-  u32x4 v;
-  asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(off) : "memory");
-  return v;
-}
-__device__ __forceinline__ void lds_write16(uint32_t off, u32x4 v) {
-  asm volatile("ds_write_b128 %0, %1" ::"v"(off), "v"(v) : "memory");
-}
 // loads requested above stay above: the compiler would rather sink them to where they are used
 __device__ __forceinline__ void requested() { asm volatile("" ::: "memory"); }
 // The next of a row of chunks that are requested together, or the same again: the compiler must not see that it may be the
@@ -75,9 +50,6 @@ __device__ __forceinline__ const char *next_chunk(const char *chunk, bool more, 
   asm volatile("" : "+s"(chunk));
   return as_global(chunk);
 }
-// makes v "produced here" for the compiler, so nothing that uses it moves above a preceding wait
-__device__ __forceinline__ void pin(u32x4 &v) { asm volatile("" : "+v"(v)); }
-
 // q = n / d and rem = n % d for n < 2^24 (exact in fp32) from a reciprocal computed once: the float estimate of
 // the quotient is off by at most one.  An integer division by a run-time divisor costs some 35 vector
 // instructions, and the kernels' address set-up does several per lane before the first load can be issued.

@@ -140,7 +140,7 @@ struct ExpandArgs {
   int64_t v_tstride, partial_tstride;
   PoolDev pool;
   const uint16_t *scales;
-  int T, h_out, kmax, slot, n_ochunks;
+  int T, h_out, kmax, n_ochunks;
   float inv_h_out;            // 1 / h_out
   int compensate;             // every tile takes its own adapter's product minus the merged adapter's (one target)
 };

@@ -47,9 +47,9 @@ __device__ __forceinline__ f32x4 shrink_tile_sum(const float *lds, int nblk, int
 }
 
 // What a lane without anything to fetch reads, as far as the steps of a batch reach.
-__device__ const __align__(128) uint16_t g_shrink_zeros[3 * 8 * SHRINK_KSTEP + SHRINK_KSTEP] = {};
+__device__ const __align__(128) uint16_t g_shrink_zeros[12 * SHRINK_KSTEP + SHRINK_KSTEP] = {};
 constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1; }
-// Leaves the four waves' shares of the fp32 result of K range [kbeg, kend) in `lds` (shrink_lds_floats(MB * NB) floats,
+// Leaves the waves' shares of the fp32 result of K range [kbeg, kend) in `lds` (shrink_lds_floats(MB * NB) floats,
 // 16-byte aligned), for shrink_tile_sum to add up (rows = tokens of the tile, columns = rank); every thread of the
 // workgroup must call it, none may still be reading `lds`, and all have passed a barrier when it returns.
 // U: K steps in flight per wave.  The order of the sums does not depend on it.
@@ -68,6 +68,7 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
   constexpr int BLKS = MB + NB;                         // 16-row blocks of a K step, x first
   constexpr bool MANY = NB > 2;
   constexpr bool WHOLE = MB == 1 || NB <= 2;            // has a loop of its own for whole batches
+  static_assert(WAVES * (U - 1) <= 12, "a batch's steps reach past g_shrink_zeros");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, kg = lane >> 4;           // MFMA operand roles
   const int grow = lane >> 3, gcol = lane & 7;          // loader roles: row within a group of 8, 16-byte chunk
