@@ -30,7 +30,9 @@ constexpr int64_t MAX_GRID_TILES = 65535;   // tiles of one launch: grid y is 16
 constexpr int EXP_V_BATCH = 3;     // chunks of v a thread requests together
 __host__ __device__ constexpr int expand_v_chunks(int kb) { return kb * 4 + 1; }   // LDS chunks of a v row, odd
 
-// Waves per SIMD the register allocator has to leave room for: as many as do without spills.
+// Waves per SIMD the register allocator has to leave room for: as many as do without spills of vector registers.  (Rank above 64
+// with outputs narrower than SMALL_WIDE: 16 look-ups' masks do not fit the scalar registers either, 27 scalars with partial sums and 58
+// with COMP stand in lanes of vector registers.  250 calls of such ranks with 256 to 1536 outputs take 0.83 of the time of masked loads.)
 constexpr int expand_min_waves(int kb, bool partial, bool comp) {
   return comp || partial ? 1 : kb == 1 ? 6 : kb == 2 ? 5 : 1;
 }
@@ -57,8 +59,8 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
   constexpr int MBU = COMP && KB == 4 ? 1 : EXP_MBU;   // two rank-128 operand sets leave registers for one block
   constexpr int VC = KB * 4, VLD = expand_v_chunks(KB);
   __shared__ __align__(16) float stage[4][8][STAGE_LD];
-  // The tile's v rows, with COMP the merged adapter's behind them, and its token indices.  (As small as they can be: 96 tokens of
-  // rank 64 are 31.6 KB a workgroup in all, five on a compute unit.)
+  // The tile's v rows, with COMP the merged adapter's behind them, and its token indices.  (96 tokens of rank 64
+  // are 22.9 KB a workgroup in all, which seven would fit; registers leave room for five.)
   extern __shared__ __align__(16) unsigned char s_v[];
 
   const int tile_idx = (int)blockIdx.y, z = (int)blockIdx.z;

@@ -287,8 +287,9 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
 
 // All of K in one workgroup of eight waves, 32 or 64 tokens: no partials, no second launch (or wait for the other chunks).  The
 // tile list may be one of taller tiles, whose pieces of 16 * MB tokens the workgroups take.  csrc/one_call_tiles.h has the rule.
-// Bound by what a compute unit takes in and by HBM: 7000 tokens over 32 adapters, 4096 wide, rank 32 read 57 MB in 17.4 us (3.3
-// TB/s).  The shrink alone, cold x, 128-token tiles in four chunks and the launch that sums them / this: rank 32 22.9 / 17.4 us,
+// Bound by launch, look-ups, first loads and the final sums, which nothing hides with one workgroup a compute unit (130 registers at rank
+// 32), and between them by what a compute unit takes in: 7000 tokens over 32 adapters, 4096 wide, rank 32 read 57 MB in 17.4 us,
+// 3.3 TB/s over the whole launch.  The shrink alone, cold x, 128-token tiles in four chunks and the launch that sums them / this: rank 32 22.9 / 17.4 us,
 // rank 16 17.1 / 14.4; four waves instead of eight with the same 32 tokens 19.6 / 16.4 (6749 tokens, rank 32).  Four K steps in
 // flight a wave instead of two gain nothing at 4096 and lose where they leave a remainder (7000 tokens, 3072 wide, rank 8
 // 10.8 / 12.1).
@@ -330,9 +331,10 @@ __device__ const __align__(128) uint16_t g_zero_line[64] = {};
 // is needed.  A K step of 64 is requested into registers as whole 128-byte lines, every wave its own x rows and a quarter
 // of the adapter's A rows, two steps before it is used, and handed over through two LDS stages; one barrier per step.
 //
-// Bound by memory: x once, A once per 128 tokens, the partials, and the y lines the expand before it still has to
-// write back.  With the loads alone 17.1 of 17.9 us, with the products alone 12.3, one step only 6.6 (5254 tokens of rank 64, one
-// target in four chunks); a deeper ring, K starts spread over the channels, ids by XCD and contiguous pool rows change
+// Bound by a fixed part (launch, look-ups, first step, partials: one step only takes 6.6 of 17.9 us; 5254 tokens of rank 64, one target in
+// four chunks) and then by a stream of loads at 4.3 TB/s: 43 MB of x and 5.4 MB of partials in the other 11.3 us, A again per 128 tokens
+// from L2 and the y lines that the expand before it still has to write back on top.  With the loads alone 17.1 of the 17.9 us, with
+// the products alone 12.3; a deeper ring, K starts spread over the channels, ids by XCD and contiguous pool rows change
 // nothing.  Direct global -> LDS loads into a three-stage ring (one or two workgroups a compute unit instead of three, LDS turn
 // of the result, zero rows read for a narrower adapter's rank) / now, behind the same expand: three targets of 5254 tokens of
 // rank 64 37.2 / 33.4 us, 5401 tokens over ranks 8-64, one target 20.4 / 19.6, two 29.5 / 25.6, three 34.5 / 30.7, `down` of 11008
@@ -533,7 +535,7 @@ __global__ __launch_bounds__(256, MBW == 2 ? 2 : 1) void shrink_gemm_kernel(cons
 // waves split the tokens, the waves of a pair the rank columns.  One step is in flight, and a step's operands are read half by
 // half, so that two workgroups share a compute unit up to 192 columns (two steps in flight at three targets of rank 64: 154
 // registers, one workgroup, 5401 tokens over ranks 8-64 32.3 us against 29.3 now).
-// Bound by memory and by what is not yet or no more streaming: launch, look-ups, first step, partials (6.6 us of one target).
+// Bound as the four-wave tile: 6.6 us of launch, look-ups, first step and partials (of one target), then the stream of x.
 // 4430 tokens of rank 64, 4096 wide, four chunks, per target / together: two targets 25.8 / 23.3 us, three 33.3 / 27.5; 5401 tokens
 // over ranks 8-64 25.4 / 23.6, 30.6 / 29.3.  One target of rank 128, four waves (280 registers, one workgroup a compute unit) /
 // eight, the whole op: 3000 tokens over 64 adapters, 5120 wide 47.8 / 43.0; 113 shapes 0.965 in the mean.  (Up to rank 64 one target is
