@@ -131,8 +131,8 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
   auto start_of = [&](int a) -> int64_t { return SMALL ? s_astart[a] : a_start[a]; };
   // A token's adapter, -1 where the plan leaves the token out, and the adapter's usable rank.  A compensation plan keeps
   // the tokens of adapters without a usable rank: they have no product of their own, but the merged one comes off them.
-  // (Looked up once: inside adapter_of the compiler's code for tables in global memory dropped those tokens all the same.)
-  const bool keep_rankless = merged >= 0 && usable_rank(a_len[merged]) > 0;
+  // (Looked up once, below: inside adapter_of the compiler's code for tables in global memory dropped those tokens all the same.)
+  bool keep_rankless = false;
   auto adapter_of = [&](int64_t a64, int &r) -> int {
     r = 0;
     if (a64 < 0 || a64 >= A || a64 == merged) return -1;
@@ -182,6 +182,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     }
   }
   __syncthreads();
+  if (merged >= 0) keep_rankless = rank_of(merged) > 0;
   for (int i = part * THREADS + tid; i < n_flag_words; i += n_parts * THREADS) plan[off_counters + i] = 0;
 
   // 1. histogram of the tokens per row.  A step of one adapter (most of a prefill batch) is one addition: 64 lanes that add to
@@ -447,16 +448,17 @@ int launch_plan(hipStream_t st, const PlanSet &set, int n_plans, const PlanLayou
   const bool few = L.T <= 1024 && A <= 512;
   // Parts and rows.  One compute unit is bound by the instructions of the scatter and by its own stores (126 KB of plan for 5400
   // tokens); counting all tokens again in every part is cheap beside that.  us a build, back to back in a graph, 1 part / several:
-  // 300 tokens over 300 adapters 9.1 / 8.3, 512 over 32 6.7 / 6.4, 1024 over 128 9.4 / 7.5 (4 parts; 256 tokens 5.7 / 6.4), 5401 over 32 (8
-  // parts) 15.2 / 10.9, 6749 over 24 17.0 / 11.3, 20000 over 128 38.6 / 20.3; 512 to 2048 adapters, where counting them again costs more:
+  // 300 tokens over 300 adapters 9.1 / 8.3, 512 over 32 6.7 / 6.4 (behind other kernels 6.2 / 6.2, over 4 5.7 / 6.0), 1024 over 128 9.4 / 7.5
+  // (4 parts; 256 tokens 5.7 / 6.4), 5401 over 32 (8 parts) 15.2 / 10.9, 6749 over 24 17.0 / 11.3, 20000 over 128 38.6 / 20.3; 512 to 2048 adapters, where counting them again costs more:
   // 800 tokens over 600 8.4 / 8.8, 1000 9.8 / 9.4.  16 rows instead of 32: 1500 tokens 8.4 / 8.8, 5401 11.3 / 10.9, 8192 14.0 / 13.0.
   // (4 or 16 parts are equal to 8; 512 threads 0.5 us slower from 5000 tokens.)
   // The code of one part (PARTS off) against that of several, both with one part: one token 5.1 / 5.4, 64 over 600 adapters 7.6 / 8.3, over
   // 2000 9.0 / 10.8, over 4000 12.9 / 15.5; above 2048 adapters 600 tokens 20.5 / 20.5, 4000 64.6 / 58.0.
   int parts = 1, rows = PLAN_WAVES;
   if (few) {
-    rows = L.T > 256 ? 8 : PLAN_THREADS_SMALL / 64;
-    parts = L.T > 256 ? 4 : 1;
+    const bool several = L.T > 512 || (L.T > 256 && A > 32);
+    rows = several ? 8 : PLAN_THREADS_SMALL / 64;
+    parts = several ? 4 : 1;
   } else if (A <= PLAN_SMALL_A && L.T > 900) {
     rows = L.T > 4096 ? 32 : 16;
     parts = 8;
@@ -469,7 +471,7 @@ int launch_plan(hipStream_t st, const PlanSet &set, int n_plans, const PlanLayou
                      a_len, (int)L.T, A, n_slots, set.bm_s[0], set.bm_e[0], W, set, L.off_perm, L.off_padapter, L.off_prank,                \
                      L.off_tiles_s, L.off_tiles_e, L.off_counters, L.off_scratch,                                 \
                      (int)(L.off_scratch - L.off_counters), merged)
-  if (few && parts == 1) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL, false);
+  if (few && L.T <= 256) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL, false);
   else if (few) MLORA_LAUNCH_PLAN(true, PLAN_THREADS_SMALL, true);
   else if (small_a && parts > 1) MLORA_LAUNCH_PLAN(true, PLAN_THREADS, true);
   else if (small_a) MLORA_LAUNCH_PLAN(true, PLAN_THREADS, false);
