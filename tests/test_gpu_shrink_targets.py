@@ -76,3 +76,39 @@ def test_both_sides_of_the_rule(dev, T, h_in, ksplit, rank, n, together):
     for z in range(n):
         plan.apply(ys[n + z], x, pool.key_buffer, pool.value_buffer, *idx, z, pool.a_scaling)
         assert ys[z].any() and torch.equal(ys[z], ys[n + z]), z
+
+
+@pytest.mark.parametrize("T,ranks", [(5401, (16, 8, 8, 16)), (5402, (32, 8, 24, 16)), (5403, (64, 8, 40, 16)), (5901, (128, 8, 72, 40))])
+@pytest.mark.parametrize("h_in,ksplit", [(1032, 4), (1024, 2), (4104, 4), (520, 3)])
+@pytest.mark.parametrize("n", [2, 3])
+def test_together(dev, T, ranks, h_in, ksplit, n):
+    """Calls that do go together: adapters of several rank classes with short last tiles, K remainders, rank rows outside the index
+    or the pool, against separate calls (same bits) and the oracle."""
+    T = T if ksplit == 4 else T * 4 // ksplit
+    A, R = len(ranks), max(ranks)
+    assert _lib.lib().mlora_targets_together(T, A, R, 128, ksplit, n) == 1
+    g = torch.Generator().manual_seed(T + h_in)
+    dtype = torch.bfloat16 if T % 2 else torch.float16
+    lens = torch.tensor([T // 3 + 1, T // 6 + 127, 129, 0])
+    lens[3] = T - int(lens.sum()) - 7
+    ids = torch.cat([torch.repeat_interleave(torch.arange(A), lens), torch.full((7,), -1)])[torch.randperm(T, generator=g)]
+    pool = W.make_pool(list(ranks), h_in, 72, dtype, g, True, std=0.05, heads=1, extra_rows=1)
+    spare = pool.key_buffer.shape[0] - 1   # zeros for the oracle, out of the pool's bounds for the op
+    pool.key_buffer[-1], pool.value_buffer[-1] = 0, 0
+    pool.a_loc[pool.a_loc == spare] = 0
+    seen = pool.a_loc.clone()
+    for slot in range(3):
+        at = int(pool.a_start[slot]) + ranks[slot] * slot + 2 * slot + 1
+        seen[at], pool.a_loc[at] = spare, (-1, spare + 1, 1 << 40)[slot]
+    x = torch.randn(T, h_in, generator=g).to(dtype)
+    y0 = torch.randn(T, 72, generator=g).to(dtype)
+    pd, xd = pool.to(dev), x.to(dev)
+    idx = (pd.a_start, pd.a_len, pd.a_loc)
+    plan = LoraPlan(ids.to(dev), *idx[:2], R, hidden=h_in, bm_shrink=128, bm_expand=32, ksplit=ksplit, reduce_in_expand=False, one_launch=False)
+    ys = [y0.to(dev) for _ in range(2 * n)]
+    plan.apply_multi(ys[:n], xd, pd.key_buffer, pd.value_buffer, *idx, list(range(n)), pd.a_scaling)
+    for z in range(n):
+        plan.apply(ys[n + z], xd, pd.key_buffer, pd.value_buffer, *idx, z, pd.a_scaling)
+        assert torch.equal(ys[z], ys[n + z]), z
+    want = O.lora_op(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, seen, ids, n - 1, pool.a_scaling)
+    assert_parity(ys[n - 1].cpu(), want, f"{T} {h_in} {ksplit} {ranks}")

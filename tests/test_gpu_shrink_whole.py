@@ -1,7 +1,6 @@
-"""Shrinks of one target over a few thousand tokens, all of K in one workgroup of eight waves: at the edges of the rule that
-takes them (4480 tokens; one round of 32-token pieces, or of 64-token ones up to rank 16; 5120 wide), of the pieces and of K,
+"""Shrinks of one target over a few thousand tokens, all of K in one workgroup of eight waves: at the edges of the pieces and of K,
 through every entry point that writes such a result and over plans of other tile heights, against the oracle at the
-tolerance of the whole op."""
+tolerance of the whole op; then on both sides of every bound of the rule that takes them."""
 import pytest
 import torch
 
@@ -20,14 +19,14 @@ pytestmark = pytest.mark.gpu
     (4800, 8, (8, 8)),
     (5001, 1032, (32, 8, 24)),
     (4700, 5120, (16, 8)),
-    (6080, 3080, (32, 16)),         # 191 pieces with rank above 16 and more than 3072 wide: the table's; 192
+    (6080, 3080, (32, 16)),         # too few pieces with rank above 16 and more than 3072 wide: the table's tiles
     (6112, 3080, (32, 16)),
     (6000, 584, (64, 40, 8, 16, 128)),
     (4600, 1096, (32,) * 100),      # a tail per adapter
     (8191, 264, (16,)),             # the last of one round of 32-token pieces
-    (12000, 264, (16, 8, 8)),       # 64-token pieces
+    (12000, 264, (16, 8, 8)),       # past it and too narrow for 64-token ones: the table's tiles
     (16383, 136, (8,)),
-    (16448, 136, (8,)),             # past both rounds: the table's tiles
+    (16448, 136, (8,)),
 ])
 def test_entry_points(dev, T, h_in, ranks):
     from valora_amd.atmm_ops import dispatch_bgmv as dispatch_sgmm, shrink_accumulate
