@@ -1,0 +1,82 @@
+"""Launches that write y on to memory at once (from 2 MB of y on, 3 MB where the op is one launch) against the same tokens in
+batches below that size: the same bits, for tiles of odd and even token counts, widths that end inside a line and inside a
+chunk, tokens without an adapter, and nothing written beside the rows."""
+import pytest
+import torch
+
+from oracle import lora_oracle as O
+from valora_amd import workloads as W
+from valora_amd.merge import DeLoraPlan
+from valora_amd.plan import LoraPlan
+
+from _util import REL_L2
+
+pytestmark = pytest.mark.gpu
+H_IN = 264
+
+
+def _case(T, h_out, ranks, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    pool = W.make_pool(ranks, H_IN, h_out, dtype, g, True, n_slots=2, std=0.05, scalings=[0.5 + 0.25 * i for i in range(len(ranks))],
+                       heads=1, extra_rows=2)
+    ids = torch.randint(-1, len(ranks), (T,), generator=g)
+    x, y = torch.randn(T, H_IN, generator=g).to(dtype), torch.randn(T, h_out, generator=g).to(dtype)
+    return pool, ids, x, y
+
+
+def _framed(y):
+    frame = torch.full((y.size(0) + 2, y.size(1)), 7.0, dtype=y.dtype, device=y.device)
+    frame[1:-1] = y
+    return frame
+
+
+def _both(dev, make_plan, call, pool, ids, x, y0, least):
+    """The whole batch, and its two halves; the former writes through, the latter do not."""
+    T, h_out = y0.shape
+    assert T * h_out * 2 >= least > (T + 1) // 2 * h_out * 2
+    whole, parts = _framed(y0), _framed(y0)
+    call(make_plan(ids), whole[1:-1], x)
+    for a, b in ((0, T // 2), (T // 2, T)):
+        call(make_plan(ids[a:b].contiguous()), parts[1 + a:1 + b], x[a:b])
+    assert torch.equal(whole, parts)
+    assert bool((whole[0] == 7).all() and (whole[-1] == 7).all())
+    none = ids < 0
+    assert torch.equal(whole[1:-1][none], y0[none])
+    return whole[1:-1]
+
+
+@pytest.mark.parametrize("h_out", [1640, 4104, 4184])
+@pytest.mark.parametrize("ranks", [[16, 8], [32, 24, 8], [64, 40, 8], [128, 72, 16]])
+@pytest.mark.parametrize("bm,one", [(16, False), (48, False), (16, True)])
+def test_same_bits_as_smaller_batches(dev, h_out, ranks, bm, one):
+    if one and max(ranks) > 64:
+        pytest.skip("the one-launch op takes ranks up to 64")
+    least = (3 if one and max(ranks) <= 32 else 2) << 20
+    T = least // (2 * h_out) + 3
+    dtype = torch.bfloat16 if h_out == 4104 else torch.float16
+    print(T, h_out, ranks, bm, one, flush=True)
+    pool, ids, x, y0 = _case(T, h_out, ranks, dtype, h_out + ranks[0])
+    p = pool.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    got = _both(dev, lambda i: LoraPlan(i, *idx[:2], max(ranks), n_slots=2, hidden=H_IN, bm_shrink=16, bm_expand=bm, one_launch=one, ksplit=2),
+                lambda plan, y, xs: plan.apply(y, xs, p.key_buffer, p.value_buffer, *idx, 1, p.a_scaling),
+                p, ids.to(dev), x.to(dev), y0.to(dev), least)
+    want = O.lora_op(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1, pool.a_scaling, n_slots=2)
+    # one rounding of y, and one of v on its way through B
+    assert O.rel_l2(got.cpu(), want) <= (REL_L2 if dtype is torch.float16 else 8 * REL_L2)
+
+
+@pytest.mark.parametrize("ranks", [[16, 8], [32, 24, 8], [64, 40, 8], [128, 72, 16]])
+@pytest.mark.parametrize("bm", [16, 48])
+def test_compensation_same_bits_as_smaller_batches(dev, ranks, bm):
+    h_out = 4104
+    T = (2 << 20) // (2 * h_out) + 3
+    pool, ids, x, y0 = _case(T, h_out, ranks, torch.float16, ranks[0] + bm)
+    p = pool.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    got = _both(dev, lambda i: DeLoraPlan(i, 1, *idx[:2], max(ranks), H_IN, n_slots=2, bm_shrink=16, bm_expand=bm, ksplit=2),
+                lambda plan, y, xs: plan.apply(y, xs, p.key_buffer, p.value_buffer, *idx, 1, p.a_scaling),
+                p, ids.to(dev), x.to(dev), y0.to(dev), 2 << 20)
+    want = O.delora_compensate(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1, 1, pool.a_scaling,
+                               n_slots=2)
+    assert O.rel_l2(got.cpu(), want) <= REL_L2

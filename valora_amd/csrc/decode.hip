@@ -122,11 +122,12 @@ __device__ __forceinline__ ItemId item_of(int n_producers, int n_consumers, int 
 // output by token (no turn through LDS), its chunk loads not behind its B loads, and the shrink's loads without masks, cold layers,
 // rank 16, before / now: one target of one token 6.4 / 5.7 us, of 256 9.6 / 9.6, 11008 wide 15.1 / 14.1; q+k+v of 256 21.2 / 19.9, of
 // 512 23.7 / 22.1.
+// THROUGH: y is written through (expand_core.h; a form of its own: the flag would take a scalar register of which there are none left).
 // The leading scalar parameters repeat what the first dependent loads need (the tile records, the `done` words, the
 // id layout): the library is built with kernel-argument preloading, which hands the first 8 dwords of the
 // argument list to the wave in registers at launch, so the tile record can be requested without waiting for a load
 // of the argument block first (0.35 us of a 10.3 us op).
-template <typename T, int NB, bool WIDE>
+template <typename T, int NB, bool WIDE, bool THROUGH>
 __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_base, uint32_t *done_base, int h_n_producers,
                                                         int h_n_consumers, int h_n_tiles, int h_shrink_ids,
                                                         DecodeArgs a) {
@@ -245,7 +246,7 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
   SmallY<KB> yy[DEC_CH];
   u32x4 raw[DEC_CH][SmallB<KB>::LOADS];
 #pragma unroll
-  for (int c = 0; c < DEC_CH; ++c) small_load_y(yy[c], as_global(y), tok, on, o_wave + c * 256u, (uint32_t)h_out, lane);
+  for (int c = 0; c < DEC_CH; ++c) small_load_y(yy[c], as_global(y), tok, o_wave + c * 256u, (uint32_t)h_out, lane);
   requested();
 #pragma unroll
   for (int c = 0; c < DEC_CH; ++c) small_load_b<KB, WIDE>(pool, lane, rows[c], raw[c]);
@@ -304,7 +305,7 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
     f32x4 acc[4];
     small_product<T, KB>(raw[c], vfrag, rk, lane, acc);
     small_add<T, KB>(yy[c], acc, scale);
-    small_store_y(yy[c]);
+    small_store_y(yy[c], lane, cnt, THROUGH);
   }
   // the tile's last expand item tops the tile's `done` word up to the launch's weight
   if (tid == 0 && item == h_n_consumers - 1) add_device(done_base + tile_idx, DECODE_LAUNCH_WEIGHT - (uint32_t)n_producers);
@@ -312,13 +313,18 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
 
 template <typename T>
 int launch_decode_t(hipStream_t st, const DecodeArgs &a, int nb, dim3 grid, int shrink_ids) {
-#define MLORA_DECODE(NB, WIDE)                                                                                                  \
-  hipLaunchKernelGGL((decode_kernel<T, NB, WIDE>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, \
+  const bool through = write_through(a.e, THROUGH_BYTES_ONE_LAUNCH);
+#define MLORA_DECODE_FORM(NB, WIDE, THROUGH)                                                                                    \
+  hipLaunchKernelGGL((decode_kernel<T, NB, WIDE, THROUGH>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, \
                      a.n_tiles, shrink_ids, a)
-  if (nb == 1) MLORA_DECODE(1, false);
-  else if (a.e.h_out >= SMALL_WIDE) MLORA_DECODE(2, true);
-  else MLORA_DECODE(2, false);
+#define MLORA_DECODE(NB, WIDE)                  \
+  if (through) MLORA_DECODE_FORM(NB, WIDE, true); \
+  else MLORA_DECODE_FORM(NB, WIDE, false)
+  if (nb == 1) { MLORA_DECODE(1, false); }
+  else if (a.e.h_out >= SMALL_WIDE) { MLORA_DECODE(2, true); }
+  else { MLORA_DECODE(2, false); }
 #undef MLORA_DECODE
+#undef MLORA_DECODE_FORM
   return check_launch("decode_kernel");
 }
 

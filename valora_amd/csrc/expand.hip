@@ -46,6 +46,8 @@ constexpr int expand_min_waves(int kb, bool partial, bool comp) {
 // 108.8 / 99.4; 5401 tokens over ranks 8-64 24.8 / 22.6, 57.9 / 54.5, 93.0 / 90.9; 10000 tokens over 8 adapters of rank 128, shrink and
 // expand 106 / 92.  (Of the 109 us, B and v together were 29, v alone 8.  One more or one less waves' worth of registers spills or gains
 // nothing; 16 instead of 8 staged tokens, 8.7 KB more LDS, 1 % slower.)
+// y written through instead of left dirty in the L2s for the end of the kernel: 5401 tokens over ranks 8-64, one target of 4096
+// columns 25.7 / 23.1, three 54.6 / 51.9, two of 11008 93.3 / 90.9 (with non-temporal stores the same as with plain ones).
 // COMP: the compensation of a request whose base weights hold another adapter (csrc/api.hip, mlora_lora_compensate):
 // y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), where v' is the "target" 1 matrix of the same positions:
 // both products in one pass over y.
@@ -67,12 +69,13 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
   int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
+  int through = may_write_through(KB, WIDE) ? p.through : 0;
   uint16_t *y = p.ys[z];
   const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
   int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
   float inv_h_out = p.inv_h_out;
   asm volatile("" : "+s"(ad), "+s"(r), "+s"(pos0), "+s"(cnt), "+s"(astart), "+s"(slot), "+s"(kmax), "+s"(w_rows), "+s"(v_by_pos),
-                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out));
+                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out), "+s"(through));
   if (COMP) cnt = abs(cnt);                  // (negative: no usable rank of its own, r = 0)
   if (cnt <= 0) return;                      // records past the last tile are zero
   y = as_global(y);
@@ -232,7 +235,10 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 #pragma unroll
           for (int i = 0; i < 8; ++i) f[i] += sc * srow[i];
           yv[b][h] = pack8<T>(f);
-          if (last && ocol_ok && row0 + rr0 + 8 * h < cnt) store16(yp[b][h], yv[b][h]);
+          if (last && ocol_ok && row0 + rr0 + 8 * h < cnt) {
+            if (may_write_through(KB, WIDE) && through) store16_through(yp[b][h], yv[b][h]);
+            else store16(yp[b][h], yv[b][h]);
+          }
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           __builtin_amdgcn_wave_barrier();
         }
@@ -265,12 +271,13 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
   int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
+  int through = may_write_through(KB, WIDE) ? p.through : 0;
   uint16_t *y = p.ys[z];
   const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
   int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
   float inv_h_out = p.inv_h_out;
   asm volatile("" : "+s"(ad), "+s"(r), "+s"(pos0), "+s"(cnt), "+s"(astart), "+s"(slot), "+s"(kmax), "+s"(w_rows), "+s"(v_by_pos),
-                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out));
+                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out), "+s"(through));
   if (COMP) cnt = abs(cnt);                  // (negative: no usable rank of its own, r = 0)
   if (cnt <= 0) return;                      // records past the last tile are zero
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -314,7 +321,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   else
     load_v(v + z * v_tstride, pool.rk, vfrag);
   SmallY<KB> yy;
-  small_load_y(yy, y, tok, on, o_wave, (uint32_t)h_out, lane);
+  small_load_y(yy, y, tok, o_wave, (uint32_t)h_out, lane);
   requested();
   u32x4 raw[SmallB<KB>::LOADS];
   small_load_b<KB, WIDE>(pool, lane, rows, raw);
@@ -335,7 +342,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
     small_product<T, KB>(raw, vfrag, pool.rk, lane, acc);
     small_add<T, KB>(yy, acc, scale);
   }
-  small_store_y(yy);
+  small_store_y(yy, lane, cnt, may_write_through(KB, WIDE) && through);
 }
 
 template <typename T, int KB>
@@ -402,8 +409,13 @@ int launch_expand_t(hipStream_t st, const ExpandArgs &a, int max_rank, int bm, i
 
 }  // namespace
 
-int launch_expand(hipStream_t st, const ExpandArgs &a, int max_rank, int64_t grid_tiles, int bm_expand, mlora_dtype dt) {
+int launch_expand(hipStream_t st, const ExpandArgs &args, int max_rank, int64_t grid_tiles, int bm_expand, mlora_dtype dt) {
   if (grid_tiles <= 0) return MLORA_OK;
+  ExpandArgs a = args;
+  // (ranks above 64 in tiles of a few tokens read so much more than they write that it only costs: 512 tokens over 128 adapters of
+  // rank 128, a pass of 8 calls 837 / 846 us; from about five a tile on 0.97 to 1.00)
+  const bool mostly_reads = bm_expand == 16 && max_rank > 64 && a.T < 5 * grid_tiles;
+  a.through = !mostly_reads && write_through(a, THROUGH_BYTES);
   if (bm_expand == 16)
     return dt == MLORA_F16 ? launch_small_t<_Float16>(st, a, max_rank, grid_tiles) : launch_small_t<__bf16>(st, a, max_rank, grid_tiles);
   return dt == MLORA_F16 ? launch_expand_t<_Float16>(st, a, max_rank, bm_expand, grid_tiles)

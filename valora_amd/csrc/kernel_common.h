@@ -23,6 +23,13 @@ __device__ __forceinline__ To as(const From &v) {
 // One global_load_dwordx4 / global_store_dwordx4.  Addresses must be 16-byte aligned.
 __device__ __forceinline__ u32x4 load16(const uint16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
 __device__ __forceinline__ void store16(uint16_t *p, u32x4 v) { *reinterpret_cast<u32x4 *>(p) = v; }
+// The same, on to memory at once instead of leaving a dirty line in the XCD's L2.  The L2s write their dirty lines back when a
+// kernel ends, with nothing else to do: 2.4 us of a launch that updates tens of MB.  Pays for whole 128-byte lines (pieces of
+// 16 bytes are written to memory one by one); csrc/expand_core.h has the rule.
+__device__ __forceinline__ void store16_through(uint16_t *p, u32x4 v) {
+  typedef __attribute__((address_space(1))) u32x4 *GP;
+  __builtin_amdgcn_global_store_b128((GP)(uintptr_t)p, v, "agent");
+}
 
 // A pointer that went through an inline asm operand has lost what the compiler knew about it; telling it again that
 // the memory is global keeps its loads and stores on the global path (flat accesses count against two wait counters)

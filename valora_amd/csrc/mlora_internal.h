@@ -143,6 +143,7 @@ struct ExpandArgs {
   int T, h_out, kmax, n_ochunks;
   float inv_h_out;            // 1 / h_out
   int compensate;             // every tile takes its own adapter's product minus the merged adapter's (one target)
+  int through;                // y goes on to memory at once (set by the launchers, csrc/expand_core.h)
 };
 
 
