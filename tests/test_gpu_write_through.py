@@ -46,11 +46,9 @@ def _both(dev, make_plan, call, pool, ids, x, y0, least):
 
 
 @pytest.mark.parametrize("h_out", [1640, 4104, 4184])
-@pytest.mark.parametrize("ranks", [[16, 8], [32, 24, 8], [64, 40, 8], [128, 72, 16]])
-@pytest.mark.parametrize("bm,one", [(16, False), (48, False), (16, True)])
+@pytest.mark.parametrize("ranks,bm,one", [(r, bm, one) for r in ([16, 8], [32, 24, 8], [64, 40, 8], [128, 72, 16])
+                                          for bm, one in ((16, False), (48, False), (16, True)) if not one or max(r) <= 64])
 def test_same_bits_as_smaller_batches(dev, h_out, ranks, bm, one):
-    if one and max(ranks) > 64:
-        pytest.skip("the one-launch op takes ranks up to 64")
     least = (3 if one and max(ranks) <= 32 else 2) << 20
     T = least // (2 * h_out) + 3
     dtype = torch.bfloat16 if h_out == 4104 else torch.float16

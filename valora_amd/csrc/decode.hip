@@ -246,7 +246,7 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
   SmallY<KB> yy[DEC_CH];
   u32x4 raw[DEC_CH][SmallB<KB>::LOADS];
 #pragma unroll
-  for (int c = 0; c < DEC_CH; ++c) small_load_y(yy[c], as_global(y), tok, o_wave + c * 256u, (uint32_t)h_out, lane);
+  for (int c = 0; c < DEC_CH; ++c) small_load_y(yy[c], as_global(y), tok, on, o_wave + c * 256u, (uint32_t)h_out, lane);
   requested();
 #pragma unroll
   for (int c = 0; c < DEC_CH; ++c) small_load_b<KB, WIDE>(pool, lane, rows[c], raw[c]);
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
     f32x4 acc[4];
     small_product<T, KB>(raw[c], vfrag, rk, lane, acc);
     small_add<T, KB>(yy[c], acc, scale);
-    small_store_y(yy[c], lane, cnt, THROUGH);
+    small_store_y(yy[c], lane, cnt, o_wave + c * 256u, (uint32_t)h_out, THROUGH);
   }
   // the tile's last expand item tops the tile's `done` word up to the launch's weight
   if (tid == 0 && item == h_n_consumers - 1) add_device(done_base + tile_idx, DECODE_LAUNCH_WEIGHT - (uint32_t)n_producers);
@@ -313,7 +313,8 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
 
 template <typename T>
 int launch_decode_t(hipStream_t st, const DecodeArgs &a, int nb, dim3 grid, int shrink_ids) {
-  const bool through = write_through(a.e, THROUGH_BYTES_ONE_LAUNCH);
+  // (with a few tokens a tile an item's y is too little to gain: 256 tokens over 64 adapters, a pass of 32 layers 928 / 931 us)
+  const bool through = a.s.T >= 5 * a.n_tiles && write_through(a.e, THROUGH_BYTES_ONE_LAUNCH);
 #define MLORA_DECODE_FORM(NB, WIDE, THROUGH)                                                                                    \
   hipLaunchKernelGGL((decode_kernel<T, NB, WIDE, THROUGH>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, \
                      a.n_tiles, shrink_ids, a)

@@ -69,7 +69,8 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
   int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
-  int through = may_write_through(KB, WIDE) ? p.through : 0;
+  constexpr bool MAY_THROUGH = KB < 4 || WIDE;
+  int through = MAY_THROUGH ? p.through : 0;
   uint16_t *y = p.ys[z];
   const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
   int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
@@ -236,7 +237,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
           for (int i = 0; i < 8; ++i) f[i] += sc * srow[i];
           yv[b][h] = pack8<T>(f);
           if (last && ocol_ok && row0 + rr0 + 8 * h < cnt) {
-            if (may_write_through(KB, WIDE) && through) store16_through(yp[b][h], yv[b][h]);
+            if (MAY_THROUGH && through) store16_through(yp[b][h], yv[b][h]);
             else store16(yp[b][h], yv[b][h]);
           }
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
   int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
-  int through = may_write_through(KB, WIDE) ? p.through : 0;
+  int through = KB < 4 ? p.through : 0;
   uint16_t *y = p.ys[z];
   const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
   int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   else
     load_v(v + z * v_tstride, pool.rk, vfrag);
   SmallY<KB> yy;
-  small_load_y(yy, y, tok, o_wave, (uint32_t)h_out, lane);
+  small_load_y(yy, y, tok, on, o_wave, (uint32_t)h_out, lane);
   requested();
   u32x4 raw[SmallB<KB>::LOADS];
   small_load_b<KB, WIDE>(pool, lane, rows, raw);
@@ -342,7 +343,7 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
     small_product<T, KB>(raw, vfrag, pool.rk, lane, acc);
     small_add<T, KB>(yy, acc, scale);
   }
-  small_store_y(yy, lane, cnt, may_write_through(KB, WIDE) && through);
+  small_store_y(yy, lane, cnt, o_wave, (uint32_t)h_out, KB < 4 && through);
 }
 
 template <typename T, int KB>
@@ -412,10 +413,7 @@ int launch_expand_t(hipStream_t st, const ExpandArgs &a, int max_rank, int bm, i
 int launch_expand(hipStream_t st, const ExpandArgs &args, int max_rank, int64_t grid_tiles, int bm_expand, mlora_dtype dt) {
   if (grid_tiles <= 0) return MLORA_OK;
   ExpandArgs a = args;
-  // (ranks above 64 in tiles of a few tokens read so much more than they write that it only costs: 512 tokens over 128 adapters of
-  // rank 128, a pass of 8 calls 837 / 846 us; from about five a tile on 0.97 to 1.00)
-  const bool mostly_reads = bm_expand == 16 && max_rank > 64 && a.T < 5 * grid_tiles;
-  a.through = !mostly_reads && write_through(a, THROUGH_BYTES);
+  a.through = write_through(a, THROUGH_BYTES);
   if (bm_expand == 16)
     return dt == MLORA_F16 ? launch_small_t<_Float16>(st, a, max_rank, grid_tiles) : launch_small_t<__bf16>(st, a, max_rank, grid_tiles);
   return dt == MLORA_F16 ? launch_expand_t<_Float16>(st, a, max_rank, bm_expand, grid_tiles)

@@ -245,30 +245,30 @@ __device__ __forceinline__ void small_v_partials(const float *tile, uint32_t row
   }
 }
 // Bytes of y from which a launch writes it through (store16_through).  Cold layers, whole op, 140 shapes: tall tiles (4.8 MB of y and more)
-// 0.95 to 0.99 of the time, 1.01 at worst; 16-token tiles of two launches 0.95 to 0.99 from 2.5 MB on and 0.98 to 1.02 at 1 to 2 MB; one
+// 0.95 to 0.99 of the time, 1.01 at worst; 16-token tiles of two launches up to rank 64 0.95 to 0.99 from 2.5 MB on, 0.98 to 1.02 at 1 to 2 MB; one
 // launch 0.91 to 0.98 from 4.7 MB on (1201 tokens of rank 16, two targets of 8192 columns 26.9 / 24.7 us), 1.00 at 1 to 2.5 MB, and 1.05 for
 // a few tokens, where the way to memory is longer than the write-back of what little there is.
 constexpr int64_t THROUGH_BYTES = (int64_t)2 << 20, THROUGH_BYTES_ONE_LAUNCH = (int64_t)3 << 20;
 inline int write_through(const ExpandArgs &a, int64_t least) { return (int64_t)a.T * a.h_out * a.n_targets * 2 >= least; }
-// (Ranks above 64 with outputs narrower than SMALL_WIDE have no scalar register to spare for the choice.)
-constexpr bool may_write_through(int kb, bool wide) { return kb < 4 || wide; }
+// Not in 16-token tiles above rank 64, which read much more than they write (512 tokens over 128 adapters of rank 128, q+k+v 79.2 / 80.4
+// us, and 80.0 with the choice alone), nor above rank 64 with outputs narrower than SMALL_WIDE (no scalar register is left for the choice).
 
 // The lane's outputs of y: 16 from o_wave + 16 * (lane / 16) on, in two 16-byte halves.
 template <int KB>
 struct SmallY {
   u32x4 v[2];
   uint16_t *p;
-  bool col[2];   // whether there are such columns
+  bool ok[2];
 };
 template <int KB>
-__device__ __forceinline__ void small_load_y(SmallY<KB> &s, uint16_t *y, int tok, uint32_t o_wave, uint32_t h_out, int lane) {
+__device__ __forceinline__ void small_load_y(SmallY<KB> &s, uint16_t *y, int tok, bool on, uint32_t o_wave, uint32_t h_out, int lane) {
   const uint32_t o = o_wave + (uint32_t)(lane >> 4) * (KB ? 16u : 8u);
   constexpr uint32_t H = KB ? 8u : 32u;
   s.p = reinterpret_cast<uint16_t *>(reinterpret_cast<char *>(y) + (uint64_t)(uint32_t)tok * (h_out * 2u)) + o;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    s.col[h] = o + H * h < h_out;
-    s.v[h] = load16(s.col[h] ? s.p + h * (KB ? 8 : 32) : y);   // (lanes without a token read the first one's row)
+    s.ok[h] = on && o + H * h < h_out;
+    s.v[h] = load16(o + H * h < h_out ? s.p + h * (KB ? 8 : 32) : y);   // (lanes without a token read the first one's row)
   }
 }
 template <typename T, int KB>
@@ -288,12 +288,12 @@ __device__ __forceinline__ uint32_t lane_pair(uint32_t x) { return (uint32_t)__b
 // of one half writes pieces of lines.  That is all the same to the L2; on their way to memory the lanes of a pair, two tokens of the
 // same columns, exchange a half first: every store then writes whole lines of one token.
 template <int KB>
-__device__ __forceinline__ void small_store_y(const SmallY<KB> &s, int lane, int cnt, bool through) {
+__device__ __forceinline__ void small_store_y(const SmallY<KB> &s, int lane, int cnt, uint32_t o_wave, uint32_t h_out, bool through) {
   constexpr int H = KB ? 8 : 32;
   if (!through) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
-      if (s.col[h] && (lane & 15) < cnt) store16(s.p + h * H, s.v[h]);
+      if (s.ok[h]) store16(s.p + h * H, s.v[h]);
     return;
   }
   const bool odd = lane & 1;
@@ -305,7 +305,7 @@ __device__ __forceinline__ void small_store_y(const SmallY<KB> &s, int lane, int
   const uint64_t other = (uint64_t)lane_pair((uint32_t)own) | (uint64_t)lane_pair((uint32_t)(own >> 32)) << 32;
   uint16_t *const even_row = reinterpret_cast<uint16_t *>(odd ? other : own) + (odd ? H : 0);
   uint16_t *const odd_row = reinterpret_cast<uint16_t *>(odd ? own : other) + (odd ? H : 0);
-  const bool col = odd ? s.col[1] : s.col[0];
+  const bool col = o_wave + (uint32_t)((lane >> 4) * (KB ? 16 : 8) + (odd ? H : 0)) < h_out;
   const int m = lane & 15;
   if (col && (m & ~1) < cnt) store16_through(even_row, odd ? got : s.v[0]);
   if (col && (m | 1) < cnt) store16_through(odd_row, odd ? s.v[1] : got);
