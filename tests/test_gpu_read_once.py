@@ -1,0 +1,57 @@
+"""Launches whose operands are read as lines that nobody reads again (the rules stand beside the kernels) against the same tokens
+in calls that the rules leave out: the same bits, and the oracle's result."""
+import pytest
+import torch
+
+from oracle import lora_oracle as O
+from valora_amd import workloads as W
+from valora_amd.plan import LoraPlan
+
+from _util import REL_L2
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(T, n, rank, h_in, h_out, dtype, seed):
+    g = torch.Generator().manual_seed(seed)
+    ranks = [max(8, rank - 8 * (i % 3)) for i in range(n)]
+    pool = W.make_pool(ranks, h_in, h_out, dtype, g, True, n_slots=2, std=0.05, scalings=[0.5 + 0.25 * (i % 4) for i in range(n)],
+                       heads=1, extra_rows=2)
+    ids = torch.randint(-1, n, (T,), generator=g)
+    return pool, ids, torch.randn(T, h_in, generator=g).to(dtype), torch.randn(T, h_out, generator=g).to(dtype)
+
+
+def _oracle(pool, ids, x, y):
+    return O.lora_op(y, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1, pool.a_scaling, n_slots=2)
+
+
+def _bound(dtype):
+    return REL_L2 if dtype is torch.float16 else 8 * REL_L2   # one rounding of y, and one of v on its way through B
+
+
+@pytest.mark.parametrize("rank,one,ksplit", [(r, one, k) for r in (16, 32, 64, 128) for one in (False, True) for k in (1, 4)
+                                             if not one or (r <= 32 and k > 1)])
+@pytest.mark.parametrize("odd", [0, 64, -128])   # K ranges that are whole batches of steps, or end in the middle of one
+def test_rows_of_a_in_small_tiles(dev, rank, one, ksplit, odd):
+    """4 MB of A and more in the whole batch, less in each half."""
+    n, T = 40, 43
+    h_in = 65536 // rank + odd
+    dtype = torch.bfloat16 if odd else torch.float16
+    print(rank, one, ksplit, h_in, flush=True)
+    rp = rank
+    assert ((T + 15) // 16 + n) * rp * h_in * 2 >= 4 << 20 > ((T + 31) // 32 + (T + 1) // 2) * rp * h_in * 2
+    pool, ids, x, y0 = _case(T, n, rank, h_in, 264, dtype, rank + odd)
+    p, xd = pool.to(dev), x.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+
+    def call(a, b, y):
+        plan = LoraPlan(ids[a:b].to(dev).contiguous(), *idx[:2], rank, n_slots=2, hidden=h_in, bm_shrink=16, bm_expand=16, one_launch=one,
+                        ksplit=ksplit)
+        plan.apply(y, xd[a:b], p.key_buffer, p.value_buffer, *idx, 1, p.a_scaling)
+
+    whole, halves = y0.to(dev), y0.to(dev)
+    call(0, T, whole)
+    call(0, T // 2, halves[: T // 2])
+    call(T // 2, T, halves[T // 2:])
+    assert torch.equal(whole, halves)
+    assert O.rel_l2(whole.cpu(), _oracle(pool, ids, x, y0)) <= _bound(dtype)

@@ -22,6 +22,9 @@ __device__ __forceinline__ To as(const From &v) {
 
 // One global_load_dwordx4 / global_store_dwordx4.  Addresses must be 16-byte aligned.
 __device__ __forceinline__ u32x4 load16(const uint16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
+// The same for what nobody reads again soon: the line is the first to leave the caches.  Only where a wave reads whole lines at once: of a
+// line read piece by piece it costs a second fetch (B of the expand: 512 tokens over 128 adapters of rank 128, a pass 839 / 912 us).
+__device__ __forceinline__ u32x4 load16_once(const uint16_t *p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p)); }
 __device__ __forceinline__ void store16(uint16_t *p, u32x4 v) { *reinterpret_cast<u32x4 *>(p) = v; }
 // The same, on to memory at once instead of leaving a dirty line in the XCD's L2.  The L2s write their dirty lines back when a
 // kernel ends, with nothing else to do: 2.4 us of a launch that updates tens of MB.  Pays for whole 128-byte lines (pieces of

@@ -131,7 +131,7 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
 // spill 4 and 28 registers; three / two: 4000 tokens over 32 adapters of rank 32, four chunks 12.8 / 11.6 us, eight 12.9 / 11.4; 8000 over
 // 64 of rank 16 18.4 / 16.0, of rank 32 20.6 / 18.7.)
 constexpr int shrink_min_waves(int mb, int nb) { return mb + nb <= 3 ? 4 : nb == 8 ? 3 - mb : mb == 4 ? 2 : 3; }
-template <typename T, int MB, int NB>
+template <typename T, int MB, int NB, bool ONCE = false>
 __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
                                                      int h_n_tiles, ShrinkArgs args_in) {
   int tile_idx, z_idx, s;
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
     on[it] = row[it] < cnt && c4[it] < quarter;
     tok[it] = (p.out_by_token && on[it]) ? perm[pos0 + row[it]] : 0;
   }
-  shrink_tile_to_lds<T, MB, NB>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, kbeg, kend, s_tile);
+  shrink_tile_to_lds<T, MB, NB, shrink_steps(MB + NB), 4, ONCE>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, kbeg, kend, s_tile);
   if (p.ksplit == 1) {
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it)
@@ -725,14 +725,23 @@ int launch_gemm_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
 }
 
 template <typename T, int MB>
-int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
+int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, int max_rank, dim3 grid) {
+  constexpr bool MAY_ONCE = MB == 1;
+  const bool once = MAY_ONCE && !a.compensate && shrink_reads_once(a, a.n_tiles, max_rank);
+#define MLORA_SHRINK_FORM(MBX, NB, ONCE) \
+  hipLaunchKernelGGL((shrink_kernel<T, MBX, NB, ONCE>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a)
+#define MLORA_SHRINK(MBX, NB)                         \
+  if (once) MLORA_SHRINK_FORM(MBX, NB, MAY_ONCE);     \
+  else MLORA_SHRINK_FORM(MBX, NB, false)
   switch (nb) {
-    case 1: hipLaunchKernelGGL((shrink_kernel<T, MB, 1>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
-    case 2: hipLaunchKernelGGL((shrink_kernel<T, MB, 2>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
-    case 4: hipLaunchKernelGGL((shrink_kernel<T, MB, 4>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
-    case 8: hipLaunchKernelGGL((shrink_kernel<T, (MB > 2 ? 2 : MB), 8>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a); break;
+    case 1: MLORA_SHRINK(MB, 1); break;
+    case 2: MLORA_SHRINK(MB, 2); break;
+    case 4: MLORA_SHRINK(MB, 4); break;
+    case 8: MLORA_SHRINK((MB > 2 ? 2 : MB), 8); break;
     default: return fail(MLORA_ERR_NO_KERNEL, "shrink: no kernel for rank blocks=%d", nb);
   }
+#undef MLORA_SHRINK
+#undef MLORA_SHRINK_FORM
   return check_launch("shrink_kernel");
 }
 
@@ -773,11 +782,11 @@ int launch_whole(hipStream_t st, const ShrinkArgs &a, int bm, int nb, int64_t ti
 }
 
 template <typename T>
-int launch_shrink_t(hipStream_t st, const ShrinkArgs &a, int bm, int nb, dim3 grid) {
+int launch_shrink_t(hipStream_t st, const ShrinkArgs &a, int bm, int nb, int max_rank, dim3 grid) {
   switch (bm) {
-    case 16: return launch_shrink_nb<T, 1>(st, a, nb, grid);
-    case 32: return launch_shrink_nb<T, 2>(st, a, nb, grid);
-    case 64: return launch_shrink_nb<T, 4>(st, a, nb, grid);
+    case 16: return launch_shrink_nb<T, 1>(st, a, nb, max_rank, grid);
+    case 32: return launch_shrink_nb<T, 2>(st, a, nb, max_rank, grid);
+    case 64: return launch_shrink_nb<T, 4>(st, a, nb, max_rank, grid);
     case 128: return launch_gemm_nb<T, 2>(st, a, nb, grid);
     case 256: return launch_gemm_nb<T, 4>(st, a, nb, grid);
     default: return fail(MLORA_ERR_NO_KERNEL, "shrink: tile height %d not in {16,32,64,128,256}", bm);
@@ -847,8 +856,8 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   }
   if (a.reduce_here)
     grid = dim3((unsigned)(8 * a.ksplit), (unsigned)a.n_targets, (unsigned)(grid_tiles / 8));   // at most 4096 tokens (csrc/api.hip)
-  return dt == MLORA_F16 ? launch_shrink_t<_Float16>(st, a, bm, nb, grid)
-                         : launch_shrink_t<__bf16>(st, a, bm, nb, grid);
+  return dt == MLORA_F16 ? launch_shrink_t<_Float16>(st, a, bm, nb, max_rank, grid)
+                         : launch_shrink_t<__bf16>(st, a, bm, nb, max_rank, grid);
 }
 
 }  // namespace mlora

@@ -53,11 +53,12 @@ constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1;
 // 16-byte aligned), for shrink_tile_sum to add up (rows = tokens of the tile, columns = rank); every thread of the
 // workgroup must call it, none may still be reading `lds`, and all have passed a barrier when it returns.
 // U: K steps in flight per wave.  The order of the sums does not depend on it.
+// ONCE: the rows of A have no other reader (shrink_reads_once).
 // Bound by the instructions of one wave in a row, and by what a compute unit takes in.  Rows that are not there are a choice of
 // address, not a mask: a mask, four zeroed registers and a branch around each of a batch's 16 loads took 1400 cycles to issue.
 // One target, cold layers, masked / like this: 1 token of rank 16 4.9 / 4.0 us, 256 over 64 adapters 6.7 / 5.7, 200 over 16 of rank 32
 // 7.6 / 6.5, 77 over ranks 8-64 8.8 / 7.9, 256 over 64 of rank 64 11.6 / 10.9, 512 over 128 of rank 128 29.5 / 28.4.
-template <typename T, int MB, int NB, int U = shrink_steps(MB + NB), int WAVES = 4>
+template <typename T, int MB, int NB, int U = shrink_steps(MB + NB), int WAVES = 4, bool ONCE = false>
 __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ x, int h_in, const PoolDev &pool,
                                                    int slot, const int32_t *__restrict__ perm, int r, int pos0,
                                                    int cnt, int astart, int kbeg, int kend,
@@ -176,8 +177,13 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const uint16_t *const src = rp[b][u] + (MANY && b >= MB ? kb0 & step[b < MB ? 0 : b - MB][u] : kb0);
+        if (ONCE && b >= MB) {
 #pragma unroll
-        for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16(src + uu * WAVES * SHRINK_KSTEP);
+          for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16_once(src + uu * WAVES * SHRINK_KSTEP);
+        } else {
+#pragma unroll
+          for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16(src + uu * WAVES * SHRINK_KSTEP);
+        }
       }
     requested();
     use();
@@ -211,6 +217,17 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
 #pragma unroll
     for (int i = 0; i < 4; ++i) dst[(b * 4 + i) * 64 + lane] = acc[b / NB][b % NB][i];
   __syncthreads();
+}
+
+// Whether A's rows are read as lines that nobody reads again (load16_once): few tokens a tile, so that most adapters have one tile; more
+// of A than an L2 holds (one token over 8 adapters, a pass of 64 calls 379 / 398 us with it, 900 tokens over 12 adapters with their
+// compensation 585 / 664); rows of whole lines; and not rank 8 alone, where the lanes of the other eight rows read the last one again (128
+// adapters, 0.993).   Cold layers, without / with, a pass: 512 tokens
+// over 128 adapters of rank 128 864 / 841 us, 256 over 64 of rank 16 928 / 922, 77 over ranks 8-64 617 / 608; 18 batches of 14 to 900
+// tokens 1.024 times as fast in the mean (60 over 16 of rank 64 64.7 / 57.7).
+inline bool shrink_reads_once(const ShrinkArgs &a, int64_t n_tiles, int max_rank) {
+  return max_rank > 8 && a.T < 5 * n_tiles && n_tiles * a.rp * a.h_in * a.n_targets * 2 >= ((int64_t)4 << 20) && !(a.h_in & 63) &&
+         !(reinterpret_cast<uintptr_t>(a.pool.w) & 127u);
 }
 
 }  // namespace mlora
