@@ -249,7 +249,13 @@ __device__ __forceinline__ void small_v_partials(const float *tile, uint32_t row
 // launch 0.91 to 0.98 from 4.7 MB on (1201 tokens of rank 16, two targets of 8192 columns 26.9 / 24.7 us), 1.00 at 1 to 2.5 MB, and 1.05 for
 // a few tokens, where the way to memory is longer than the write-back of what little there is.
 constexpr int64_t THROUGH_BYTES = (int64_t)2 << 20, THROUGH_BYTES_ONE_LAUNCH = (int64_t)3 << 20;
-inline int write_through(const ExpandArgs &a, int64_t least) { return (int64_t)a.T * a.h_out * a.n_targets * 2 >= least; }
+// And only rows of whole 128-byte lines: a line that two waves store a piece of each goes to memory twice (6700 tokens of rank 64, 4128
+// and 8224 columns, a pass of two layers 804 us without, 922 with).
+inline int write_through(const ExpandArgs &a, int64_t least) {
+  uintptr_t ends = 0;
+  for (int z = 0; z < a.n_targets; ++z) ends |= reinterpret_cast<uintptr_t>(a.ys[z]);
+  return (int64_t)a.T * a.h_out * a.n_targets * 2 >= least && !(a.h_out & 63) && !(ends & 127u);
+}
 // Not in 16-token tiles above rank 64, which read much more than they write (512 tokens over 128 adapters of rank 128, q+k+v 79.2 / 80.4
 // us, and 80.0 with the choice alone), nor above rank 64 with outputs narrower than SMALL_WIDE (no scalar register is left for the choice).
 
