@@ -48,10 +48,14 @@ constexpr int expand_min_waves(int kb, bool partial, bool comp) {
 // nothing; 16 instead of 8 staged tokens, 8.7 KB more LDS, 1 % slower.)
 // y written through instead of left dirty in the L2s for the end of the kernel: 5401 tokens over ranks 8-64, one target of 4096
 // columns 25.7 / 23.1, three 54.6 / 51.9, two of 11008 93.3 / 90.9 (with non-temporal stores the same as with plain ones).
+// THROUGH: y is written through (expand_core.h), and read as lines that nobody reads again (load16_once), so that the caches keep B and v: a
+// pass of two layers, plain reads / these, 5401 tokens over ranks 8-64 682 / 675 us, 14000 over ranks 8-64, 5120 wide 786 / 744, 7000 of rank
+// 128 411 / 404; 15 prefill batches 1.011 in the mean, 0.99 at worst (1600 tokens).  (A form of its own: above rank 64 no scalar
+// register is left for a flag.  In 16-token tiles such reads are 0.995.)
 // COMP: the compensation of a request whose base weights hold another adapter (csrc/api.hip, mlora_lora_compensate):
 // y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), where v' is the "target" 1 matrix of the same positions:
 // both products in one pass over y.
-template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP>
+template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP, bool THROUGH>
 __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expand_kernel(const int32_t *tiles_base, const int32_t *perm,
                                                                                     const int64_t *a_loc, int h_n_loc, int h_out,
                                                                                     ExpandArgs p) {
@@ -69,14 +73,12 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
   int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
-  constexpr bool MAY_THROUGH = KB < 4 || WIDE;
-  int through = MAY_THROUGH ? p.through : 0;
   uint16_t *y = p.ys[z];
   const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
   int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
   float inv_h_out = p.inv_h_out;
   asm volatile("" : "+s"(ad), "+s"(r), "+s"(pos0), "+s"(cnt), "+s"(astart), "+s"(slot), "+s"(kmax), "+s"(w_rows), "+s"(v_by_pos),
-                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out), "+s"(through));
+                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out));
   if (COMP) cnt = abs(cnt);                  // (negative: no usable rank of its own, r = 0)
   if (cnt <= 0) return;                      // records past the last tile are zero
   y = as_global(y);
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         yp[b][h] = ycol + (uint64_t)(uint32_t)t[b][h] * (uint32_t)h_out;
-        yv[b][h] = load16(yp[b][h]);
+        yv[b][h] = THROUGH ? load16_once(yp[b][h]) : load16(yp[b][h]);
       }
   };
   u32x4 bfrag[4 * KB], bfrag2[COMP ? 4 * KB : 1];
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
           for (int i = 0; i < 8; ++i) f[i] += sc * srow[i];
           yv[b][h] = pack8<T>(f);
           if (last && ocol_ok && row0 + rr0 + 8 * h < cnt) {
-            if (MAY_THROUGH && through) store16_through(yp[b][h], yv[b][h]);
+            if (THROUGH) store16_through(yp[b][h], yv[b][h]);
             else store16(yp[b][h], yv[b][h]);
           }
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -383,12 +385,15 @@ int launch_expand_kb(hipStream_t st, const ExpandArgs &a, int bm, int64_t tiles)
   // an index without entries: the kernel reads one all the same, and drops it
   const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
   const int lds = bm * ((a.compensate ? 2 : 1) * expand_v_chunks(KB) * 16 + 4);
-#define MLORA_EXPAND(WIDE, PARTIAL, COMP)                                                                       \
-  hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP>), grid, dim3(256), lds, st, records,            \
+#define MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, THROUGH)                                                         \
+  hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH>), grid, dim3(256), lds, st, records,   \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
+#define MLORA_EXPAND(WIDE, PARTIAL, COMP)                               \
+  if (a.through) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, true);          \
+  else MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, false)
 #define MLORA_EXPAND_WIDTH(PARTIAL, COMP)                     \
-  if (a.h_out >= SMALL_WIDE) MLORA_EXPAND(true, PARTIAL, COMP); \
-  else MLORA_EXPAND(false, PARTIAL, COMP)
+  if (a.h_out >= SMALL_WIDE) { MLORA_EXPAND(true, PARTIAL, COMP); } \
+  else { MLORA_EXPAND(false, PARTIAL, COMP); }
   for (int64_t t0 = 0; t0 < tiles; t0 += MAX_GRID_TILES) {
     const int32_t *records = a.plan + a.off_tiles + t0 * TILE_WORDS;
     const dim3 grid((unsigned)a.n_ochunks, (unsigned)(tiles - t0 < MAX_GRID_TILES ? tiles - t0 : MAX_GRID_TILES), (unsigned)a.n_targets);
@@ -398,6 +403,7 @@ int launch_expand_kb(hipStream_t st, const ExpandArgs &a, int bm, int64_t tiles)
   }
 #undef MLORA_EXPAND_WIDTH
 #undef MLORA_EXPAND
+#undef MLORA_EXPAND_FORM
   return check_launch("expand_kernel");
 }
 

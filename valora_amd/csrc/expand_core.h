@@ -257,7 +257,7 @@ inline int write_through(const ExpandArgs &a, int64_t least) {
   return (int64_t)a.T * a.h_out * a.n_targets * 2 >= least && !(a.h_out & 63) && !(ends & 127u);
 }
 // Not in 16-token tiles above rank 64, which read much more than they write (512 tokens over 128 adapters of rank 128, q+k+v 79.2 / 80.4
-// us, and 80.0 with the choice alone), nor above rank 64 with outputs narrower than SMALL_WIDE (no scalar register is left for the choice).
+// us, and 80.0 with the choice alone).
 
 // The lane's outputs of y: 16 from o_wave + 16 * (lane / 16) on, in two 16-byte halves.
 template <int KB>
