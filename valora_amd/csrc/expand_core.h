@@ -288,8 +288,6 @@ __device__ __forceinline__ void small_add(SmallY<KB> &s, const f32x4 (&acc)[4], 
     s.v[h] = pack8<T>(f);
   }
 }
-// The value of the other lane of a pair (lanes 2i and 2i + 1)
-__device__ __forceinline__ uint32_t lane_pair(uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true); }
 // cnt: tokens of the tile; through: wave-uniform (launch_expand, launch_decode).  A lane's halves lie 16 or 64 bytes apart, so that a store
 // of one half writes pieces of lines.  That is all the same to the L2; on their way to memory the lanes of a pair, two tokens of the
 // same columns, exchange a half first: every store then writes whole lines of one token.

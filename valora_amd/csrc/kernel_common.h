@@ -34,6 +34,9 @@ __device__ __forceinline__ void store16_through(uint16_t *p, u32x4 v) {
   __builtin_amdgcn_global_store_b128((GP)(uintptr_t)p, v, "agent");
 }
 
+// The value of the other lane of a pair (lanes 2i and 2i + 1)
+__device__ __forceinline__ uint32_t lane_pair(uint32_t x) { return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0xb1, 0xf, 0xf, true); }
+
 // A pointer that went through an inline asm operand has lost what the compiler knew about it; telling it again that
 // the memory is global keeps its loads and stores on the global path (flat accesses count against two wait counters)
 template <typename P>

@@ -117,6 +117,8 @@ struct ShrinkArgs {
   int prp;                    // row stride of the partials in that mode: whole 128-byte lines per row
   int n_tiles;                // upper bound of the tile count
   unsigned long long *arrive; // [tiles][MLORA_MAX_TARGETS] arrival words, zero between launches
+  int x_once;                 // 128- and 256-token tiles: one workgroup of a K chunk reads a row of x (set by the launcher)
+  int partial_through;        // and its partials go on to memory at once (set by the launcher)
   int whole;                  // 32 or 64: all of K in one workgroup of so many tokens (no taller than the plan's tiles), else 0
   int compensate;             // "target" 1 is the plan's merged adapter over all positions (host side: the kernels get a
                               // flag in their leading arguments, csrc/shrink.hip)

@@ -110,7 +110,7 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
     f32x4 q[BATCH];
 #pragma unroll
     for (int u = 0; u < BATCH; ++u) {
-      q[u] = *reinterpret_cast<const f32x4 *>(chunk + at);
+      q[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(chunk + at));   // (nobody reads them again)
       chunk = next_chunk(chunk, s0 + u + 1 < h_ksplit, stride);
     }
     requested();
@@ -344,8 +344,22 @@ constexpr int GEMM_KC = 64;                             // K elements of a step:
 constexpr int gemm_stage_bytes(int nb, int mbw) { return (64 * mbw + 16 * nb) * GEMM_KC * 2; }
 constexpr int GEMM_AHEAD = 2;                           // steps requested before the first is used
 
-// One tile and one K chunk, NB 16-row blocks of rank (of the tile's own adapter), MBW 16-token blocks per wave.
-template <typename T, int NB, int MBW>
+// Two 16-column blocks of a token row's fp32 partial, as the products leave them (four columns a lane, `row` the same for four lanes),
+// written through to memory (store16_through): the lanes of a pair, two rows, exchange a block first, so that a store writes whole
+// lines.  at: column 4 * kg of the first block in row `row & ~1`, `rp` floats in front of the next row's.  All lanes take part.
+__device__ __forceinline__ void store_partials_through(float *at, int rp, const f32x4 &first, const f32x4 &second, int row, int cnt, bool odd) {
+  const u32x4 lo = as<u32x4>(first), hi = as<u32x4>(second), give = odd ? lo : hi;
+  u32x4 got;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) got[i] = lane_pair(give[i]);
+  uint16_t *const dst = reinterpret_cast<uint16_t *>(at + (odd ? 16 : 0));
+  if ((row & ~1) < cnt) store16_through(dst, odd ? got : lo);
+  if ((row | 1) < cnt) store16_through(dst + 2 * rp, odd ? hi : got);
+}
+
+// One tile and one K chunk, NB 16-row blocks of rank (of the tile's own adapter), MBW 16-token blocks per wave.  ONCE: the rows of x have
+// no other reader (launch_shrink).
+template <typename T, int NB, int MBW, bool ONCE>
 __device__ __forceinline__ void shrink_gemm_tile(const ShrinkArgs &p, int s, int r, int pos0, int cnt, int astart, unsigned char *lds) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
@@ -399,7 +413,7 @@ __device__ __forceinline__ void shrink_gemm_tile(const ShrinkArgs &p, int s, int
   auto request = [&](int step, u32x4 (&x)[XG], u32x4 (&a)[APW]) {
     const int off = kbeg + step * KC;
 #pragma unroll
-    for (int g = 0; g < XG; ++g) x[g] = load16(xp[g] + off);
+    for (int g = 0; g < XG; ++g) x[g] = ONCE ? load16_once(xp[g] + off) : load16(xp[g] + off);
 #pragma unroll
     for (int i = 0; i < APW; ++i) a[i] = load16(ap[i] + (off & astep[i]));
     requested();
@@ -493,6 +507,14 @@ __device__ __forceinline__ void shrink_gemm_tile(const ShrinkArgs &p, int s, int
 #pragma unroll
   for (int mb = 0; mb < MBW; ++mb) {
     const int row = wrow0 + mb * 16 + lrow;
+    if constexpr (NB >= 2)
+      if (p.partial_through) {
+        float *const part = as_global(p.partial) + ((int64_t)s * p.T + pos0 + (row & ~1)) * p.rp + kg * 4;
+#pragma unroll
+        for (int nb = 0; nb < NB; nb += 2)
+          if (nb * 16 < p.rp) store_partials_through(part + nb * 16, p.rp, acc[mb][nb], acc[mb][nb + 1], row, cnt, lane & 1);
+        continue;
+      }
     if (row < cnt) {
       if (p.ksplit == 1) {
         const int t = p.out_by_token ? perm[pos0 + row] : 0;
@@ -511,7 +533,7 @@ __device__ __forceinline__ void shrink_gemm_tile(const ShrinkArgs &p, int s, int
   }
 }
 
-template <typename T, int NB, int MBW>
+template <typename T, int NB, int MBW, bool ONCE>
 __global__ __launch_bounds__(256, MBW == 2 ? 2 : 1) void shrink_gemm_kernel(const int32_t *tiles_base, int h_flags, ShrinkArgs args_in) {
   // grid (K chunks, targets, tiles).  The workgroup id mod 8 selects the XCD, so
   // with the K chunk as the fast index the tiles of an adapter that share a K chunk of A, and the
@@ -525,9 +547,9 @@ __global__ __launch_bounds__(256, MBW == 2 ? 2 : 1) void shrink_gemm_kernel(cons
   if ((h_flags & SHRINK_COMPENSATE) && z_idx == 1) merged_tile(p.plan, tile_idx, 64 * MBW, r, pos0, cnt, astart);
   if (cnt <= 0) return;   // records past the last tile are zero
   // (a narrow adapter among wide ones takes the loads and products of its own rank)
-  if (NB > 1 && r <= 16) shrink_gemm_tile<T, 1, MBW>(p, s, r, pos0, cnt, astart, lds);
-  else if (NB > 2 && r <= 32) shrink_gemm_tile<T, 2, MBW>(p, s, r, pos0, cnt, astart, lds);
-  else shrink_gemm_tile<T, NB, MBW>(p, s, r, pos0, cnt, astart, lds);
+  if (NB > 1 && r <= 16) shrink_gemm_tile<T, 1, MBW, ONCE>(p, s, r, pos0, cnt, astart, lds);
+  else if (NB > 2 && r <= 32) shrink_gemm_tile<T, 2, MBW, ONCE>(p, s, r, pos0, cnt, astart, lds);
+  else shrink_gemm_tile<T, NB, MBW, ONCE>(p, s, r, pos0, cnt, astart, lds);
 }
 
 // The same tile in eight waves, for NT targets of a call together (x is requested, written to LDS and read from it once for all
@@ -545,7 +567,7 @@ constexpr int targets_half(int nt, int nb) { return (nt * nb + 1) / 2; }   // 16
 constexpr int targets_stage_bytes(int nt, int nb) { return (TARGETS_ROWS + 32 * targets_half(nt, nb)) * GEMM_KC * 2; }
 
 // One tile and one K chunk, NB 16-row blocks of rank (of the tile's own adapter) for each of NT targets.
-template <typename T, int NT, int NB>
+template <typename T, int NT, int NB, bool ONCE>
 __device__ __forceinline__ void shrink_targets_tile(const ShrinkArgs &p, int s, int r, int pos0, int cnt, int astart, unsigned char *lds) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
@@ -596,7 +618,7 @@ __device__ __forceinline__ void shrink_targets_tile(const ShrinkArgs &p, int s, 
   auto request = [&](int step) {
     const int off = kbeg + step * KC;
 #pragma unroll
-    for (int g = 0; g < XG; ++g) rx[g] = load16(xp[g] + off);
+    for (int g = 0; g < XG; ++g) rx[g] = ONCE ? load16_once(xp[g] + off) : load16(xp[g] + off);
 #pragma unroll
     for (int i = 0; i < APW; ++i) ra[i] = load16(ap[i] + (off & astep[i]));
     requested();
@@ -671,6 +693,17 @@ __device__ __forceinline__ void shrink_targets_tile(const ShrinkArgs &p, int s, 
 #pragma unroll
   for (int mb = 0; mb < 2; ++mb) {
     const int row = trow0 + mb * 16 + lrow;
+    if constexpr (NB >= 2 && HB % 2 == 0)
+      if (p.partial_through) {
+        float *const part = as_global(p.partial) + ((int64_t)s * p.T + pos0 + (row & ~1)) * p.rp + kg * 4;
+#pragma unroll
+        for (int b = 0; b < HB; b += 2) {
+          const int z = (b0 + b) / NB, nb = (b0 + b) % NB;
+          if (z < NT && nb * 16 < p.rp)
+            store_partials_through(part + z * p.partial_tstride + nb * 16, p.rp, acc[mb][b], acc[mb][b + 1], row, cnt, lane & 1);
+        }
+        continue;
+      }
     if (row < cnt) {
       if (NT == 1 && p.ksplit == 1) {                   // (targets go together only where K is split)
         const int t = p.out_by_token ? perm[pos0 + row] : 0;
@@ -694,7 +727,7 @@ __device__ __forceinline__ void shrink_targets_tile(const ShrinkArgs &p, int s, 
   }
 }
 
-template <typename T, int NT, int NB>
+template <typename T, int NT, int NB, bool ONCE>
 __global__ __launch_bounds__(512, NT * NB <= 12 ? 4 : 2) void shrink_targets_kernel(const int32_t *tiles_base, int h_flags, ShrinkArgs args_in) {
   // grid (K chunks, groups of NT targets, tiles)
   const ShrinkArgs p = NT == 1 ? select_target(args_in, blockIdx.y) : args_in;
@@ -705,22 +738,26 @@ __global__ __launch_bounds__(512, NT * NB <= 12 ? 4 : 2) void shrink_targets_ker
   if (NT == 1 && (h_flags & SHRINK_COMPENSATE) && blockIdx.y == 1) merged_tile(p.plan, (int)blockIdx.z, TARGETS_ROWS, r, pos0, cnt, astart);
   if (cnt <= 0) return;   // records past the last tile are zero
   // (a narrow adapter among wide ones takes the loads and products of its own rank)
-  if (NB > 1 && r <= 16) shrink_targets_tile<T, NT, 1>(p, s, r, pos0, cnt, astart, lds);
-  else if (NB > 2 && r <= 32) shrink_targets_tile<T, NT, 2>(p, s, r, pos0, cnt, astart, lds);
-  else if (NB > 4 && r <= 64) shrink_targets_tile<T, NT, 4>(p, s, r, pos0, cnt, astart, lds);
-  else shrink_targets_tile<T, NT, NB>(p, s, r, pos0, cnt, astart, lds);
+  if (NB > 1 && r <= 16) shrink_targets_tile<T, NT, 1, ONCE>(p, s, r, pos0, cnt, astart, lds);
+  else if (NB > 2 && r <= 32) shrink_targets_tile<T, NT, 2, ONCE>(p, s, r, pos0, cnt, astart, lds);
+  else if (NB > 4 && r <= 64) shrink_targets_tile<T, NT, 4, ONCE>(p, s, r, pos0, cnt, astart, lds);
+  else shrink_targets_tile<T, NT, NB, ONCE>(p, s, r, pos0, cnt, astart, lds);
 }
 
 inline int head_flags(const ShrinkArgs &a) { return a.reduce_here | (a.compensate ? SHRINK_COMPENSATE : 0); }
 
 template <typename T, int MBW>
 int launch_gemm_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
+#define MLORA_GEMM(NB)                                                                                                             \
+  if (a.x_once) hipLaunchKernelGGL((shrink_gemm_kernel<T, NB, MBW, true>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); \
+  else hipLaunchKernelGGL((shrink_gemm_kernel<T, NB, MBW, false>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a)
   switch (nb) {
-    case 1: hipLaunchKernelGGL((shrink_gemm_kernel<T, 1, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
-    case 2: hipLaunchKernelGGL((shrink_gemm_kernel<T, 2, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
-    case 4: hipLaunchKernelGGL((shrink_gemm_kernel<T, 4, MBW>), grid, dim3(256), 0, st, a.plan + a.off_tiles, head_flags(a), a); break;
+    case 1: MLORA_GEMM(1); break;
+    case 2: MLORA_GEMM(2); break;
+    case 4: MLORA_GEMM(4); break;
     default: return fail(MLORA_ERR_NO_KERNEL, "shrink: no kernel for rank blocks=%d", nb);
   }
+#undef MLORA_GEMM
   return check_launch("shrink_gemm_kernel");
 }
 
@@ -748,15 +785,16 @@ int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, int max_rank, 
 template <typename T, int NT>
 int launch_targets(hipStream_t st, const ShrinkArgs &a, int nb, int64_t tiles) {
   const dim3 grid((unsigned)a.ksplit, (unsigned)(a.n_targets / NT), (unsigned)tiles);
-#define MLORA_TARGETS(NB) \
-  hipLaunchKernelGGL((shrink_targets_kernel<T, NT, NB>), grid, dim3(512), 0, st, a.plan + a.off_tiles, head_flags(a), a)
+#define MLORA_TARGETS(NB)                                                                                                            \
+  if (a.x_once) hipLaunchKernelGGL((shrink_targets_kernel<T, NT, NB, true>), grid, dim3(512), 0, st, a.plan + a.off_tiles, head_flags(a), a); \
+  else hipLaunchKernelGGL((shrink_targets_kernel<T, NT, NB, false>), grid, dim3(512), 0, st, a.plan + a.off_tiles, head_flags(a), a)
   if constexpr (NT == 1) {   // (above rank 64)
     MLORA_TARGETS(8);
   } else {
-    if (nb == 1) MLORA_TARGETS(1);
-    else if (nb == 2) MLORA_TARGETS(2);
-    else if (nb == 4) MLORA_TARGETS(4);
-    else MLORA_TARGETS(8);
+    if (nb == 1) { MLORA_TARGETS(1); }
+    else if (nb == 2) { MLORA_TARGETS(2); }
+    else if (nb == 4) { MLORA_TARGETS(4); }
+    else { MLORA_TARGETS(8); }
   }
 #undef MLORA_TARGETS
   return check_launch("shrink_targets_kernel");
@@ -831,8 +869,10 @@ bool shrink_targets_together(int64_t T, int64_t adapters, int64_t max_rank, int 
   return many ? least >= 176 && (usual <= 232 || usual > 704) : least >= 160 && (usual <= 256 || usual > 336);
 }
 
-int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int64_t grid_tiles,
+int launch_shrink(hipStream_t st, const ShrinkArgs &args, int bm, int max_rank, int64_t grid_tiles,
                   mlora_dtype dt) {
+  ShrinkArgs a = args;
+  a.x_once = a.partial_through = 0;
   int nb = (max_rank + 15) / 16;
   nb = nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : 8;
   if (nb == 8 && (bm == 64 || bm == 256)) return fail(MLORA_ERR_NO_KERNEL, "shrink: rank > 64 needs tile height 16, 32 or 128");
@@ -848,7 +888,16 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &a, int bm, int max_rank, int
   if (bm >= 128) {
     if (grid_tiles > 65535) return fail(MLORA_ERR_NO_KERNEL, "shrink: grid too large");   // (4M tokens of 8192 adapters have 40960)
     grid = dim3((unsigned)a.ksplit, (unsigned)a.n_targets, (unsigned)grid_tiles);
-    if (!a.compensate && shrink_targets_together(a.T, grid_tiles - (a.T + 127) / 128, max_rank, bm, a.ksplit, a.n_targets)) {
+    const bool together = !a.compensate && shrink_targets_together(a.T, grid_tiles - (a.T + 127) / 128, max_rank, bm, a.ksplit, a.n_targets);
+    // x is read as lines that nobody reads again (load16_once) where that is so: not by one target's workgroups after another's, nor where
+    // the caller's next call reads it; in rows of whole lines.  Partials are written through in whole lines likewise, instead of left in the
+    // L2s for the end of the kernel, and the launch that sums them reads them once.  A pass of two layers, before / now: 4430 tokens of rank 64
+    // 664 / 636 us, 5401 over ranks 8-64 678 / 667, 7000 of rank 128 407 / 398, 14000 over ranks 8-64, 5120 wide 785 / 763; one-call entry
+    // points (partials only) 1600 of rank 64 199 / 184, 7000 of rank 128 500 / 490, and with x read so 515; 15 prefill batches 1.016 in the
+    // mean, 0.99 at worst (2800 tokens of ranks 32 and 48, whose partials are no whole lines).
+    a.x_once = !a.out_by_token && (a.n_targets == 1 || together) && !(a.h_in & 63) && !(reinterpret_cast<uintptr_t>(a.x) & 127u);
+    a.partial_through = a.ksplit > 1 && (a.rp & 31) == 0 && (reinterpret_cast<uintptr_t>(a.partial) & 127u) == 0;
+    if (together) {
       if (a.n_targets == 3) return dt == MLORA_F16 ? launch_targets<_Float16, 3>(st, a, nb, grid_tiles) : launch_targets<__bf16, 3>(st, a, nb, grid_tiles);
       return dt == MLORA_F16 ? launch_targets<_Float16, 2>(st, a, nb, grid_tiles) : launch_targets<__bf16, 2>(st, a, nb, grid_tiles);
     }
