@@ -87,3 +87,56 @@ def test_tall_tiles(dev, ranks, bm, targets, ksplit):
     for t in range(targets):
         want = O.lora_op(y0[t], x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, t, pool.a_scaling, n_slots=3)
         assert O.rel_l2(got[0][t].cpu(), want) <= _bound(dtype)
+
+
+@pytest.mark.parametrize("T,A,bm_s,bm_e,merged", [(1, 5, 16, 16, None), (60, 40, 16, 16, None), (300, 9, 16, 48, None), (900, 64, 16, 32, None),
+                                                  (700, 3000, 16, 16, None), (5000, 600, 64, 16, None), (250, 12, 16, 16, 2)])
+def test_record_says_which_tile_is_its_adapters_only_one(dev, T, A, bm_s, bm_e, merged):
+    from valora_amd.merge import DeLoraPlan
+    g = torch.Generator().manual_seed(T + A)
+    a_len = (torch.randint(1, 9, (A,), generator=g) * 16)
+    a_start = torch.cumsum(a_len, 0) - a_len
+    index = (a_start.to(dev), a_len.to(dev))
+
+    def check(plan, ids):
+        for tiles, bm in ((plan.tiles_shrink().cpu().tolist(), bm_s), (plan.tiles_expand().cpu().tolist(), bm_e)):
+            assert tiles
+            for t in tiles:
+                assert t[5:] == [len(tiles) if sum(u[0] == t[0] for u in tiles) == 1 else 0, 0, 0], (t, bm)
+
+    hot = torch.where(torch.rand(T, generator=g) < 0.5, torch.tensor(A // 2), torch.randint(0, A, (T,), generator=g))
+    one = torch.full((T,), A - 1)
+    kw = dict(n_slots=2, bm_shrink=bm_s, bm_expand=bm_e)
+    plan = LoraPlan(hot.to(dev), *index, 64, hidden=4096, **kw) if merged is None else DeLoraPlan(hot.to(dev), merged, *index, 64, 4096, **kw).plan
+    check(plan, hot)
+    plan.rebuild(one.to(dev))
+    check(plan, one)
+
+
+@pytest.mark.parametrize("rank", [16, 32, 64, 128])
+@pytest.mark.parametrize("ksplit", [1, 4])
+@pytest.mark.parametrize("shared", [0.0, 0.5, 1.0])   # of the tokens on one adapter, whose tiles share its A
+def test_adapters_of_one_tile_among_others(dev, rank, ksplit, shared):
+    """A on 128-byte lines against the same A beside them, which is read the plain way."""
+    n, T, h_in, h_out = 60, 90, 2048 if rank > 16 else 4096, 72
+    g = torch.Generator().manual_seed(rank + ksplit)
+    pool, _, x, y0 = _case(T, n, rank, h_in, h_out, torch.float16, rank)
+    ids = torch.where(torch.rand(T, generator=g) < shared, torch.tensor(7), torch.arange(T) % n)
+    print(rank, ksplit, shared, flush=True)
+    p, xd, idsd = pool.to(dev), x.to(dev), ids.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    plan = LoraPlan(idsd, *idx[:2], rank, n_slots=2, hidden=h_in, bm_shrink=16, bm_expand=16, one_launch=False, ksplit=ksplit)
+    tiles = plan.tiles_shrink().cpu()
+    some = shared < 1.0   # (batches that the rule takes: enough tiles, some of which are their adapter's only one)
+    assert bool((tiles[:, 5] > 0).any()) == some and tiles.size(0) * rank * h_in * 2 >= (4 << 20 if some else 0)
+    got = []
+    for off in (0, 8):
+        room = torch.empty(p.key_buffer.numel() + off, dtype=torch.float16, device=dev)
+        kb = room[off:].view(p.key_buffer.shape)
+        assert (kb.data_ptr() % 128 == 0) == (off == 0)
+        kb.copy_(p.key_buffer)
+        y = y0.to(dev)
+        plan.apply(y, xd, kb, p.value_buffer, *idx, 1, p.a_scaling)
+        got.append(y)
+    assert torch.equal(got[0], got[1])
+    assert O.rel_l2(got[0].cpu(), _oracle(pool, ids, x, y0)) <= REL_L2

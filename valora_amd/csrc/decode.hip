@@ -122,13 +122,12 @@ __device__ __forceinline__ ItemId item_of(int n_producers, int n_consumers, int 
 // output by token (no turn through LDS), its chunk loads not behind its B loads, and the shrink's loads without masks, cold layers,
 // rank 16, before / now: one target of one token 6.4 / 5.7 us, of 256 9.6 / 9.6, 11008 wide 15.1 / 14.1; q+k+v of 256 21.2 / 19.9, of
 // 512 23.7 / 22.1.
-// ONCE: A's rows are read as lines that nobody reads again (shrink_reads_once).
 // THROUGH: y is written through (expand_core.h; a form of its own: the flag would take a scalar register of which there are none left).
 // The leading scalar parameters repeat what the first dependent loads need (the tile records, the `done` words, the
 // id layout): the library is built with kernel-argument preloading, which hands the first 8 dwords of the
 // argument list to the wave in registers at launch, so the tile record can be requested without waiting for a load
 // of the argument block first (0.35 us of a 10.3 us op).
-template <typename T, int NB, bool WIDE, bool THROUGH, bool ONCE>
+template <typename T, int NB, bool WIDE, bool THROUGH>
 __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_base, uint32_t *done_base, int h_n_producers,
                                                         int h_n_consumers, int h_n_tiles, int h_shrink_ids,
                                                         DecodeArgs a) {
@@ -191,7 +190,7 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
     const int kbeg = s * kchunk;
     const int kend = min(h_in, kbeg + kchunk);
     const int slot = z == 0 ? sl0 : z == 1 ? sl1 : z == 2 ? sl2 : sl3;
-    shrink_tile_to_lds<T, 1, NB, shrink_steps(1 + NB), 4, ONCE>(x, h_in, pool, slot, perm, r, pos0, cnt, astart, kbeg, kend, s_buf);
+    shrink_tile_to_lds<T, 1, NB>(x, h_in, pool, slot, perm, r, pos0, cnt, astart, kbeg, kend, s_buf);
     if (wave == 0) {
       // wave 0 alone writes the partial and then the stamp: no barrier, and nothing else of its own in flight
       // (no division: 16 rows x 4 quarters of a rank block are the lanes)
@@ -313,18 +312,15 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
 }
 
 template <typename T>
-int launch_decode_t(hipStream_t st, const DecodeArgs &a, int max_rank, dim3 grid, int shrink_ids) {
-  const int nb = (max_rank + 15) / 16;
+int launch_decode_t(hipStream_t st, const DecodeArgs &a, int nb, dim3 grid, int shrink_ids) {
   // (with a few tokens a tile an item's y is too little to gain: 256 tokens over 64 adapters, a pass of 32 layers 928 / 931 us)
   const bool through = a.s.T >= 5 * a.n_tiles && write_through(a.e, THROUGH_BYTES_ONE_LAUNCH);
-  const bool once = !through && shrink_reads_once(a.s, a.n_tiles, max_rank);   // (A is read once with so few tokens a tile that y is not written through)
-#define MLORA_DECODE_FORM(NB, WIDE, THROUGH, ONCE)                                                                              \
-  hipLaunchKernelGGL((decode_kernel<T, NB, WIDE, THROUGH, ONCE>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, \
+#define MLORA_DECODE_FORM(NB, WIDE, THROUGH)                                                                                    \
+  hipLaunchKernelGGL((decode_kernel<T, NB, WIDE, THROUGH>), grid, dim3(256), 0, st, a.s.plan + a.e.off_tiles, a.done, a.n_producers, a.n_consumers, \
                      a.n_tiles, shrink_ids, a)
 #define MLORA_DECODE(NB, WIDE)                  \
-  if (through) MLORA_DECODE_FORM(NB, WIDE, true, false); \
-  else if (once) MLORA_DECODE_FORM(NB, WIDE, false, true); \
-  else MLORA_DECODE_FORM(NB, WIDE, false, false)
+  if (through) MLORA_DECODE_FORM(NB, WIDE, true); \
+  else MLORA_DECODE_FORM(NB, WIDE, false)
   if (nb == 1) { MLORA_DECODE(1, false); }
   else if (a.e.h_out >= SMALL_WIDE) { MLORA_DECODE(2, true); }
   else { MLORA_DECODE(2, false); }
@@ -353,8 +349,8 @@ int launch_decode(hipStream_t st, const DecodeArgs &a, int max_rank, mlora_dtype
   const int64_t total = shrink_ids + groups * 8 * a.n_consumers;
   if (total > 0x7fffffff) return fail(MLORA_ERR_NO_KERNEL, "one-launch op: grid too large");
   dim3 grid((unsigned)total);
-  return dt == MLORA_F16 ? launch_decode_t<_Float16>(st, a, max_rank, grid, (int)shrink_ids)
-                         : launch_decode_t<__bf16>(st, a, max_rank, grid, (int)shrink_ids);
+  return dt == MLORA_F16 ? launch_decode_t<_Float16>(st, a, nb, grid, (int)shrink_ids)
+                         : launch_decode_t<__bf16>(st, a, nb, grid, (int)shrink_ids);
 }
 
 }  // namespace mlora

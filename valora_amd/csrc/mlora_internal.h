@@ -15,7 +15,8 @@ namespace mlora {
 // perm[p]     token index at sorted position p (tokens grouped by adapter, original order kept
 //             inside a group); positions >= hdr[H_NACTIVE] are unused
 // padapter[p] adapter of position p;  prank[p] its rank
-// tile        {adapter, rank, first position, token count, a_start[adapter], 0, 0, 0}; in a compensation plan the tile of
+// tile        {adapter, rank, first position, token count, a_start[adapter], alone, 0, 0}; alone: the number of tiles of the list where
+//             this is the adapter's only one, 0 where the adapter has more; in a compensation plan the tile of
 //             an adapter without a usable rank has rank 0 and its token count with a minus sign: the kernels leave it as
 //             they leave an empty record, but for the compensating expand, which takes the merged adapter off its tokens
 // done, stamps  the hand-off words of the one-launch op (csrc/decode.hip): per tile a word that numbers the launches
@@ -119,6 +120,7 @@ struct ShrinkArgs {
   unsigned long long *arrive; // [tiles][MLORA_MAX_TARGETS] arrival words, zero between launches
   int x_once;                 // 128- and 256-token tiles: one workgroup of a K chunk reads a row of x (set by the launcher)
   int partial_through;        // and its partials go on to memory at once (set by the launcher)
+  int once_tiles;             // 16-token tiles: A of an adapter's only tile is read as lines that nobody reads again from so many tiles on (set by the launchers)
   int whole;                  // 32 or 64: all of K in one workgroup of so many tokens (no taller than the plan's tiles), else 0
   int compensate;             // "target" 1 is the plan's merged adapter over all positions (host side: the kernels get a
                               // flag in their leading arguments, csrc/shrink.hip)

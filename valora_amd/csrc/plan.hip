@@ -321,12 +321,12 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     const int n_tiles = pass ? n_te : n_ts;
     const int bm = pass ? bm_e : bm_s;
     const int32_t *toff = pass ? toff_e : toff_s;
-    auto put_record = [&](int i, int4 head, int32_t start) {   // the lists begin on 32-byte boundaries of a 16-byte aligned buffer
+    auto put_record = [&](int i, int4 head, int32_t start, int32_t alone) {   // the lists begin on 32-byte boundaries of a 16-byte aligned buffer
       static_assert(TILE_WORDS == 8, "two 16-byte stores");
       for (int list = 0; list < (one_list ? 2 : 1); ++list) {
         int4 *tl = reinterpret_cast<int4 *>(plan + (pass || list ? off_tiles_e : off_tiles_s) + (int64_t)i * TILE_WORDS);
         tl[0] = head;
-        tl[1] = int4{start, 0, 0, 0};
+        tl[1] = int4{start, alone, 0, 0};
       }
     };
     // the kernels' grids are sized with the upper bound of the tile count: records past the last
@@ -334,7 +334,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
     const int upper = (T + bm - 1) / bm + min(A, T);
     for (int i = tid * n_parts + part; i < upper; i += THREADS * n_parts) {
       if (i >= n_tiles) {
-        put_record(i, int4{0, 0, 0, 0}, 0);
+        put_record(i, int4{0, 0, 0, 0}, 0, 0);
         continue;
       }
       int lo = 0, hi = A;  // first adapter with toff > i
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(THREADS) void plan_kernel(
       // any other row outside the pool.
       // (no usable rank, compensation plans only: the count is negative, so whoever has no use for the tile leaves)
       const int r = rank_of(a), n = min(bm, c - k * bm);
-      put_record(i, int4{a, r, gstart[a] + k * bm, r > 0 ? n : -n}, start_word(st));
+      put_record(i, int4{a, r, gstart[a] + k * bm, r > 0 ? n : -n}, start_word(st), c <= bm ? n_tiles : 0);
     }
   }
   if (part == 0 && tid == 0) {

@@ -131,7 +131,9 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
 // spill 4 and 28 registers; three / two: 4000 tokens over 32 adapters of rank 32, four chunks 12.8 / 11.6 us, eight 12.9 / 11.4; 8000 over
 // 64 of rank 16 18.4 / 16.0, of rank 32 20.6 / 18.7.)
 constexpr int shrink_min_waves(int mb, int nb) { return mb + nb <= 3 ? 4 : nb == 8 ? 3 - mb : mb == 4 ? 2 : 3; }
-template <typename T, int MB, int NB, bool ONCE = false>
+// ONCE: a tile that is its adapter's only one may read A as lines that nobody reads again (shrink_once_tiles).  A form of its own: with both
+// loops in one kernel a call of a few tokens takes 3.78 us instead of 3.62.
+template <typename T, int MB, int NB, bool ONCE>
 __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
                                                      int h_n_tiles, ShrinkArgs args_in) {
   int tile_idx, z_idx, s;
@@ -162,6 +164,7 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
   __shared__ int s_last;
 
   int r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
+  const int until_once = ONCE ? p.once_tiles - 1 - tile_alone(tile) : 1;
   if (compensate && z_idx == 1) merged_tile(p.plan, tile_idx, 16 * MB, r, pos0, cnt, astart);
   if (cnt <= 0) return;   // records past the last tile are zero
   const int32_t *__restrict__ perm = p.plan + p.off_perm;
@@ -180,7 +183,7 @@ __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(c
     on[it] = row[it] < cnt && c4[it] < quarter;
     tok[it] = (p.out_by_token && on[it]) ? perm[pos0 + row[it]] : 0;
   }
-  shrink_tile_to_lds<T, MB, NB, shrink_steps(MB + NB), 4, ONCE>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, kbeg, kend, s_tile);
+  shrink_tile_to_lds<T, MB, NB, shrink_steps(MB + NB), 4, ONCE>(p.x, p.h_in, p.pool, p.slot, perm, r, pos0, cnt, astart, kbeg, kend, s_tile, until_once);
   if (p.ksplit == 1) {
 #pragma unroll
     for (int it = 0; it < ITEMS; ++it)
@@ -762,14 +765,13 @@ int launch_gemm_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
 }
 
 template <typename T, int MB>
-int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, int max_rank, dim3 grid) {
+int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
   constexpr bool MAY_ONCE = MB == 1;
-  const bool once = MAY_ONCE && !a.compensate && shrink_reads_once(a, a.n_tiles, max_rank);
+#define MLORA_SHRINK(MBX, NB)                                                                     \
+  if (MAY_ONCE && a.once_tiles <= a.n_tiles) MLORA_SHRINK_FORM(MBX, NB, MAY_ONCE);                \
+  else MLORA_SHRINK_FORM(MBX, NB, false)
 #define MLORA_SHRINK_FORM(MBX, NB, ONCE) \
   hipLaunchKernelGGL((shrink_kernel<T, MBX, NB, ONCE>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a)
-#define MLORA_SHRINK(MBX, NB)                         \
-  if (once) MLORA_SHRINK_FORM(MBX, NB, MAY_ONCE);     \
-  else MLORA_SHRINK_FORM(MBX, NB, false)
   switch (nb) {
     case 1: MLORA_SHRINK(MB, 1); break;
     case 2: MLORA_SHRINK(MB, 2); break;
@@ -820,11 +822,11 @@ int launch_whole(hipStream_t st, const ShrinkArgs &a, int bm, int nb, int64_t ti
 }
 
 template <typename T>
-int launch_shrink_t(hipStream_t st, const ShrinkArgs &a, int bm, int nb, int max_rank, dim3 grid) {
+int launch_shrink_t(hipStream_t st, const ShrinkArgs &a, int bm, int nb, dim3 grid) {
   switch (bm) {
-    case 16: return launch_shrink_nb<T, 1>(st, a, nb, max_rank, grid);
-    case 32: return launch_shrink_nb<T, 2>(st, a, nb, max_rank, grid);
-    case 64: return launch_shrink_nb<T, 4>(st, a, nb, max_rank, grid);
+    case 16: return launch_shrink_nb<T, 1>(st, a, nb, grid);
+    case 32: return launch_shrink_nb<T, 2>(st, a, nb, grid);
+    case 64: return launch_shrink_nb<T, 4>(st, a, nb, grid);
     case 128: return launch_gemm_nb<T, 2>(st, a, nb, grid);
     case 256: return launch_gemm_nb<T, 4>(st, a, nb, grid);
     default: return fail(MLORA_ERR_NO_KERNEL, "shrink: tile height %d not in {16,32,64,128,256}", bm);
@@ -873,6 +875,7 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &args, int bm, int max_rank, 
                   mlora_dtype dt) {
   ShrinkArgs a = args;
   a.x_once = a.partial_through = 0;
+  a.once_tiles = bm == 16 ? shrink_once_tiles(a, a.n_tiles, max_rank) : 0x7fffffff;
   int nb = (max_rank + 15) / 16;
   nb = nb <= 1 ? 1 : nb <= 2 ? 2 : nb <= 4 ? 4 : 8;
   if (nb == 8 && (bm == 64 || bm == 256)) return fail(MLORA_ERR_NO_KERNEL, "shrink: rank > 64 needs tile height 16, 32 or 128");
@@ -905,8 +908,8 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &args, int bm, int max_rank, 
   }
   if (a.reduce_here)
     grid = dim3((unsigned)(8 * a.ksplit), (unsigned)a.n_targets, (unsigned)(grid_tiles / 8));   // at most 4096 tokens (csrc/api.hip)
-  return dt == MLORA_F16 ? launch_shrink_t<_Float16>(st, a, bm, nb, max_rank, grid)
-                         : launch_shrink_t<__bf16>(st, a, bm, nb, max_rank, grid);
+  return dt == MLORA_F16 ? launch_shrink_t<_Float16>(st, a, bm, nb, grid)
+                         : launch_shrink_t<__bf16>(st, a, bm, nb, grid);
 }
 
 }  // namespace mlora

@@ -16,6 +16,8 @@
 // rank rows gathered through loc_indicies, fp32 accumulation).
 #pragma once
 
+#include <type_traits>
+
 #include "kernel_common.h"
 
 namespace mlora {
@@ -46,6 +48,13 @@ __device__ __forceinline__ f32x4 shrink_tile_sum(const float *lds, int nblk, int
   return (w0 + w2) + (w1 + w3);
 }
 
+// Word 5 of a tile's record on the scalar path (as constant memory: the plan is not written while it is in use; left to itself the
+// compiler takes a vector load).
+__device__ __forceinline__ int tile_alone(const int32_t *tile) {
+  typedef __attribute__((address_space(4))) const int32_t *CP;
+  return *(CP)(uintptr_t)(tile + 5);
+}
+
 // What a lane without anything to fetch reads, as far as the steps of a batch reach.
 __device__ const __align__(128) uint16_t g_shrink_zeros[12 * SHRINK_KSTEP + SHRINK_KSTEP] = {};
 constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1; }
@@ -53,27 +62,29 @@ constexpr int shrink_steps(int blks) { return blks <= 2 ? 4 : blks <= 5 ? 2 : 1;
 // 16-byte aligned), for shrink_tile_sum to add up (rows = tokens of the tile, columns = rank); every thread of the
 // workgroup must call it, none may still be reading `lds`, and all have passed a barrier when it returns.
 // U: K steps in flight per wave.  The order of the sums does not depend on it.
-// ONCE: the rows of A have no other reader (shrink_reads_once).
+// until_once (wave-uniform, only looked at with MAY_ONCE): negative where the rows of A have no other reader (shrink_once_tiles).
 // Bound by the instructions of one wave in a row, and by what a compute unit takes in.  Rows that are not there are a choice of
 // address, not a mask: a mask, four zeroed registers and a branch around each of a batch's 16 loads took 1400 cycles to issue.
 // One target, cold layers, masked / like this: 1 token of rank 16 4.9 / 4.0 us, 256 over 64 adapters 6.7 / 5.7, 200 over 16 of rank 32
 // 7.6 / 6.5, 77 over ranks 8-64 8.8 / 7.9, 256 over 64 of rank 64 11.6 / 10.9, 512 over 128 of rank 128 29.5 / 28.4.
-template <typename T, int MB, int NB, int U = shrink_steps(MB + NB), int WAVES = 4, bool ONCE = false>
+template <typename T, int MB, int NB, int U = shrink_steps(MB + NB), int WAVES = 4, bool MAY_ONCE = false>
 __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ x, int h_in, const PoolDev &pool,
                                                    int slot, const int32_t *__restrict__ perm, int r, int pos0,
                                                    int cnt, int astart, int kbeg, int kend,
-                                                   float *lds) {
+                                                   float *lds, int until_once = 1) {
   using Tr = Traits<T>;
   using vec8 = typename Tr::vec8;
   constexpr int NBLK = MB * NB;
   constexpr int BLKS = MB + NB;                         // 16-row blocks of a K step, x first
   constexpr bool MANY = NB > 2;
+  constexpr bool PINNED = MB == 1 && NB > 4;
   constexpr bool WHOLE = MB == 1 || NB <= 2;            // has a loop of its own for whole batches
   static_assert(WAVES * (U - 1) <= 12, "a batch's steps reach past g_shrink_zeros");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int lrow = lane & 15, kg = lane >> 4;           // MFMA operand roles
   const int grow = lane >> 3, gcol = lane & 7;          // loader roles: row within a group of 8, 16-byte chunk
   const int64_t base = (int64_t)astart + (int64_t)r * slot;
+  if (MAY_ONCE) asm volatile("" : "+s"(until_once));   // (requested with the rest, not in front of the first batch)
 
   // This lane's row pointers (already at its chunk).  All look-ups are requested together, one round trip: those with
   // nothing to look up read an address that is always there instead of branching around the load.
@@ -112,6 +123,9 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
       all = all && ok[nb][u];
       rp[MB + nb][u] = pool.w + (uint64_t)(uint32_t)(ok[nb][u] ? prow[nb][u] : 0) * (uint32_t)h_in + gcol * 8;
       step[nb][u] = ok[nb][u] ? -1 : 0;
+      // (PINNED: kept in its register, not as a condition in two scalar ones, of which there are none left: 46 and more stood in lanes of
+      // vector registers.  512 tokens of rank 128 on one adapter, a pass 242 / 238 us)
+      if (PINNED) asm("" : "+v"(step[nb][u]));
       if (MANY && !ok[nb][u]) rp[MB + nb][u] = as_global(g_shrink_zeros) + gcol * 8;
     }
   }
@@ -169,25 +183,30 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
   };
   // The trip counts must be wave-uniform: MFMA ignores EXEC, so a lane that left a loop early would still feed its stale
   // registers into the matrix core.
-  // Whole batches: a load is an instruction, the steps of a batch are offsets in it.
+  // Whole batches: a load is an instruction, the steps of a batch are offsets in it.  (A loop for either kind of A: with a branch in one
+  // loop 900 tokens of rank 128 on one adapter take 277 us a pass, with two 269.)
   int kb0 = kbeg + wave * SHRINK_KSTEP;
-  for (; plain && kb0 + (WAVES * (U - 1) + 1) * SHRINK_KSTEP <= kend; kb0 += WAVES * SHRINK_KSTEP * U) {
+  auto whole_batches = [&](auto a_once) {
+    for (; plain && kb0 + (WAVES * (U - 1) + 1) * SHRINK_KSTEP <= kend; kb0 += WAVES * SHRINK_KSTEP * U) {
 #pragma unroll
-    for (int b = 0; b < BLKS; ++b)
+      for (int b = 0; b < BLKS; ++b)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const uint16_t *const src = rp[b][u] + (MANY && b >= MB ? kb0 & step[b < MB ? 0 : b - MB][u] : kb0);
-        if (ONCE && b >= MB) {
+        for (int u = 0; u < 2; ++u) {
+          const uint16_t *const src = rp[b][u] + (MANY && b >= MB ? kb0 & step[b < MB ? 0 : b - MB][u] : kb0);
+          if (decltype(a_once)::value && b >= MB) {
 #pragma unroll
-          for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16_once(src + uu * WAVES * SHRINK_KSTEP);
-        } else {
+            for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16_once(src + uu * WAVES * SHRINK_KSTEP);
+          } else {
 #pragma unroll
-          for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16(src + uu * WAVES * SHRINK_KSTEP);
+            for (int uu = 0; uu < U; ++uu) buf[uu * BLKS + b][u] = load16(src + uu * WAVES * SHRINK_KSTEP);
+          }
         }
-      }
-    requested();
-    use();
-  }
+      requested();
+      use();
+    }
+  };
+  if (MAY_ONCE && until_once < 0) whole_batches(std::true_type{});
+  else whole_batches(std::false_type{});
   // what is left of the chunk, less than a batch (or all of it, where a rank row lies outside the index or the pool): steps and
   // lanes past its end read zeros, and so do rows that are not there
   for (; kb0 < kend; kb0 += WAVES * SHRINK_KSTEP * U) {
@@ -200,7 +219,7 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
           const int nb = b < MB ? 0 : b - MB;
-          buf[uu * BLKS + b][u] = load16(as_global(kok && (b < MB || ok[nb][u]) ? rp[b][u] + k : g_shrink_zeros));
+          buf[uu * BLKS + b][u] = load16(as_global(kok && (b < MB || (PINNED ? step[nb][u] != 0 : ok[nb][u])) ? rp[b][u] + k : g_shrink_zeros));
         }
     }
     requested();
@@ -219,15 +238,20 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
   __syncthreads();
 }
 
-// Whether A's rows are read as lines that nobody reads again (load16_once): few tokens a tile, so that most adapters have one tile; more
-// of A than an L2 holds (one token over 8 adapters, a pass of 64 calls 379 / 398 us with it, 900 tokens over 12 adapters with their
-// compensation 585 / 664); rows of whole lines; and not rank 8 alone, where the lanes of the other eight rows read the last one again (128
-// adapters, 0.993).   Cold layers, without / with, a pass: 512 tokens
-// over 128 adapters of rank 128 864 / 841 us, 256 over 64 of rank 16 928 / 922, 77 over ranks 8-64 617 / 608; 18 batches of 14 to 900
-// tokens 1.024 times as fast in the mean (60 over 16 of rank 64 64.7 / 57.7).
-inline bool shrink_reads_once(const ShrinkArgs &a, int64_t n_tiles, int max_rank) {
-  return max_rank > 8 && a.T < 5 * n_tiles && n_tiles * a.rp * a.h_in * a.n_targets * 2 >= ((int64_t)4 << 20) && !(a.h_in & 63) &&
-         !(reinterpret_cast<uintptr_t>(a.pool.w) & 127u);
+// From how many tiles of the list on A is read as lines that nobody reads again (load16_once), by a tile that is its adapter's only one;
+// shrink_kernel, 16-token tiles.  The record says whether it is, and of how many: the host knows the resident adapters, not those that a
+// batch touches, and where tiles share A such loads lose most (512 tokens of rank 128 on one of 128 adapters, a pass 243 us without, 299 with
+// them; 900 of rank 32 on four 354 / 385).  From 4 MB of A on, more than an L2 holds (one token over 8 adapters, a pass of 64 calls
+// 379 / 398); in rows of whole lines; not for rank 8 alone, where the lanes of the other eight rows read the last one again (128
+// adapters, 0.993); nor for batches of five tokens a tile and more.  A pass, plain loads / this: 512 tokens over 128 adapters of rank 128
+// 633 / 611 us, 900 over 128 of rank 64 563 / 537, 77 over ranks 8-64 473 / 456; twelve batches of 14 to 900 tokens 1.026 in the mean, and
+// twelve of as many tokens on one to four of up to 128 adapters 1.00 to 1.09 (what is above 1.02 is y written through)
+// (the one-launch op, which has no scalar register left for it, reads A the plain way: 256 tokens over 64 adapters of rank 16, a pass
+// of 16 layers 453 us, 450 with such loads).
+inline int shrink_once_tiles(const ShrinkArgs &a, int64_t n_tiles, int max_rank) {
+  const int64_t tile_bytes = (int64_t)a.rp * a.h_in * a.n_targets * 2;
+  if (max_rank <= 8 || a.compensate || a.T >= 5 * n_tiles || (a.h_in & 63) || (reinterpret_cast<uintptr_t>(a.pool.w) & 127u)) return 0x7fffffff;
+  return (int)((((int64_t)4 << 20) + tile_bytes - 1) / tile_bytes);
 }
 
 }  // namespace mlora
