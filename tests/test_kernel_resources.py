@@ -66,3 +66,29 @@ def test_scalar_spills_are_the_known_ones(tmp_path):
         assert number("private_segment_fixed_size") == 0, symbol
         allowed = max((n for pattern, n in known.items() if re.search(pattern, symbol)), default=0)
         assert number("sgpr_spill_count") <= allowed, (symbol, number("sgpr_spill_count"))
+
+
+def kernel_code(tmp_path, pattern):
+    """(symbol, its instructions) of the library's kernels whose symbol matches."""
+    objdump = os.path.join(LLVM, "llvm-objdump")
+    if not shutil.which(objdump):
+        pytest.skip("needs the toolchain's llvm-objdump")
+    for _ in kernel_metadata(tmp_path):   # (leaves the device images behind)
+        pass
+    for f in sorted(tmp_path.glob("*.co")):
+        if re.search(pattern.encode(), f.read_bytes()):
+            text = subprocess.run([objdump, "-d", "--no-show-raw-insn", str(f)], check=True, capture_output=True, text=True).stdout
+            for part in re.split(r"\n(?=[0-9a-f]+ <)", text):
+                name = re.match(r"[0-9a-f]+ <(\S+)>:", part)
+                if name and re.search(pattern, name.group(1)):
+                    yield name.group(1), part
+
+
+def test_small_expand_stores_y_one_way(tmp_path):
+    """A launch that writes y through and one that does not are different kernels: with both kinds in one, every launch of a few tokens
+    pays for the exchange of halves that only the former need (0.15 of 3.6 us)."""
+    kinds = {}
+    for symbol, code in kernel_code(tmp_path, "expand_small_kernel"):
+        stores = re.findall(r"global_store_dwordx4 [^\n]*", code)
+        kinds.setdefault(frozenset("sc1" in s for s in stores), []).append(symbol)
+    assert set(kinds) == {frozenset([True]), frozenset([False])}, {k: len(v) for k, v in kinds.items()}

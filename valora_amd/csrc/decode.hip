@@ -305,7 +305,8 @@ __global__ __launch_bounds__(256, 3) void decode_kernel(const int32_t *tiles_bas
     f32x4 acc[4];
     small_product<T, KB>(raw[c], vfrag, rk, lane, acc);
     small_add<T, KB>(yy[c], acc, scale);
-    small_store_y(yy[c], lane, cnt, o_wave + c * 256u, (uint32_t)h_out, THROUGH);
+    if constexpr (!THROUGH) small_store_y(yy[c]);
+    else if (o_wave + c * 256u < (uint32_t)h_out) small_store_y_through(yy[c], lane, cnt);
   }
   // the tile's last expand item tops the tile's `done` word up to the launch's weight
   if (tid == 0 && item == h_n_consumers - 1) add_device(done_base + tile_idx, DECODE_LAUNCH_WEIGHT - (uint32_t)n_producers);

@@ -263,7 +263,9 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 constexpr int small_min_waves(int kb, bool wide, bool comp) {   // as many as do without spills
   return comp ? (kb <= 1 ? 7 : 1) : kb <= 1 ? 8 : kb == 2 ? (wide ? 6 : 5) : (wide ? 4 : 3);
 }
-template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP>
+// THROUGH: y is written through (expand_core.h), up to rank 64.  A form of its own here as well: the exchange of halves behind a flag costs the
+// others 0.12 to 0.18 us a launch (5 tokens of rank 16, two targets of 14336 columns 3.62 / 3.50 us, one of 4096 4.48 / 4.30).
+template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP, bool THROUGH>
 __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_small_kernel(const int32_t *tiles_base, const int32_t *perm,
                                                                                          const int64_t *a_loc, int h_n_loc, int h_out,
                                                                                          ExpandArgs p) {
@@ -274,13 +276,12 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
   const int32_t *__restrict__ tile = tiles_base + (int64_t)tile_idx * TILE_WORDS;
   int ad = tile[0], r = tile[1], pos0 = tile[2], cnt = tile[3], astart = tile[4];
   int slot = p.slots[z], kmax = p.kmax, w_rows = (int)p.w_rows_t[z], v_by_pos = p.v_by_pos;
-  int through = KB < 4 ? p.through : 0;
   uint16_t *y = p.ys[z];
   const uint16_t *w = p.ws[z], *v = p.v, *scales = p.scales;
   int64_t v_tstride = p.v_tstride, v_stride = p.v_stride;
   float inv_h_out = p.inv_h_out;
   asm volatile("" : "+s"(ad), "+s"(r), "+s"(pos0), "+s"(cnt), "+s"(astart), "+s"(slot), "+s"(kmax), "+s"(w_rows), "+s"(v_by_pos),
-                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out), "+s"(through));
+                    "+s"(y), "+s"(w), "+s"(v), "+s"(scales), "+s"(v_tstride), "+s"(v_stride), "+s"(inv_h_out));
   if (COMP) cnt = abs(cnt);                  // (negative: no usable rank of its own, r = 0)
   if (cnt <= 0) return;                      // records past the last tile are zero
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -345,19 +346,23 @@ __global__ __launch_bounds__(256, small_min_waves(KB, WIDE, COMP)) void expand_s
     small_product<T, KB>(raw, vfrag, pool.rk, lane, acc);
     small_add<T, KB>(yy, acc, scale);
   }
-  small_store_y(yy, lane, cnt, o_wave, (uint32_t)h_out, KB < 4 && through);
+  if constexpr (THROUGH) small_store_y_through(yy, lane, cnt);
+  else small_store_y(yy);
 }
 
 template <typename T, int KB>
 int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
   // an index without entries: the kernel reads one all the same, and drops it
   const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
-#define MLORA_SMALL(WIDE, PARTIAL, COMP)                                                                        \
-  hipLaunchKernelGGL((expand_small_kernel<T, KB, WIDE, PARTIAL, COMP>), grid, dim3(256), 0, st, records,        \
+#define MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, THROUGH)                                                           \
+  hipLaunchKernelGGL((expand_small_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH>), grid, dim3(256), 0, st, records, \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
-#define MLORA_SMALL_WIDTH(PARTIAL, COMP)                             \
-  if (KB > 0 && a.h_out >= SMALL_WIDE) MLORA_SMALL((KB > 0), PARTIAL, COMP); \
-  else MLORA_SMALL(false, PARTIAL, COMP)
+#define MLORA_SMALL(WIDE, PARTIAL, COMP)                                                          \
+  if (KB < 4 && a.through) MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, (KB < 4));                       \
+  else MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, false)
+#define MLORA_SMALL_WIDTH(PARTIAL, COMP)                                           \
+  if (KB > 0 && a.h_out >= SMALL_WIDE) { MLORA_SMALL((KB > 0), PARTIAL, COMP); }   \
+  else { MLORA_SMALL(false, PARTIAL, COMP); }
   // Exactly as many workgroups as there are records: what stands behind the last one is no record (the words of the one-launch
   // op do, and a call of that kind leaves them non-zero).  More tiles than a grid's y takes (a million tokens) are several launches.
   for (int64_t t0 = 0; t0 < tiles; t0 += MAX_GRID_TILES) {
@@ -369,6 +374,7 @@ int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
   }
 #undef MLORA_SMALL_WIDTH
 #undef MLORA_SMALL
+#undef MLORA_SMALL_FORM
   return check_launch("expand_small_kernel");
 }
 
@@ -388,8 +394,8 @@ int launch_expand_kb(hipStream_t st, const ExpandArgs &a, int bm, int64_t tiles)
 #define MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, THROUGH)                                                         \
   hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH>), grid, dim3(256), lds, st, records,   \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
-#define MLORA_EXPAND(WIDE, PARTIAL, COMP)                               \
-  if (a.through) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, true);          \
+#define MLORA_EXPAND(WIDE, PARTIAL, COMP)                                  \
+  if (a.through) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, true);             \
   else MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, false)
 #define MLORA_EXPAND_WIDTH(PARTIAL, COMP)                     \
   if (a.h_out >= SMALL_WIDE) { MLORA_EXPAND(true, PARTIAL, COMP); } \

@@ -250,15 +250,13 @@ __device__ __forceinline__ void small_v_partials(const float *tile, uint32_t row
 // a few tokens, where the way to memory is longer than the write-back of what little there is.
 constexpr int64_t THROUGH_BYTES = (int64_t)2 << 20, THROUGH_BYTES_ONE_LAUNCH = (int64_t)3 << 20;
 // And only rows of whole 128-byte lines: a line that two waves store a piece of each goes to memory twice (6700 tokens of rank 64, 4128
-// and 8224 columns, a pass of two layers 804 us without, 922 with).
+// and 8224 columns, a pass of two layers 804 us without, 922 with).  Not in 16-token tiles above rank 64 (csrc/expand.hip), which read
+// much more than they write (512 tokens over 128 adapters of rank 128, q+k+v 79.2 / 80.4 us, and 80.0 with the choice alone).
 inline int write_through(const ExpandArgs &a, int64_t least) {
   uintptr_t ends = 0;
   for (int z = 0; z < a.n_targets; ++z) ends |= reinterpret_cast<uintptr_t>(a.ys[z]);
   return (int64_t)a.T * a.h_out * a.n_targets * 2 >= least && !(a.h_out & 63) && !(ends & 127u);
 }
-// Not in 16-token tiles above rank 64, which read much more than they write (512 tokens over 128 adapters of rank 128, q+k+v 79.2 / 80.4
-// us, and 80.0 with the choice alone).
-
 // The lane's outputs of y: 16 from o_wave + 16 * (lane / 16) on, in two 16-byte halves.
 template <int KB>
 struct SmallY {
@@ -288,18 +286,19 @@ __device__ __forceinline__ void small_add(SmallY<KB> &s, const f32x4 (&acc)[4], 
     s.v[h] = pack8<T>(f);
   }
 }
-// cnt: tokens of the tile; through: wave-uniform (launch_expand, launch_decode).  A lane's halves lie 16 or 64 bytes apart, so that a store
-// of one half writes pieces of lines.  That is all the same to the L2; on their way to memory the lanes of a pair, two tokens of the
-// same columns, exchange a half first: every store then writes whole lines of one token.
 template <int KB>
-__device__ __forceinline__ void small_store_y(const SmallY<KB> &s, int lane, int cnt, uint32_t o_wave, uint32_t h_out, bool through) {
-  constexpr int H = KB ? 8 : 32;
-  if (!through) {
+__device__ __forceinline__ void small_store_y(const SmallY<KB> &s) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-      if (s.ok[h]) store16(s.p + h * H, s.v[h]);
-    return;
-  }
+  for (int h = 0; h < 2; ++h)
+    if (s.ok[h]) store16(s.p + h * (KB ? 8 : 32), s.v[h]);
+}
+// The same, written through, where rows are whole lines (write_through) and the wave's outputs are there; cnt: tokens of the tile.  A
+// lane's halves lie 16 or 64 bytes apart, so that a store of one half writes pieces of lines.  That is all the same to the L2; on their way
+// to memory the lanes of a pair, two tokens of the same columns, exchange a half first: every store then writes whole lines of one token.
+template <int KB>
+__device__ __forceinline__ void small_store_y_through(const SmallY<KB> &s, int lane, int cnt) {
+  constexpr int H = KB ? 8 : 32;
+  const int m = lane & 15;
   const bool odd = lane & 1;
   const u32x4 give = odd ? s.v[0] : s.v[1];
   u32x4 got;
@@ -309,10 +308,8 @@ __device__ __forceinline__ void small_store_y(const SmallY<KB> &s, int lane, int
   const uint64_t other = (uint64_t)lane_pair((uint32_t)own) | (uint64_t)lane_pair((uint32_t)(own >> 32)) << 32;
   uint16_t *const even_row = reinterpret_cast<uint16_t *>(odd ? other : own) + (odd ? H : 0);
   uint16_t *const odd_row = reinterpret_cast<uint16_t *>(odd ? own : other) + (odd ? H : 0);
-  const bool col = o_wave + (uint32_t)((lane >> 4) * (KB ? 16 : 8) + (odd ? H : 0)) < h_out;
-  const int m = lane & 15;
-  if (col && (m & ~1) < cnt) store16_through(even_row, odd ? got : s.v[0]);
-  if (col && (m | 1) < cnt) store16_through(odd_row, odd ? s.v[1] : got);
+  if ((m & ~1) < cnt) store16_through(even_row, odd ? got : s.v[0]);
+  if ((m | 1) < cnt) store16_through(odd_row, odd ? s.v[1] : got);
 }
 
 }  // namespace mlora
