@@ -92,3 +92,10 @@ def test_small_expand_stores_y_one_way(tmp_path):
         stores = re.findall(r"global_store_dwordx4 [^\n]*", code)
         kinds.setdefault(frozenset("sc1" in s for s in stores), []).append(symbol)
     assert set(kinds) == {frozenset([True]), frozenset([False])}, {k: len(v) for k, v in kinds.items()}
+
+
+def test_compensation_has_no_form_that_writes_y_through(tmp_path):
+    """How much of y a compensation writes is not known at the launch; template arguments ..., COMP, THROUGH."""
+    forms = {s for s, _ in kernel_metadata(tmp_path) if re.search(r"\d+expand_(small_)?kernelI", s)}
+    assert any(re.search(r"Lb0ELb1EEE", s) for s in forms) and any(re.search(r"Lb1ELb0EEE", s) for s in forms)
+    assert not [s for s in forms if re.search(r"Lb1ELb1EEE", s)]

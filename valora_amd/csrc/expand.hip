@@ -358,7 +358,7 @@ int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
   hipLaunchKernelGGL((expand_small_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH>), grid, dim3(256), 0, st, records, \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
 #define MLORA_SMALL(WIDE, PARTIAL, COMP)                                                          \
-  if (KB < 4 && a.through) MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, (KB < 4));                       \
+  if (KB < 4 && !COMP && a.through) MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, (KB < 4 && !COMP));     \
   else MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, false)
 #define MLORA_SMALL_WIDTH(PARTIAL, COMP)                                           \
   if (KB > 0 && a.h_out >= SMALL_WIDE) { MLORA_SMALL((KB > 0), PARTIAL, COMP); }   \
@@ -395,7 +395,7 @@ int launch_expand_kb(hipStream_t st, const ExpandArgs &a, int bm, int64_t tiles)
   hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH>), grid, dim3(256), lds, st, records,   \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
 #define MLORA_EXPAND(WIDE, PARTIAL, COMP)                                  \
-  if (a.through) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, true);             \
+  if (!COMP && a.through) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, !COMP);   \
   else MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, false)
 #define MLORA_EXPAND_WIDTH(PARTIAL, COMP)                     \
   if (a.h_out >= SMALL_WIDE) { MLORA_EXPAND(true, PARTIAL, COMP); } \
