@@ -99,3 +99,9 @@ def test_compensation_has_no_form_that_writes_y_through(tmp_path):
     forms = {s for s, _ in kernel_metadata(tmp_path) if re.search(r"\d+expand_(small_)?kernelI", s)}
     assert any(re.search(r"Lb0ELb1EEE", s) for s in forms) and any(re.search(r"Lb1ELb0EEE", s) for s in forms)
     assert not [s for s in forms if re.search(r"Lb1ELb1EEE", s)]
+
+
+def test_partials_are_read_once_in_a_form_of_their_own(tmp_path):
+    """Rows of the partials that are no whole lines, and a compensation's, are read the plain way: some launch has no non-temporal load."""
+    kinds = {bool(re.search(r"global_load_dwordx4 [^\n]*\bnt\b", code)) for _, code in kernel_code(tmp_path, "shrink_reduce_kernel")}
+    assert kinds == {True, False}

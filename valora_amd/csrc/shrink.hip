@@ -85,7 +85,8 @@ __device__ __forceinline__ void store_v4(const ShrinkArgs &p, int pos, int t, in
 // Bound by a launch and three round trips (arguments, chunks, store): a few MB.  Four or eight chunks are requested before any
 // is used, beside the row's look-ups; no division.  With 64-bit divisions, a round trip per conditional chunk and 2-byte stores:
 // 7600 tokens of rank 32 in four chunks 3.5 us a launch, now 2.7.
-template <typename T>
+// ONCE: the chunks are read as lines that nobody reads again (launch_shrink_reduce).
+template <typename T, bool ONCE>
 __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_plan, const float *h_partial, int h_quarter, float h_inv_quarter,
                                                             int h_flags, int h_ksplit, ShrinkArgs args_in) {
   const ShrinkArgs p = select_target(args_in, blockIdx.y);
@@ -110,7 +111,9 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
     f32x4 q[BATCH];
 #pragma unroll
     for (int u = 0; u < BATCH; ++u) {
-      q[u] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(chunk + at));   // (nobody reads them again)
+      const f32x4 *const src = reinterpret_cast<const f32x4 *>(chunk + at);
+      if constexpr (ONCE) q[u] = __builtin_nontemporal_load(src);
+      else q[u] = *src;
       chunk = next_chunk(chunk, s0 + u + 1 < h_ksplit, stride);
     }
     requested();
@@ -839,10 +842,18 @@ int launch_shrink_reduce(hipStream_t st, const ShrinkArgs &a, mlora_dtype dt) {
   if (a.T <= 0) return MLORA_OK;
   const int quarter = (int)(a.rp >> 2), rows = 256 / quarter;   // at most 32 quarters
   const dim3 grid((unsigned)((a.T + rows - 1) / rows), (unsigned)a.n_targets);
-#define MLORA_REDUCE(T) \
-  hipLaunchKernelGGL(shrink_reduce_kernel<T>, grid, dim3(256), 0, st, a.plan, a.partial, quarter, 1.f / (float)quarter, head_flags(a), a.ksplit, a)
-  if (dt == MLORA_F16) MLORA_REDUCE(_Float16);
-  else MLORA_REDUCE(__bf16);
+  // Partials are read as lines that nobody reads again where rows are whole lines (in others two workgroups share some: 2965 tokens of ranks
+  // 16-48, a pass of three layers 259 us with such loads, 257 without), but not in compensations, which read few of them (a pass with / without:
+  // 6368 tokens over ranks 16-64, 466 of them not the merged adapter's 751 / 746 us, 2657 1073 / 1059; 2817 of rank 128, 2 505 / 497).
+  const bool once = !a.compensate && (a.rp & 31) == 0 && (reinterpret_cast<uintptr_t>(a.partial) & 127u) == 0;
+#define MLORA_REDUCE_FORM(T, ONCE) \
+  hipLaunchKernelGGL((shrink_reduce_kernel<T, ONCE>), grid, dim3(256), 0, st, a.plan, a.partial, quarter, 1.f / (float)quarter, head_flags(a), a.ksplit, a)
+#define MLORA_REDUCE(T)                   \
+  if (once) MLORA_REDUCE_FORM(T, true);   \
+  else MLORA_REDUCE_FORM(T, false)
+  if (dt == MLORA_F16) { MLORA_REDUCE(_Float16); }
+  else { MLORA_REDUCE(__bf16); }
+#undef MLORA_REDUCE_FORM
 #undef MLORA_REDUCE
   return check_launch("shrink_reduce_kernel");
 }
