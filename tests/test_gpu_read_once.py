@@ -4,6 +4,7 @@ import pytest
 import torch
 
 from oracle import lora_oracle as O
+from valora_amd import _lib
 from valora_amd import workloads as W
 from valora_amd.plan import LoraPlan
 
@@ -33,14 +34,18 @@ def _bound(dtype):
                                              if not one or (r <= 32 and k > 1)])
 @pytest.mark.parametrize("odd", [0, 64, -128])   # K ranges that are whole batches of steps, or end in the middle of one
 def test_rows_of_a_in_small_tiles(dev, rank, one, ksplit, odd):
-    """4 MB of A and more in the whole batch, less in each half."""
-    n, T = 40, 43
+    """4 MB of A and more in the whole batch, less in each half; every adapter has one tile.  (The one-launch op reads A the plain way
+    whatever the size.)"""
+    n, T = 44, 47
     h_in = 65536 // rank + odd
     dtype = torch.bfloat16 if odd else torch.float16
     print(rank, one, ksplit, h_in, flush=True)
     rp = rank
-    assert ((T + 15) // 16 + n) * rp * h_in * 2 >= 4 << 20 > ((T + 31) // 32 + (T + 1) // 2) * rp * h_in * 2
-    pool, ids, x, y0 = _case(T, n, rank, h_in, 264, dtype, rank + odd)
+    pool, _, x, y0 = _case(T, n, rank, h_in, 264, dtype, rank + odd)
+    ids = torch.arange(T) * 7 % n
+    ids[5] = -1
+    tiles = [len(set(part.tolist()) - {-1}) for part in (ids, ids[:T // 2], ids[T // 2:])]
+    assert tiles[0] * rp * h_in * 2 >= 4 << 20 > max(tiles[1:]) * rp * h_in * 2
     p, xd = pool.to(dev), x.to(dev)
     idx = (p.a_start, p.a_len, p.a_loc)
 
@@ -61,7 +66,8 @@ def test_rows_of_a_in_small_tiles(dev, rank, one, ksplit, odd):
                                               for bm in (128, 256) for t in (1, 2, 3) if bm == 128 or (max(r) <= 64 and t == 1)])
 @pytest.mark.parametrize("ksplit", [1, 2, 4])
 def test_tall_tiles(dev, ranks, bm, targets, ksplit):
-    """x on 128-byte lines against the same x beside them, which is read, and whose partial sums are written, the plain way."""
+    """x and scratch on 128-byte lines; the same with x beside them, which is read the plain way; and with scratch beside them, whose partial
+    sums are written and read the plain way."""
     T, h_in, h_out = 5861, 576, 72       # two and three targets in four chunks share a workgroup
     g = torch.Generator().manual_seed(ranks[0] + bm + targets)
     dtype = torch.bfloat16 if ranks[0] == 64 else torch.float16
@@ -83,7 +89,16 @@ def test_tall_tiles(dev, ranks, bm, targets, ksplit):
         y = y0.to(dev)
         plan.apply_multi(list(y.unbind(0)), xd, p.key_buffer, p.value_buffer, *idx, list(range(targets)), p.a_scaling)
         got.append(y)
-    assert torch.equal(got[0], got[1])
+    xd, y = x.to(dev), y0.to(dev)
+    assert xd.data_ptr() % 128 == plan.scratch.data_ptr() % 128 == 0
+    tg = (_lib.Target * targets)(*[_lib.Target(_lib.ptr(y[i]), _lib.ptr(p.value_buffer), p.value_buffer.numel() // h_out, i) for i in range(targets)])
+    _lib.check(_lib.lib().mlora_lora_apply_multi(_lib.current_stream(dev), plan.handle, _lib.c_void_p(plan.scratch.data_ptr() + 16),
+                                                 plan.scratch.numel() - 16, _lib.ptr(xd), T, h_in, h_out, max(ranks),
+                                                 _lib.make_pool(p.key_buffer, *idx, h_in, 3), targets, tg, _lib.ptr(p.a_scaling), plan.ksplit,
+                                                 plan.flags, _lib.dtype_code(dtype)))
+    torch.cuda.synchronize()
+    got.append(y)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])
     for t in range(targets):
         want = O.lora_op(y0[t], x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, t, pool.a_scaling, n_slots=3)
         assert O.rel_l2(got[0][t].cpu(), want) <= _bound(dtype)

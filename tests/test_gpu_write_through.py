@@ -1,5 +1,7 @@
 """Launches that write y on to memory at once (from 2 MB of y on, 3 MB where the op is one launch) against the same tokens in
-batches below that size: the same bits, for tiles of odd and even token counts, widths that end inside a chunk, tokens without an adapter, and nothing written beside the rows."""
+batches below that size: the same bits, for tiles of odd and even token counts, widths that end inside a chunk, tokens without an
+adapter, and nothing written beside the rows.  16-token tiles above rank 64 and compensations are never written through: their cases hold that
+large batches give the bits of small ones all the same."""
 import pytest
 import torch
 
@@ -30,7 +32,7 @@ def _framed(y):
 
 
 def _both(dev, make_plan, call, pool, ids, x, y0, least):
-    """The whole batch, and its two halves; the former writes through, the latter do not."""
+    """The whole batch, and its two halves; the former is above the size from which y is written through, the latter are below."""
     T, h_out = y0.shape
     assert T * h_out * 2 >= least > (T + 1) // 2 * h_out * 2
     whole, parts = _framed(y0), _framed(y0)
@@ -77,3 +79,42 @@ def test_compensation_same_bits_as_smaller_batches(dev, ranks, bm):
     want = O.delora_compensate(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1, 1, pool.a_scaling,
                                n_slots=2)
     assert O.rel_l2(got.cpu(), want) <= REL_L2
+
+
+@pytest.mark.parametrize("h_out", [1600, 4128])   # the latter's rows are no whole lines: never written through
+@pytest.mark.parametrize("targets", [2, 3])
+@pytest.mark.parametrize("ranks,bm,one", [([16, 8], 16, True), ([32, 24, 8], 16, True), ([32, 24, 8], 16, False), ([64, 40, 8], 16, False),
+                                          ([16, 8], 48, False), ([64, 40, 8], 48, False), ([128, 72, 16], 48, False)])
+def test_targets_count_together_and_one_beside_lines(dev, h_out, targets, ranks, bm, one):
+    """Targets that reach the size only together, all on 128-byte lines; the same with the last one beside them, which is written, with the
+    others, the plain way; and the targets one by one, below the size.  Nothing beside the rows."""
+    least = (3 if one else 2) << 20
+    T = least // (2 * h_out * targets) + 5
+    assert T * h_out * 2 * targets >= least > T * h_out * 2
+    pool, ids, x, y0 = _case(T, h_out, ranks, torch.float16, targets + ranks[0])
+    print(T, h_out, targets, ranks, bm, one, flush=True)
+    p, xd = pool.to(dev), x.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    plan = LoraPlan(ids.to(dev), *idx[:2], max(ranks), n_slots=2, hidden=H_IN, bm_shrink=16, bm_expand=bm, one_launch=one, ksplit=2)
+    slots = [z % 2 for z in range(targets)]
+
+    def run(offs, calls):
+        rooms = [torch.full(((T + 2) * h_out + 64,), 7.0, dtype=torch.float16, device=dev) for _ in offs]
+        rows = [room[off:off + (T + 2) * h_out].view(T + 2, h_out) for room, off in zip(rooms, offs)]
+        ys = [r[1:-1].copy_(y0.to(dev)) for r in rows]
+        if h_out % 64 == 0:
+            assert [y.data_ptr() % 128 == 0 for y in ys] == [off % 64 == 0 for off in offs]
+        for zs in calls:
+            plan.apply_multi([ys[z] for z in zs], xd, p.key_buffer, p.value_buffer, *idx, [slots[z] for z in zs], p.a_scaling)
+        for y, room, off in zip(ys, rooms, offs):
+            a = off + h_out
+            assert bool((room[:a] == 7).all() and (room[a + T * h_out:] == 7).all())
+        return torch.stack(ys)
+
+    together = list(range(targets))
+    got = run([0] * targets, [together])
+    assert torch.equal(got, run([0] * (targets - 1) + [8], [together]))
+    assert torch.equal(got, run([0] * targets, [[z] for z in together]))
+    for z in together:
+        want = O.lora_op(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, slots[z], pool.a_scaling, n_slots=2)
+        assert O.rel_l2(got[z].cpu(), want) <= REL_L2
