@@ -95,10 +95,12 @@ def test_small_expand_stores_y_one_way(tmp_path):
 
 
 def test_compensation_has_no_form_that_writes_y_through(tmp_path):
-    """How much of y a compensation writes is not known at the launch; template arguments ..., COMP, THROUGH."""
-    forms = {s for s, _ in kernel_metadata(tmp_path) if re.search(r"\d+expand_(small_)?kernelI", s)}
-    assert any(re.search(r"Lb0ELb1EEE", s) for s in forms) and any(re.search(r"Lb1ELb0EEE", s) for s in forms)
-    assert not [s for s in forms if re.search(r"Lb1ELb1EEE", s)]
+    """How much of y a compensation writes is not known at the launch."""
+    args = {"expand_kernel": r"Lb(\d)ELb(\d)ELb\dEEE", "expand_small_kernel": r"Lb(\d)ELb(\d)EEE"}   # ..., COMP, THROUGH (, ONCE)
+    symbols = [s for s, _ in kernel_metadata(tmp_path)]
+    for kernel, last in args.items():
+        forms = {re.search(last, s).groups() for s in symbols if re.search(r"\d+" + kernel + "I", s)}
+        assert forms == {("0", "0"), ("0", "1"), ("1", "0")}, kernel
 
 
 def test_partials_are_read_once_in_a_form_of_their_own(tmp_path):

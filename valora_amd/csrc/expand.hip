@@ -46,16 +46,19 @@ constexpr int expand_min_waves(int kb, bool partial, bool comp) {
 // 108.8 / 99.4; 5401 tokens over ranks 8-64 24.8 / 22.6, 57.9 / 54.5, 93.0 / 90.9; 10000 tokens over 8 adapters of rank 128, shrink and
 // expand 106 / 92.  (Of the 109 us, B and v together were 29, v alone 8.  One more or one less waves' worth of registers spills or gains
 // nothing; 16 instead of 8 staged tokens, 8.7 KB more LDS, 1 % slower.)
-// y written through instead of left dirty in the L2s for the end of the kernel: 5401 tokens over ranks 8-64, one target of 4096
-// columns 25.7 / 23.1, three 54.6 / 51.9, two of 11008 93.3 / 90.9 (with non-temporal stores the same as with plain ones).
-// THROUGH: y is written through (expand_core.h), and read as lines that nobody reads again (load16_once), so that the caches keep B and v: a
-// pass of two layers, plain reads / these, 5401 tokens over ranks 8-64 682 / 675 us, 14000 over ranks 8-64, 5120 wide 786 / 744, 7000 of rank
-// 128 411 / 404; 15 prefill batches 1.011 in the mean, 0.99 at worst (1600 tokens).  (A form of its own: above rank 64 no scalar
-// register is left for a flag.  In 16-token tiles such reads are 0.995.)
+// THROUGH: y is written through (write_through, expand_core.h) instead of left dirty in the L2s for the end of the kernel.  A pass, plain /
+// through (with ONCE where it is on): 5401 tokens over ranks 8-64, seven projections of 4096 and 11008, 686 / 664 us; 5254 of rank 64 660 / 638;
+// 14000 over ranks 8-64, 5120 wide 1878 / 1840; 3887 of rank 64 whose chunks are summed here (PARTIAL) 340 / 334; 1200 of rank 64 433 / 421.
+// What it gives stands mostly in the next launch: of the first batch three targets of 4096 columns take 60.9 / 57.5 us, two of 11008
+// 97.1 / 93.1, one 24.5 / 22.1, but 49.6, 87.7 and 20.8 where the shrinks read x the plain way, which lose more than that (csrc/shrink.hip).
+// ONCE: and y is read as lines that nobody reads again (load16_once), so that the caches keep B and v, from ONCE_BYTES on; not where
+// the chunks are summed here (0.996).  A pass, plain reads / these: 5401 tokens over ranks 8-64 676 / 664 us, 14000 1870 / 1840, 7000 of
+// rank 128 604 / 596; with less of y in a launch they lose: 1200 tokens of rank 64, 3072 wide, in calls of one target 395 / 406, 2600
+// 520 / 530.  (Forms of their own: above rank 64 no scalar register is left for a flag.  In 16-token tiles such reads are 0.995.)
 // COMP: the compensation of a request whose base weights hold another adapter (csrc/api.hip, mlora_lora_compensate):
 // y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), where v' is the "target" 1 matrix of the same positions:
 // both products in one pass over y.
-template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP, bool THROUGH>
+template <typename T, int KB, bool WIDE, bool PARTIAL, bool COMP, bool THROUGH, bool ONCE>
 __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expand_kernel(const int32_t *tiles_base, const int32_t *perm,
                                                                                     const int64_t *a_loc, int h_n_loc, int h_out,
                                                                                     ExpandArgs p) {
@@ -181,7 +184,7 @@ __global__ __launch_bounds__(256, expand_min_waves(KB, PARTIAL, COMP)) void expa
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         yp[b][h] = ycol + (uint64_t)(uint32_t)t[b][h] * (uint32_t)h_out;
-        yv[b][h] = THROUGH ? load16_once(yp[b][h]) : load16(yp[b][h]);
+        yv[b][h] = ONCE ? load16_once(yp[b][h]) : load16(yp[b][h]);
       }
   };
   u32x4 bfrag[4 * KB], bfrag2[COMP ? 4 * KB : 1];
@@ -391,12 +394,14 @@ int launch_expand_kb(hipStream_t st, const ExpandArgs &a, int bm, int64_t tiles)
   // an index without entries: the kernel reads one all the same, and drops it
   const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
   const int lds = bm * ((a.compensate ? 2 : 1) * expand_v_chunks(KB) * 16 + 4);
-#define MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, THROUGH)                                                         \
-  hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH>), grid, dim3(256), lds, st, records,   \
+  const bool once = a.through && write_through(a, ONCE_BYTES);
+#define MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, THROUGH, ONCE)                                                         \
+  hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH, ONCE>), grid, dim3(256), lds, st, records,   \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
-#define MLORA_EXPAND(WIDE, PARTIAL, COMP)                                  \
-  if (!COMP && a.through) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, !COMP);   \
-  else MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, false)
+#define MLORA_EXPAND(WIDE, PARTIAL, COMP)                                                             \
+  if (!COMP && !PARTIAL && once) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, !COMP, (!COMP && !PARTIAL));  \
+  else if (!COMP && a.through) MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, !COMP, false);                  \
+  else MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, false, false)
 #define MLORA_EXPAND_WIDTH(PARTIAL, COMP)                     \
   if (a.h_out >= SMALL_WIDE) { MLORA_EXPAND(true, PARTIAL, COMP); } \
   else { MLORA_EXPAND(false, PARTIAL, COMP); }
