@@ -68,7 +68,8 @@ def test_rows_of_a_in_small_tiles(dev, rank, one, ksplit, odd):
 def test_tall_tiles(dev, ranks, bm, targets, ksplit):
     """x and scratch on 128-byte lines; the same with x beside them, which is read the plain way; and with scratch beside them, whose partial
     sums are written and read the plain way."""
-    T, h_in, h_out = 5861, 576, 72       # two and three targets in four chunks share a workgroup
+    T, h_in, h_out = 5861, 3008, 72      # two and three targets in four chunks share a workgroup; more of x than the L2s hold
+    assert T * h_in * 2 >= 32 << 20
     g = torch.Generator().manual_seed(ranks[0] + bm + targets)
     dtype = torch.bfloat16 if ranks[0] == 64 else torch.float16
     pool = W.make_pool(ranks, h_in, h_out, dtype, g, True, n_slots=3, std=0.05, scalings=[0.5 + 0.25 * i for i in range(len(ranks))],

@@ -118,3 +118,27 @@ def test_targets_count_together_and_one_beside_lines(dev, h_out, targets, ranks,
     for z in together:
         want = O.lora_op(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, slots[z], pool.a_scaling, n_slots=2)
         assert O.rel_l2(got[z].cpu(), want) <= REL_L2
+
+
+@pytest.mark.parametrize("ranks", [[16, 8], [32, 24, 8], [64, 40, 8], [128, 72, 16]])
+@pytest.mark.parametrize("bm,h_out", [(48, 4160), (64, 1600)])
+def test_more_of_y_than_the_l2s_hold(dev, ranks, bm, h_out):
+    """y that is read as lines that nobody reads again as well, against the same y beside 128-byte lines, which is read and written the plain way."""
+    T = (32 << 20) // (2 * h_out) + 7
+    pool, ids, x, y0 = _case(T, h_out, ranks, torch.bfloat16, ranks[0])
+    print(T, h_out, ranks, bm, flush=True)
+    p, xd = pool.to(dev), x.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    plan = LoraPlan(ids.to(dev), *idx[:2], max(ranks), n_slots=2, hidden=H_IN, bm_shrink=16, bm_expand=bm, one_launch=False, ksplit=1)
+    got = []
+    for off in (0, 8):
+        room = torch.full(((T + 2) * h_out + 64,), 7.0, dtype=torch.bfloat16, device=dev)
+        y = room[off + h_out:off + (T + 1) * h_out].view(T, h_out)
+        assert (y.data_ptr() % 128 == 0) == (off == 0)
+        y.copy_(y0)
+        plan.apply(y, xd, p.key_buffer, p.value_buffer, *idx, 1, p.a_scaling)
+        assert bool((room[:off + h_out] == 7).all() and (room[off + (T + 1) * h_out:] == 7).all())
+        got.append(y)
+    assert torch.equal(got[0], got[1])
+    want = O.lora_op(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1, pool.a_scaling, n_slots=2)
+    assert O.rel_l2(got[0].cpu(), want) <= 8 * REL_L2

@@ -51,10 +51,11 @@ constexpr int expand_min_waves(int kb, bool partial, bool comp) {
 // 14000 over ranks 8-64, 5120 wide 1878 / 1840; 3887 of rank 64 whose chunks are summed here (PARTIAL) 340 / 334; 1200 of rank 64 433 / 421.
 // What it gives stands mostly in the next launch: of the first batch three targets of 4096 columns take 60.9 / 57.5 us, two of 11008
 // 97.1 / 93.1, one 24.5 / 22.1, but 49.6, 87.7 and 20.8 where the shrinks read x the plain way, which lose more than that (csrc/shrink.hip).
-// ONCE: and y is read as lines that nobody reads again (load16_once), so that the caches keep B and v, from ONCE_BYTES on; not where
-// the chunks are summed here (0.996).  A pass, plain reads / these: 5401 tokens over ranks 8-64 676 / 664 us, 14000 1870 / 1840, 7000 of
-// rank 128 604 / 596; with less of y in a launch they lose: 1200 tokens of rank 64, 3072 wide, in calls of one target 395 / 406, 2600
-// 520 / 530.  (Forms of their own: above rank 64 no scalar register is left for a flag.  In 16-token tiles such reads are 0.995.)
+// ONCE: and y is read as lines that nobody reads again (load16_once), so that the caches keep B and v, from L2_BYTES on, since less
+// of it stays there until it is written; not where the chunks are summed here (0.996).  A pass, plain reads / these: 5401 tokens over
+// ranks 8-64 676 / 664 us, 14000 1870 / 1840, 7000 of rank 128 604 / 596; with less of y in a launch they lose: 1200 tokens of rank 64, 3072
+// wide, in calls of one target 395 / 406, 2600 520 / 530.  (Forms of their own: above rank 64 no scalar register is left for a flag.  In
+// 16-token tiles such reads are 0.995.)
 // COMP: the compensation of a request whose base weights hold another adapter (csrc/api.hip, mlora_lora_compensate):
 // y = T(T(y + own scale * v B_own) - merged scale * v' B_merged), where v' is the "target" 1 matrix of the same positions:
 // both products in one pass over y.
@@ -394,7 +395,7 @@ int launch_expand_kb(hipStream_t st, const ExpandArgs &a, int bm, int64_t tiles)
   // an index without entries: the kernel reads one all the same, and drops it
   const int64_t *a_loc = a.pool.a_loc_len > 0 ? a.pool.a_loc : reinterpret_cast<const int64_t *>(a.plan + a.off_perm);
   const int lds = bm * ((a.compensate ? 2 : 1) * expand_v_chunks(KB) * 16 + 4);
-  const bool once = a.through && write_through(a, ONCE_BYTES);
+  const bool once = a.through && write_through(a, L2_BYTES);
 #define MLORA_EXPAND_FORM(WIDE, PARTIAL, COMP, THROUGH, ONCE)                                                         \
   hipLaunchKernelGGL((expand_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH, ONCE>), grid, dim3(256), lds, st, records,   \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)

@@ -249,9 +249,6 @@ __device__ __forceinline__ void small_v_partials(const float *tile, uint32_t row
 // launch 0.91 to 0.98 from 4.7 MB on (1201 tokens of rank 16, two targets of 8192 columns 26.9 / 24.7 us), 1.00 at 1 to 2.5 MB, and 1.05 for
 // a few tokens, where the way to memory is longer than the write-back of what little there is.
 constexpr int64_t THROUGH_BYTES = (int64_t)2 << 20, THROUGH_BYTES_ONE_LAUNCH = (int64_t)3 << 20;
-// And from which a tall expand reads it as lines that nobody reads again: what the eight L2s hold together.  Less of it stays there, read the
-// plain way, until it is written.
-constexpr int64_t ONCE_BYTES = (int64_t)32 << 20;
 // Either only in rows of whole 128-byte lines: a line that two waves store a piece of each goes to memory twice (6700 tokens of rank 64, 4128
 // and 8224 columns, a pass of two layers 804 us without, 922 with).  Not in 16-token tiles above rank 64 (csrc/expand.hip), which read
 // much more than they write (512 tokens over 128 adapters of rank 128, q+k+v 79.2 / 80.4 us, and 80.0 with the choice alone).  Nor in

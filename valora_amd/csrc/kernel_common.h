@@ -22,6 +22,7 @@ __device__ __forceinline__ To as(const From &v) {
 
 // One global_load_dwordx4 / global_store_dwordx4.  Addresses must be 16-byte aligned.
 __device__ __forceinline__ u32x4 load16(const uint16_t *p) { return *reinterpret_cast<const u32x4 *>(p); }
+constexpr int64_t L2_BYTES = (int64_t)32 << 20;   // what the L2s of the eight XCDs hold together
 // The same for what nobody reads again soon: the line is the first to leave the caches.  Only where a wave reads whole lines at once: of a
 // line read piece by piece it costs a second fetch (B of the expand: 512 tokens over 128 adapters of rank 128, a pass 839 / 912 us).
 __device__ __forceinline__ u32x4 load16_once(const uint16_t *p) { return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p)); }

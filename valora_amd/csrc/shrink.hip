@@ -338,10 +338,9 @@ __device__ const __align__(128) uint16_t g_zero_line[64] = {};
 // of the adapter's A rows, two steps before it is used, and handed over through two LDS stages; one barrier per step.
 //
 // Bound by a fixed part (launch, look-ups, first step, partials: one step only takes 6.6 of 17.9 us; 5254 tokens of rank 64, one target in
-// four chunks) and then by a stream of loads at 4.3 TB/s: 43 MB of x and 5.4 MB of partials in the other 11.3 us, A again per 128 tokens
-// from L2 and the y lines that the expand before it still has to write back on top.  With the loads alone 17.1 of the 17.9 us, with
-// the products alone 12.3; a deeper ring, K starts spread over the channels, ids by XCD and contiguous pool rows change
-// nothing.  Direct global -> LDS loads into a three-stage ring (one or two workgroups a compute unit instead of three, LDS turn
+// four chunks, 16.7 since x is read once and partials are written through, launch_shrink) and then by a stream of loads at 4.3 TB/s: 43 MB
+// of x, and A again per 128 tokens from L2.  Of the 17.9 us, 17.1 with the loads alone, 12.3 with the products alone; a deeper ring, K starts
+// spread over the channels, ids by XCD and contiguous pool rows change nothing.  Direct global -> LDS loads into a three-stage ring (one or two workgroups a compute unit instead of three, LDS turn
 // of the result, zero rows read for a narrower adapter's rank) / now, behind the same expand: three targets of 5254 tokens of
 // rank 64 37.2 / 33.4 us, 5401 tokens over ranks 8-64, one target 20.4 / 19.6, two 29.5 / 25.6, three 34.5 / 30.7, `down` of 11008
 // 56.6 / 54.9 (targets together: shrink_targets_kernel, below).  (The chunks summed inside the launch by the last to arrive: 20.4
@@ -842,7 +841,8 @@ int launch_shrink_reduce(hipStream_t st, const ShrinkArgs &a, mlora_dtype dt) {
   if (a.T <= 0) return MLORA_OK;
   const int quarter = (int)(a.rp >> 2), rows = 256 / quarter;   // at most 32 quarters
   const dim3 grid((unsigned)((a.T + rows - 1) / rows), (unsigned)a.n_targets);
-  // Partials are read as lines that nobody reads again where rows are whole lines (in others two workgroups share some: 2965 tokens of ranks
+  // Partials are read as lines that nobody reads again (a pass, plain / so: 5254 tokens of rank 64 643 / 638 us, 7000 of rank 128 604 / 596,
+  // 9000 of rank 64 635 / 625) where rows are whole lines (in others two workgroups share some: 2965 tokens of ranks
   // 16-48, a pass of three layers 259 us with such loads, 257 without), but not in compensations, which read few of them (a pass with / without:
   // 6368 tokens over ranks 16-64, 466 of them not the merged adapter's 751 / 746 us, 2657 1073 / 1059; 2817 of rank 128, 2 505 / 497).
   const bool once = !a.compensate && (a.rp & 31) == 0 && (reinterpret_cast<uintptr_t>(a.partial) & 127u) == 0;
@@ -904,12 +904,14 @@ int launch_shrink(hipStream_t st, const ShrinkArgs &args, int bm, int max_rank, 
     grid = dim3((unsigned)a.ksplit, (unsigned)a.n_targets, (unsigned)grid_tiles);
     const bool together = !a.compensate && shrink_targets_together(a.T, grid_tiles - (a.T + 127) / 128, max_rank, bm, a.ksplit, a.n_targets);
     // x is read as lines that nobody reads again (load16_once) where that is so: not by one target's workgroups after another's, nor where
-    // the caller's next call reads it; in rows of whole lines.  Partials are written through in whole lines likewise, instead of left in the
-    // L2s for the end of the kernel, and the launch that sums them reads them once.  A pass of two layers, before / now: 4430 tokens of rank 64
-    // 664 / 636 us, 5401 over ranks 8-64 678 / 667, 7000 of rank 128 407 / 398, 14000 over ranks 8-64, 5120 wide 785 / 763; one-call entry
-    // points (partials only) 1600 of rank 64 199 / 184, 7000 of rank 128 500 / 490, and with x read so 515; 15 prefill batches 1.016 in the
-    // mean, 0.99 at worst (2800 tokens of ranks 32 and 48, whose partials are no whole lines).
-    a.x_once = !a.out_by_token && (a.n_targets == 1 || together) && !(a.h_in & 63) && !(reinterpret_cast<uintptr_t>(a.x) & 127u);
+    // the caller's next call reads it (7000 tokens of rank 128 in one-call entry points 490 / 515 us a pass); in rows of whole lines; and
+    // from so much of x on that the L2s do not keep it anyway.  A pass, plain / so: 5254 tokens of rank 64, seven projections of 4096 and 11008,
+    // 661 / 638 us, 5401 over ranks 8-64 669 / 664, 14000, 5120 wide 1865 / 1841, 9000 of rank 64 in 256-token tiles 628 / 622; 2600 (21 MB of
+    // x) 620 / 624, 1200 421 / 423.  (It is `down`, 119 MB of x, that gains, 55.6 / 40.0 us; the expands behind lose 8 us of three targets.)
+    // Partials are written through in whole lines instead of left in the L2s for the end of the kernel.  A pass, plain / through: 5254 tokens
+    // of rank 64 644 / 638, 7000 of rank 128 604 / 596, 1200 of rank 64 433 / 421, in one-call entry points 2600 of it 531 / 521; 3887 of rank
+    // 64 whose expand sums them, once for every column chunk, 337 / 334; compensations of 6368 tokens over ranks 16-64 1081 / 1074.
+    a.x_once = !a.out_by_token && (a.n_targets == 1 || together) && (int64_t)a.T * a.h_in * 2 >= L2_BYTES && !(a.h_in & 63) && !(reinterpret_cast<uintptr_t>(a.x) & 127u);
     a.partial_through = a.ksplit > 1 && (a.rp & 31) == 0 && (reinterpret_cast<uintptr_t>(a.partial) & 127u) == 0;
     if (together) {
       if (a.n_targets == 3) return dt == MLORA_F16 ? launch_targets<_Float16, 3>(st, a, nb, grid_tiles) : launch_targets<__bf16, 3>(st, a, nb, grid_tiles);
