@@ -34,18 +34,14 @@ def _bound(dtype):
                                              if not one or (r <= 32 and k > 1)])
 @pytest.mark.parametrize("odd", [0, 64, -128])   # K ranges that are whole batches of steps, or end in the middle of one
 def test_rows_of_a_in_small_tiles(dev, rank, one, ksplit, odd):
-    """4 MB of A and more in the whole batch, less in each half; every adapter has one tile.  (The one-launch op reads A the plain way
-    whatever the size.)"""
-    n, T = 44, 47
+    """4 MB of A and more by the bound over the adapters of the index in the whole batch, less in each half."""
+    n, T = 40, 43
     h_in = 65536 // rank + odd
     dtype = torch.bfloat16 if odd else torch.float16
     print(rank, one, ksplit, h_in, flush=True)
     rp = rank
-    pool, _, x, y0 = _case(T, n, rank, h_in, 264, dtype, rank + odd)
-    ids = torch.arange(T) * 7 % n
-    ids[5] = -1
-    tiles = [len(set(part.tolist()) - {-1}) for part in (ids, ids[:T // 2], ids[T // 2:])]
-    assert tiles[0] * rp * h_in * 2 >= 4 << 20 > max(tiles[1:]) * rp * h_in * 2
+    assert ((T + 15) // 16 + n) * rp * h_in * 2 >= 4 << 20 > ((T + 31) // 32 + (T + 1) // 2) * rp * h_in * 2
+    pool, ids, x, y0 = _case(T, n, rank, h_in, 264, dtype, rank + odd)
     p, xd = pool.to(dev), x.to(dev)
     idx = (p.a_start, p.a_len, p.a_loc)
 
@@ -62,10 +58,73 @@ def test_rows_of_a_in_small_tiles(dev, rank, one, ksplit, odd):
     assert O.rel_l2(whole.cpu(), _oracle(pool, ids, x, y0)) <= _bound(dtype)
 
 
+@pytest.mark.parametrize("rank", [16, 32, 64, 128])
+@pytest.mark.parametrize("ksplit", [1, 4])
+@pytest.mark.parametrize("odd", [0, 64, -128])   # K ranges that are whole batches of steps, or end in the middle of one
+def test_rows_of_a_in_tiles_alone_with_their_adapter(dev, rank, ksplit, odd):
+    """4 MB of A and more in the whole batch, less in each half; every adapter has one tile."""
+    n, T = 44, 47
+    h_in = 65536 // rank + odd
+    dtype = torch.bfloat16 if odd else torch.float16
+    print(rank, ksplit, h_in, flush=True)
+    rp = rank
+    pool, _, x, y0 = _case(T, n, rank, h_in, 264, dtype, rank + odd)
+    ids = torch.arange(T) * 7 % n
+    ids[5] = -1
+    tiles = [len(set(part.tolist()) - {-1}) for part in (ids, ids[:T // 2], ids[T // 2:])]
+    assert tiles[0] * rp * h_in * 2 >= 4 << 20 > max(tiles[1:]) * rp * h_in * 2
+    p, xd = pool.to(dev), x.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+
+    def call(a, b, y):
+        plan = LoraPlan(ids[a:b].to(dev).contiguous(), *idx[:2], rank, n_slots=2, hidden=h_in, bm_shrink=16, bm_expand=16, one_launch=False,
+                        ksplit=ksplit)
+        plan.apply(y, xd[a:b], p.key_buffer, p.value_buffer, *idx, 1, p.a_scaling)
+
+    whole, halves = y0.to(dev), y0.to(dev)
+    call(0, T, whole)
+    call(0, T // 2, halves[: T // 2])
+    call(T // 2, T, halves[T // 2:])
+    assert torch.equal(whole, halves)
+    assert O.rel_l2(whole.cpu(), _oracle(pool, ids, x, y0)) <= _bound(dtype)
+
+
 @pytest.mark.parametrize("ranks,bm,targets", [(r, bm, t) for r in ([16, 8], [32, 24, 8], [48, 16], [64, 40, 8], [128, 72, 16])
                                               for bm in (128, 256) for t in (1, 2, 3) if bm == 128 or (max(r) <= 64 and t == 1)])
 @pytest.mark.parametrize("ksplit", [1, 2, 4])
 def test_tall_tiles(dev, ranks, bm, targets, ksplit):
+    """x on 128-byte lines against the same x beside them."""
+    T, h_in, h_out = 5861, 576, 72       # two and three targets in four chunks share a workgroup
+    g = torch.Generator().manual_seed(ranks[0] + bm + targets)
+    dtype = torch.bfloat16 if ranks[0] == 64 else torch.float16
+    pool = W.make_pool(ranks, h_in, h_out, dtype, g, True, n_slots=3, std=0.05, scalings=[0.5 + 0.25 * i for i in range(len(ranks))],
+                       heads=1, extra_rows=2)
+    ids = torch.randint(-1, len(ranks), (T,), generator=g)
+    x, y0 = torch.randn(T, h_in, generator=g).to(dtype), torch.randn(targets, T, h_out, generator=g).to(dtype)
+    print(ranks, bm, targets, ksplit, flush=True)
+    p, idsd = pool.to(dev), ids.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    plan = LoraPlan(idsd, *idx[:2], max(ranks), n_slots=3, hidden=h_in, bm_shrink=bm, bm_expand=64, one_launch=False, ksplit=ksplit,
+                    reduce_in_expand=False)
+    got = []
+    for off in (0, 8):
+        room = torch.empty(T * h_in + off, dtype=dtype, device=dev)
+        xd = room[off:].view(T, h_in)
+        assert (xd.data_ptr() % 128 == 0) == (off == 0)
+        xd.copy_(x)
+        y = y0.to(dev)
+        plan.apply_multi(list(y.unbind(0)), xd, p.key_buffer, p.value_buffer, *idx, list(range(targets)), p.a_scaling)
+        got.append(y)
+    assert torch.equal(got[0], got[1])
+    for t in range(targets):
+        want = O.lora_op(y0[t], x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, t, pool.a_scaling, n_slots=3)
+        assert O.rel_l2(got[0][t].cpu(), want) <= _bound(dtype)
+
+
+@pytest.mark.parametrize("ranks,bm,targets", [(r, bm, t) for r in ([16, 8], [32, 24, 8], [48, 16], [64, 40, 8], [128, 72, 16])
+                                              for bm in (128, 256) for t in (1, 2, 3) if bm == 128 or (max(r) <= 64 and t == 1)])
+@pytest.mark.parametrize("ksplit", [1, 2, 4])
+def test_tall_tiles_of_more_x_than_the_l2s_hold(dev, ranks, bm, targets, ksplit):
     """x and scratch on 128-byte lines; the same with x beside them, which is read the plain way; and with scratch beside them, whose partial
     sums are written and read the plain way."""
     T, h_in, h_out = 5861, 3008, 72      # two and three targets in four chunks share a workgroup; more of x than the L2s hold
