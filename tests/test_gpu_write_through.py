@@ -1,7 +1,7 @@
 """Launches that write y on to memory at once (from 2 MB of y on, 3 MB where the op is one launch) against the same tokens in
 batches below that size: the same bits, for tiles of odd and even token counts, widths that end inside a chunk, tokens without an
-adapter, and nothing written beside the rows.  16-token tiles above rank 64 and compensations are never written through: their cases hold that
-large batches give the bits of small ones all the same."""
+adapter, and nothing written beside the rows.  16-token tiles above rank 64 and tall ones of compensations are never written through:
+their cases hold that large batches give the bits of small ones all the same."""
 import pytest
 import torch
 
@@ -76,6 +76,27 @@ def test_compensation_same_bits_as_smaller_batches(dev, ranks, bm):
     got = _both(dev, lambda i: DeLoraPlan(i, 1, *idx[:2], max(ranks), H_IN, n_slots=2, bm_shrink=16, bm_expand=bm, ksplit=2),
                 lambda plan, y, xs: plan.apply(y, xs, p.key_buffer, p.value_buffer, *idx, 1, p.a_scaling),
                 p, ids.to(dev), x.to(dev), y0.to(dev), 2 << 20)
+    want = O.delora_compensate(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1, 1, pool.a_scaling,
+                               n_slots=2)
+    assert O.rel_l2(got.cpu(), want) <= REL_L2
+
+
+@pytest.mark.parametrize("ranks", [[16, 8], [32, 24, 8], [64, 40, 8]])
+@pytest.mark.parametrize("h_out,odd", [(1600, 2), (4160, 3), (4288, 5)])
+@pytest.mark.parametrize("own", [0.03, 0.6])   # of the tokens, not the merged adapter's
+def test_compensation_of_small_tiles(dev, ranks, h_out, odd, own):
+    """4 MB of y and more, of which half counts; with some tokens of no rank of their own."""
+    T = (4 << 20) // (2 * h_out) + odd
+    g = torch.Generator().manual_seed(h_out + ranks[0])
+    ranks = ranks + [0]
+    pool, _, x, y0 = _case(T, h_out, ranks, torch.float16, h_out)
+    ids = torch.where(torch.rand(T, generator=g) < own, torch.randint(-1, len(ranks), (T,), generator=g), torch.tensor(1))
+    print(T, h_out, ranks, own, flush=True)
+    p = pool.to(dev)
+    idx = (p.a_start, p.a_len, p.a_loc)
+    got = _both(dev, lambda i: DeLoraPlan(i, 1, *idx[:2], max(ranks), H_IN, n_slots=2, bm_shrink=16, bm_expand=16, ksplit=2),
+                lambda plan, y, xs: plan.apply(y, xs, p.key_buffer, p.value_buffer, *idx, 1, p.a_scaling),
+                p, ids.to(dev), x.to(dev), y0.to(dev), 4 << 20)
     want = O.delora_compensate(y0, x, pool.key_buffer, pool.value_buffer, pool.a_start, pool.a_len, pool.a_loc, ids, 1, 1, pool.a_scaling,
                                n_slots=2)
     assert O.rel_l2(got.cpu(), want) <= REL_L2

@@ -362,7 +362,7 @@ int launch_small_kb(hipStream_t st, const ExpandArgs &a, int64_t tiles) {
   hipLaunchKernelGGL((expand_small_kernel<T, KB, WIDE, PARTIAL, COMP, THROUGH>), grid, dim3(256), 0, st, records, \
                      a.plan + a.off_perm, a_loc, (int)a.pool.a_loc_len, a.h_out, a)
 #define MLORA_SMALL(WIDE, PARTIAL, COMP)                                                          \
-  if (KB < 4 && !COMP && a.through) MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, (KB < 4 && !COMP));     \
+  if (KB < 4 && a.through) MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, (KB < 4));                       \
   else MLORA_SMALL_FORM(WIDE, PARTIAL, COMP, false)
 #define MLORA_SMALL_WIDTH(PARTIAL, COMP)                                           \
   if (KB > 0 && a.h_out >= SMALL_WIDE) { MLORA_SMALL((KB > 0), PARTIAL, COMP); }   \

@@ -252,14 +252,17 @@ constexpr int64_t THROUGH_BYTES = (int64_t)2 << 20, THROUGH_BYTES_ONE_LAUNCH = (
 // Either only in rows of whole 128-byte lines: a line that two waves store a piece of each goes to memory twice (6700 tokens of rank 64, 4128
 // and 8224 columns, a pass of two layers 804 us without, 922 with).  Not in 16-token tiles above rank 64 (csrc/expand.hip), which read
 // much more than they write (512 tokens over 128 adapters of rank 128, q+k+v 79.2 / 80.4 us, and 80.0 with the choice alone).  Nor in
-// compensations: the merged adapter's tokens are not written, most of the batch in earnest, and the host does not know how many they are.  A
-// pass, plain / through: 2817 tokens of rank 128, 2 of them not the merged adapter's 505 / 512 us, 737 of them 665 / 676; 6368 over ranks
-// 16-64, 466 751 / 749, 2657 1073 / 1066; 1000 of rank 16, 95 435 / 433; twelve such batches the same in the mean.  (Tokens without an adapter are counted: of
-// 1000 tokens of rank 16 in one launch, half of them without, a pass of 8 layers 236 / 226, 95 % of them 155 / 159.)
+// tall tiles of compensations: the merged adapter's tokens are not written, most of the batch in earnest, and the host does not know how many they
+// are.  A pass, plain / through: 2817 tokens of rank 128, 2 of them not the merged adapter's 505 / 512 us, 737 of them 665 / 676; 6368 over
+// ranks 16-64, 466 751 / 749, 2657 1073 / 1066.  In 16-token tiles up to rank 64 it pays there as well, whatever their number, from half as
+// many bytes on: 918 tokens over ranks 16-64, 306 not the merged adapter's 557 / 542, 1100 of rank 32, 958 of them 677 / 654 and 39 of them
+// 354 / 348, 600 of rank 16, 44 of them 268 / 269, 900 of rank 64, 33 of them 401 / 405 (the worst of ten).
+// (Tokens without an adapter are counted: of 1000 tokens of rank 16 in one launch, half of them without, a pass of 8 layers 236 / 226, 95 %
+// of them 155 / 159.)
 inline int write_through(const ExpandArgs &a, int64_t least) {
   uintptr_t ends = 0;
   for (int z = 0; z < a.n_targets; ++z) ends |= reinterpret_cast<uintptr_t>(a.ys[z]);
-  return !a.compensate && (int64_t)a.T * a.h_out * a.n_targets * 2 >= least && !(a.h_out & 63) && !(ends & 127u);
+  return (int64_t)(a.compensate ? a.T / 2 : a.T) * a.h_out * a.n_targets * 2 >= least && !(a.h_out & 63) && !(ends & 127u);
 }
 // The lane's outputs of y: 16 from o_wave + 16 * (lane / 16) on, in two 16-byte halves.
 template <int KB>
