@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void shrink_reduce_kernel(const int32_t *h_pla
 // spill 4 and 28 registers; three / two: 4000 tokens over 32 adapters of rank 32, four chunks 12.8 / 11.6 us, eight 12.9 / 11.4; 8000 over
 // 64 of rank 16 18.4 / 16.0, of rank 32 20.6 / 18.7.)
 constexpr int shrink_min_waves(int mb, int nb) { return mb + nb <= 3 ? 4 : nb == 8 ? 3 - mb : mb == 4 ? 2 : 3; }
-// ONCE: a tile that is its adapter's only one may read A as lines that nobody reads again (shrink_once_tiles).  A form of its own: with both
+// ONCE: a tile that is its adapter's only one may read A as lines that nobody reads again (shrink_once_tiles), above rank 16.  A form of its own: with both
 // loops in one kernel a call of a few tokens takes 3.78 us instead of 3.62.
 template <typename T, int MB, int NB, bool ONCE>
 __global__ __launch_bounds__(256, shrink_min_waves(MB, NB)) void shrink_kernel(const int32_t *tiles_base, int h_ksplit, int h_n_targets, int h_reduce_here,
@@ -770,7 +770,7 @@ template <typename T, int MB>
 int launch_shrink_nb(hipStream_t st, const ShrinkArgs &a, int nb, dim3 grid) {
   constexpr bool MAY_ONCE = MB == 1;
 #define MLORA_SHRINK(MBX, NB)                                                                     \
-  if (MAY_ONCE && a.once_tiles <= a.n_tiles) MLORA_SHRINK_FORM(MBX, NB, MAY_ONCE);                \
+  if (MAY_ONCE && NB > 1 && a.once_tiles <= a.n_tiles) MLORA_SHRINK_FORM(MBX, NB, (MAY_ONCE && NB > 1)); \
   else MLORA_SHRINK_FORM(MBX, NB, false)
 #define MLORA_SHRINK_FORM(MBX, NB, ONCE) \
   hipLaunchKernelGGL((shrink_kernel<T, MBX, NB, ONCE>), grid, dim3(256), 0, st, a.plan + a.off_tiles, a.ksplit, a.n_targets, head_flags(a), a.n_tiles, a)

@@ -242,15 +242,16 @@ __device__ __forceinline__ void shrink_tile_to_lds(const uint16_t *__restrict__ 
 // shrink_kernel, 16-token tiles.  The record says whether it is, and of how many: the host knows the resident adapters, not those that a
 // batch touches, and where tiles share A such loads lose most (512 tokens of rank 128 on one of 128 adapters, a pass 243 us without, 299 with
 // them; 900 of rank 32 on four 354 / 385).  From 4 MB of A on, more than an L2 holds (one token over 8 adapters, a pass of 64 calls
-// 379 / 398); in rows of whole lines; not for rank 8 alone, where the lanes of the other eight rows read the last one again (128
-// adapters, 0.993); nor for batches of five tokens a tile and more.  A pass, plain loads / this: 512 tokens over 128 adapters of rank 128
+// 379 / 398); in rows of whole lines; above rank 16, up to which the look at the flag takes 0.12 us of a launch of 5 and the loads give no more
+// (256 tokens over 64 adapters of rank 16, a pass of 256 one-call launches 1518 us plain, 1536 with them; rank 8 alone 0.993); and not for
+// batches of five tokens a tile and more.  A pass, plain loads / this: 512 tokens over 128 adapters of rank 128
 // 633 / 611 us, 900 over 128 of rank 64 563 / 537, 77 over ranks 8-64 473 / 456; twelve batches of 14 to 900 tokens 1.026 in the mean, and
 // twelve of as many tokens on one to four of up to 128 adapters 1.00 to 1.09 (what is above 1.02 is y written through)
 // (the one-launch op, which has no scalar register left for it, reads A the plain way: 256 tokens over 64 adapters of rank 16, a pass
 // of 16 layers 453 us, 450 with such loads).
 inline int shrink_once_tiles(const ShrinkArgs &a, int64_t n_tiles, int max_rank) {
   const int64_t tile_bytes = (int64_t)a.rp * a.h_in * a.n_targets * 2;
-  if (max_rank <= 8 || a.compensate || a.T >= 5 * n_tiles || (a.h_in & 63) || (reinterpret_cast<uintptr_t>(a.pool.w) & 127u)) return 0x7fffffff;
+  if (max_rank <= 16 || a.compensate || a.T >= 5 * n_tiles || (a.h_in & 63) || (reinterpret_cast<uintptr_t>(a.pool.w) & 127u)) return 0x7fffffff;
   return (int)((((int64_t)4 << 20) + tile_bytes - 1) / tile_bytes);
 }
 
